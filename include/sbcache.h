@@ -350,6 +350,17 @@ typedef struct sb_gla_recurrent_args {
 
 int sb_gla_recurrent(const sb_gla_recurrent_args *args);
 
+/* The same call with long prompts cut into segments that run side by side (few prompts x heads leave most of the GPU
+ * idle otherwise). sb_gla_prompt_segments: how many segments the library would cut this call's longest prompt into
+ * (1 = not at all); sb_gla_prompt_workspace_bytes: scratch memory that takes (device, 16-byte aligned, contents
+ * irrelevant before and after; calls whose scratch memory overlaps must be ordered); sb_gla_prompt_segmented: the
+ * call, cut into at most n_segments pieces. args->seq_len bounds the prompts' lengths as in sb_gla_recurrent. A
+ * segment starts from a state that was formed in fp32 from its predecessors' contributions, so results agree with
+ * the uncut call within fp32 rounding of the state. n_segments < 2: sb_gla_recurrent. */
+int32_t sb_gla_prompt_segments(const sb_gla_recurrent_args *args);
+size_t sb_gla_prompt_workspace_bytes(const sb_gla_recurrent_args *args, int32_t n_segments);
+int sb_gla_prompt_segmented(const sb_gla_recurrent_args *args, int32_t n_segments, void *workspace, size_t workspace_bytes);
+
 /* Gate range check of the block form above. No counterpart in the reference (fla's kernel gives no such
  * signal). *hits = number of times the matrix-core GLA launches made with SB_GLA_CHECK_GATES on the current
  * device met gates beyond the range stated at `flags` (one per prompt, head, 32 key dims and pair of 16-token blocks concerned), since

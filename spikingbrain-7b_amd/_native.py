@@ -176,6 +176,9 @@ EXPORTS = {
     "sb_swa_decode": (C.c_int, [C.POINTER(SwaDecodeArgs)]),
     "sb_swa_decode_static": (C.c_int, [C.POINTER(SwaDecodeArgs)]),
     "sb_gla_recurrent": (C.c_int, [C.POINTER(GlaRecurrentArgs)]),
+    "sb_gla_prompt_segments": (i32, [C.POINTER(GlaRecurrentArgs)]),
+    "sb_gla_prompt_workspace_bytes": (sz, [C.POINTER(GlaRecurrentArgs), i32]),
+    "sb_gla_prompt_segmented": (C.c_int, [C.POINTER(GlaRecurrentArgs), i32, vp, sz]),
     "sb_gla_gate_range_hits": (C.c_int, [C.POINTER(C.c_int64), C.c_int32]),
     "sb_copy_blocks": (C.c_int, [vp, vp, i64, i64, i64, vp]),
     "sb_window_shift": (C.c_int, [C.POINTER(WindowShiftArgs)]),

@@ -66,6 +66,11 @@ struct GlaChunkParams {
   // final state. One state per head: G = jn = 1, j0 = 0, write_state = 1.
   int G, jn, j0, write_state;
   unsigned int *range_hits;  // device counter of (wavefront, pair of blocks) events whose gates reached the exponent clamp
+  // Prompts cut into segments (0: not cut): seg_tokens tokens each, n_seg of them for the longest prompt. ws holds
+  // per (row, state head, segment) the state in register order, 16384 floats, and behind all of those the
+  // segments' total log-decays, 128 floats each (log2 units).
+  int seg_tokens, n_seg;
+  float *ws;
 };
 
 constexpr int kCB = 16;      // tokens per block
@@ -117,8 +122,11 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float x) { return __builtin_bit_
 
 // kCheck: report gates beyond the block form's range (SB_GLA_CHECK_GATES); a build of its own, because even this
 // little extra work shifts the register allocation of a kernel that runs at the edge of its budget (0-4 % slower).
-template <bool kStateF32, int GDT, bool kCheck>
+// kSeg: the workgroup runs one segment of its prompt, from the state gla_segment_scan_kernel left in the workspace
+// for it; the workgroup of a prompt's last segment stores the final state.
+template <bool kStateF32, int GDT, bool kCheck, bool kSeg>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gla_chunk_kernel(const GlaChunkParams p) {
+  const int seg = kSeg ? (int)blockIdx.y : 0;
   const int b = blockIdx.x / p.H;
   const int hh = blockIdx.x - b * p.H;
   const int hk = hh / p.jn;
@@ -133,6 +141,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     qo = t0 * p.q_st; ko = t0 * p.k_st; vo = t0 * p.v_st; go = t0 * p.g_st; oo = t0 * p.o_st;
   } else {
     qo = b * p.q_sb; ko = b * p.k_sb; vo = b * p.v_sb; go = b * p.g_sb; oo = b * p.o_sb;
+  }
+  bool last_segment = true;
+  if constexpr (kSeg) {
+    const int64_t t0 = (int64_t)seg * p.seg_tokens;
+    last_segment = T <= t0 + p.seg_tokens;
+    T = (int)min((int64_t)p.seg_tokens, T - t0);
+    qo += t0 * p.q_st; ko += t0 * p.k_st; vo += t0 * p.v_st; go += t0 * p.g_st; oo += t0 * p.o_st;
   }
   if (T <= 0) return;
   qo += h * p.q_sh; ko += hk * p.k_sh; vo += hk * p.v_sh; go += hk * p.g_sh; oo += h * p.o_sh;
@@ -151,16 +166,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   auto state_index = [&](int rt, int nt, int i) {
     return (32 * (rt >> 1) + 8 * g + 4 * (rt & 1) + i) * 128 + 32 * w + 16 * nt + c;
   };
+  if constexpr (kSeg) {
+    const int Hk = p.H / p.jn;
+    const f32x4_t *src = reinterpret_cast<const f32x4_t *>(p.ws + (((int64_t)b * Hk + hk) * p.n_seg + seg) * 16384) + tid;
 #pragma unroll
-  for (int rt = 0; rt < 8; ++rt)
+    for (int rt = 0; rt < 8; ++rt)
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
+      for (int nt = 0; nt < 2; ++nt) S[rt][nt] = src[(2 * rt + nt) * 256];
+  } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int idx = state_index(rt, nt, i);
-        S[rt][nt][i] = kStateF32 ? reinterpret_cast<const float *>(sbase)[idx]
-                                 : bf16_to_f32(reinterpret_cast<const uint16_t *>(sbase)[idx]);
-      }
+    for (int rt = 0; rt < 8; ++rt)
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int idx = state_index(rt, nt, i);
+          S[rt][nt][i] = kStateF32 ? reinterpret_cast<const float *>(sbase)[idx]
+                                   : bf16_to_f32(reinterpret_cast<const uint16_t *>(sbase)[idx]);
+        }
+  }
 
   // ---- block inputs in registers: 8 dims of one token's q, k, v (bf16) and gate ---------------------------
   constexpr int kGateBytes = GDT == SB_F32 ? 4 : 2;
@@ -385,7 +409,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if (__builtin_amdgcn_ballot_w64(worst < -kMaxExp * kLog2e) != 0 && tid == 0) atomicAdd(p.range_hits, 1u);
   }
 
-  if (!p.write_state) return;
+  if (kSeg ? (!last_segment || hh % p.jn != 0) : !p.write_state) return;
 #pragma unroll
   for (int rt = 0; rt < 8; ++rt)
 #pragma unroll
@@ -398,6 +422,220 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
 }
 
+
+// ---- prompts cut into segments -----------------------------------------------------------------------------------
+// Few chains (one prompt: 28 of them) leave most CUs idle, so long prompts are cut: the segments' own contributions
+// to the state (from a zero start) and total decays are formed side by side (gla_segment_state_kernel), a scan over
+// the segments turns them into the state each one starts from (gla_segment_scan_kernel), and gla_chunk_kernel<kSeg>
+// then runs all segments at once. Segments are whole pairs of blocks, so the operands of a pair are those of the
+// uncut prompt. k, v and the gate are read twice; what is bought is n_seg times as many workgroups.
+
+// One workgroup per (row, state head, segment but the last): S_loc = sum over the segment's tokens of
+// (k_s exp(B_end - B_s))^T v_s, with the operand arithmetic, the tiles and the pairing of gla_chunk_kernel but
+// without its outputs (16 matrix instructions per wavefront and block instead of 30, no q).
+struct StateStage {
+  uint16_t ks[kCB][kRow];
+  uint16_t kl[kCB][kRow];
+  uint16_t vs[kCB][kRow];
+  float dec[128];
+};
+
+template <int GDT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gla_segment_state_kernel(const GlaChunkParams p) {
+  const int seg = blockIdx.y;
+  const int Hk = p.H;   // state heads here
+  const int b = blockIdx.x / Hk;
+  const int hk = blockIdx.x - b * Hk;
+  if (p.slot_idx && p.slot_idx[b] < 0) return;
+  int T = p.T;
+  int64_t ko, vo, go;
+  if (p.cu) {
+    const int64_t t0 = p.cu[b];
+    T = p.cu[b + 1] - (int)t0;
+    ko = t0 * p.k_st; vo = t0 * p.v_st; go = t0 * p.g_st;
+  } else {
+    ko = b * p.k_sb; vo = b * p.v_sb; go = b * p.g_sb;
+  }
+  const int64_t s0 = (int64_t)seg * p.seg_tokens;
+  if (T <= s0 + p.seg_tokens) return;   // a prompt's last segment hands nothing on
+  ko += s0 * p.k_st + hk * p.k_sh; vo += s0 * p.v_st + hk * p.v_sh; go += s0 * p.g_st + hk * p.g_sh;
+
+  const int tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const int g = lane >> 4, c = lane & 15;
+  const int r = tid >> 4;
+
+  __shared__ __attribute__((aligned(16))) StateStage stage[2];
+
+  f32x4_t S[8][2];
+#pragma unroll
+  for (int rt = 0; rt < 8; ++rt)
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) S[rt][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  constexpr int kGateBytes = GDT == SB_F32 ? 4 : 2;
+  const char *gb = reinterpret_cast<const char *>(p.g) + go * kGateBytes;
+  const char *kb = reinterpret_cast<const char *>(p.k + ko), *vb_ = reinterpret_cast<const char *>(p.v + vo);
+  const int64_t g_row = p.g_st * kGateBytes, k_row = p.k_st * 2, v_row = p.v_st * 2;
+  struct BlockIn {
+    uint4 k, v;
+    uint4 g[kGateBytes / 2];
+  };
+  auto fetch = [&](int t0, BlockIn &in) {   // (every block of such a segment is whole)
+    in.k = load16(rows_from(kb + t0 * k_row), c * (int)k_row + r * 16);
+    in.v = load16(rows_from(vb_ + t0 * v_row), c * (int)v_row + r * 16);
+    const __amdgpu_buffer_rsrc_t gr = rows_from(gb + t0 * g_row);
+#pragma unroll
+    for (int j = 0; j < kGateBytes / 2; ++j) in.g[j] = load16(gr, c * (int)g_row + r * 8 * kGateBytes + 16 * j);
+  };
+  float carry[8], total[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) carry[i] = total[i] = 0.f;
+  auto prepare = [&](const BlockIn &in, StateStage &st, auto second_tag) {
+    constexpr bool kSecond = decltype(second_tag)::value;
+    float B[8], tot[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float x;
+      if constexpr (GDT == SB_F32) x = __uint_as_float(word(in.g[i >> 2], i & 3));
+      else if constexpr (GDT == SB_BF16) x = (i & 1) ? bf16_hi(word(in.g[0], i >> 1)) : bf16_lo(word(in.g[0], i >> 1));
+      else x = (i & 1) ? f16_hi(word(in.g[0], i >> 1)) : f16_lo(word(in.g[0], i >> 1));
+      x *= kLog2e;
+      x += row_shr<1>(x);
+      x += row_shr<2>(x);
+      x += row_shr<4>(x);
+      x += row_shr<8>(x);
+      if constexpr (kSecond) x += carry[i];
+      B[i] = x;
+      tot[i] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane | 15) << 2, __builtin_bit_cast(int, x)));
+    }
+    float kf[8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      kf[2 * i] = bf16_lo(word(in.k, i));
+      kf[2 * i + 1] = bf16_hi(word(in.k, i));
+    }
+    uint32_t ks[4], kl[4];
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {
+      const float x0 = kf[i] * fast_exp2(fminf(-B[i], kMaxExp * kLog2e)), x1 = kf[i + 1] * fast_exp2(fminf(-B[i + 1], kMaxExp * kLog2e));
+      const uint32_t h = Mma<BF16>::pack(x0, x1);
+      ks[i / 2] = h;
+      kl[i / 2] = Mma<BF16>::pack(x0 - __uint_as_float(h << 16), x1 - __uint_as_float(h & 0xffff0000u));
+    }
+    *reinterpret_cast<uint4 *>(&st.ks[c][8 * r]) = make_uint4(ks[0], ks[1], ks[2], ks[3]);
+    *reinterpret_cast<uint4 *>(&st.kl[c][8 * r]) = make_uint4(kl[0], kl[1], kl[2], kl[3]);
+    *reinterpret_cast<uint4 *>(&st.vs[c][8 * r]) = in.v;
+    if constexpr (kSecond) {
+      *reinterpret_cast<float4 *>(&st.dec[8 * r]) = make_float4(fast_exp2(tot[0]), fast_exp2(tot[1]), fast_exp2(tot[2]), fast_exp2(tot[3]));
+      *reinterpret_cast<float4 *>(&st.dec[8 * r + 4]) = make_float4(fast_exp2(tot[4]), fast_exp2(tot[5]), fast_exp2(tot[6]), fast_exp2(tot[7]));
+#pragma unroll
+      for (int i = 0; i < 8; ++i) total[i] += tot[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) carry[i] = tot[i];
+    }
+  };
+  auto multiply = [&](const StateStage &st, auto second_tag) {
+    constexpr bool kSecond = decltype(second_tag)::value;
+    uint4 vb[2];
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+      const uint2 x = load_transposed(&st.vs[4 * g + (c >> 2)][32 * w + 16 * nt + 4 * (c & 3)]);
+      vb[nt] = make_uint4(x.x, x.y, x.x, x.y);
+    }
+#pragma unroll
+    for (int rt = 0; rt < 8; ++rt) {
+      const int tok = 4 * g + (c >> 2), dims = 32 * (rt >> 1) + 8 * (c & 3) + 4 * (rt & 1);
+      const uint2 h2 = load_transposed(&st.ks[tok][dims]);
+      const uint2 l2 = load_transposed(&st.kl[tok][dims]);
+      const uint4 ka = make_uint4(h2.x, h2.y, l2.x, l2.y);
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) S[rt][nt] = Mma<BF16>::run(ka, vb[nt], S[rt][nt]);
+      if constexpr (kSecond) {
+        const float4 dc = *reinterpret_cast<const float4 *>(&st.dec[32 * (rt >> 1) + 8 * g + 4 * (rt & 1)]);
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+          S[rt][nt][0] *= dc.x; S[rt][nt][1] *= dc.y; S[rt][nt][2] *= dc.z; S[rt][nt][3] *= dc.w;
+        }
+      }
+    }
+  };
+
+  const int n_blocks = p.seg_tokens / kCB;   // a whole number of pairs
+  const std::false_type kFirst{};
+  const std::true_type kSecond{};
+  BlockIn in;
+  fetch(0, in);
+  prepare(in, stage[0], kFirst);
+  fetch(kCB, in);
+  for (int blk = 0; blk < n_blocks; blk += 2) {
+    __syncthreads();
+    multiply(stage[0], kFirst);
+    prepare(in, stage[1], kSecond);
+    fetch(min(blk + 2, n_blocks - 1) * kCB, in);
+    __syncthreads();
+    multiply(stage[1], kSecond);
+    prepare(in, stage[0], kFirst);
+    fetch(min(blk + 3, n_blocks - 1) * kCB, in);
+  }
+  const int64_t at = ((int64_t)b * Hk + hk) * p.n_seg + seg;
+  f32x4_t *dst = reinterpret_cast<f32x4_t *>(p.ws + at * 16384) + tid;
+#pragma unroll
+  for (int rt = 0; rt < 8; ++rt)
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) dst[(2 * rt + nt) * 256] = S[rt][nt];
+  if (c == 0) {   // every lane of the row holds the totals of its 8 dims
+    float4 *d = reinterpret_cast<float4 *>(p.ws + (int64_t)gridDim.x * p.n_seg * 16384 + at * 128 + 8 * r);
+    d[0] = make_float4(total[0], total[1], total[2], total[3]);
+    d[1] = make_float4(total[4], total[5], total[6], total[7]);
+  }
+}
+
+// Grid (rows x state heads, 16 accumulator tiles): thread tid of workgroup (., tile) owns the four state elements
+// that thread tid of the other two kernels holds in that tile. In place: S_loc of a segment becomes the state the
+// segment starts from. A few segments' contributions are requested together, ahead of the chain over them.
+template <bool kStateF32>
+__global__ __launch_bounds__(256) void gla_segment_scan_kernel(const GlaChunkParams p) {
+  const int Hk = p.H;
+  const int b = blockIdx.x / Hk;
+  const int hk = blockIdx.x - b * Hk;
+  const int64_t slot = p.slot_idx ? (int64_t)p.slot_idx[b] : (int64_t)b;
+  if (slot < 0) return;
+  const int T = p.cu ? p.cu[b + 1] - p.cu[b] : p.T;
+  const int n = (T + p.seg_tokens - 1) / p.seg_tokens;   // segments of this prompt
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, c = lane & 15;
+  const int rt = blockIdx.y >> 1, nt = blockIdx.y & 1;
+  const int row = 32 * (rt >> 1) + 8 * g + 4 * (rt & 1);
+  const char *sbase = reinterpret_cast<const char *>(p.state) + (slot * p.s_slot + (int64_t)hk * p.s_head) * (kStateF32 ? 4 : 2);
+  f32x4_t S;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int idx = (row + i) * 128 + 32 * w + 16 * nt + c;
+    S[i] = kStateF32 ? reinterpret_cast<const float *>(sbase)[idx] : bf16_to_f32(reinterpret_cast<const uint16_t *>(sbase)[idx]);
+  }
+  const int64_t at0 = (int64_t)blockIdx.x * p.n_seg;
+  f32x4_t *const ws = reinterpret_cast<f32x4_t *>(p.ws + at0 * 16384) + blockIdx.y * 256 + tid;
+  const float *const decay = p.ws + (int64_t)gridDim.x * p.n_seg * 16384 + at0 * 128 + row;
+  constexpr int kAhead = 4;
+  for (int s0 = 0; s0 < n; s0 += kAhead) {
+    f32x4_t loc[kAhead], d[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const int s = min(s0 + j, n - 1);   // (the last segment's entry is not used: it hands nothing on)
+      loc[j] = ws[(int64_t)s * 4096];
+      d[j] = *reinterpret_cast<const f32x4_t *>(decay + s * 128);
+    }
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j)
+      if (s0 + j < n) {
+        ws[(int64_t)(s0 + j) * 4096] = S;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S[i] = fmaf(fast_exp2(d[j][i]), S[i], loc[j][i]);
+      }
+  }
+}
 
 // ---- one pass for a whole GQA group (shared states) -----------------------------------------------------------
 // One workgroup per (sequence, state head): the state is advanced ONCE per block and the outputs of all G query
@@ -415,8 +653,9 @@ struct GroupStage {
   float dec[128];
 };
 
-template <bool kStateF32, int GDT>
+template <bool kStateF32, int GDT, bool kSeg>
 __global__ __launch_bounds__(256) void gla_chunk_group_kernel(const GlaChunkParams p) {
+  const int seg = kSeg ? (int)blockIdx.y : 0;
   const int b = blockIdx.x / p.H;   // p.H: state heads here
   const int hk = blockIdx.x - b * p.H;
   const int G = p.G;
@@ -430,6 +669,13 @@ __global__ __launch_bounds__(256) void gla_chunk_group_kernel(const GlaChunkPara
     qo = t0 * p.q_st; ko = t0 * p.k_st; vo = t0 * p.v_st; go = t0 * p.g_st; oo = t0 * p.o_st;
   } else {
     qo = b * p.q_sb; ko = b * p.k_sb; vo = b * p.v_sb; go = b * p.g_sb; oo = b * p.o_sb;
+  }
+  bool last_segment = true;
+  if constexpr (kSeg) {
+    const int64_t t0 = (int64_t)seg * p.seg_tokens;
+    last_segment = T <= t0 + p.seg_tokens;
+    T = (int)min((int64_t)p.seg_tokens, T - t0);
+    qo += t0 * p.q_st; ko += t0 * p.k_st; vo += t0 * p.v_st; go += t0 * p.g_st; oo += t0 * p.o_st;
   }
   if (T <= 0) return;
   qo += (int64_t)hk * G * p.q_sh; ko += hk * p.k_sh; vo += hk * p.v_sh; go += hk * p.g_sh; oo += (int64_t)hk * G * p.o_sh;
@@ -448,16 +694,24 @@ __global__ __launch_bounds__(256) void gla_chunk_group_kernel(const GlaChunkPara
   auto state_index = [&](int rt, int nt, int i) {
     return (32 * (rt >> 1) + 8 * g + 4 * (rt & 1) + i) * 128 + 32 * w + 16 * nt + c;
   };
+  if constexpr (kSeg) {
+    const f32x4_t *src = reinterpret_cast<const f32x4_t *>(p.ws + ((int64_t)blockIdx.x * p.n_seg + seg) * 16384) + tid;
 #pragma unroll
-  for (int rt = 0; rt < 8; ++rt)
+    for (int rt = 0; rt < 8; ++rt)
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
+      for (int nt = 0; nt < 2; ++nt) S[rt][nt] = src[(2 * rt + nt) * 256];
+  } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int idx = state_index(rt, nt, i);
-        S[rt][nt][i] = kStateF32 ? reinterpret_cast<const float *>(sbase)[idx]
-                                 : bf16_to_f32(reinterpret_cast<const uint16_t *>(sbase)[idx]);
-      }
+    for (int rt = 0; rt < 8; ++rt)
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int idx = state_index(rt, nt, i);
+          S[rt][nt][i] = kStateF32 ? reinterpret_cast<const float *>(sbase)[idx]
+                                   : bf16_to_f32(reinterpret_cast<const uint16_t *>(sbase)[idx]);
+        }
+  }
 
   constexpr int kGateBytes = GDT == SB_F32 ? 4 : 2;
   const char *gb = reinterpret_cast<const char *>(p.g) + go * kGateBytes;
@@ -686,6 +940,7 @@ __global__ __launch_bounds__(256) void gla_chunk_group_kernel(const GlaChunkPara
       }
     }
   }
+  if (!last_segment) return;
 #pragma unroll
   for (int rt = 0; rt < 8; ++rt)
 #pragma unroll
@@ -745,13 +1000,8 @@ extern "C" int sb_gla_gate_range_hits(int64_t *hits, int32_t reset) {
 
 namespace sb_host {
 
-// Launch for bf16 q/k/v/out; g of any built type. Grid: one workgroup per (row, head).
-// Returns SB_OK, or an error when the device's hit counter cannot be located (nothing is launched then).
-int launch_gla_chunk(const sb_gla_recurrent_args *a, int64_t groups, int heads, int G, int jn, int j0, int write_state) {
+static GlaChunkParams fill(const sb_gla_recurrent_args *a, int heads, int G, int jn, int j0, int write_state) {
   GlaChunkParams p;
-  const bool check = (a->flags & SB_GLA_CHECK_GATES) != 0;
-  p.range_hits = check ? range_hits_ptr() : nullptr;
-  if (check && !p.range_hits) return SB_ERR_INVALID;
   p.q = (const uint16_t *)a->q; p.k = (const uint16_t *)a->k; p.v = (const uint16_t *)a->v; p.g = a->g;
   p.state = a->state; p.out = (uint16_t *)a->out; p.slot_idx = a->slot_idx; p.cu = a->cu_seqlens;
   p.H = heads; p.T = a->seq_len; p.scale = a->scale;
@@ -762,12 +1012,25 @@ int launch_gla_chunk(const sb_gla_recurrent_args *a, int64_t groups, int heads, 
   p.g_sb = a->g_stride_b; p.g_sh = a->g_stride_h; p.g_st = a->g_stride_t;
   p.o_sb = a->out_stride_b; p.o_sh = a->out_stride_h; p.o_st = a->out_stride_t;
   p.s_slot = a->state_stride_slot; p.s_head = a->state_stride_head;
+  p.range_hits = nullptr;
+  p.seg_tokens = p.n_seg = 0;
+  p.ws = nullptr;
+  return p;
+}
+
+// Launch for bf16 q/k/v/out; g of any built type. Grid: one workgroup per (row, head).
+// Returns SB_OK, or an error when the device's hit counter cannot be located (nothing is launched then).
+int launch_gla_chunk(const sb_gla_recurrent_args *a, int64_t groups, int heads, int G, int jn, int j0, int write_state) {
+  GlaChunkParams p = fill(a, heads, G, jn, j0, write_state);
+  const bool check = (a->flags & SB_GLA_CHECK_GATES) != 0;
+  p.range_hits = check ? range_hits_ptr() : nullptr;
+  if (check && !p.range_hits) return SB_ERR_INVALID;
   const dim3 grid((unsigned)groups), block(256);
   hipStream_t st = (hipStream_t)a->stream;
 #define SB_LAUNCH(F32S, GDT)                                                                     \
   do {                                                                                           \
-    if (check) hipLaunchKernelGGL((gla_chunk_kernel<F32S, GDT, true>), grid, block, 0, st, p);   \
-    else hipLaunchKernelGGL((gla_chunk_kernel<F32S, GDT, false>), grid, block, 0, st, p);        \
+    if (check) hipLaunchKernelGGL((gla_chunk_kernel<F32S, GDT, true, false>), grid, block, 0, st, p);   \
+    else hipLaunchKernelGGL((gla_chunk_kernel<F32S, GDT, false, false>), grid, block, 0, st, p);        \
   } while (0)
   if (a->state_dtype == SB_F32) {
     if (a->g_dtype == SB_F32) SB_LAUNCH(true, SB_F32);
@@ -782,35 +1045,22 @@ int launch_gla_chunk(const sb_gla_recurrent_args *a, int64_t groups, int heads, 
   return SB_OK;
 }
 
-// Shared states, one pass: grid = one workgroup per (row, state head), each forming the outputs of its G query
-// heads. SB_ERR_UNSUPPORTED (nothing launched) where the group's head offsets do not fit the kernel's 32-bit
-// in-block offsets; the caller then takes the launches per query head.
-int launch_gla_chunk_group(const sb_gla_recurrent_args *a, int state_heads, int G) {
-  if (G < 2 || G > kMaxGroup) return SB_ERR_UNSUPPORTED;
-  if ((int64_t)G * a->q_stride_h * 2 >= (1LL << 30) || (int64_t)G * a->out_stride_h * 2 >= (1LL << 30) ||
-      a->q_stride_h < 0 || a->out_stride_h < 0)
-    return SB_ERR_UNSUPPORTED;
-  GlaChunkParams p;
-  p.range_hits = nullptr;
-  p.q = (const uint16_t *)a->q; p.k = (const uint16_t *)a->k; p.v = (const uint16_t *)a->v; p.g = a->g;
-  p.state = a->state; p.out = (uint16_t *)a->out; p.slot_idx = a->slot_idx; p.cu = a->cu_seqlens;
-  p.H = state_heads; p.T = a->seq_len; p.scale = a->scale;
-  p.G = G; p.jn = 1; p.j0 = 0; p.write_state = 1;
-  p.q_sb = a->q_stride_b; p.q_sh = a->q_stride_h; p.q_st = a->q_stride_t;
-  p.k_sb = a->k_stride_b; p.k_sh = a->k_stride_h; p.k_st = a->k_stride_t;
-  p.v_sb = a->v_stride_b; p.v_sh = a->v_stride_h; p.v_st = a->v_stride_t;
-  p.g_sb = a->g_stride_b; p.g_sh = a->g_stride_h; p.g_st = a->g_stride_t;
-  p.o_sb = a->out_stride_b; p.o_sh = a->out_stride_h; p.o_st = a->out_stride_t;
-  p.s_slot = a->state_stride_slot; p.s_head = a->state_stride_head;
-  const dim3 grid((unsigned)(a->batch * (int64_t)state_heads)), block(256);
+static bool group_fits(const sb_gla_recurrent_args *a, int G) {
+  return G >= 2 && G <= kMaxGroup && a->q_stride_h >= 0 && a->out_stride_h >= 0 && (int64_t)G * a->q_stride_h * 2 < (1LL << 30) &&
+         (int64_t)G * a->out_stride_h * 2 < (1LL << 30);
+}
+
+template <bool kSeg>
+static int launch_group_kernel(const sb_gla_recurrent_args *a, const GlaChunkParams &p, dim3 grid) {
+  const dim3 block(256);
   hipStream_t st = (hipStream_t)a->stream;
   constexpr int kLds = 2 * (int)sizeof(GroupStage);
-#define SB_LAUNCH(F32S, GDT)                                                                                  \
-  do {                                                                                                        \
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gla_chunk_group_kernel<F32S, GDT>),    \
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, kLds);                     \
-    if (e != hipSuccess) return fail((int)e, "gla_chunk_group_kernel: %s", hipGetErrorString(e));             \
-    hipLaunchKernelGGL((gla_chunk_group_kernel<F32S, GDT>), grid, block, kLds, st, p);                        \
+#define SB_LAUNCH(F32S, GDT)                                                                                     \
+  do {                                                                                                           \
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gla_chunk_group_kernel<F32S, GDT, kSeg>), \
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, kLds);                        \
+    if (e != hipSuccess) return fail((int)e, "gla_chunk_group_kernel: %s", hipGetErrorString(e));                \
+    hipLaunchKernelGGL((gla_chunk_group_kernel<F32S, GDT, kSeg>), grid, block, kLds, st, p);                     \
   } while (0)
   if (a->state_dtype == SB_F32) {
     if (a->g_dtype == SB_F32) SB_LAUNCH(true, SB_F32);
@@ -823,6 +1073,52 @@ int launch_gla_chunk_group(const sb_gla_recurrent_args *a, int state_heads, int 
   }
 #undef SB_LAUNCH
   return SB_OK;
+}
+
+// Prompts cut into n_seg segments of seg_tokens tokens (a multiple of 2 blocks); ws: see GlaChunkParams. With shared
+// states the segments fill the machine, so the one-pass kernel per group runs them (it does 0.4 x the work; per query
+// head where its strides do not fit, again in one launch: no head reads the state cache the last segments store into).
+int launch_gla_chunk_segments(const sb_gla_recurrent_args *a, int G, int n_seg, int seg_tokens, float *ws) {
+  const int Hk = a->num_heads / G;
+  GlaChunkParams p = fill(a, Hk, G, G, 0, 1);
+  p.seg_tokens = seg_tokens; p.n_seg = n_seg; p.ws = ws;
+  const dim3 block(256);
+  const unsigned chains = (unsigned)(a->batch * (int64_t)Hk);
+  hipStream_t st = (hipStream_t)a->stream;
+  const dim3 sgrid(chains, (unsigned)(n_seg - 1));
+  if (a->g_dtype == SB_F32) hipLaunchKernelGGL((gla_segment_state_kernel<SB_F32>), sgrid, block, 0, st, p);
+  else if (a->g_dtype == SB_BF16) hipLaunchKernelGGL((gla_segment_state_kernel<SB_BF16>), sgrid, block, 0, st, p);
+  else hipLaunchKernelGGL((gla_segment_state_kernel<SB_F16>), sgrid, block, 0, st, p);
+  if (int rc = check_launch("gla_segment_state_kernel")) return rc;
+  if (a->state_dtype == SB_F32) hipLaunchKernelGGL((gla_segment_scan_kernel<true>), dim3(chains, 16), block, 0, st, p);
+  else hipLaunchKernelGGL((gla_segment_scan_kernel<false>), dim3(chains, 16), block, 0, st, p);
+  if (int rc = check_launch("gla_segment_scan_kernel")) return rc;
+  if (group_fits(a, G) && !(a->flags & SB_GLA_PER_HEAD)) {
+    const int rc = launch_group_kernel<true>(a, p, dim3(chains, (unsigned)n_seg));
+    return rc ? rc : check_launch("gla_chunk_group_kernel");
+  }
+  p.H = a->num_heads;
+  const dim3 grid((unsigned)(a->batch * (int64_t)a->num_heads), (unsigned)n_seg);
+#define SB_LAUNCH(F32S, GDT) hipLaunchKernelGGL((gla_chunk_kernel<F32S, GDT, false, true>), grid, block, 0, st, p)
+  if (a->state_dtype == SB_F32) {
+    if (a->g_dtype == SB_F32) SB_LAUNCH(true, SB_F32);
+    else if (a->g_dtype == SB_BF16) SB_LAUNCH(true, SB_BF16);
+    else SB_LAUNCH(true, SB_F16);
+  } else {
+    if (a->g_dtype == SB_F32) SB_LAUNCH(false, SB_F32);
+    else if (a->g_dtype == SB_BF16) SB_LAUNCH(false, SB_BF16);
+    else SB_LAUNCH(false, SB_F16);
+  }
+#undef SB_LAUNCH
+  return check_launch("gla_chunk_kernel");
+}
+
+// Shared states, one pass: grid = one workgroup per (row, state head), each forming the outputs of its G query
+// heads. SB_ERR_UNSUPPORTED (nothing launched) where the group's head offsets do not fit the kernel's 32-bit
+// in-block offsets; the caller then takes the launches per query head.
+int launch_gla_chunk_group(const sb_gla_recurrent_args *a, int state_heads, int G) {
+  if (!group_fits(a, G)) return SB_ERR_UNSUPPORTED;
+  return launch_group_kernel<false>(a, fill(a, state_heads, G, 1, 0, 1), dim3((unsigned)(a->batch * (int64_t)state_heads)));
 }
 
 }  // namespace sb_host

@@ -502,6 +502,7 @@ void launch_sequence(const GlaParams &p, dim3 grid, hipStream_t st) {
 namespace sb_host {
 int launch_gla_chunk(const sb_gla_recurrent_args *a, int64_t groups, int heads, int G, int jn, int j0, int write_state);
 int launch_gla_chunk_group(const sb_gla_recurrent_args *a, int state_heads, int G);
+int launch_gla_chunk_segments(const sb_gla_recurrent_args *a, int G, int n_seg, int seg_tokens, float *ws);
 }
 
 // Shared states: (row, state head) groups from which a prompt launch takes one workgroup per group.
@@ -510,11 +511,11 @@ constexpr int64_t kGroupPassMinGroups = 112;
 // Calls of this many steps or more (and every packed call) with bf16 q, k, v run on the matrix cores.
 constexpr int kChunkKernelMinSteps = 32;
 
-extern "C" int sb_gla_recurrent(const sb_gla_recurrent_args *a) {
+static int check_args(const sb_gla_recurrent_args *a) {
   using namespace sb_host;
   if (!a) return fail(SB_ERR_INVALID, "sb_gla_recurrent: null args");
   if (a->batch < 0 || a->seq_len < 0) return fail(SB_ERR_INVALID, "sb_gla_recurrent: negative size");
-  if (a->batch == 0 || a->seq_len == 0 || a->num_heads == 0) return SB_OK;
+  if (a->batch == 0 || a->seq_len == 0 || a->num_heads == 0) return SB_OK;   // (nothing to do: the callers look again)
   if (!a->q || !a->k || !a->v || !a->g || !a->state || !a->out)
     return fail(SB_ERR_INVALID, "sb_gla_recurrent: null tensor pointer");
   if (a->head_dim != 128)
@@ -535,6 +536,84 @@ extern "C" int sb_gla_recurrent(const sb_gla_recurrent_args *a) {
   if (a->q_heads_per_state < 0 || G > kMaxGroup || a->num_heads % G)
     return fail(SB_ERR_INVALID, "sb_gla_recurrent: q_heads_per_state %d must be 0..%d and divide num_heads %d",
                 a->q_heads_per_state, kMaxGroup, a->num_heads);
+  return SB_OK;
+}
+
+namespace {
+// Whether a call runs on the matrix cores in block form: bf16, 32 steps or more or packed, and q, k, v, g movable as
+// 16-byte pieces and out as 8-byte pieces.
+bool block_form(const sb_gla_recurrent_args *a) {
+  auto pieces = [](const void *ptr, int64_t per16, int64_t sb_, int64_t sh, int64_t st) {
+    return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0 && sb_ % per16 == 0 && sh % per16 == 0 && st % per16 == 0;
+  };
+  return a->dtype == SB_BF16 && !(a->flags & SB_GLA_VECTOR_ONLY) && (a->cu_seqlens || a->seq_len >= kChunkKernelMinSteps) &&
+         pieces(a->q, 8, a->q_stride_b, a->q_stride_h, a->q_stride_t) && pieces(a->k, 8, a->k_stride_b, a->k_stride_h, a->k_stride_t) &&
+         pieces(a->v, 8, a->v_stride_b, a->v_stride_h, a->v_stride_t) &&
+         pieces(a->g, a->g_dtype == SB_F32 ? 4 : 8, a->g_stride_b, a->g_stride_h, a->g_stride_t) &&
+         pieces(a->out, 8, a->out_stride_b, a->out_stride_h, a->out_stride_t);
+}
+// Tokens per segment of a prompt cut into n segments: whole pairs of 16-token blocks.
+int segment_tokens(int seq_len, int n) { return ((seq_len + n - 1) / n + 31) / 32 * 32; }
+}  // namespace
+
+// Where the line lies (28 : 28 and 28 : 4 heads, fp32 state and gate, us per call uncut -> cut into n, measured):
+// * one state per head: two workgroups fit a CU and a cut prompt does 1.6 x the work, so it pays while 512
+//   workgroups allow four segments (18 at one prompt), of 64 tokens or more: 1 x 512 46 -> 28 (8), 1 x 3001 233 -> 63
+//   (16), 1 x 8192 691 -> 148, 2 x 2048 161 -> 75, 4 x 4096 358 -> 300; six prompts 371 -> 402 (3). The two extra
+//   launches cost about 15 us: 4 x 600 54 -> 57;
+// * shared states: the one-pass kernel per group fills a CU by itself and beats a workgroup per query head as soon as
+//   there are enough of them: 1 x 512 87 -> 27 (16), 1 x 8192 1250 -> 72 (64), 4 x 4096 684 -> 121, 16 x 8192 1738 -> 786
+//   (4), 26 x 4096 1230 -> 766 (2).
+extern "C" int32_t sb_gla_prompt_segments(const sb_gla_recurrent_args *a) {
+  if (!a || a->batch <= 0 || a->num_heads <= 0 || a->seq_len < 256 || !block_form(a) ||
+      (a->flags & (SB_GLA_CHECK_GATES | SB_GLA_PER_HEAD | SB_GLA_GROUP_PASS)))
+    return 1;
+  const int G = a->q_heads_per_state > 1 ? a->q_heads_per_state : 1;
+  const int64_t chains = a->batch * (int64_t)(a->num_heads / G);
+  if (chains == 0) return 1;
+  int64_t n;
+  if (G > 1) {
+    n = 256 / chains < a->seq_len / 48 ? 256 / chains : a->seq_len / 48;
+    if (n < 2) return 1;
+  } else {
+    n = 512 / chains < a->seq_len / 64 ? 512 / chains : a->seq_len / 64;
+    if (n < 4 || a->seq_len < (n < 8 ? 1024 : 512)) return 1;
+  }
+  const int seg = segment_tokens(a->seq_len, (int)n);
+  return (a->seq_len + seg - 1) / seg;
+}
+
+extern "C" size_t sb_gla_prompt_workspace_bytes(const sb_gla_recurrent_args *a, int32_t n_segments) {
+  if (!a || n_segments < 2) return 0;
+  const int G = a->q_heads_per_state > 1 ? a->q_heads_per_state : 1;
+  return (size_t)(a->batch * (a->num_heads / G)) * (size_t)n_segments * (16384 + 128) * sizeof(float);
+}
+
+extern "C" int sb_gla_prompt_segmented(const sb_gla_recurrent_args *a, int32_t n_segments, void *workspace, size_t workspace_bytes) {
+  using namespace sb_host;
+  if (n_segments < 2) return sb_gla_recurrent(a);
+  if (int rc = check_args(a)) return rc;
+  if (a->batch == 0 || a->seq_len == 0 || a->num_heads == 0) return SB_OK;
+  if (!block_form(a) || (a->flags & SB_GLA_CHECK_GATES))
+    return fail(SB_ERR_UNSUPPORTED, "sb_gla_prompt_segmented: only calls that run in block form, without the gate check, can be cut");
+  const int G = a->q_heads_per_state > 1 ? a->q_heads_per_state : 1;
+  const int seg = segment_tokens(a->seq_len, n_segments);
+  const int n = (a->seq_len + seg - 1) / seg;
+  if (n < 2) return sb_gla_recurrent(a);
+  if (n > 65535 || a->batch * (int64_t)a->num_heads > 0x7fffffffLL)
+    return fail(SB_ERR_UNSUPPORTED, "sb_gla_prompt_segmented: too many segments or chains");
+  if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 15u) || workspace_bytes < sb_gla_prompt_workspace_bytes(a, n))
+    return fail(SB_ERR_WORKSPACE, "sb_gla_prompt_segmented: workspace of %zu bytes (16-byte aligned) needed, got %zu",
+                sb_gla_prompt_workspace_bytes(a, n), workspace ? workspace_bytes : (size_t)0);
+  return launch_gla_chunk_segments(a, G, n, seg, static_cast<float *>(workspace));
+}
+
+extern "C" int sb_gla_recurrent(const sb_gla_recurrent_args *a) {
+  using namespace sb_host;
+  if (int rc = check_args(a)) return rc;
+  if (a->batch == 0 || a->seq_len == 0 || a->num_heads == 0) return SB_OK;
+  const int64_t groups = a->batch * (int64_t)a->num_heads;
+  const int G = a->q_heads_per_state > 1 ? a->q_heads_per_state : 1;
   const int Hk = a->num_heads / G;
 
   GlaParams p;
@@ -562,17 +641,7 @@ extern "C" int sb_gla_recurrent(const sb_gla_recurrent_args *a) {
                           quad_aligned(a->v, a->dtype, p.v_sb, p.v_sh, p.v_st) &&
                           quad_aligned(a->g, a->g_dtype, p.g_sb, p.g_sh, p.g_st) &&
                           quad_aligned(a->out, a->dtype, p.o_sb, p.o_sh, p.o_st);
-  // the matrix-core kernel moves q, k, v, g as 16-byte pieces and out as 8-byte pieces
-  auto piece_aligned = [](const void *ptr, int64_t per16, int64_t sb_, int64_t sh, int64_t st) {
-    return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0 && sb_ % per16 == 0 && sh % per16 == 0 && st % per16 == 0;
-  };
-  const int64_t g_per16 = a->g_dtype == SB_F32 ? 4 : 8;
-  const bool pieces_ok = piece_aligned(a->q, 8, p.q_sb, p.q_sh, p.q_st) && piece_aligned(a->k, 8, p.k_sb, p.k_sh, p.k_st) &&
-                         piece_aligned(a->v, 8, p.v_sb, p.v_sh, p.v_st) &&
-                         piece_aligned(a->g, g_per16, p.g_sb, p.g_sh, p.g_st) &&
-                         piece_aligned(a->out, 8, p.o_sb, p.o_sh, p.o_st);
-  if (a->dtype == SB_BF16 && pieces_ok && !(a->flags & SB_GLA_VECTOR_ONLY) &&
-      (a->cu_seqlens || a->seq_len >= kChunkKernelMinSteps)) {
+  if (block_form(a)) {
     // Shared states: the heads of a group each carry the recurrence for their own outputs (that keeps
     // one workgroup per query head busy), all reading the group's state. The group's first head stores
     // the final state, in a launch of its own behind the others so that no head reads a state already

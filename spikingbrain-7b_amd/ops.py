@@ -765,8 +765,9 @@ def gla_recurrent(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
     and accumulation in fp32, bf16 operand rounding on the output path); vector_only=True keeps them on
     the step-by-step fp32 kernel. check_gates=True: the block form counts gates beyond its range (see
     gla_gate_range_hits). per_head (shared states, block form): True = one workgroup per query head, False = one
-    per group of query heads (the state advanced once for the group), None = chosen by the number of groups; the
-    results are the same bits either way.
+    per group of query heads (the state advanced once for the group); the results are the same bits either way.
+    None = chosen by the library, which also cuts long prompts of a few sequences into segments that run side by
+    side (results within fp32 rounding of the state).
     Shared states: k, v, g may come with Hkv < H heads (H a multiple of Hkv, up to 8 query heads per kv
     head) and state as [slots, Hkv, D, D]: query head h then works on head h // (H // Hkv) of them, which is
     the reference's repeat_kv of k, v and the gate (hf_7B_model/gla_attention.py:147-149) without the
@@ -814,8 +815,20 @@ def gla_recurrent(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
         flags=(N.SB_GLA_VECTOR_ONLY if vector_only else 0) | (N.SB_GLA_CHECK_GATES if check_gates else 0)
         | (0 if per_head is None else (N.SB_GLA_PER_HEAD if per_head else N.SB_GLA_GROUP_PASS)),
         q_heads_per_state=H // Hk, **_event_args(profile_events))
-    N.check(N.lib().sb_gla_recurrent(C.byref(a)), "gla_recurrent")
+    _launch_gla(a, dev)
     return out
+
+
+def _launch_gla(a, dev: torch.device) -> None:
+    """Enqueue the recurrence; long prompts of a few sequences are cut into segments that run side by side, with
+    scratch memory from torch's allocator (stream-ordered, and part of the graph under capture)."""
+    L = N.lib()
+    n = L.sb_gla_prompt_segments(C.byref(a)) if a.seq_len > 1 else 1
+    if n > 1:
+        ws = torch.empty(L.sb_gla_prompt_workspace_bytes(C.byref(a), n), dtype=torch.uint8, device=dev)
+        N.check(L.sb_gla_prompt_segmented(C.byref(a), n, ws.data_ptr(), ws.numel()), "gla_recurrent")
+    else:
+        N.check(L.sb_gla_recurrent(C.byref(a)), "gla_recurrent")
 
 
 def _state_heads(num_q_heads: int, num_k_heads: int) -> int:
@@ -879,7 +892,7 @@ def gla_recurrent_packed(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: t
         flags=(N.SB_GLA_VECTOR_ONLY if vector_only else 0) | (N.SB_GLA_CHECK_GATES if check_gates else 0)
         | (0 if per_head is None else (N.SB_GLA_PER_HEAD if per_head else N.SB_GLA_GROUP_PASS)),
         q_heads_per_state=H // Hk)
-    N.check(N.lib().sb_gla_recurrent(C.byref(a)), "gla_recurrent")
+    _launch_gla(a, dev)
     return out
 
 
