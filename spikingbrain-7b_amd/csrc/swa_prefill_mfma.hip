@@ -6,8 +6,8 @@
 // the end of the key sequence).
 //
 // Work decomposition
-//   grid = (query tiles of 64 tokens, kv heads); a workgroup covers up to 4 query heads of the kv head
-//   (a wider GQA group takes several launches, 7 = 4 + 3). Every wavefront owns two "column blocks" of
+//   grid = (query tiles of 64 tokens, kv heads, groups of 4 or 3 query heads of the kv head); a workgroup covers one
+//   of those groups (7 = 4 + 3; a last group of 1 or 2 heads takes a launch of its own). Every wavefront owns two "column blocks" of
 //   16 tokens x 1 head (32 score columns, no padding): a pair of heads is served by 4 wavefronts (one
 //   per 16-token sub-tile), an odd last head by 2 wavefronts (two sub-tiles each) - 8 wavefronts for 4
 //   heads, 6 for 3. At 256 registers per wavefront two of them share a SIMD.
@@ -85,9 +85,6 @@ struct PrefillParams {
   int meta_bias_off;
 };
 
-#ifndef SB_PREFILL_HEADS
-#define SB_PREFILL_HEADS 4
-#endif
 constexpr int kRowPad = 288;   // LDS row stride of a K chunk: 256 B of data + 32 B (16-byte operand loads of 16 rows: measured 1.6 x the rate of a 272 B stride)
 constexpr int kRowPadV = 288;  // of a V chunk: 256 B + 32 B (transposing loads: 4 rows x 32 B at a time)
 constexpr int kStageK = 32 * kRowPad, kStageV = 32 * kRowPadV;
@@ -107,10 +104,11 @@ constexpr float kRaise = 8.f;
 // NHEADS query heads of one kv head per workgroup; wavefronts own two column blocks each
 // (a column block = 16 tokens x 1 head): head pairs are served by 4 wavefronts (one per 16-token
 // sub-tile, both heads of the pair), an odd last head by 2 wavefronts (two sub-tiles each).
+// NHEADS = 4 also serves 3 heads (the last four wavefronts then own one column block each): blockIdx.z picks the
+// group of four or three, so that the two groups of a GQA group of 7 are one launch.
 template <int NHEADS>
 struct Shape {
-  static constexpr int kPairs = NHEADS / 2;
-  static constexpr int kWaves = 4 * kPairs + 4 * (NHEADS % 2);
+  static constexpr int kWaves = 4 * (NHEADS / 2) + 4 * (NHEADS % 2);
   static constexpr int kFetchWaves = kWaves == 8 ? 8 : (kWaves < 4 ? kWaves : 4);   // wavefronts that move K/V into LDS
   static constexpr int kLoads = 8 / kFetchWaves;                // 4-row loads per fetching lane, per K and per V
 };
@@ -160,6 +158,8 @@ void swa_prefill_kernel(const PrefillParams p) {
   const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if (tile >= p.num_tiles) return;
   const int kvh = blockIdx.y;
+  const int head_begin = p.head_begin + (NHEADS == 4 ? 4 * (int)blockIdx.z : 0);
+  const int nheads = NHEADS == 4 ? min(4, p.G - head_begin) : NHEADS;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
@@ -194,9 +194,9 @@ void swa_prefill_kernel(const PrefillParams p) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
       ts[b] = wave & 3;
-      hd[b] = NB == 2 ? 2 * (wave >> 2) + b : NHEADS - 1;
+      hd[b] = NB == 2 ? 2 * (wave >> 2) + b : nheads - 1;
     }
-    const int head0 = kvh * p.G + p.head_begin;
+    const int head0 = kvh * p.G + head_begin;
     // (rows past the end of the sequence repeat its last token; they are never stored)
     const int jw0 = min(q0 + 16 * ts[0], Lq - 1);            // first and last token of the wavefront
     const int jw_last = min(q0 + 16 * ts[NB - 1] + 15, Lq - 1);
@@ -592,11 +592,13 @@ void swa_prefill_kernel(const PrefillParams p) {
       }
     }
   };
-  if constexpr (NHEADS % 2 == 1) {
-    if (wave >= 4 * S::kPairs) run(std::integral_constant<int, 1>{});
-    else if constexpr (NHEADS > 1) run(std::integral_constant<int, 2>{});
-  } else {
+  if constexpr (NHEADS == 1) {
+    run(std::integral_constant<int, 1>{});
+  } else if constexpr (NHEADS == 2) {
     run(std::integral_constant<int, 2>{});
+  } else {
+    if ((nheads & 1) && wave >= 4) run(std::integral_constant<int, 1>{});
+    else run(std::integral_constant<int, 2>{});
   }
 }
 
@@ -605,7 +607,6 @@ void launch_prefill_q(int nh, dim3 grid, hipStream_t st, const PrefillParams &p)
   switch (nh) {
     case 1: hipLaunchKernelGGL((swa_prefill_kernel<E, 1, KVQ, PAGED>), grid, dim3(64 * Shape<1>::kWaves), 0, st, p); break;
     case 2: hipLaunchKernelGGL((swa_prefill_kernel<E, 2, KVQ, PAGED>), grid, dim3(64 * Shape<2>::kWaves), 0, st, p); break;
-    case 3: hipLaunchKernelGGL((swa_prefill_kernel<E, 3, KVQ, PAGED>), grid, dim3(64 * Shape<3>::kWaves), 0, st, p); break;
     default: hipLaunchKernelGGL((swa_prefill_kernel<E, 4, KVQ, PAGED>), grid, dim3(64 * Shape<4>::kWaves), 0, st, p); break;
   }
 }
@@ -713,10 +714,15 @@ extern "C" int sb_swa_prefill(const sb_swa_prefill_args *a) {
     p.meta_sr = a->meta_stride_row * 2; p.meta_sh = a->meta_stride_head * 2;
   }
 
-  const dim3 grid((unsigned)((a->num_tiles + 7) / 8 * 8), (unsigned)a->num_kv_heads);
-  for (int h0 = 0; h0 < p.G; h0 += SB_PREFILL_HEADS) {  // a GQA group is covered SB_PREFILL_HEADS heads at a time
+  // Groups of four heads, and a last one of three, are one launch (workgroups of eight wavefronts each); a last group
+  // of one or two heads runs workgroups of four and is a launch of its own.
+  for (int h0 = 0; h0 < p.G;) {
+    const int left = p.G - h0;
+    const int groups = left >= 3 ? left / 4 + (left % 4 == 3) : 1;
+    const int nh = left >= 3 ? 4 : left;
     p.head_begin = h0;
-    const int nh = p.G - h0 < SB_PREFILL_HEADS ? p.G - h0 : SB_PREFILL_HEADS;
+    h0 += nh * groups;
+    const dim3 grid((unsigned)((a->num_tiles + 7) / 8 * 8), (unsigned)a->num_kv_heads, (unsigned)groups);
     if (a->dtype == SB_BF16) launch_prefill<BF16>(a->kv_quant, nh, grid, (hipStream_t)a->stream, p);
     else launch_prefill<F16>(a->kv_quant, nh, grid, (hipStream_t)a->stream, p);
     const int rc = check_launch("swa_prefill_kernel");

@@ -6,6 +6,7 @@ from __future__ import annotations
 import ctypes as C
 from typing import Dict, Optional, Tuple
 
+import numpy as np
 import torch
 
 from . import _native as N
@@ -504,6 +505,7 @@ def plan_decode_split(num_rows: int, num_kv_heads: int, max_seq_len: int, window
 
 
 PREFILL_TILE = 64  # query tokens per workgroup of the prefill kernel
+PREFILL_CONTIGUOUS_TILES = 1024  # lists of this many tiles keep sequence order
 
 
 class PrefillPlan:
@@ -519,21 +521,34 @@ class PrefillPlan:
         seq_lens_k = query_lens if seq_lens_k is None else [int(x) for x in seq_lens_k]
         if len(seq_lens_k) != len(query_lens):
             raise ValueError("query_lens and seq_lens_k must have one entry per sequence")
-        cu, tile_seq, tile_q0 = [0], [], []
-        for s, (lq, lk) in enumerate(zip(query_lens, seq_lens_k)):
-            if lq < 0 or lk < lq:
-                raise ValueError(f"sequence {s}: {lq} queries need at least as many keys, got {lk}")
-            cu.append(cu[-1] + lq)
-            for q0 in range(0, lq, PREFILL_TILE):
-                tile_seq.append(s)
-                tile_q0.append(q0)
-        S, T = len(query_lens), len(tile_seq)
-        packed = torch.tensor(cu + seq_lens_k + tile_seq + tile_q0, dtype=torch.int32).to(device, non_blocking=False)
+        lq, lk = np.asarray(query_lens, dtype=np.int64), np.asarray(seq_lens_k, dtype=np.int64)
+        bad = np.nonzero((lq < 0) | (lk < lq))[0]
+        if bad.size:
+            s = int(bad[0])
+            raise ValueError(f"sequence {s}: {lq[s]} queries need at least as many keys, got {lk[s]}")
+        S = len(query_lens)
+        cu = np.concatenate([[0], np.cumsum(lq)])
+        n = -(-lq // PREFILL_TILE)
+        T = int(n.sum())
+        tile_seq = np.repeat(np.arange(S), n)
+        tile_q0 = (np.arange(T) - np.repeat(np.cumsum(n) - n, n)) * PREFILL_TILE
+        if 0 < T < PREFILL_CONTIGUOUS_TILES:
+            # The kernel gives XCD x the x-th contiguous eighth of the list. Tiles late in a long sequence see the
+            # most keys: they are dealt out in turn, latest first, so that the XCDs get equal shares and the
+            # longest workgroups start first. (Long lists stay in sequence order: an XCD's neighbouring tiles
+            # then share their keys in its L2, and there are enough of them to even out.)
+            order = np.argsort(-(tile_q0 + (lk - lq)[tile_seq]), kind="stable")
+            per_xcd = -(-T // 8)
+            k = np.arange(8 * per_xcd)
+            at = (k % 8) * per_xcd + k // 8
+            at = at[at < T]
+            tile_seq[at], tile_q0[at] = tile_seq[order], tile_q0[order]
+        packed = torch.from_numpy(np.concatenate([cu, lk, tile_seq, tile_q0]).astype(np.int32)).to(device, non_blocking=False)
         self.cu_seqlens_q = packed[:S + 1]
         self.seq_lens_k = packed[S + 1:2 * S + 1]
         self.tile_seq = packed[2 * S + 1:2 * S + 1 + T]
         self.tile_q0 = packed[2 * S + 1 + T:]
-        self.num_tiles, self.total_q, self.num_seqs = T, cu[-1], S
+        self.num_tiles, self.total_q, self.num_seqs = T, int(cu[-1]), S
         self.max_k, self.total_k = max(seq_lens_k, default=0), sum(seq_lens_k)
 
 
