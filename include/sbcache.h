@@ -400,6 +400,33 @@ typedef struct sb_window_shift_args {
 
 int sb_window_shift(const sb_window_shift_args *args);
 
+/* Both halves of a layer's cache: the shift of `k` and that of `v` (which must not touch each other's dst), as one
+ * launch where they move the same rows of the same strides on one stream, else as two. */
+int sb_window_shift_pair(const sb_window_shift_args *k, const sb_window_shift_args *v);
+
+/* ------------------------------------------------------------------------------------
+ * Per-row lengths and per-sequence bounds of a dense, left-padded batch, as sb_swa_decode / sb_swa_prefill take
+ * them: what window_attention.py:190-206 works out from the attention mask, in one launch.
+ * mask: [batch, mask_cols] integers of mask_elem_bytes (1, 2, 4 or 8) each, 0 = padding (a prefix), strides in
+ * elements; NULL = no padding. With pad[b] = num_keys - (non-zero entries of mask row b):
+ *   seq_lens[b * num_queries + j] = num_keys - num_queries + 1 + j
+ *   row_seq [b * num_queries + j] = b
+ *   key_lo  [b * num_queries + j] = pad[b]
+ *   kv_start[b]                   = b * kv_step
+ * Outputs may be NULL (not wanted).
+ * ------------------------------------------------------------------------------------ */
+typedef struct sb_dense_rows_args {
+  const void *mask;
+  int32_t *seq_lens, *row_seq, *key_lo;
+  int64_t *kv_start;
+  int64_t batch, num_queries, num_keys, kv_step;
+  int64_t mask_cols, mask_stride_row, mask_stride_col;
+  int32_t mask_elem_bytes;
+  void *stream;
+} sb_dense_rows_args;
+
+int sb_dense_rows(const sb_dense_rows_args *args);
+
 /* ------------------------------------------------------------------------------------
  * Causal sliding-window attention over many query tokens per sequence (prompt prefill,
  * chunked prefill over the paged cache, multi-token decode); bf16 / fp16, head_size 128,

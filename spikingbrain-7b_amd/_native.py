@@ -94,6 +94,15 @@ class WindowShiftArgs(C.Structure):
     ]
 
 
+class DenseRowsArgs(C.Structure):
+    _fields_ = [
+        ("mask", vp), ("seq_lens", vp), ("row_seq", vp), ("key_lo", vp), ("kv_start", vp),
+        ("batch", i64), ("num_queries", i64), ("num_keys", i64), ("kv_step", i64),
+        ("mask_cols", i64), ("mask_stride_row", i64), ("mask_stride_col", i64),
+        ("mask_elem_bytes", i32), ("stream", vp),
+    ]
+
+
 class SwaPrefillArgs(C.Structure):
     _fields_ = [
         ("q", vp), ("k", vp), ("v", vp), ("out", vp),
@@ -182,6 +191,8 @@ EXPORTS = {
     "sb_gla_gate_range_hits": (C.c_int, [C.POINTER(C.c_int64), C.c_int32]),
     "sb_copy_blocks": (C.c_int, [vp, vp, i64, i64, i64, vp]),
     "sb_window_shift": (C.c_int, [C.POINTER(WindowShiftArgs)]),
+    "sb_window_shift_pair": (C.c_int, [C.POINTER(WindowShiftArgs), C.POINTER(WindowShiftArgs)]),
+    "sb_dense_rows": (C.c_int, [C.POINTER(DenseRowsArgs)]),
     "sb_swa_prefill": (C.c_int, [C.POINTER(SwaPrefillArgs)]),
     "sb_window_advance": (C.c_int, [C.POINTER(WindowAdvanceArgs)]),
     "sb_lse_merge": (C.c_int, [C.POINTER(LseMergeArgs)]),

@@ -82,34 +82,36 @@ class Cache(_HFCache):
 
     # -- sliding-window storage ---------------------------------------------------------
     @staticmethod
-    def _new_buffer(rows: torch.Tensor, window: Optional[int]) -> _WindowBuffer:
-        """Store `rows` [B, H, n, D] (already truncated) in a fresh buffer."""
+    def _new_buffer(rows: torch.Tensor, window: Optional[int]) -> Tuple[_WindowBuffer, tuple]:
+        """A fresh buffer for `rows` [B, H, n, D] (already truncated), and the copy that fills it."""
         B, H, n, D = rows.shape
         storage = torch.empty((B, H, _capacity_for(n, window), D), dtype=rows.dtype, device=rows.device)
-        ops.window_shift(None, storage, rows, keep_rows=0, src_row0=0, dst_row0=0)
-        return _WindowBuffer(storage, 0, n)
+        return _WindowBuffer(storage, 0, n), (None, storage, rows, 0, 0, 0)
+
+    @classmethod
+    def _new_buffers(cls, k: torch.Tensor, v: torch.Tensor, window: Optional[int]):
+        (kb, k_copy), (vb, v_copy) = cls._new_buffer(k, window), cls._new_buffer(v, window)
+        ops.window_shift_pair(k_copy, v_copy)
+        return kb, vb
 
     @staticmethod
-    def _push(buf: _WindowBuffer, rows: torch.Tensor, drop: int, window: Optional[int]) -> None:
-        """Drop the `drop` oldest live rows and append `rows` behind the rest."""
+    def _push(buf: _WindowBuffer, rows: torch.Tensor, drop: int, window: Optional[int]) -> Tuple[tuple, _WindowBuffer]:
+        """Drop the `drop` oldest live rows and append `rows` behind the rest: the copy that takes, and what the buffer
+        is once it has been made."""
         n = rows.shape[2]
         keep = buf.length - drop
         cap = buf.storage.shape[2]
         if buf.start + buf.length + n <= cap:
-            ops.window_shift(None, buf.storage, rows, keep_rows=0, src_row0=0, dst_row0=buf.start + buf.length)
-            buf.start += drop
-        elif keep + n <= buf.start + drop:
+            return ((None, buf.storage, rows, 0, 0, buf.start + buf.length),
+                    _WindowBuffer(buf.storage, buf.start + drop, keep + n))
+        if keep + n <= buf.start + drop:
             # compaction: kept rows move to the front of the same buffer; every destination row
             # (kept + new) lies below the first source row, so the copy cannot race with itself
-            ops.window_shift(buf.storage, buf.storage, rows, keep_rows=keep, src_row0=buf.start + drop, dst_row0=0)
-            buf.start = 0
+            storage = buf.storage
         else:
             B, H, _, D = buf.storage.shape
             storage = torch.empty((B, H, _capacity_for(keep + n, window), D), dtype=rows.dtype, device=rows.device)
-            ops.window_shift(buf.storage, storage, rows, keep_rows=keep, src_row0=buf.start + drop, dst_row0=0)
-            buf.storage = storage
-            buf.start = 0
-        buf.length = keep + n
+        return (buf.storage, storage, rows, keep, buf.start + drop, 0), _WindowBuffer(storage, 0, keep + n)
 
     def update(
         self,
@@ -136,8 +138,7 @@ class Cache(_HFCache):
                 if window_size is not None and input_size > window_size:
                     k_new = k_new[..., -window_size:, :]
                     v_new = v_new[..., -window_size:, :]
-                kb = self._new_buffer(k_new, window_size)
-                vb = self._new_buffer(v_new, window_size)
+                kb, vb = self._new_buffers(k_new, v_new, window_size)
                 self._buffers[len(self.states)] = (kb, vb)
                 attn_state = (kb.view(), vb.view())
             state = dict(recurrent_state=recurrent_state, attn_state=attn_state, conv_state=conv_state)
@@ -152,7 +153,7 @@ class Cache(_HFCache):
                     old = state["attn_state"]
                     if old is None:
                         raise TypeError("'NoneType' object is not iterable")  # what unpacking None raises
-                    bufs = (self._new_buffer(old[0], window_size), self._new_buffer(old[1], window_size))
+                    bufs = self._new_buffers(old[0], old[1], window_size)
                     self._buffers[layer_idx] = bufs
                 kb, vb = bufs
                 # cache.py:96: the window slides only when the stored length EQUALS the window;
@@ -162,8 +163,10 @@ class Cache(_HFCache):
                     raise RuntimeError(
                         f"cannot roll {input_size} new rows into a window of {kb.length}: the reference's "
                         "slice-assign would fail with a shape mismatch here")
-                self._push(kb, attn_state[0], drop, window_size)
-                self._push(vb, attn_state[1], drop, window_size)
+                k_copy, kb = self._push(kb, attn_state[0], drop, window_size)
+                v_copy, vb = self._push(vb, attn_state[1], drop, window_size)
+                ops.window_shift_pair(k_copy, v_copy)
+                self._buffers[layer_idx] = (kb, vb)
                 state["attn_state"] = (kb.view(), vb.view())
             if conv_state is not None:
                 state["conv_state"] = conv_state

@@ -937,10 +937,9 @@ def stream_copy(dst: torch.Tensor, src: torch.Tensor) -> None:
     N.check(N.lib().sb_stream_copy(N.ptr(dst), N.ptr(src), nbytes, N.stream_ptr(dev)), "stream_copy")
 
 
-def window_shift(src: Optional[torch.Tensor], dst: torch.Tensor, fresh: Optional[torch.Tensor], *, keep_rows: int,
-                 src_row0: int, dst_row0: int) -> None:
-    """dst[..., dst_row0 : dst_row0+keep_rows, :] = src[..., src_row0 : src_row0+keep_rows, :] and the
-    n rows of fresh behind them; src/dst are [B, H, cap, D] contiguous, fresh is [B, H, n, D]."""
+def _window_shift_args(src: Optional[torch.Tensor], dst: torch.Tensor, fresh: Optional[torch.Tensor], keep_rows: int,
+                       src_row0: int, dst_row0: int):
+    """The call's arguments, and the (possibly re-laid-out) fresh rows that must live until it is enqueued."""
     dev = N.require_gpu(src, dst, fresh)
     B, H, cap_d, D = dst.shape
     if not dst.is_contiguous() or (src is not None and not src.is_contiguous()):
@@ -954,15 +953,58 @@ def window_shift(src: Optional[torch.Tensor], dst: torch.Tensor, fresh: Optional
             fresh = fresh.contiguous()
     if dst_row0 + keep_rows + n_new > cap_d:
         raise ValueError("window_shift would write past the destination capacity")
-    a = N.WindowShiftArgs(
+    return N.WindowShiftArgs(
         src=N.ptr(src), dst=N.ptr(dst), fresh=N.ptr(fresh), planes=B * H, keep_rows=keep_rows,
         src_row0=src_row0, dst_row0=dst_row0, n_new=n_new, row_bytes=D * esz,
         src_stride_plane_bytes=0 if src is None else src.stride(1) * esz,
         dst_stride_plane_bytes=dst.stride(1) * esz,
         fresh_stride_plane_bytes=0 if fresh is None else fresh.stride(1) * esz,
         fresh_stride_row_bytes=0 if fresh is None else fresh.stride(2) * esz,
-        stream=N.stream_ptr(dev))
+        stream=N.stream_ptr(dev)), fresh
+
+
+def window_shift(src: Optional[torch.Tensor], dst: torch.Tensor, fresh: Optional[torch.Tensor], *, keep_rows: int,
+                 src_row0: int, dst_row0: int) -> None:
+    """dst[..., dst_row0 : dst_row0+keep_rows, :] = src[..., src_row0 : src_row0+keep_rows, :] and the
+    n rows of fresh behind them; src/dst are [B, H, cap, D] contiguous, fresh is [B, H, n, D]."""
+    a, _fresh = _window_shift_args(src, dst, fresh, keep_rows, src_row0, dst_row0)
     N.check(N.lib().sb_window_shift(C.byref(a)), "window_shift")
+
+
+def window_shift_pair(k: tuple, v: tuple) -> None:
+    """window_shift for a layer's K and V, each (src, dst, fresh, keep_rows, src_row0, dst_row0): one launch where both
+    move the same rows of the same strides."""
+    ak, _k = _window_shift_args(*k)
+    av, _v = _window_shift_args(*v)
+    N.check(N.lib().sb_window_shift_pair(C.byref(ak), C.byref(av)), "window_shift")
+
+
+def dense_rows(batch: int, num_queries: int, num_keys: int, kv_step: int, device: torch.device,
+               mask: Optional[torch.Tensor] = None):
+    """What a dense, left-padded batch of `num_queries` queries over `num_keys` keys each is to the attention kernels:
+    (seq_lens, row_seq, key_lo or None, kv_start): int32 [batch * num_queries] (query j sits at key index
+    num_keys - num_queries + j; padding = num_keys minus the non-zero entries of the sequence's mask row) and
+    int64 [batch] (b * kv_step). mask: [>= batch, n], zeros marking a prefix of padding. One launch."""
+    R = batch * num_queries
+    if mask is not None:
+        N.require_gpu(mask)
+        if mask.device != device:
+            raise RuntimeError(f"tensors on different devices: {device} and {mask.device}")
+        if mask.dim() != 2 or mask.shape[0] < batch:
+            raise ValueError(f"mask must be 2-D with a row per sequence ({batch}), got {tuple(mask.shape)}")
+        if mask.dtype.is_floating_point or mask.dtype.is_complex:   # (-0.0 is a zero with bits set)
+            mask = mask != 0
+    buf = torch.empty(batch + (3 * R + 1) // 2, dtype=torch.int64, device=device)
+    rows = buf[batch:].view(torch.int32)
+    kv_start, seq_lens, row_seq, key_lo = buf[:batch], rows[:R], rows[R:2 * R], rows[2 * R:3 * R]
+    a = N.DenseRowsArgs(
+        mask=N.ptr(mask), seq_lens=N.ptr(seq_lens), row_seq=N.ptr(row_seq),
+        key_lo=None if mask is None else N.ptr(key_lo), kv_start=N.ptr(kv_start), batch=batch, num_queries=num_queries,
+        num_keys=num_keys, kv_step=kv_step, mask_cols=0 if mask is None else mask.shape[1],
+        mask_stride_row=0 if mask is None else mask.stride(0), mask_stride_col=0 if mask is None else mask.stride(1),
+        mask_elem_bytes=1 if mask is None else mask.element_size(), stream=N.stream_ptr(device))
+    N.check(N.lib().sb_dense_rows(C.byref(a)), "dense_rows")
+    return seq_lens, row_seq, None if mask is None else key_lo, kv_start
 
 
 def window_advance(n_tokens: torch.Tensor, lo: torch.Tensor, hi: torch.Tensor, ring: torch.Tensor,

@@ -36,14 +36,13 @@ def _uniform_plan(B: int, Q: int, K: int, dev: torch.device):
     return plan
 
 
-def _kv_start_rows(k: torch.Tensor) -> Optional[torch.Tensor]:
-    """Row offset of each batch entry, in units of k.stride(2); None if it is not a whole number."""
-    B = k.shape[0]
-    if B == 1:
-        return torch.zeros(1, dtype=torch.int64, device=k.device)
+def _kv_step_rows(k: torch.Tensor) -> Optional[int]:
+    """Distance of two batch entries in units of k.stride(2); None if it is not a whole number."""
+    if k.shape[0] == 1:
+        return 0
     if k.stride(2) == 0 or k.stride(0) % k.stride(2) != 0:
         return None
-    return torch.arange(B, dtype=torch.int64, device=k.device) * (k.stride(0) // k.stride(2))
+    return k.stride(0) // k.stride(2)
 
 
 def sliding_window_attention(
@@ -89,28 +88,25 @@ def sliding_window_attention(
         window_left = sliding_window if flavour == "flash" else sliding_window - 1
 
     k, v = key_states, value_states
-    if k.stride(3) != 1 or v.stride() != k.stride() or _kv_start_rows(k) is None:
+    if k.stride(3) != 1 or v.stride() != k.stride() or _kv_step_rows(k) is None:
         k, v = k.contiguous(), v.contiguous()
-    kv_start = _kv_start_rows(k)
 
     q_rows = query_states.transpose(1, 2).reshape(B * Q, Hq, D)
     dev = q_rows.device
+    # left padding: zeros form a prefix of a sequence's mask
+    keep = None if attention_mask is None else attention_mask[:, -K:]
+    pad = None
+    if keep is not None and keep.dim() != 2:
+        pad, keep = (K - (keep != 0).sum(dim=1)).to(torch.int32).contiguous(), None
     if Q >= PREFILL_MIN_QUERIES and q_rows.dtype in (torch.bfloat16, torch.float16) and D == 128:
-        # prompt-sized query runs go to the matrix-core kernel (64-token tiles)
-        pad = None
-        if attention_mask is not None:
-            pad = (K - (attention_mask[:, -K:] != 0).sum(dim=1)).to(torch.int32).contiguous()
+        # prompt-sized query runs go to the matrix-core kernel (64-token tiles): one bound per sequence
+        _, _, key_lo, kv_start = ops.dense_rows(B, 1, K, _kv_step_rows(k), dev, keep)
         out = ops.swa_prefill_attention(
-            q_rows, k, v, plan=_uniform_plan(B, Q, K, dev), kv_start=kv_start, key_lo=pad,
+            q_rows, k, v, plan=_uniform_plan(B, Q, K, dev), kv_start=kv_start, key_lo=key_lo if pad is None else pad,
             kv_strides=(k.stride(2), k.stride(1)), num_kv_heads=Hkv, window_left=window_left, scale=D ** -0.5)
         return out.view(B, Q, Hq, D)
-    j = torch.arange(Q, device=dev, dtype=torch.int32)
-    seq_lens_row = (K - Q + 1 + j).repeat(B)                       # query j sits at key index K - Q + j
-    row_seq = torch.arange(B, device=dev, dtype=torch.int32).repeat_interleave(Q)
-    key_lo = None
-    if attention_mask is not None:
-        keep = attention_mask[:, -K:]
-        pad = (K - (keep != 0).sum(dim=1)).to(torch.int32)         # left padding: zeros form a prefix
+    seq_lens_row, row_seq, key_lo, kv_start = ops.dense_rows(B, Q, K, _kv_step_rows(k), dev, keep)
+    if pad is not None:
         key_lo = pad.repeat_interleave(Q)
     out = ops.swa_decode_attention(
         q_rows, k, v, seq_lens_row, kv_start=kv_start, row_seq=row_seq, key_lo=key_lo,
