@@ -25,6 +25,7 @@ SB_GLA_VECTOR_ONLY = 1
 SB_GLA_CHECK_GATES = 2
 SB_GLA_PER_HEAD = 4
 SB_GLA_GROUP_PASS = 8
+SB_GLA_ZERO_SKIPPED = 16
 SB_SWA_DECODE_STATIC_SCRATCH_BYTES = 8 << 20
 ABI_VERSION = 3
 

@@ -34,6 +34,7 @@ struct GlaParams {
   // index hh of the grid stands for state head hk = hh / jn and query head hk * G + j0 + hh % jn, and the
   // final state is stored only if write_state. One state per head: G = jn = 1, j0 = 0, write_state = 1.
   int G, jn, j0, write_state;
+  int zero_skipped;  // one-step kernels: rows without a state get zero outputs (else: left as they are)
 };
 
 // (state head, query head) of head index hh of the launch
@@ -110,9 +111,12 @@ __global__ __launch_bounds__(256, kOneStep ? 4 : 3) void gla_recurrent_kernel(co
   const int b = blockIdx.x / p.H;
   const int h = blockIdx.x - b * p.H;
   const int64_t slot = p.slot_idx ? (int64_t)p.slot_idx[b] : (int64_t)b;
-  if (slot < 0) return;  // no state for this row: nothing read, nothing written
-
   const int tid = threadIdx.x;
+  if (slot < 0) {  // no state for this row: nothing read, at most a zero output written
+    // (a fill of the whole output in front of the kernel cost a launch of its own: 6 rows 22.0 -> 17.6 us a call)
+    if (kOneStep && p.zero_skipped && tid < 128) store_scalar(p.out, b * p.o_sb + h * p.o_sh + tid, p.dtype, 0.f);
+    return;
+  }
   const int col4 = tid & 31;  // columns 4*col4 .. 4*col4+3
   const int rg = tid >> 5;    // row within a pass
 
@@ -212,12 +216,16 @@ __global__ __launch_bounds__(256, kOneStep ? 4 : 3) void gla_recurrent_grouped_k
   const int b = blockIdx.x / Hk;
   const int hk = blockIdx.x - b * Hk;
   const int64_t slot = p.slot_idx ? (int64_t)p.slot_idx[b] : (int64_t)b;
-  if (slot < 0) return;
-
   const int tid = threadIdx.x;
   const int col4 = tid & 31;
   const int rg = tid >> 5;
   const int G = p.G;
+  if (slot < 0) {  // as in the kernel above
+    if (kOneStep && p.zero_skipped)
+      for (int idx = tid; idx < G * 128; idx += 256)
+        store_scalar(p.out, b * p.o_sb + (hk * G + (idx >> 7)) * p.o_sh + (idx & 127), p.dtype, 0.f);
+    return;
+  }
 
   // the step's vectors in LDS: rows 0 .. G-1 = the group's q heads (scaled), then k, v, exp(g)
   __shared__ __attribute__((aligned(16))) float s_vec[kMaxGroup + 3][128];
@@ -630,6 +638,9 @@ extern "C" int sb_gla_recurrent(const sb_gla_recurrent_args *a) {
 
   p.cu = a->cu_seqlens;
   p.G = G; p.jn = 1; p.j0 = 0; p.write_state = 1;
+  p.zero_skipped = (a->flags & SB_GLA_ZERO_SKIPPED) != 0;
+  if (p.zero_skipped && (a->seq_len != 1 || a->cu_seqlens))
+    return fail(SB_ERR_UNSUPPORTED, "sb_gla_recurrent: SB_GLA_ZERO_SKIPPED is for calls of one step");
 
   // the prompt kernel moves q, k, v, g, out as 4-element vectors
   auto quad_aligned = [](const void *ptr, int dt, int64_t sb_, int64_t sh, int64_t st) {

@@ -36,8 +36,7 @@ def my_fused_recurrent_gla(
     q, k, v, g: [B, H, 1, D]; kv_caches: [slots, H, D, D]; slot_idx: [B] int (-1 = skip the row).
     Returns o [B, H, D] (my_fused_recurrent.py:117-119). `initial_state`, `output_final_state`
     and `reverse` are accepted and ignored, as in the reference (:88-119 never reads them).
-    Rows whose slot is -1 keep whatever the output buffer held (the reference leaves them
-    uninitialised); here the buffer starts zeroed.
+    The outputs of rows whose slot is -1 are zero (the reference leaves them uninitialised).
 
     Shared states (not in the reference, which repeats k, v and the gate to all query heads before this
     call, gla_attention.py:264-267): k, v, g [B, Hkv, 1, D] and kv_caches [slots, Hkv, D, D] with H a
@@ -51,8 +50,7 @@ def my_fused_recurrent_gla(
         scale = D ** -0.5
     if slot_idx is not None and slot_idx.dtype != torch.int32:
         slot_idx = slot_idx.to(torch.int32)
-    out = torch.zeros((B, H, 1, D), dtype=q.dtype, device=q.device)
-    ops.gla_recurrent(q, k, v, g, kv_caches, slot_idx, scale, out)
+    out = ops.gla_recurrent(q, k, v, g, kv_caches, slot_idx, scale, zero_skipped=True)
     return out.view(B, H, D)
 
 

@@ -772,10 +772,11 @@ def gla_gate_range_hits(reset: bool = False) -> int:
 def gla_recurrent(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor, state: torch.Tensor,
                   slot_idx: Optional[torch.Tensor] = None, scale: Optional[float] = None,
                   out: Optional[torch.Tensor] = None, vector_only: bool = False, profile_events=None,
-                  check_gates: bool = False, per_head: Optional[bool] = None) -> torch.Tensor:
+                  check_gates: bool = False, per_head: Optional[bool] = None,
+                  zero_skipped: bool = False) -> torch.Tensor:
     """q, k, v, g [B, H, T, D] (any batch/head/time strides, contiguous D); state
     [slots, H, D, D] fp32 or bf16, updated in place; returns o [B, H, T, D] in q's dtype.
-    Rows with slot_idx == -1 are skipped (state and output untouched).
+    Rows with slot_idx == -1 are skipped (state and output untouched; zero_skipped=True, one step only: output zero).
     Calls of 32 steps or more with bf16 q/k/v run 16 tokens at a time on the matrix cores (state, gates
     and accumulation in fp32, bf16 operand rounding on the output path); vector_only=True keeps them on
     the step-by-step fp32 kernel. check_gates=True: the block form counts gates beyond its range (see
@@ -828,7 +829,8 @@ def gla_recurrent(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
         state_stride_slot=state.stride(0), state_stride_head=state.stride(1),
         num_slots=state.shape[0], stream=N.stream_ptr(dev),
         flags=(N.SB_GLA_VECTOR_ONLY if vector_only else 0) | (N.SB_GLA_CHECK_GATES if check_gates else 0)
-        | (0 if per_head is None else (N.SB_GLA_PER_HEAD if per_head else N.SB_GLA_GROUP_PASS)),
+        | (0 if per_head is None else (N.SB_GLA_PER_HEAD if per_head else N.SB_GLA_GROUP_PASS))
+        | (N.SB_GLA_ZERO_SKIPPED if zero_skipped else 0),
         q_heads_per_state=H // Hk, **_event_args(profile_events))
     _launch_gla(a, dev)
     return out

@@ -338,3 +338,24 @@ def test_step_by_step_prompt_kernel_every_element_type(sb, dev, dtype, gdtype, T
         assert np.abs(o.double().cpu().numpy() - ref_o).max() <= 1e-4 * max(1.0, np.abs(ref_o).max())
     else:
         assert out_close(o.float().cpu().numpy(), ref_o, dtype)
+
+
+@pytest.mark.parametrize("shared", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_decode_outputs_of_rows_without_a_slot_are_zero(sb, dev, shared, dtype):
+    """The kernel itself writes them (one step, either kernel); many-step calls refuse the request."""
+    g = torch.Generator().manual_seed(3)
+    B, H, Hk, D = 5, 8, 2 if shared else 8, 128
+    q = torch.randn(B, H, 1, D, generator=g).to(dtype).to(dev)
+    k, v = (torch.randn(B, Hk, 1, D, generator=g).to(dtype).to(dev) for _ in range(2))
+    gate = -torch.rand(B, Hk, 1, D, generator=g).to(dev)
+    state = torch.randn(4, Hk, D, D, generator=g).to(dev)
+    slots = torch.tensor([-1, 2, -1, 0, -1], dtype=torch.int32, device=dev)
+    wide = torch.full((B, H, 1, 2 * D), 7.0, dtype=dtype, device=dev)     # outputs with a stride: nothing beside them changes
+    sb.ops.gla_recurrent(q, k, v, gate, state.clone(), slots, out=wide[..., :D], zero_skipped=True)
+    o = sb.my_fused_recurrent_gla(q, k, v, gate, state.clone(), slots)
+    assert torch.equal(wide[..., 0, :D], o) and bool((wide[..., D:] == 7).all())
+    assert bool((o[[0, 2, 4]] == 0).all()) and bool((o[[1, 3]] != 0).any())
+    with pytest.raises(NotImplementedError):
+        sb.ops.gla_recurrent(q.expand(-1, -1, 2, -1), k.expand(-1, -1, 2, -1), v.expand(-1, -1, 2, -1),
+                             gate.expand(-1, -1, 2, -1), state, slots, zero_skipped=True)
