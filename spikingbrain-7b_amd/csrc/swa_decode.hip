@@ -377,7 +377,11 @@ __global__ __launch_bounds__(256) void swa_decode_split_kernel(const DecodeParam
 }
 
 // One workgroup of head_size threads per (query row, query head): log-sum-exp merge of the splits.
-template <typename E>
+// kBatch splits per trip to memory, every load of a trip issued before any is used: the kernel is latency and little
+// else, so the host takes the batch that covers the split count in one or two trips. The arithmetic goes four
+// splits at a time in the same order whatever the batch (same bits); from four to four the running sums are
+// rescaled to the new maximum.
+template <typename E, int kBatch>
 __global__ __launch_bounds__(256) void swa_decode_merge_kernel(const DecodeParams p) {
   const int64_t rh = blockIdx.x;  // r*Hq + hq
   const int64_t r = rh / p.Hq;
@@ -385,37 +389,49 @@ __global__ __launch_bounds__(256) void swa_decode_merge_kernel(const DecodeParam
   const int d = threadIdx.x;
   const float *ml = p.ws_ml + rh * p.n_split * 2;
   const float *acc = p.ws_acc + rh * p.n_split * p.D + d;
-  // Four splits per trip, every load of a trip issued before any is used: with the usual split counts
-  // the kernel is one round trip to memory. Across trips the running sums are rescaled to the new maximum.
   float tot = 0.f, L = 0.f, M = kNegInf;
-  for (int s0 = 0; s0 < p.n_split; s0 += 4) {
-    float ms[4], ls[4], av[4];
+  for (int b0 = 0; b0 < p.n_split; b0 += kBatch) {
+    float ms[kBatch], ls[kBatch], av[kBatch];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int s = min(s0 + j, p.n_split - 1);
+    for (int j = 0; j < kBatch; ++j) {
+      const int s = min(b0 + j, p.n_split - 1);
       ms[j] = ml[2 * s];
       ls[j] = ml[2 * s + 1];
       av[j] = acc[(int64_t)s * p.D];
     }
-    float Mn = M;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (s0 + j < p.n_split) Mn = fmaxf(Mn, ms[j]);
-    if (Mn != kNegInf) {
-      const float keep = (M == kNegInf) ? 0.f : fast_exp2(M - Mn);
-      tot *= keep;
-      L *= keep;
+    for (int j0 = 0; j0 < kBatch; j0 += 4) {
+      const int s0 = b0 + j0;
+      if (s0 < p.n_split) {
+        float Mn = M;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float f = (s0 + j >= p.n_split || ms[j] == kNegInf) ? 0.f : fast_exp2(ms[j] - Mn);
-        tot = fmaf(av[j], f, tot);
-        L = fmaf(ls[j], f, L);
+        for (int j = 0; j < 4; ++j)
+          if (s0 + j < p.n_split) Mn = fmaxf(Mn, ms[j0 + j]);
+        if (Mn != kNegInf) {
+          const float keep = (M == kNegInf) ? 0.f : fast_exp2(M - Mn);
+          tot *= keep;
+          L *= keep;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float f = (s0 + j >= p.n_split || ms[j0 + j] == kNegInf) ? 0.f : fast_exp2(ms[j0 + j] - Mn);
+            tot = fmaf(av[j0 + j], f, tot);
+            L = fmaf(ls[j0 + j], f, L);
+          }
+        }
+        M = Mn;
       }
     }
-    M = Mn;
   }
   store_out<E>(p.out, r * p.o_sr + (int64_t)hq * p.o_sh + d, L > 0.f ? tot / L : 0.f);
   if (d == 0 && p.lse) p.lse[rh] = L > 0.f ? (M + log2f(L)) * kLn2 : kNegInf;
+}
+
+template <typename E>
+void launch_merge(dim3 grid, dim3 block, hipStream_t st, const DecodeParams &p) {
+  if (p.n_split <= 4) hipLaunchKernelGGL((swa_decode_merge_kernel<E, 4>), grid, block, 0, st, p);
+  else if (p.n_split <= 8) hipLaunchKernelGGL((swa_decode_merge_kernel<E, 8>), grid, block, 0, st, p);
+  else if (p.n_split <= 16) hipLaunchKernelGGL((swa_decode_merge_kernel<E, 16>), grid, block, 0, st, p);
+  else hipLaunchKernelGGL((swa_decode_merge_kernel<E, 32>), grid, block, 0, st, p);
 }
 
 // Merge for the balanced split: the partials of row r are numbers w + r for the workgroups w whose
@@ -636,16 +652,26 @@ static double split_cost(int64_t wgs, int64_t n, int64_t chunks, int64_t cus) {
   return (double)full * round_cost(per_wg, cus, cus) + (rest ? round_cost(per_wg, rest, cus) : 0.0);
 }
 
+// Estimated duration (us) of a fixed split whose workgroups all run at once. A workgroup's chunk costs it what its
+// wavefronts take to issue and compute it (1.8 us, however many chunks are in flight: register sets for two or three
+// chunks ahead changed nothing) and up to 0.84 us more where all CUs share the memory system; every split is one more
+// partial to store and merge. Fitted to 120 launches of 1 .. 64 rows of 300 .. 4097 keys (rms 7 %).
+static double one_round_us(int64_t wgs, int64_t n, int64_t chunks, int64_t cus) {
+  const double fill = (double)(wgs * n) / (double)cus;
+  return 5.7 + (double)((chunks + n - 1) / n) * (1.82 + 0.84 * fill * fill) + (n > 1 ? 0.14 * (double)n : 0.0);
+}
+// Windows of at most this many chunks are left whole.
+constexpr int64_t kWholeChunks = 11;
+
 extern "C" int32_t sb_swa_decode_auto_split(int64_t num_rows, int32_t num_kv_heads,
                                             int32_t max_seq_len, int32_t window_left) {
   if (num_rows <= 0 || num_kv_heads <= 0 || max_seq_len <= 0) return 1;
   int64_t keys = max_seq_len;
   if (window_left >= 0 && keys > (int64_t)window_left + 1) keys = (int64_t)window_left + 1;
   const int64_t chunks = (keys + 31) / 32 + 1;  // +1: an unaligned window touches one more chunk
-  // A split is one workgroup per (row, group of up to 4 kv heads). Take the split count with the lowest
-  // estimated duration (rows x splits just above a multiple of the CU count pay a whole extra round),
-  // leaving every workgroup at least 8 chunks (256 keys) so that its fixed cost stays small next to the
-  // streaming; ties go to more splits (more CUs streaming).
+  // A split is one workgroup per (row, group of up to 4 kv heads). Where rows x splits takes more than one round
+  // over the CUs: the split count with the lowest estimated duration (just above a multiple of the CU count costs a
+  // whole extra round), leaving every workgroup at least 8 chunks; ties go to more splits (more CUs streaming).
   const int64_t wgs = num_rows * ((num_kv_heads + 3) / 4);
   const int64_t cus = device_cu_count();
   int64_t cap = chunks / 8;
@@ -655,6 +681,18 @@ extern "C" int32_t sb_swa_decode_auto_split(int64_t num_rows, int32_t num_kv_hea
   double best_cost = split_cost(wgs, 1, chunks, cus);
   for (int64_t n = 2; n <= cap; ++n) {
     const double c = split_cost(wgs, n, chunks, cus);
+    if (c <= best_cost) { best = n; best_cost = c; }
+  }
+  if (wgs * best > cus || chunks <= kWholeChunks) return (int32_t)best;
+  // One round: the CUs that 8 chunks a workgroup would leave idle are worth more than the partials they add. Measured
+  // with 8 chunks or more each -> without that bound (us per call): 1 row x 4097 keys 24.1 -> 17.1 (15 -> 43 splits),
+  // 8 x 4097 27.5 -> 22.3 (15 -> 26), 1 x 2000 21.1 -> 12.9 (8 -> 32), 16 x 1000 22.5 -> 14.7 (4 -> 16),
+  // 64 x 600 28.3 -> 21.6 (2 -> 4); INT8 8 x 4097 21.3 -> 18.1.
+  const int64_t run = keys < max_seq_len ? chunks : chunks - 1;  // (a window that starts at the first key is aligned)
+  best = 1;
+  best_cost = one_round_us(wgs, 1, run, cus);
+  for (int64_t n = 2; n <= 64 && n <= run && wgs * n <= cus; ++n) {
+    const double c = one_round_us(wgs, n, run, cus);
     if (c <= best_cost) { best = n; best_cost = c; }
   }
   return (int32_t)best;
@@ -974,9 +1012,9 @@ extern "C" int sb_swa_decode(const sb_swa_decode_args *a) {
     return check_launch("swa_decode_merge_balanced_kernel");
   }
   const dim3 mblock((unsigned)a->head_size);
-  if (a->dtype == SB_BF16) hipLaunchKernelGGL(swa_decode_merge_kernel<BF16>, mgrid, mblock, 0, st, p);
-  else if (a->dtype == SB_F16) hipLaunchKernelGGL(swa_decode_merge_kernel<F16>, mgrid, mblock, 0, st, p);
-  else hipLaunchKernelGGL(swa_decode_merge_kernel<F32>, mgrid, mblock, 0, st, p);
+  if (a->dtype == SB_BF16) launch_merge<BF16>(mgrid, mblock, st, p);
+  else if (a->dtype == SB_F16) launch_merge<F16>(mgrid, mblock, st, p);
+  else launch_merge<F32>(mgrid, mblock, st, p);
   return check_launch("swa_decode_merge_kernel");
 }
 
@@ -1002,6 +1040,10 @@ extern "C" int sb_swa_decode_static(const sb_swa_decode_args *a) {
   if (n_split < 0) return fail(SB_ERR_INVALID, "sb_swa_decode_static: negative n_split");
   if (n_split == 0)
     n_split = sb_swa_decode_auto_split(a->num_rows, a->num_kv_heads, a->max_seq_len, a->window_left);
+  // (chosen here: never more partials than the library's scratch holds)
+  while (a->n_split == 0 && n_split > 1 && sb_swa_decode_workspace_bytes(a->num_rows, a->num_q_heads, a->head_size, n_split) >
+                                               (size_t)SB_SWA_DECODE_STATIC_SCRATCH_BYTES)
+    --n_split;
   const size_t need = sb_swa_decode_workspace_bytes(a->num_rows, a->num_q_heads, a->head_size, n_split);
   if (need > (size_t)SB_SWA_DECODE_STATIC_SCRATCH_BYTES)
     return fail(SB_ERR_WORKSPACE,

@@ -450,7 +450,9 @@ __global__ __launch_bounds__(256, 1) void swa_decode_stream_kernel(const DecodeP
       }
     }
     reset();
-    if (any && next.valid) load_row(next.r);
+    if constexpr (kBalanced) {  // (a run of the fixed split is one segment)
+      if (any && next.valid) load_row(next.r);
+    }
   };
 
   if (cb >= ce) {  // fixed split: a part of the row with no chunks still owes the merge its (empty) partial

@@ -114,3 +114,17 @@ def test_wrappers_refuse_cpu_tensors(sb):
     cache = torch.zeros(4, 16, 4, 128, dtype=torch.bfloat16)
     with pytest.raises(RuntimeError, match="no CPU path"):
         sb.ops.kv_append(k, k, cache, cache, torch.zeros(2, dtype=torch.int64))
+
+
+def test_auto_split_of_one_round(sb):
+    """Shapes whose workgroups run at once: never more of them than CUs (256 where the device cannot be asked), never more
+    splits than chunks or 64, and the partials of 28 heads fit the library's own scratch."""
+    L = sb._native.lib()
+    for rows in range(1, 257):
+        for keys, wl in ((200, 4096), (321, 4096), (352, 4096), (353, 4096), (600, 512), (1000, -1), (4097, 4096), (20000, 4096)):
+            n = L.sb_swa_decode_auto_split(rows, 4, keys, wl)
+            visible = min(keys, wl + 1) if wl >= 0 else keys
+            assert 1 <= n <= min(64, visible // 32 + 2)
+            if rows <= 64:
+                assert rows * n <= 256
+                assert L.sb_swa_decode_workspace_bytes(rows, 28, 128, n) <= sb._native.SB_SWA_DECODE_STATIC_SCRATCH_BYTES

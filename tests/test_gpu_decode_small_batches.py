@@ -1,0 +1,55 @@
+"""Small decode batches: split counts at the edges of the merge kernel's batches (4, 8, 16, 32 partials per trip), in fp32
+against float64 attention (2e-6 of the largest value: 32-bit sums over at most 700 keys), and the bf16 stream kernel at
+the split the library chooses against the same rows unsplit (both round fp32 results to bf16: one last place, 2^-7)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+HQ, HKV, D, BS = 8, 2, 128, 16
+
+
+def _problem(dev, dtype, lens, seed):
+    g = torch.Generator().manual_seed(seed)
+    need = [(n + BS - 1) // BS for n in lens]
+    perm = torch.randperm(sum(need), generator=g).int()
+    tables = torch.zeros(len(lens), max(need), dtype=torch.int32)
+    at = 0
+    for b, n in enumerate(need):
+        tables[b, :n] = perm[at:at + n]
+        at += n
+    kv = torch.randn(2, sum(need), BS, HKV, D, generator=g).to(dtype)
+    q = torch.randn(len(lens), HQ, D, generator=g).to(dtype)
+    return q, kv, tables, torch.tensor(lens, dtype=torch.int32)
+
+
+def _reference(q, kv, tables, lens, window):
+    out = []
+    for b, n in enumerate(lens):
+        rows = kv[:, tables[b].long()].flatten(1, 2)[:, max(0, n - 1 - window):n].double()
+        k, v = rows.repeat_interleave(HQ // HKV, dim=2).unbind(0)
+        p = torch.softmax(torch.einsum("hd,khd->hk", q[b].double(), k) * D ** -0.5, -1)
+        out.append(torch.einsum("hk,khd->hd", p, v))
+    return torch.stack(out)
+
+
+@pytest.mark.parametrize("n_split", [2, 4, 5, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 65])
+def test_merge_of_many_partials(sb, dev, n_split):
+    lens = [700, 33, 1, 512, 97]          # rows with fewer chunks than splits leave empty partials
+    q, kv, tables, sl = _problem(dev, torch.float32, lens, n_split)
+    kvd = kv.to(dev)
+    out, lse = sb.ops.swa_decode_attention(q.to(dev), kvd[0], kvd[1], sl.to(dev), block_table=tables.to(dev), window_left=650,
+                                           n_split=n_split, balanced=False, return_lse=True)
+    ref = _reference(q, kv, tables, lens, 650)
+    assert (out.cpu().double() - ref).abs().max() <= 2e-6 * ref.abs().max() and torch.isfinite(lse).all()
+
+
+@pytest.mark.parametrize("rows", [1, 3, 17])
+@pytest.mark.parametrize("length", [350, 353, 600, 1000, 2048])
+def test_chosen_split_matches_unsplit_rows(sb, dev, rows, length):
+    lens = [max(1, length - 37 * i) for i in range(rows)]
+    q, kv, tables, sl = _problem(dev, torch.bfloat16, lens, length)
+    q, kv, tables, sl = q.to(dev), kv.to(dev), tables.to(dev), sl.to(dev)
+    assert sb._native.lib().sb_swa_decode_auto_split(rows, HKV, tables.shape[1] * BS, 1024) > 1
+    one, auto = (sb.ops.swa_decode_attention(q, kv[0], kv[1], sl, block_table=tables, window_left=1024, n_split=n, balanced=False)
+                 for n in (1, 0))
+    assert ((auto.float() - one.float()).abs() <= 2 ** -7 * one.float().abs() + 2 ** -9 * one.float().abs().max()).all()
