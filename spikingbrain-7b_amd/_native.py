@@ -279,7 +279,8 @@ def require_gpu(*tensors: torch.Tensor) -> torch.device:
 
 
 def stream_ptr(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    # torch.cuda.current_stream(dev).cuda_stream without the Stream object (1.3 us of a 15 us call)
+    return torch._C._cuda_getCurrentRawStream(dev.index if dev.index is not None else torch.cuda.current_device())
 
 
 def ptr(t: Optional[torch.Tensor]) -> Optional[int]:

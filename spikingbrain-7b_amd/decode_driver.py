@@ -23,7 +23,7 @@ import torch
 
 from . import ops
 from .block_manager import DeviceWindowState, WindowBlockManager
-from .meta_attention import MetaAttentionBackend, MetaAttentionImpl, MetaAttentionMetadata
+from .meta_attention import MetaAttentionBackend, MetaAttentionImpl, MetaAttentionMetadata, _flat, _rows_of
 
 
 class HybridDecodeCache:
@@ -223,17 +223,17 @@ class HybridDecodeCache:
         if self.kv_quant == "int8":
             codes, scales = self.kv_caches[layer_idx // 2], self.kv_scales[layer_idx // 2]
             n = q.shape[0]
-            ops.kv_append_int8(k, v, codes[0], codes[1], scales[0], scales[1], meta.slot_mapping.flatten()[:n])
+            ops.kv_append_int8(k, v, codes[0], codes[1], scales[0], scales[1], _rows_of(_flat(meta.slot_mapping), 0, n))
             return ops.swa_decode_attention(
-                q, codes[0], codes[1], meta.seq_lens_tensor[:n], block_table=meta.block_tables, window_left=self.wl,
+                q, codes[0], codes[1], _rows_of(meta.seq_lens_tensor, 0, n), block_table=meta.block_tables, window_left=self.wl,
                 scale=self.D ** -0.5, out=out, max_seq_len=meta.max_decode_seq_len or None,
                 k_scale=scales[0], v_scale=scales[1])
         if self.kv_quant == "fp8":
             codes = self.kv_caches[layer_idx // 2]
             n = q.shape[0]
-            ops.kv_append_fp8(k, v, codes[0], codes[1], meta.slot_mapping.flatten()[:n], 1.0, 1.0)
+            ops.kv_append_fp8(k, v, codes[0], codes[1], _rows_of(_flat(meta.slot_mapping), 0, n), 1.0, 1.0)
             return ops.swa_decode_attention(
-                q, codes[0], codes[1], meta.seq_lens_tensor[:n], block_table=meta.block_tables, window_left=self.wl,
+                q, codes[0], codes[1], _rows_of(meta.seq_lens_tensor, 0, n), block_table=meta.block_tables, window_left=self.wl,
                 scale=self.D ** -0.5, out=out, max_seq_len=meta.max_decode_seq_len or None, fp8_scales=(1.0, 1.0))
         return self.impl.forward(self._layer, q, k, v, None, None, None, self.kv_caches[layer_idx // 2], meta, out)
 

@@ -379,6 +379,23 @@ class MetaAttentionMetadataBuilder:
         )
 
 
+# A layer call of a small decode step costs more host time than GPU time, and each view, slice or flatten of a tensor
+# 1 to 2 us of it: these make one only where it changes something.
+def _heads(t: torch.Tensor, heads: int, size: int) -> torch.Tensor:
+    """t.view(-1, heads, size)."""
+    return t if t.dim() == 3 and t.shape[1] == heads and t.shape[2] == size else t.view(-1, heads, size)
+
+
+def _rows_of(t: torch.Tensor, start: int, stop: int) -> torch.Tensor:
+    """t[start:stop] for 0 <= start <= stop."""
+    return t if start == 0 and stop >= t.shape[0] else t[start:stop]
+
+
+def _flat(t: torch.Tensor) -> torch.Tensor:
+    """t.flatten()."""
+    return t if t.dim() == 1 else t.flatten()
+
+
 class MetaAttentionImpl:
     """meta_attention.py:611-982.
 
@@ -490,11 +507,11 @@ class MetaAttentionImpl:
                 raise AssertionError(f"key2/value2 must hold num_meta_tokens = {self.num_meta_tokens} rows")
 
         window_left = self.sliding_window[0]
-        query = query.view(-1, self.num_heads, self.head_size)
-        output = output.view(-1, self.num_heads, self.head_size)
+        query = _heads(query, self.num_heads, self.head_size)
+        output = _heads(output, self.num_heads, self.head_size)
         if key is not None:
-            key = key.view(-1, self.num_kv_heads, self.head_size)
-            value = value.view(-1, self.num_kv_heads, self.head_size)
+            key = _heads(key, self.num_kv_heads, self.head_size)
+            value = _heads(value, self.num_kv_heads, self.head_size)
 
         # A pure decode step (one new token per sequence, the hot loop) appends and attends in ONE
         # launch: the attention kernel takes the newest K/V row from `key`/`value` and stores it at
@@ -518,15 +535,15 @@ class MetaAttentionImpl:
             if fp8_kv and key_cache.dtype not in (torch.uint8, torch.float8_e4m3fn):
                 raise ValueError(f"an fp8 kv-cache must be a uint8 or float8_e4m3fn tensor, got {key_cache.dtype}")
             if key is not None and value is not None and fp8_kv:
-                ops.kv_append_fp8(key, value, key_cache, value_cache, attn_metadata.slot_mapping.flatten(),
+                ops.kv_append_fp8(key, value, key_cache, value_cache, _flat(attn_metadata.slot_mapping),
                                   k_scale_f, v_scale_f)
             elif key is not None and value is not None and int8_kv:
                 # rows are quantised on their way in: 128 code bytes + one scale per (token, kv head)
                 ops.kv_append_int8(key, value, key_cache, value_cache, scales["k_scale"], scales["v_scale"],
-                                   attn_metadata.slot_mapping.flatten())
+                                   _flat(attn_metadata.slot_mapping))
             elif key is not None and value is not None and not fuse_append:
                 # all new K/V of the step (prefill and decode tokens) go in with one launch (:790-799)
-                ops.kv_append(key, value, key_cache, value_cache, attn_metadata.slot_mapping.flatten())
+                ops.kv_append(key, value, key_cache, value_cache, _flat(attn_metadata.slot_mapping))
 
         num_prefill_query_tokens = attn_metadata.num_prefill_tokens
         num_decode_query_tokens = attn_metadata.num_decode_tokens
@@ -545,8 +562,8 @@ class MetaAttentionImpl:
                 options = dict(softcap=self.logits_soft_cap, alibi_slopes=self.alibi_slopes,
                                meta_bias=(num_prefill_query_tokens, num_prefill_query_tokens + self.num_meta_tokens))
             output[:self.num_meta_tokens] = ops.meta_token_attention(query2, key2, value2, self.scale, **options)[0]
-        prefill_output = output[num_meta_prefill_tokens - num_prefill_query_tokens:num_meta_prefill_tokens]
-        decode_output = output[num_meta_prefill_tokens:]
+        prefill_output = _rows_of(output, num_meta_prefill_tokens - num_prefill_query_tokens, num_meta_prefill_tokens)
+        decode_output = _rows_of(output, num_meta_prefill_tokens, output.shape[0])
 
         # The kernels take the meta rows into their own softmax (meta_k/meta_v), over element and byte-code
         # caches alike (the reference runs a second attention over them and merges by log-sum-exp).
@@ -567,15 +584,15 @@ class MetaAttentionImpl:
                 prefill_kv["meta_bias"] = (0, num_meta_prefill_tokens)
                 decode_kv["meta_bias"] = (0, num_decode_query_tokens)
 
-        decode_query = query[num_prefill_query_tokens:]
-        query = query[:num_prefill_query_tokens]
+        decode_query = _rows_of(query, num_prefill_query_tokens, query.shape[0])
+        query = _rows_of(query, 0, num_prefill_query_tokens)
         assert query.shape[0] == num_prefill_query_tokens
         assert decode_query.shape[0] == num_decode_query_tokens
 
         if prefill_meta := attn_metadata.prefill_metadata:
             if kv_cache.numel() == 0 or prefill_meta.block_tables is None or prefill_meta.block_tables.numel() == 0:
                 # plain prompt run: keys and values are the in-flight tensors (:835-884)
-                pk, pv = key[:num_prefill_query_tokens], value[:num_prefill_query_tokens]
+                pk, pv = _rows_of(key, 0, num_prefill_query_tokens), _rows_of(value, 0, num_prefill_query_tokens)
                 if int8_kv:   # attend to what the cache will hold: the rows as quantize_sym returns them
                     pk, pv = ops.quantize_sym(pk), ops.quantize_sym(pv)
                 elif fp8_kv:  # scaled_fp8_quant of the prompt's keys and values (:853-869)
@@ -604,8 +621,8 @@ class MetaAttentionImpl:
                 n = decode_query.shape[0]
                 fused = {}
                 if fuse_append:
-                    fused = dict(new_key=key[:n], new_value=value[:n],
-                                 new_slot_mapping=decode_meta.slot_mapping.flatten()[:n].contiguous())
+                    fused = dict(new_key=_rows_of(key, 0, n), new_value=_rows_of(value, 0, n),
+                                 new_slot_mapping=_rows_of(_flat(decode_meta.slot_mapping), 0, n).contiguous())
                 if decode_meta._decode_balanced is None:
                     host_lens = decode_meta.host_seq_lens
                     decode_meta._decode_balanced = bool(
@@ -613,7 +630,7 @@ class MetaAttentionImpl:
                         ops.plan_decode_split(n, self.num_kv_heads, decode_meta.max_decode_seq_len or max(host_lens[:n]),
                                               window_left, host_lens[:n]))
                 ops.swa_decode_attention(
-                    decode_query, key_cache, value_cache, decode_meta.seq_lens_tensor[:n],
+                    decode_query, key_cache, value_cache, _rows_of(decode_meta.seq_lens_tensor, 0, n),
                     block_table=decode_meta.block_tables, window_left=window_left, scale=self.scale,
                     out=decode_output, max_seq_len=decode_meta.max_decode_seq_len or None,
                     balanced=False if byte_kv else decode_meta._decode_balanced, **scales, **fused, **decode_kv)

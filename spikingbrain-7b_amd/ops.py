@@ -24,10 +24,10 @@ _workspaces: Dict[Tuple[torch.device, int], torch.Tensor] = {}
 _graph_workspaces: Dict[Tuple[torch.device, int], list] = {}
 
 
-def _capture_id(dev: torch.device) -> int:
-    """Sequence number of the stream capture torch's current stream is part of, 0 if none."""
+def _capture_id(stream: int) -> int:
+    """Sequence number of the stream capture `stream` is part of, 0 if none."""
     cid = C.c_uint64(0)
-    N.check(N.lib().sb_stream_capture_id(N.stream_ptr(dev), C.byref(cid)), "stream_capture_id")
+    N.check(N.lib().sb_stream_capture_id(stream, C.byref(cid)), "stream_capture_id")
     return cid.value
 
 
@@ -43,7 +43,8 @@ def _new_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
 def _workspace(dev: torch.device, nbytes: int) -> Optional[torch.Tensor]:
     if nbytes == 0:
         return None
-    cap = _capture_id(dev)
+    stream = N.stream_ptr(dev)
+    cap = _capture_id(stream)
     if cap:
         # (allocated inside the capture: the 64 KiB counter fill becomes a node of the graph and runs at every
         # replay, which is harmless: the counters are zero between launches anyway)
@@ -52,7 +53,7 @@ def _workspace(dev: torch.device, nbytes: int) -> Optional[torch.Tensor]:
             # (a smaller buffer handed out earlier in this capture stays in the list: earlier nodes use it)
             owned.append(_new_workspace(dev, nbytes))
         return owned[-1]
-    key = (dev, N.stream_ptr(dev))
+    key = (dev, stream)
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = _new_workspace(dev, nbytes)
@@ -325,6 +326,7 @@ def swa_decode_attention(
         n_split = 2  # the balanced split always goes through partial results and the merge
     ws_bytes = L.sb_swa_decode_workspace_bytes(R, Hq, D, n_split)
     ws = _workspace(dev, ws_bytes)
+    q_strides, out_strides = q.stride(), out.stride()
     a = N.SwaDecodeArgs(
         q=N.ptr(q), k_cache=N.ptr(key_cache), v_cache=N.ptr(value_cache), out=N.ptr(out), lse=N.ptr(lse),
         block_table=N.ptr(block_table), kv_start=N.ptr(kv_start), row_seq=N.ptr(row_seq),
@@ -337,8 +339,8 @@ def swa_decode_attention(
         | (N.SB_DECODE_MERGE_IN_KERNEL if merge_in_kernel else 0) | (N.SB_DECODE_PER_SEGMENT if per_segment else 0)
         | ((int(pipeline_depth) & 7) << 4),
         scale=float(scale),
-        q_stride_row=q.stride(0), q_stride_head=q.stride(1),
-        out_stride_row=out.stride(0), out_stride_head=out.stride(1),
+        q_stride_row=q_strides[0], q_stride_head=q_strides[1],
+        out_stride_row=out_strides[0], out_stride_head=out_strides[1],
         kv_stride_block=kv_strides[0], kv_stride_row=kv_strides[1], kv_stride_head=kv_strides[2],
         block_table_stride=bt_stride, stream=N.stream_ptr(dev),
         k_scale=N.ptr(k_scale), v_scale=N.ptr(v_scale),
@@ -816,17 +818,18 @@ def gla_recurrent(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
         if out.shape != q.shape or out.dtype != q.dtype:
             raise ValueError("out must match q in shape and dtype")
         _inner_contiguous(out, "out")
+    sq, sk, sv, sg, so, ss = q.stride(), k.stride(), v.stride(), g.stride(), out.stride(), state.stride()
     a = N.GlaRecurrentArgs(
         q=N.ptr(q), k=N.ptr(k), v=N.ptr(v), g=N.ptr(g), state=N.ptr(state), out=N.ptr(out),
         slot_idx=N.ptr(slot_idx), batch=B, num_heads=H, seq_len=T, head_dim=D,
         dtype=N.dtype_code(q.dtype), g_dtype=N.dtype_code(g.dtype), state_dtype=N.dtype_code(state.dtype),
         scale=float(scale),
-        q_stride_b=q.stride(0), q_stride_h=q.stride(1), q_stride_t=q.stride(2),
-        k_stride_b=k.stride(0), k_stride_h=k.stride(1), k_stride_t=k.stride(2),
-        v_stride_b=v.stride(0), v_stride_h=v.stride(1), v_stride_t=v.stride(2),
-        g_stride_b=g.stride(0), g_stride_h=g.stride(1), g_stride_t=g.stride(2),
-        out_stride_b=out.stride(0), out_stride_h=out.stride(1), out_stride_t=out.stride(2),
-        state_stride_slot=state.stride(0), state_stride_head=state.stride(1),
+        q_stride_b=sq[0], q_stride_h=sq[1], q_stride_t=sq[2],
+        k_stride_b=sk[0], k_stride_h=sk[1], k_stride_t=sk[2],
+        v_stride_b=sv[0], v_stride_h=sv[1], v_stride_t=sv[2],
+        g_stride_b=sg[0], g_stride_h=sg[1], g_stride_t=sg[2],
+        out_stride_b=so[0], out_stride_h=so[1], out_stride_t=so[2],
+        state_stride_slot=ss[0], state_stride_head=ss[1],
         num_slots=state.shape[0], stream=N.stream_ptr(dev),
         flags=(N.SB_GLA_VECTOR_ONLY if vector_only else 0) | (N.SB_GLA_CHECK_GATES if check_gates else 0)
         | (0 if per_head is None else (N.SB_GLA_PER_HEAD if per_head else N.SB_GLA_GROUP_PASS))
