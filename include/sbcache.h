@@ -502,6 +502,19 @@ typedef struct sb_swa_prefill_args {
 
 int sb_swa_prefill(const sb_swa_prefill_args *args);
 
+/* The same call with the keys of a tile cut into parts that run side by side (a few tiles leave most of the GPU idle
+ * otherwise: a chunk of 200 prompt tokens behind a full window is 4 tiles). sb_swa_prefill_parts: how many parts the
+ * library would cut this call's longest walk into (1 = not at all); max_keys bounds seq_lens_k.
+ * sb_swa_prefill_workspace_bytes: scratch memory that takes (device, 16-byte aligned, contents irrelevant before and
+ * after; calls whose scratch memory overlaps must be ordered), total_q being the packed query rows (cu_seqlens_q's last
+ * entry). sb_swa_prefill_parted: the call. Every part keeps its softmax in fp32 and the parts are put together in fp32.
+ * n_parts < 2: sb_swa_prefill with max_keys known (workspace unused). A walk longer than max_keys allows is still
+ * walked whole. */
+int32_t sb_swa_prefill_parts(const sb_swa_prefill_args *args, int64_t max_keys);
+size_t sb_swa_prefill_workspace_bytes(const sb_swa_prefill_args *args, int64_t total_q, int32_t n_parts);
+int sb_swa_prefill_parted(const sb_swa_prefill_args *args, int64_t total_q, int64_t max_keys, int32_t n_parts,
+                          void *workspace, size_t workspace_bytes);
+
 /* ------------------------------------------------------------------------------------
  * Per-row symmetric INT8 K/V (W8ASpike/window_attention.py:183-186 with quantize_sym, :227-237):
  *   scale = clamp(max|row| / 127, 1e-5, 1e4); code = clamp(round_half_even(x / scale), -128, 127)

@@ -6,8 +6,9 @@
 // the end of the key sequence).
 //
 // Work decomposition
-//   grid = (query tiles of 64 tokens, kv heads, groups of 4 or 3 query heads of the kv head); a workgroup covers one
-//   of those groups (7 = 4 + 3; a last group of 1 or 2 heads takes a launch of its own). Every wavefront owns two "column blocks" of
+//   grid = (query tiles of 64 tokens, kv heads, groups of 4 or 3 query heads of the kv head, or of 2 and 1 in small
+//   calls; parts of the tile's keys); a workgroup covers one of those groups (7 = 4 + 3 = 2 + 2 + 2 + 1; behind groups of
+//   four a last group of 1 or 2 heads takes a launch of its own). Every wavefront owns two "column blocks" of
 //   16 tokens x 1 head (32 score columns, no padding): a pair of heads is served by 4 wavefronts (one
 //   per 16-token sub-tile), an odd last head by 2 wavefronts (two sub-tiles each) - 8 wavefronts for 4
 //   heads, 6 for 3. At 256 registers per wavefront two of them share a SIMD.
@@ -84,7 +85,33 @@ struct PrefillParams {
   ScoreOptions opt;          // soft cap / ALiBi slopes, applied to every raw score in front of the mask
   // ALiBi term of meta row j for packed query row t: -slope * |meta_bias_off + t - j|, meta_bias_off = row0 + meta_len - rows
   int meta_bias_off;
+  // Key split: a tile's walk is cut into up to n_parts parts of part_chunks chunks (the last part takes what is left),
+  // a workgroup each; a tile that fits one part stores its output itself, the others fp32 partials: numerators
+  // [query row, query head, n_parts, 128] and (reference point, denominator) [query row, query head, n_parts, 2].
+  int n_parts, part_chunks;
+  float *ws_acc;
+  float *ws_ml;
 };
+
+// The walk of a tile in 32-key chunks: every chunk that holds a key some token of the tile can see.
+struct Walk {
+  int lo, hi;  // keys [lo, hi)
+  int ch_begin, ch_end;
+};
+__device__ __forceinline__ Walk tile_walk(const PrefillParams &p, int seq, int q0, int Lq, int Lk) {
+  Walk w;
+  const int shift = Lk - Lq;  // query j sits at key index shift + j
+  const int klo = p.key_lo ? max(p.key_lo[seq], 0) : 0;
+  w.hi = shift + min(q0 + 63, Lq - 1) + 1;
+  // (kept inside the sequence even when padding hides every key: such rows end up fully masked)
+  w.lo = min(max(p.window_left >= 0 ? shift + q0 - p.window_left : 0, klo), w.hi - 1);
+  w.ch_begin = w.lo >> 5;
+  w.ch_end = ((w.hi - 1) >> 5) + 1;
+  return w;
+}
+__device__ __forceinline__ int tile_parts(const PrefillParams &p, const Walk &w) {
+  return min(p.n_parts, (w.ch_end - w.ch_begin + p.part_chunks - 1) / p.part_chunks);
+}
 
 constexpr int kRowPad = 288;   // LDS row stride of a K chunk: 256 B of data + 32 B (16-byte operand loads of 16 rows: measured 1.6 x the rate of a 272 B stride)
 constexpr int kRowPadV = 288;  // of a V chunk: 256 B + 32 B (transposing loads: 4 rows x 32 B at a time)
@@ -105,8 +132,8 @@ constexpr float kRaise = 8.f;
 // NHEADS query heads of one kv head per workgroup; wavefronts own two column blocks each
 // (a column block = 16 tokens x 1 head): head pairs are served by 4 wavefronts (one per 16-token
 // sub-tile, both heads of the pair), an odd last head by 2 wavefronts (two sub-tiles each).
-// NHEADS = 4 also serves 3 heads (the last four wavefronts then own one column block each): blockIdx.z picks the
-// group of four or three, so that the two groups of a GQA group of 7 are one launch.
+// NHEADS = 4 also serves 3 heads (the last four wavefronts then own one column block each) and NHEADS = 2 one, so that
+// all groups of a GQA group of 7 are one launch either way.
 template <int NHEADS>
 struct Shape {
   static constexpr int kWaves = 4 * (NHEADS / 2) + 4 * (NHEADS % 2);
@@ -163,11 +190,12 @@ void swa_prefill_kernel(const PrefillParams p) {
   const int width = min(p.bucket, per_xcd - bucket * p.bucket);   // tiles of this bucket
   const int in_bucket = at - bucket * p.bucket * per_tile;
   const int pair = in_bucket / width;
-  const int tile = (blockIdx.x & 7) * per_xcd + bucket * p.bucket + (in_bucket - pair * width);
+  // (the parts of a tile go to XCDs one after the other: a call of one tile would otherwise run on one of them)
+  const int tile = ((blockIdx.x + blockIdx.y) & 7) * per_xcd + bucket * p.bucket + (in_bucket - pair * width);
   if (tile >= p.num_tiles) return;
   const int head_group = pair / p.Hkv, kvh = pair - head_group * p.Hkv;
-  const int head_begin = p.head_begin + 4 * head_group;
-  const int nheads = NHEADS == 4 ? min(4, p.G - head_begin) : NHEADS;
+  const int head_begin = p.head_begin + NHEADS * head_group;
+  const int nheads = min(NHEADS, p.G - head_begin);
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
@@ -183,15 +211,17 @@ void swa_prefill_kernel(const PrefillParams p) {
   const int wl = p.window_left;
 
   // keys any token of this workgroup can see: [wg_lo, wg_hi)
-  const int j_last = min(q0 + 63, Lq - 1);
-  const int wg_hi = shift + j_last + 1;
+  const Walk walk = tile_walk(p, seq, q0, Lq, Lk);
+  const int wg_lo = walk.lo, wg_hi = walk.hi;
   const int klo = p.key_lo ? max(p.key_lo[seq], 0) : 0;
-  // (kept inside the sequence even when padding hides every key: such rows end up fully masked)
-  const int wg_lo = min(max(wl >= 0 ? shift + q0 - wl : 0, klo), wg_hi - 1);
   const int first_tile = wg_lo >> 4, last_tile = (wg_hi - 1) >> 4;
-  const int ch_begin = wg_lo >> 5, ch_end = ((wg_hi - 1) >> 5) + 1;
+  // this workgroup's part of the walk
+  const int part = blockIdx.y, parts = tile_parts(p, walk);
+  if (part >= parts) return;  // (the whole workgroup, ahead of every barrier)
+  const int ch_begin = walk.ch_begin + part * p.part_chunks;
+  const int ch_end = part + 1 == parts ? walk.ch_end : ch_begin + p.part_chunks;
   const int n_walk = ch_end - ch_begin;  // the walk: index x is window chunk ch_begin + x
-  const int meta_chunks = (p.meta_len + 31) >> 5;
+  const int meta_chunks = part == 0 ? (p.meta_len + 31) >> 5 : 0;
 
   // Everything from here on is written for NB column blocks per wavefront: two for the wavefronts of a head
   // pair, one for those of an odd last head (four wavefronts, one per 16-token sub-tile).
@@ -586,7 +616,14 @@ void swa_prefill_kernel(const PrefillParams p) {
       float lt = l[b];
       lt += __shfl_xor(lt, 16);
       lt += __shfl_xor(lt, 32);
-      if (q0 + 16 * ts[b] + c < Lq) {
+      if (q0 + 16 * ts[b] + c < Lq && parts > 1) {
+        const int64_t rec = ((int64_t)(qrow0 + q0 + 16 * ts[b] + c) * p.Hq + head0 + hd[b]) * p.n_parts + part;
+        float *dst = p.ws_acc + rec * 128 + 4 * g;
+#pragma unroll
+        for (int mt = 0; mt < 8; ++mt)
+          *reinterpret_cast<float4 *>(dst + 16 * mt) = make_float4(acc[b][mt][0], acc[b][mt][1], acc[b][mt][2], acc[b][mt][3]);
+        if (g == 0) *reinterpret_cast<float2 *>(p.ws_ml + rec * 2) = make_float2(m[b], lt);
+      } else if (q0 + 16 * ts[b] + c < Lq) {
         const float inv = lt > 0.f ? 1.f / lt : 0.f;
         char *dst = p.out + ((int64_t)(qrow0 + q0 + 16 * ts[b] + c) * p.o_sr + (int64_t)(head0 + hd[b]) * p.o_sh +
                              4 * g) * 2;
@@ -603,11 +640,61 @@ void swa_prefill_kernel(const PrefillParams p) {
   if constexpr (NHEADS == 1) {
     run(std::integral_constant<int, 1>{});
   } else if constexpr (NHEADS == 2) {
-    run(std::integral_constant<int, 2>{});
+    if (nheads == 1) run(std::integral_constant<int, 1>{});
+    else run(std::integral_constant<int, 2>{});
   } else {
     if ((nheads & 1) && wave >= 4) run(std::integral_constant<int, 1>{});
     else run(std::integral_constant<int, 2>{});
   }
+}
+
+// Puts the parts of a tile together: a workgroup per 8 query rows of a tile and query head, 32 lanes of four dims per
+// row. A tile of one part has its output already. Latency and bytes (parts x 520 per row and head, once): with the 64
+// rows of a tile in one workgroup, eight after the other, 24 parts took 60 us instead of 9.
+template <typename E>
+__global__ __launch_bounds__(256) void swa_prefill_merge_kernel(const PrefillParams p) {
+  const int tile = blockIdx.x, head = blockIdx.y;
+  const int seq = p.tile_seq[tile], q0 = p.tile_q0[tile];
+  const int qrow0 = p.cu_q[seq], Lq = p.cu_q[seq + 1] - qrow0;
+  const int parts = tile_parts(p, tile_walk(p, seq, q0, Lq, p.seq_lens_k[seq]));
+  const int j = q0 + 8 * blockIdx.z + (threadIdx.x >> 5), d4 = threadIdx.x & 31;
+  if (parts < 2 || j >= Lq) return;
+  const int64_t rh = (int64_t)(qrow0 + j) * p.Hq + head;
+  const float2 *ml = reinterpret_cast<const float2 *>(p.ws_ml) + rh * p.n_parts;
+  const float4 *acc = reinterpret_cast<const float4 *>(p.ws_acc) + rh * p.n_parts * 32 + d4;
+  float4 tot = make_float4(0.f, 0.f, 0.f, 0.f);
+  float L = 0.f, M = kNegInf;
+  for (int s0 = 0; s0 < parts; s0 += 4) {  // four parts per trip to memory
+    float2 x[4];
+    float4 a[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int s = min(s0 + u, parts - 1);
+      x[u] = ml[s];
+      a[u] = acc[s * 32];
+    }
+    float Mn = M;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) Mn = fmaxf(Mn, x[u].x);
+    const float ref = Mn == kNegInf ? 0.f : Mn;  // (nothing visible so far: every factor is 0, and a NaN stays one)
+    const float keep = fast_exp2(M - ref);
+    tot.x *= keep; tot.y *= keep; tot.z *= keep; tot.w *= keep;
+    L *= keep;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float f = fast_exp2((s0 + u < parts ? x[u].x : kNegInf) - ref);
+      tot.x = fmaf(a[u].x, f, tot.x);
+      tot.y = fmaf(a[u].y, f, tot.y);
+      tot.z = fmaf(a[u].z, f, tot.z);
+      tot.w = fmaf(a[u].w, f, tot.w);
+      L = fmaf(x[u].y, f, L);  // (past the last part: the last one again, times 0)
+    }
+    M = Mn;
+  }
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  char *dst = p.out + ((int64_t)(qrow0 + j) * p.o_sr + (int64_t)head * p.o_sh + 4 * d4) * 2;
+  *reinterpret_cast<uint2 *>(dst) = make_uint2(E::pack(tot.x * inv, tot.y * inv), E::pack(tot.z * inv, tot.w * inv));
+  if (p.lse && d4 == 0) p.lse[rh] = L > 0.f ? (M + log2f(L)) * kLn2 : kNegInf;
 }
 
 template <typename E, int KVQ, bool PAGED>
@@ -626,9 +713,54 @@ void launch_prefill(int kv_quant, int nh, dim3 grid, hipStream_t st, const Prefi
   else launch_prefill_q<E, SB_KV_NONE, false>(nh, grid, st, p);
 }
 
-}  // namespace
+// Most 32-key chunks a tile of 64 queries walks when no sequence has more than max_keys keys.
+int64_t most_chunks(const sb_swa_prefill_args *a, int64_t max_keys) {
+  int64_t span = max_keys;
+  if (a->window_left >= 0 && span > (int64_t)a->window_left + 64) span = (int64_t)a->window_left + 64;
+  return (span + 30) / 32 + 1;
+}
 
-extern "C" int sb_swa_prefill(const sb_swa_prefill_args *a) {
+constexpr int64_t kCUs = 256;
+
+// How a call is spread over the GPU: with groups of four heads a workgroup of eight wavefronts fills a CU, and a call
+// of `wgs` of them takes as long as its longest walk while wgs <= 256. Two ways to shorten that:
+//  * pairs: workgroups of two heads and four wavefronts, two to a CU. A CU that holds one runs its chunks at 0.69 us
+//    instead of 0.9, and in whole prompts a long walk shares its CU with a short one (1 x 300 / 700 / 1000 / 1517 /
+//    2560 / 3000 tokens: 16.6 / 28.3 / 35.8 / 50.7 / 80.7 / 92.8 -> 13.1 / 21.9 / 28.2 / 42.3 / 69 / 87 us). With walks of
+//    equal length (prompt chunks behind a context) only while every CU gets one (1024 tokens behind 4200: 125 -> 97;
+//    1500: 126 -> 136), and beyond 1.5 x 256 workgroups of four heads they lose (1 x 6000: 256 -> 271);
+//  * parts: the keys of a walk cut into parts of 8 chunks or more side by side, at the price of fp32 partials and
+//    a merge (64 / 200 / 512 / 1024 tokens behind 4200: 123 -> 24 (16 parts) / 33 (8) / 49 (4) / 80 (2) us).
+struct Spread {
+  int parts;
+  bool pairs;
+};
+int64_t quad_workgroups(const sb_swa_prefill_args *a) {
+  return a->num_tiles * a->num_kv_heads * ((a->num_q_heads / a->num_kv_heads + 3) / 4);
+}
+bool pairs_pay(const sb_swa_prefill_args *a, int64_t chunks, int64_t parts) {
+  const int64_t wgs = quad_workgroups(a) * parts;
+  // (whole prompts walk two chunks per tile at most; a longer walk means a context in front of the queries)
+  const bool whole = chunks <= 2 * a->num_tiles + 2;
+  return whole && parts == 1 ? 2 * wgs <= 3 * kCUs : 2 * wgs <= kCUs;
+}
+Spread spread_of(const sb_swa_prefill_args *a, int64_t max_keys) {
+  const int64_t chunks = most_chunks(a, max_keys), wgs = quad_workgroups(a);
+  Spread best{1, pairs_pay(a, chunks, 1)};
+  double best_us = 5.0 + (best.pairs ? 0.69 : 0.9) * (double)chunks;
+  for (int64_t n = 2; n * wgs <= kCUs && 8 * n <= chunks; ++n) {
+    const bool pairs = pairs_pay(a, chunks, n);
+    const double us = 13.5 + 0.28 * (double)n + 8.0 * (double)(n * wgs) / (double)kCUs +
+                      (pairs ? 0.69 : 0.86) * (double)((chunks + n - 1) / n);
+    if (us < best_us) {
+      best = Spread{(int)n, pairs};
+      best_us = us;
+    }
+  }
+  return best;
+}
+
+int prefill(const sb_swa_prefill_args *a, int64_t max_keys, int n_parts, float *ws_acc, float *ws_ml) {
   using namespace sb_host;
   if (!a) return fail(SB_ERR_INVALID, "sb_swa_prefill: null args");
   if (a->num_tiles < 0) return fail(SB_ERR_INVALID, "sb_swa_prefill: negative num_tiles");
@@ -686,6 +818,9 @@ extern "C" int sb_swa_prefill(const sb_swa_prefill_args *a) {
   p.k_scale_tensor = a->k_scale_tensor; p.v_scale_tensor = a->v_scale_tensor; p.Hkv = a->num_kv_heads;
   p.bt_stride = a->block_table_stride;
   p.num_tiles = (int)a->num_tiles;
+  const int64_t chunks = most_chunks(a, max_keys);
+  p.n_parts = n_parts; p.part_chunks = (int)((chunks + n_parts - 1) / n_parts);
+  p.ws_acc = ws_acc; p.ws_ml = ws_ml;
   p.meta_k = p.meta_v = nullptr;
   p.meta_len = 0;
   p.meta_sr = p.meta_sh = 0;
@@ -730,19 +865,57 @@ extern "C" int sb_swa_prefill(const sb_swa_prefill_args *a) {
   // its heads); 16 x 8192 in sequence order 6.34 ms at 1 against 6.04 at 4, 6.08 at 16 and 6.13 at all (four tiles and one
   // kv head at a time keep their keys in the XCD's L2).
   p.bucket = a->num_tiles < 1024 ? 1 : 4;
+  const bool pairs = p.G > 1 && pairs_pay(a, chunks, n_parts);
   if (per_xcd * 8 * a->num_kv_heads * p.G > 0x7fffffffLL) return fail(SB_ERR_UNSUPPORTED, "sb_swa_prefill: grid too large");
   for (int h0 = 0; h0 < p.G;) {
     const int left = p.G - h0;
-    const int groups = left >= 3 ? left / 4 + (left % 4 == 3) : 1;
-    const int nh = left >= 3 ? 4 : left;
+    const int groups = pairs ? (left + 1) / 2 : (left >= 3 ? left / 4 + (left % 4 == 3) : 1);
+    const int nh = pairs ? 2 : (left >= 3 ? 4 : left);
     p.head_begin = h0;
     h0 += nh * groups;
     p.head_groups = groups;
-    const dim3 grid((unsigned)(per_xcd * 8 * a->num_kv_heads * groups));
+    const dim3 grid((unsigned)(per_xcd * 8 * a->num_kv_heads * groups), (unsigned)n_parts);
     if (a->dtype == SB_BF16) launch_prefill<BF16>(a->kv_quant, nh, grid, (hipStream_t)a->stream, p);
     else launch_prefill<F16>(a->kv_quant, nh, grid, (hipStream_t)a->stream, p);
     const int rc = check_launch("swa_prefill_kernel");
     if (rc != SB_OK) return rc;
   }
+  if (n_parts > 1) {
+    const dim3 mgrid((unsigned)a->num_tiles, (unsigned)a->num_q_heads, 8);
+    if (a->dtype == SB_BF16) hipLaunchKernelGGL(swa_prefill_merge_kernel<BF16>, mgrid, dim3(256), 0, (hipStream_t)a->stream, p);
+    else hipLaunchKernelGGL(swa_prefill_merge_kernel<F16>, mgrid, dim3(256), 0, (hipStream_t)a->stream, p);
+    return check_launch("swa_prefill_merge_kernel");
+  }
   return SB_OK;
+}
+
+}  // namespace
+
+extern "C" int sb_swa_prefill(const sb_swa_prefill_args *a) { return prefill(a, INT32_MAX, 1, nullptr, nullptr); }
+
+extern "C" int32_t sb_swa_prefill_parts(const sb_swa_prefill_args *a, int64_t max_keys) {
+  if (!a || a->num_tiles <= 0 || a->num_kv_heads <= 0 || a->num_q_heads <= 0 || max_keys <= 0) return 1;
+  return spread_of(a, max_keys < INT32_MAX ? max_keys : INT32_MAX).parts;
+}
+
+extern "C" size_t sb_swa_prefill_workspace_bytes(const sb_swa_prefill_args *a, int64_t total_q, int32_t n_parts) {
+  if (!a || n_parts < 2 || total_q <= 0 || a->num_q_heads <= 0) return 0;
+  return (size_t)total_q * (size_t)a->num_q_heads * (size_t)n_parts * (128 + 2) * sizeof(float);
+}
+
+extern "C" int sb_swa_prefill_parted(const sb_swa_prefill_args *a, int64_t total_q, int64_t max_keys, int32_t n_parts,
+                                     void *workspace, size_t workspace_bytes) {
+  using namespace sb_host;
+  if (!a) return fail(SB_ERR_INVALID, "sb_swa_prefill_parted: null args");
+  if (a->num_tiles <= 0) return sb_swa_prefill(a);
+  if (total_q <= 0 || max_keys <= 0) return fail(SB_ERR_INVALID, "sb_swa_prefill_parted: total_q and max_keys must be positive");
+  if (max_keys > INT32_MAX) max_keys = INT32_MAX;
+  if (n_parts < 2) return prefill(a, max_keys, 1, nullptr, nullptr);
+  if (n_parts > 1024 || a->num_q_heads > 65535) return fail(SB_ERR_UNSUPPORTED, "sb_swa_prefill_parted: too many parts or heads");
+  if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 15u) ||
+      workspace_bytes < sb_swa_prefill_workspace_bytes(a, total_q, n_parts))
+    return fail(SB_ERR_WORKSPACE, "sb_swa_prefill_parted: workspace of %zu bytes (16-byte aligned) needed, got %zu",
+                sb_swa_prefill_workspace_bytes(a, total_q, n_parts), workspace ? workspace_bytes : (size_t)0);
+  float *acc = static_cast<float *>(workspace);
+  return prefill(a, max_keys, n_parts, acc, acc + total_q * a->num_q_heads * n_parts * 128);
 }

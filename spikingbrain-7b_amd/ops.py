@@ -579,6 +579,7 @@ def swa_prefill_attention(
     softcap: float = 0.0,
     alibi_slopes: Optional[torch.Tensor] = None,
     meta_bias: Optional[Tuple[int, int]] = None,
+    n_parts: int = 0,
 ):
     """Causal sliding-window attention for q [total_q, Hq, D] packed sequence after sequence.
     softcap / alibi_slopes: as for swa_decode_attention; query j of a sequence sits at key position
@@ -597,7 +598,9 @@ def swa_prefill_attention(
     key_lo [S] int32: keys below key_lo[s] are invisible (left padding); a query that sees no key
     gets zeros.
     k_scale/v_scale (INT8 codes) or fp8_scales (e4m3fn codes): the paged caches are byte codes as
-    kv_append_int8 / kv_append_fp8 wrote them; rows are dequantised on their way into the kernel."""
+    kv_append_int8 / kv_append_fp8 wrote them; rows are dequantised on their way into the kernel.
+    n_parts: cut the keys of a tile into up to this many parts that run side by side (0 = chosen by the library, 1 =
+    not at all)."""
     dev = N.require_gpu(q, k, v, block_table, kv_start, key_lo, out, k_scale, v_scale)
     kv_quant = N.SB_KV_NONE
     if fp8_scales is not None:
@@ -705,7 +708,14 @@ def swa_prefill_attention(
         softcap=float(softcap), alibi_slopes=N.ptr(_slopes(alibi_slopes, Hq, dev)),
         meta_bias_row0=int(meta_bias[0]) if meta_bias else 0,
         meta_bias_rows=int(meta_bias[1]) if meta_bias else int(q.shape[0]), **meta)
-    N.check(N.lib().sb_swa_prefill(C.byref(a)), "swa_prefill")
+    L = N.lib()
+    if n_parts == 0:
+        n_parts = L.sb_swa_prefill_parts(C.byref(a), plan.max_k)
+    ws = None
+    if n_parts > 1:   # scratch memory from torch's allocator: stream-ordered, and part of the graph under capture
+        ws = torch.empty(L.sb_swa_prefill_workspace_bytes(C.byref(a), Tq, n_parts), dtype=torch.uint8, device=dev)
+    N.check(L.sb_swa_prefill_parted(C.byref(a), Tq, plan.max_k, n_parts, N.ptr(ws), 0 if ws is None else ws.numel()),
+            "swa_prefill")
     return (out, lse) if return_lse else out
 
 

@@ -1,0 +1,97 @@
+"""Prompt attention with the keys of a tile cut into parts (fp32 partials and a merge) and with workgroups of two heads:
+against float64 attention. Element outputs are rounded to bf16 from fp32 and the probabilities to bf16 on the way: 1e-2 of
+the 2-norm, the same bound as for uncut calls; cut against uncut the same, with the log-sum-exp (fp32 throughout) within
+2e-5 + the two's rounding of scores."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+D = 128
+
+
+def _reference(q, k, v, lens, ctx, window, key_lo, G):
+    outs, at, kat = [], 0, 0
+    for s, n in enumerate(lens):
+        L = n + ctx
+        qq, kk, vv = q[at:at + n].double(), k[kat:kat + L].double().repeat_interleave(G, 1), v[kat:kat + L].double().repeat_interleave(G, 1)
+        sc = torch.matmul(qq.transpose(0, 1), kk.permute(1, 2, 0).contiguous()) * D ** -0.5
+        pos, key = torch.arange(n)[:, None] + ctx, torch.arange(L)[None]
+        hide = (key > pos) | (key < key_lo[s])
+        if window >= 0:
+            hide |= key < pos - window
+        sc.masked_fill_(hide, float("-inf"))
+        p = torch.nan_to_num(torch.softmax(sc, -1))
+        outs.append(torch.matmul(p, vv.transpose(0, 1).contiguous()).transpose(0, 1))
+        at, kat = at + n, kat + L
+    return torch.cat(outs)
+
+
+@pytest.mark.parametrize("G", [1, 2, 3, 4, 5, 7, 8])
+@pytest.mark.parametrize("lens,ctx,window", [([1], 0, -1), ([65], 300, -1), ([64, 3], 257, 100), ([130, 1, 70], 0, 4096), ([40], 1000, 511)])
+@pytest.mark.parametrize("n_parts", [0, 1, 2, 3, 7, 40])
+def test_parts_and_pairs(sb, dev, G, lens, ctx, window, n_parts):
+    g = torch.Generator().manual_seed(G * 100 + n_parts)
+    Hkv, T, Lk = 2, sum(lens), sum(lens) + ctx * len(lens)
+    q, k, v = torch.randn(T, Hkv * G, D, generator=g).bfloat16(), torch.randn(Lk, Hkv, D, generator=g).bfloat16(), torch.randn(Lk, Hkv, D, generator=g).bfloat16()
+    key_lo = [(7 * s) % (n + ctx + 2) for s, n in enumerate(lens)]      # some rows see nothing: zeros
+    kv_start = torch.tensor([0] + [n + ctx for n in lens]).cumsum(0)[:-1].to(dev)
+    run = lambda parts: sb.ops.swa_prefill_attention(
+        q.to(dev), k.to(dev), v.to(dev), query_lens=lens, seq_lens_k=[n + ctx for n in lens], kv_start=kv_start,
+        key_lo=torch.tensor(key_lo, dtype=torch.int32, device=dev), window_left=window, return_lse=True, n_parts=parts)
+    out, lse = run(n_parts)
+    ref = _reference(q, k, v, lens, ctx, window, key_lo, G)
+    assert (out.cpu().double() - ref).norm() <= 1e-2 * ref.norm()
+    out1, lse1 = run(1)
+    assert torch.equal(torch.isneginf(lse), torch.isneginf(lse1))
+    ok = ~torch.isneginf(lse)
+    assert (lse[ok] - lse1[ok]).abs().max() <= 1e-4
+
+
+@pytest.mark.parametrize("kv", ["bf16", "int8", "fp8"])
+def test_paged_parts_with_meta_rows_and_options(sb, dev, kv):
+    """The parts over a paged cache (element and byte codes), with meta rows (walked by the first part) and score options."""
+    g = torch.Generator().manual_seed(5)
+    Hkv, G, bs, n, ctx = 2, 4, 16, 50, 500
+    L = n + ctx
+    blocks = (L + bs - 1) // bs
+    table = torch.randperm(blocks, generator=g).int()[None].to(dev)
+    q = torch.randn(n, Hkv * G, D, generator=g).bfloat16().to(dev)
+    kw = {}
+    if kv == "int8":
+        cache = torch.randint(-127, 128, (2, blocks, bs, Hkv, D), generator=g).to(torch.int8).to(dev)
+        sc = (torch.rand(2, blocks, Hkv, bs, generator=g) * 0.02 + 0.005).to(dev)
+        kw.update(k_scale=sc[0], v_scale=sc[1])
+    elif kv == "fp8":
+        cache = torch.randn(2, blocks, bs, Hkv, D, generator=g).to(torch.float8_e4m3fn).to(dev)
+        kw.update(fp8_scales=(0.5, 2.0))
+    else:
+        cache = torch.randn(2, blocks, bs, Hkv, D, generator=g).bfloat16().to(dev)
+    meta = torch.randn(2, 37, Hkv, D, generator=g).bfloat16().to(dev)
+    kw.update(meta_k=meta[0], meta_v=meta[1], softcap=20.0, alibi_slopes=torch.linspace(0.01, 0.3, Hkv * G, device=dev))
+    run = lambda parts: sb.ops.swa_prefill_attention(q, cache[0], cache[1], query_lens=[n], seq_lens_k=[L], block_table=table,
+                                                     window_left=400, return_lse=True, n_parts=parts, **kw)
+    one, lse1 = run(1)
+    for parts in (2, 5):
+        out, lse = run(parts)
+        assert (out.float() - one.float()).norm() <= 5e-3 * one.float().norm()   # both round the same sums to bf16
+        assert (lse - lse1).abs().max() <= 1e-4
+
+
+def test_parted_call_under_capture(sb, dev):
+    g = torch.Generator().manual_seed(9)
+    q = torch.randn(100, 28, D, generator=g).bfloat16().to(dev)
+    k, v = torch.randn(2100, 4, D, generator=g).bfloat16().to(dev), torch.randn(2100, 4, D, generator=g).bfloat16().to(dev)
+    plan, start = sb.ops.PrefillPlan([100], [2100], dev), torch.zeros(1, dtype=torch.int64, device=dev)
+    out = torch.empty_like(q)
+    run = lambda: sb.ops.swa_prefill_attention(q, k, v, plan=plan, kv_start=start, window_left=4096, out=out)
+    run()
+    eager = out.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run()
+    for _ in range(3):
+        out.zero_()
+        torch.randn(1 << 20, device=dev).sum()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
