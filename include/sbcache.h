@@ -27,7 +27,7 @@
 extern "C" {
 #endif
 
-#define SB_ABI_VERSION 3
+#define SB_ABI_VERSION 4
 
 enum sb_dtype { SB_BF16 = 0, SB_F16 = 1, SB_F32 = 2 };
 
@@ -498,6 +498,8 @@ typedef struct sb_swa_prefill_args {
   float softcap;
   const float *alibi_slopes;
   int64_t meta_bias_row0, meta_bias_rows;
+  /* kv_start as 32-bit values (the step metadata's seq_start_loc as it is); read where kv_start is NULL. */
+  const int32_t *kv_start32;
 } sb_swa_prefill_args;
 
 int sb_swa_prefill(const sb_swa_prefill_args *args);

@@ -27,7 +27,7 @@ SB_GLA_PER_HEAD = 4
 SB_GLA_GROUP_PASS = 8
 SB_GLA_ZERO_SKIPPED = 16
 SB_SWA_DECODE_STATIC_SCRATCH_BYTES = 8 << 20
-ABI_VERSION = 3
+ABI_VERSION = 4
 
 _DTYPES = {torch.bfloat16: SB_BF16, torch.float16: SB_F16, torch.float32: SB_F32}
 
@@ -120,6 +120,7 @@ class SwaPrefillArgs(C.Structure):
         ("k_scale_tensor", f32), ("v_scale_tensor", f32),
         ("meta_k", vp), ("meta_v", vp), ("meta_len", i32), ("meta_stride_row", i64), ("meta_stride_head", i64),
         ("softcap", f32), ("alibi_slopes", vp), ("meta_bias_row0", i64), ("meta_bias_rows", i64),
+        ("kv_start32", vp),
     ]
 
 

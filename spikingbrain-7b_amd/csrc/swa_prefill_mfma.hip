@@ -60,6 +60,7 @@ struct PrefillParams {
   int Hkv;
   const int32_t *block_table;
   const int64_t *kv_start;
+  const int32_t *kv_start32;
   const int32_t *key_lo;      // [S] first visible key of each sequence, or null
   const int32_t *cu_q;        // [S+1] first q/out row of each sequence
   const int32_t *seq_lens_k;  // [S] keys of each sequence (context + new tokens)
@@ -279,7 +280,7 @@ void swa_prefill_kernel(const PrefillParams p) {
     const int lrow = (wave * rows_per_wave) % 16 + (lane >> 4);            // row inside the tile, +4 per load
     const uint32_t row_bytes = (uint32_t)p.kv_sr;                          // < 2^24 (host check)
     const uint32_t lane_col = c * (KVQ == SB_KV_NONE ? 16 : 8);
-    const int64_t wg_off = (int64_t)kvh * p.kv_sh + ((!PAGED && p.kv_start) ? p.kv_start[seq] * p.kv_sr : 0);
+    const int64_t wg_off = (int64_t)kvh * p.kv_sh + (PAGED ? 0 : p.kv_start ? p.kv_start[seq] * p.kv_sr : p.kv_start32 ? p.kv_start32[seq] * p.kv_sr : 0);
     const char *const kbase = p.k + wg_off, *const vbase = p.v + wg_off;
     const int32_t *const table_row = PAGED ? p.block_table + (int64_t)seq * p.bt_stride : nullptr;
     auto walk_tile = [&](int x) __attribute__((always_inline)) {  // (past the end of the walk: the last tile again)
@@ -805,7 +806,7 @@ int prefill(const sb_swa_prefill_args *a, int64_t max_keys, int n_parts, float *
   PrefillParams p;
   p.q = (const char *)a->q; p.k = (const char *)a->k; p.v = (const char *)a->v; p.out = (char *)a->out;
   p.lse = a->lse; p.Hq = a->num_q_heads;
-  p.block_table = a->block_table; p.kv_start = a->kv_start; p.key_lo = a->key_lo;
+  p.block_table = a->block_table; p.kv_start = a->kv_start; p.kv_start32 = a->kv_start32; p.key_lo = a->key_lo;
   p.cu_q = a->cu_seqlens_q; p.seq_lens_k = a->seq_lens_k; p.tile_seq = a->tile_seq; p.tile_q0 = a->tile_q0;
   p.G = a->num_q_heads / a->num_kv_heads; p.head_begin = 0;
   p.block_size = a->block_size > 0 ? a->block_size : 16; p.window_left = a->window_left;

@@ -670,9 +670,13 @@ class MetaAttentionImpl:
             k = k.contiguous()
         plan = self._plan_for(meta, q)
         if plan is not None and plan.total_k <= k.shape[0]:
+            start = meta.seq_start_loc
+            if start.dtype == torch.int32 and start.dim() == 1 and start.is_contiguous() and start.numel() > plan.num_seqs:
+                starts = dict(kv_start32=start)
+            else:
+                starts = dict(kv_start=start.to(torch.int64)[:-1].contiguous())
             res = ops.swa_prefill_attention(q, k, v, plan=plan, window_left=window_left, scale=self.scale, out=out,
-                                            kv_start=meta.seq_start_loc.to(torch.int64)[:-1].contiguous(),
-                                            return_lse=return_lse, **meta_kv)
+                                            return_lse=return_lse, **starts, **meta_kv)
             return res[1] if return_lse else None
         row_seq, j, _ = self._rows(meta.query_start_loc, T)
         seq_lens_row = (j + 1).to(torch.int32)

@@ -580,6 +580,7 @@ def swa_prefill_attention(
     alibi_slopes: Optional[torch.Tensor] = None,
     meta_bias: Optional[Tuple[int, int]] = None,
     n_parts: int = 0,
+    kv_start32: Optional[torch.Tensor] = None,
 ):
     """Causal sliding-window attention for q [total_q, Hq, D] packed sequence after sequence.
     softcap / alibi_slopes: as for swa_decode_attention; query j of a sequence sits at key position
@@ -593,6 +594,7 @@ def swa_prefill_attention(
     paged (block_table [S, max_blocks] int32): k/v are the caches [num_blocks, block_size, Hkv, D].
     dense (block_table None): k/v are [rows, Hkv, D]; keys of sequence s start at row kv_start[s]
     (int64 device vector; default: the same packing as q, which needs seq_lens_k == query_lens).
+    kv_start32: the same as an int32 device vector, in place of kv_start.
     With kv_strides = (row, head) in elements (and num_kv_heads), k/v may be any tensors whose
     element offset for (sequence s, key i, head h) is (kv_start[s] + i)*row + h*head.
     key_lo [S] int32: keys below key_lo[s] are invisible (left padding); a query that sees no key
@@ -601,7 +603,7 @@ def swa_prefill_attention(
     kv_append_int8 / kv_append_fp8 wrote them; rows are dequantised on their way into the kernel.
     n_parts: cut the keys of a tile into up to this many parts that run side by side (0 = chosen by the library, 1 =
     not at all)."""
-    dev = N.require_gpu(q, k, v, block_table, kv_start, key_lo, out, k_scale, v_scale)
+    dev = N.require_gpu(q, k, v, block_table, kv_start, kv_start32, key_lo, out, k_scale, v_scale)
     kv_quant = N.SB_KV_NONE
     if fp8_scales is not None:
         if block_table is None or k.dtype not in (torch.float8_e4m3fn, torch.uint8) or v.dtype != k.dtype:
@@ -646,7 +648,7 @@ def swa_prefill_attention(
     else:
         bs, bt_stride = 16, 0
         if kv_strides is not None:
-            if num_kv_heads is None or kv_start is None:
+            if num_kv_heads is None or (kv_start is None and kv_start32 is None):
                 raise ValueError("kv_strides needs num_kv_heads and kv_start")
             Hkv, Dc = num_kv_heads, k.shape[-1]
             strides = (0, int(kv_strides[0]), int(kv_strides[1]))
@@ -655,11 +657,14 @@ def swa_prefill_attention(
                 raise ValueError("dense k/v must be [rows, num_kv_heads, head_size]")
             Hkv, Dc = k.shape[1], k.shape[2]
             strides = (0, k.stride(0), k.stride(1))
-            if kv_start is None:
+            if kv_start is None and kv_start32 is None:
                 if plan.total_k > k.shape[0]:
                     raise ValueError(f"k has {k.shape[0]} rows, the sequences hold {plan.total_k} keys")
-                kv_start = plan.cu_seqlens_q.to(torch.int64)
-        if kv_start.dtype != torch.int64 or not kv_start.is_contiguous() or kv_start.numel() < plan.num_seqs:
+                kv_start32 = plan.cu_seqlens_q
+        if kv_start is None:
+            if kv_start32.dtype != torch.int32 or not kv_start32.is_contiguous() or kv_start32.numel() < plan.num_seqs:
+                raise ValueError("kv_start32 must be a contiguous int32 vector with one entry per sequence")
+        elif kv_start.dtype != torch.int64 or not kv_start.is_contiguous() or kv_start.numel() < plan.num_seqs:
             raise ValueError("kv_start must be a contiguous int64 vector with one entry per sequence")
     if num_kv_heads is not None and num_kv_heads != Hkv:
         raise ValueError(f"num_kv_heads {num_kv_heads} does not match k's {Hkv}")
@@ -707,7 +712,8 @@ def swa_prefill_attention(
         v_scale_tensor=float(fp8_scales[1]) if fp8_scales is not None else 0.0,
         softcap=float(softcap), alibi_slopes=N.ptr(_slopes(alibi_slopes, Hq, dev)),
         meta_bias_row0=int(meta_bias[0]) if meta_bias else 0,
-        meta_bias_rows=int(meta_bias[1]) if meta_bias else int(q.shape[0]), **meta)
+        meta_bias_rows=int(meta_bias[1]) if meta_bias else int(q.shape[0]),
+        kv_start32=N.ptr(kv_start32) if block_table is None else None, **meta)
     L = N.lib()
     if n_parts == 0:
         n_parts = L.sb_swa_prefill_parts(C.byref(a), plan.max_k)

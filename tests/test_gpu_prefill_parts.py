@@ -47,6 +47,19 @@ def test_parts_and_pairs(sb, dev, G, lens, ctx, window, n_parts):
     assert (lse[ok] - lse1[ok]).abs().max() <= 1e-4
 
 
+def test_starts_as_32_bit_values(sb, dev):
+    g = torch.Generator().manual_seed(2)
+    lens = [70, 5, 130]
+    q, k, v = (torch.randn(sum(lens), h, D, generator=g).bfloat16().to(dev) for h in (4, 2, 2))
+    starts = torch.tensor([0] + lens).cumsum(0)
+    run = lambda **kw: sb.ops.swa_prefill_attention(q, k, v, query_lens=lens, window_left=64, **kw)
+    a = run(kv_start=starts[:-1].contiguous().to(dev))
+    assert torch.equal(a, run(kv_start32=starts.int().to(dev))) and torch.equal(a, run())
+    for bad in (starts.to(dev), starts[:2].int().to(dev)):
+        with pytest.raises(ValueError):
+            run(kv_start32=bad)
+
+
 @pytest.mark.parametrize("kv", ["bf16", "int8", "fp8"])
 def test_paged_parts_with_meta_rows_and_options(sb, dev, kv):
     """The parts over a paged cache (element and byte codes), with meta rows (walked by the first part) and score options."""
