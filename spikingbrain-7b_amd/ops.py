@@ -34,29 +34,29 @@ def _capture_id(stream: int) -> int:
 _COUNTER_BYTES = 64 << 10   # arrival counters of the in-kernel merge at the head of a workspace: zero between launches
 
 
-def _new_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
-    ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=dev)
-    ws[:_COUNTER_BYTES].zero_()   # only the counters need a known start; partials are written before they are read
-    return ws
-
-
-def _workspace(dev: torch.device, nbytes: int) -> Optional[torch.Tensor]:
+def _workspace(dev: torch.device, nbytes: int, counters: bool = False) -> Optional[torch.Tensor]:
+    """counters: the call uses the arrival counters (they need a known start; partials are written before they are read)."""
     if nbytes == 0:
         return None
     stream = N.stream_ptr(dev)
     cap = _capture_id(stream)
     if cap:
-        # (allocated inside the capture: the 64 KiB counter fill becomes a node of the graph and runs at every
-        # replay, which is harmless: the counters are zero between launches anyway)
         owned = _graph_workspaces.setdefault((dev, cap), [])
         if not owned or owned[-1].numel() < nbytes:
             # (a smaller buffer handed out earlier in this capture stays in the list: earlier nodes use it)
-            owned.append(_new_workspace(dev, nbytes))
-        return owned[-1]
+            owned.append(torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=dev))
+        ws = owned[-1]
+        if counters and not getattr(ws, "sb_counters_cleared", False):
+            # (a node of the graph, 4.5 us at every replay, and harmless there: the counters are zero between launches;
+            # captures that never merge inside the kernel go without)
+            ws[:_COUNTER_BYTES].zero_()
+            ws.sb_counters_cleared = True
+        return ws
     key = (dev, stream)
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
-        ws = _new_workspace(dev, nbytes)
+        ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=dev)
+        ws[:_COUNTER_BYTES].zero_()
         _workspaces[key] = ws
     return ws
 
@@ -325,7 +325,7 @@ def swa_decode_attention(
     if balanced and can_balance and n_split < 2:
         n_split = 2  # the balanced split always goes through partial results and the merge
     ws_bytes = L.sb_swa_decode_workspace_bytes(R, Hq, D, n_split)
-    ws = _workspace(dev, ws_bytes)
+    ws = _workspace(dev, ws_bytes, merge_in_kernel)
     q_strides, out_strides = q.stride(), out.stride()
     a = N.SwaDecodeArgs(
         q=N.ptr(q), k_cache=N.ptr(key_cache), v_cache=N.ptr(value_cache), out=N.ptr(out), lse=N.ptr(lse),
