@@ -595,6 +595,18 @@ int sb_kv_append_fp8(const sb_kv_append_fp8_args *args);
 int sb_fp8_round(const void *in, void *out, int64_t rows, int64_t row_elems, int64_t in_stride_row,
                  int64_t out_stride_row, int32_t dtype, float scale, void *stream);
 
+/* A step's append (or NULL) and up to three round trips, on `stream` (the append's own stream field is not read): one
+ * launch where all tensors are of one type, else one each. Outputs must not overlap other inputs of the call. */
+typedef struct sb_fp8_round_args {
+  const void *in;
+  void *out;
+  int64_t rows, row_elems, in_stride_row, out_stride_row;
+  int32_t dtype;
+  float scale;
+} sb_fp8_round_args;
+
+int sb_fp8_step(const sb_kv_append_fp8_args *append, const sb_fp8_round_args *rounds, int32_t n_rounds, void *stream);
+
 /* ------------------------------------------------------------------------------------
  * Merge of two attention results over disjoint key sets by their log-sum-exps, in place:
  *   lse' = lse - logsigmoid(lse - block_lse)

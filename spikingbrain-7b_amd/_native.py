@@ -158,6 +158,11 @@ class KvAppendFp8Args(C.Structure):
     ]
 
 
+class Fp8RoundArgs(C.Structure):
+    _fields_ = [("in_", vp), ("out", vp), ("rows", i64), ("row_elems", i64), ("in_stride_row", i64), ("out_stride_row", i64),
+                ("dtype", i32), ("scale", f32)]
+
+
 class QuantizeSymArgs(C.Structure):
     _fields_ = [
         ("in_", vp), ("out", vp), ("rows", i64), ("heads", i32), ("head_size", i32), ("dtype", i32),
@@ -205,6 +210,7 @@ EXPORTS = {
     "sb_quantize_sym": (C.c_int, [C.POINTER(QuantizeSymArgs)]),
     "sb_kv_append_fp8": (C.c_int, [C.POINTER(KvAppendFp8Args)]),
     "sb_fp8_round": (C.c_int, [vp, vp, i64, i64, i64, i64, i32, f32, vp]),
+    "sb_fp8_step": (C.c_int, [C.POINTER(KvAppendFp8Args), C.POINTER(Fp8RoundArgs), i32, vp]),
     "sb_stream_copy": (C.c_int, [vp, vp, i64, vp]),
     "sb_stream_capture_id": (C.c_int, [vp, C.POINTER(C.c_uint64)]),
 }

@@ -143,52 +143,95 @@ __device__ __forceinline__ uint32_t to_fp8x4(float a, float b, float c, float d,
   return (uint32_t)r;
 }
 
+struct Fp8Append {
+  const char *key, *value;
+  char *k_cache, *v_cache;
+  const int64_t *slot_mapping;
+  int64_t num_tokens;
+  int num_kv_heads, block_size;
+  int64_t key_tok_b, key_head_b, val_tok_b, val_head_b, blk_b, row_b, head_b;
+  float k_scale, v_scale;
+};
+
+// one wavefront: four heads (16 lanes each) of one token's K (which = 0) or V row
 template <int DT>
-__global__ __launch_bounds__(256) void kv_append_fp8_kernel(
-    const char *__restrict__ key, const char *__restrict__ value, char *__restrict__ k_cache,
-    char *__restrict__ v_cache, const int64_t *__restrict__ slot_mapping, int64_t num_tokens, int num_kv_heads,
-    int block_size, int64_t key_tok_b, int64_t key_head_b, int64_t val_tok_b, int64_t val_head_b, int64_t blk_b,
-    int64_t row_b, int64_t head_b, float k_scale, float v_scale) {
-  const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const int lane = threadIdx.x & 63;
-  const int64_t tok = wave >> 1;
-  const int which = (int)(wave & 1);
-  if (tok >= num_tokens) return;
-  const int64_t slot = slot_mapping[tok];
+__device__ __forceinline__ void append_fp8(const Fp8Append &p, int64_t tok, int which, int head0, int lane) {
+  const int64_t slot = p.slot_mapping[tok];
   if (slot < 0) return;
-  const int64_t blk = slot / block_size;
-  const int off = (int)(slot - blk * block_size);
-  const int h = blockIdx.y * 4 + (lane >> 4);
+  const int64_t blk = slot / p.block_size;
+  const int off = (int)(slot - blk * p.block_size);
+  const int h = head0 + (lane >> 4);
   const int piece = lane & 15;
-  if (h >= num_kv_heads) return;
+  if (h >= p.num_kv_heads) return;
   constexpr int kEsz = DT == SB_F32 ? 4 : 2;
   float x[8];
-  const char *src = which ? value + tok * val_tok_b + h * val_head_b : key + tok * key_tok_b + h * key_head_b;
+  const char *src = which ? p.value + tok * p.val_tok_b + h * p.val_head_b : p.key + tok * p.key_tok_b + h * p.key_head_b;
   load8<DT>(src + piece * 8 * kEsz, x);
-  const float sc = which ? v_scale : k_scale;
-  char *dst = (which ? v_cache : k_cache) + blk * blk_b + off * row_b + h * head_b + piece * 8;
+  const float sc = which ? p.v_scale : p.k_scale;
+  char *dst = (which ? p.v_cache : p.k_cache) + blk * p.blk_b + off * p.row_b + h * p.head_b + piece * 8;
   *reinterpret_cast<uint2 *>(dst) = make_uint2(to_fp8x4(x[0], x[1], x[2], x[3], sc), to_fp8x4(x[4], x[5], x[6], x[7], sc));
+}
+
+// The append alone (a captured decode step of 28 layers over an fp8 cache: through the kernel below, with its 300 bytes of
+// arguments, the step took 319 instead of 315 us).
+template <int DT>
+__global__ __launch_bounds__(256) void kv_append_fp8_kernel(const Fp8Append p) {
+  const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  if ((wave >> 1) >= p.num_tokens) return;
+  append_fp8<DT>(p, wave >> 1, (int)(wave & 1), blockIdx.y * 4, threadIdx.x & 63);
 }
 
 // y = e4m3fn(clamp(x / scale)) * scale rounded to the tensor's dtype: what a tensor looks like after a
 // round trip through the fp8 cache (or through scaled_fp8_quant, meta_attention.py:806-811, :853-869).
+struct Fp8Round {
+  const char *in;
+  char *out;
+  int64_t rows, in_row_b, out_row_b;
+  int row_vecs;
+  float scale;
+};
 template <int DT>
-__global__ __launch_bounds__(256) void fp8_round_kernel(const char *__restrict__ in, char *__restrict__ out,
-                                                        int64_t rows, int64_t in_row_b, int64_t out_row_b, int row_vecs,
-                                                        float scale) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t r = t / row_vecs;
-  if (r >= rows) return;
-  const int vec = (int)(t - r * row_vecs);
+__device__ __forceinline__ void round_fp8(const Fp8Round &p, int64_t t) {  // t: 8-element vector of the tensor
+  const int64_t r = t / p.row_vecs;
+  if (r >= p.rows) return;
+  const int vec = (int)(t - r * p.row_vecs);
   constexpr int kEsz = DT == SB_F32 ? 4 : 2;
+  const float scale = p.scale;
   float x[8];
-  load8<DT>(in + r * in_row_b + vec * 8 * kEsz, x);
+  load8<DT>(p.in + r * p.in_row_b + vec * 8 * kEsz, x);
   const uint32_t lo = to_fp8x4(x[0], x[1], x[2], x[3], scale), hi = to_fp8x4(x[4], x[5], x[6], x[7], scale);
   const float y[8] = {__builtin_amdgcn_cvt_f32_fp8((int)lo, 0) * scale, __builtin_amdgcn_cvt_f32_fp8((int)lo, 1) * scale,
                       __builtin_amdgcn_cvt_f32_fp8((int)lo, 2) * scale, __builtin_amdgcn_cvt_f32_fp8((int)lo, 3) * scale,
                       __builtin_amdgcn_cvt_f32_fp8((int)hi, 0) * scale, __builtin_amdgcn_cvt_f32_fp8((int)hi, 1) * scale,
                       __builtin_amdgcn_cvt_f32_fp8((int)hi, 2) * scale, __builtin_amdgcn_cvt_f32_fp8((int)hi, 3) * scale};
-  store8<DT>(out + r * out_row_b + vec * 8 * kEsz, y);
+  store8<DT>(p.out + r * p.out_row_b + vec * 8 * kEsz, y);
+}
+
+// What a step over an fp8 cache does in front of its attention, in one launch: the append and the round trips of the
+// queries and (prompts) of the keys and values attended to in flight. Workgroups [0, first[0]) append, those
+// from first[j] on round tensor j. The pieces touch different memory. As launches of their own they cost 4 to 5 us each.
+constexpr int kMaxRounds = 3;
+struct Fp8Step {
+  Fp8Append append;
+  Fp8Round round[kMaxRounds];
+  int64_t first[kMaxRounds];
+};
+template <int DT>
+__global__ __launch_bounds__(256) void fp8_step_kernel(const Fp8Step p) {
+  const int64_t b = blockIdx.x;
+  if (b < p.first[0]) {
+    const int64_t wave = b * 4 + (threadIdx.x >> 6);
+    const int groups = (p.append.num_kv_heads + 3) >> 2;
+    const int64_t tok = (wave >> 1) / groups;
+    if (tok >= p.append.num_tokens) return;
+    append_fp8<DT>(p.append, tok, (int)(wave & 1), 4 * (int)((wave >> 1) - tok * groups), threadIdx.x & 63);
+  } else if (b < p.first[1]) {
+    round_fp8<DT>(p.round[0], (b - p.first[0]) * 256 + threadIdx.x);
+  } else if (b < p.first[2]) {
+    round_fp8<DT>(p.round[1], (b - p.first[1]) * 256 + threadIdx.x);
+  } else {
+    round_fp8<DT>(p.round[2], (b - p.first[2]) * 256 + threadIdx.x);
+  }
 }
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -271,7 +314,9 @@ extern "C" int sb_quantize_sym(const sb_quantize_sym_args *a) {
   return check_launch("quantize_sym_kernel");
 }
 
-extern "C" int sb_kv_append_fp8(const sb_kv_append_fp8_args *a) {
+namespace {
+
+int check_append(const sb_kv_append_fp8_args *a) {
   using namespace sb_host;
   if (!a) return fail(SB_ERR_INVALID, "sb_kv_append_fp8: null args");
   if (a->num_tokens < 0) return fail(SB_ERR_INVALID, "sb_kv_append_fp8: negative num_tokens");
@@ -293,43 +338,92 @@ extern "C" int sb_kv_append_fp8(const sb_kv_append_fp8_args *a) {
     if (s % 8 != 0) return fail(SB_ERR_INVALID, "sb_kv_append_fp8: cache stride %lld is not 8-byte aligned", (long long)s);
   if (!aligned16(a->key) || !aligned16(a->value) || !aligned16(a->k_cache) || !aligned16(a->v_cache))
     return fail(SB_ERR_INVALID, "sb_kv_append_fp8: tensor base not 16-byte aligned");
-  const int64_t blocks = (a->num_tokens * 2 + 3) / 4;
-  if (blocks > 0x7fffffffLL) return fail(SB_ERR_UNSUPPORTED, "sb_kv_append_fp8: too many tokens");
-  const dim3 grid((unsigned)blocks, (unsigned)((a->num_kv_heads + 3) / 4));
-#define SB_ARGS                                                                                                \
-  (const char *)a->key, (const char *)a->value, (char *)a->k_cache, (char *)a->v_cache, a->slot_mapping,         \
-      a->num_tokens, a->num_kv_heads, a->block_size, a->key_stride_token *esz, a->key_stride_head *esz,          \
-      a->value_stride_token *esz, a->value_stride_head *esz, a->cache_stride_block, a->cache_stride_row,         \
-      a->cache_stride_head, a->k_scale, a->v_scale
-  hipStream_t st = (hipStream_t)a->stream;
-  if (a->dtype == SB_BF16) hipLaunchKernelGGL(kv_append_fp8_kernel<SB_BF16>, grid, dim3(256), 0, st, SB_ARGS);
-  else if (a->dtype == SB_F16) hipLaunchKernelGGL(kv_append_fp8_kernel<SB_F16>, grid, dim3(256), 0, st, SB_ARGS);
-  else hipLaunchKernelGGL(kv_append_fp8_kernel<SB_F32>, grid, dim3(256), 0, st, SB_ARGS);
-#undef SB_ARGS
-  return check_launch("kv_append_fp8_kernel");
+  if (a->num_tokens > 0x7fffffffLL) return fail(SB_ERR_UNSUPPORTED, "sb_kv_append_fp8: too many tokens");
+  return SB_OK;
+}
+
+int check_round(const sb_fp8_round_args *a) {
+  using namespace sb_host;
+  if (a->rows < 0 || a->row_elems < 0) return fail(SB_ERR_INVALID, "sb_fp8_round: negative size");
+  if (a->rows == 0 || a->row_elems == 0) return SB_OK;
+  if (!a->in || !a->out) return fail(SB_ERR_INVALID, "sb_fp8_round: null tensor pointer");
+  const int esz = elem_size(a->dtype);
+  if (!esz) return fail(SB_ERR_UNSUPPORTED, "sb_fp8_round: unknown dtype %d", a->dtype);
+  if (a->row_elems % 8 != 0 || (a->in_stride_row * esz) % 16 != 0 || (a->out_stride_row * esz) % 16 != 0 ||
+      !aligned16(a->in) || !aligned16(a->out))
+    return fail(SB_ERR_INVALID, "sb_fp8_round: rows must be whole 8-element vectors at 16-byte aligned addresses");
+  if (!(a->scale > 0.f)) return fail(SB_ERR_INVALID, "sb_fp8_round: scale must be positive");
+  return SB_OK;
+}
+
+// (a: checked, or null; r: n checked tensors, all of `dtype`)
+int launch_fp8_step(const sb_kv_append_fp8_args *a, const sb_fp8_round_args *r, int n, int dtype, hipStream_t st) {
+  using namespace sb_host;
+  const int esz = elem_size(dtype);
+  Fp8Step p = {};
+  int64_t blocks = 0;
+  if (a && a->num_tokens > 0) {
+    p.append = Fp8Append{(const char *)a->key, (const char *)a->value, (char *)a->k_cache, (char *)a->v_cache, a->slot_mapping,
+                         a->num_tokens, a->num_kv_heads, a->block_size, a->key_stride_token * esz, a->key_stride_head * esz,
+                         a->value_stride_token * esz, a->value_stride_head * esz, a->cache_stride_block, a->cache_stride_row,
+                         a->cache_stride_head, a->k_scale, a->v_scale};
+    blocks = (a->num_tokens * 2 * ((a->num_kv_heads + 3) / 4) + 3) / 4;
+    if (n == 0) {
+      const dim3 agrid((unsigned)((a->num_tokens * 2 + 3) / 4), (unsigned)((a->num_kv_heads + 3) / 4));
+      if (dtype == SB_BF16) hipLaunchKernelGGL(kv_append_fp8_kernel<SB_BF16>, agrid, dim3(256), 0, st, p.append);
+      else if (dtype == SB_F16) hipLaunchKernelGGL(kv_append_fp8_kernel<SB_F16>, agrid, dim3(256), 0, st, p.append);
+      else hipLaunchKernelGGL(kv_append_fp8_kernel<SB_F32>, agrid, dim3(256), 0, st, p.append);
+      return check_launch("kv_append_fp8_kernel");
+    }
+  }
+  for (int j = 0; j < kMaxRounds; ++j) {
+    p.first[j] = blocks;
+    if (j >= n || r[j].rows == 0 || r[j].row_elems == 0) continue;
+    p.round[j] = Fp8Round{(const char *)r[j].in, (char *)r[j].out, r[j].rows, r[j].in_stride_row * esz, r[j].out_stride_row * esz,
+                          (int)(r[j].row_elems / 8), r[j].scale};
+    blocks += (r[j].rows * (r[j].row_elems / 8) + 255) / 256;
+  }
+  if (blocks == 0) return SB_OK;
+  if (blocks > 0x7fffffffLL) return fail(SB_ERR_UNSUPPORTED, "sb_fp8_step: too many rows");
+  const dim3 grid((unsigned)blocks);
+  if (dtype == SB_BF16) hipLaunchKernelGGL(fp8_step_kernel<SB_BF16>, grid, dim3(256), 0, st, p);
+  else if (dtype == SB_F16) hipLaunchKernelGGL(fp8_step_kernel<SB_F16>, grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL(fp8_step_kernel<SB_F32>, grid, dim3(256), 0, st, p);
+  return check_launch("fp8_step_kernel");
+}
+
+}  // namespace
+
+extern "C" int sb_kv_append_fp8(const sb_kv_append_fp8_args *a) {
+  const int rc = check_append(a);
+  return rc != SB_OK ? rc : launch_fp8_step(a, nullptr, 0, a->dtype, (hipStream_t)a->stream);
 }
 
 extern "C" int sb_fp8_round(const void *in, void *out, int64_t rows, int64_t row_elems, int64_t in_stride_row,
                             int64_t out_stride_row, int32_t dtype, float scale, void *stream) {
+  const sb_fp8_round_args r = {in, out, rows, row_elems, in_stride_row, out_stride_row, dtype, scale};
+  const int rc = check_round(&r);
+  return rc != SB_OK ? rc : launch_fp8_step(nullptr, &r, 1, dtype, (hipStream_t)stream);
+}
+
+extern "C" int sb_fp8_step(const sb_kv_append_fp8_args *append, const sb_fp8_round_args *rounds, int32_t n_rounds,
+                           void *stream) {
   using namespace sb_host;
-  if (rows < 0 || row_elems < 0) return fail(SB_ERR_INVALID, "sb_fp8_round: negative size");
-  if (rows == 0 || row_elems == 0) return SB_OK;
-  if (!in || !out) return fail(SB_ERR_INVALID, "sb_fp8_round: null tensor pointer");
-  const int esz = elem_size(dtype);
-  if (!esz) return fail(SB_ERR_UNSUPPORTED, "sb_fp8_round: unknown dtype %d", dtype);
-  if (row_elems % 8 != 0 || (in_stride_row * esz) % 16 != 0 || (out_stride_row * esz) % 16 != 0 || !aligned16(in) ||
-      !aligned16(out))
-    return fail(SB_ERR_INVALID, "sb_fp8_round: rows must be whole 8-element vectors at 16-byte aligned addresses");
-  if (!(scale > 0.f)) return fail(SB_ERR_INVALID, "sb_fp8_round: scale must be positive");
-  const int row_vecs = (int)(row_elems / 8);
-  const int64_t blocks = (rows * row_vecs + 255) / 256;
-  if (blocks > 0x7fffffffLL) return fail(SB_ERR_UNSUPPORTED, "sb_fp8_round: too many rows");
-  const dim3 grid((unsigned)blocks);
-  hipStream_t st = (hipStream_t)stream;
-#define SB_ARGS (const char *)in, (char *)out, rows, in_stride_row *esz, out_stride_row *esz, row_vecs, scale
-  if (dtype == SB_BF16) hipLaunchKernelGGL(fp8_round_kernel<SB_BF16>, grid, dim3(256), 0, st, SB_ARGS);
-  else if (dtype == SB_F16) hipLaunchKernelGGL(fp8_round_kernel<SB_F16>, grid, dim3(256), 0, st, SB_ARGS);
-  else hipLaunchKernelGGL(fp8_round_kernel<SB_F32>, grid, dim3(256), 0, st, SB_ARGS);
-#undef SB_ARGS
-  return check_launch("fp8_round_kernel");
+  if (n_rounds < 0 || n_rounds > kMaxRounds || (n_rounds > 0 && !rounds))
+    return fail(SB_ERR_INVALID, "sb_fp8_step: 0 to %d tensors to round", kMaxRounds);
+  if (!append && n_rounds == 0) return SB_OK;
+  if (append)
+    if (int rc = check_append(append)) return rc;
+  const int dtype = append ? append->dtype : rounds[0].dtype;
+  bool same = true;
+  for (int j = 0; j < n_rounds; ++j) {
+    if (int rc = check_round(&rounds[j])) return rc;
+    same = same && rounds[j].dtype == dtype;
+  }
+  if (!same) {  // tensors of several types: a launch each
+    for (int j = 0; j < n_rounds; ++j)
+      if (int rc = launch_fp8_step(nullptr, &rounds[j], 1, rounds[j].dtype, (hipStream_t)stream)) return rc;
+    return append ? launch_fp8_step(append, nullptr, 0, dtype, (hipStream_t)stream) : SB_OK;
+  }
+  return launch_fp8_step(append, rounds, n_rounds, dtype, (hipStream_t)stream);
 }

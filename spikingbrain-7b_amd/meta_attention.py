@@ -391,6 +391,11 @@ def _rows_of(t: torch.Tensor, start: int, stop: int) -> torch.Tensor:
     return t if start == 0 and stop >= t.shape[0] else t[start:stop]
 
 
+def _in_flight(kv_cache, prompts) -> bool:
+    """Whether a step's prompts attend to the step's own keys and values instead of the paged cache."""
+    return kv_cache.numel() == 0 or prompts.block_tables is None or prompts.block_tables.numel() == 0
+
+
 def _flat(t: torch.Tensor) -> torch.Tensor:
     """t.flatten()."""
     return t if t.dim() == 1 else t.flatten()
@@ -522,8 +527,10 @@ class MetaAttentionImpl:
             if int8_kv:
                 raise ValueError("kv_cache_dtype says fp8 but the cache is an Int8KVCache")
             scales = dict(fp8_scales=(k_scale_f, v_scale_f))
-            # queries take the fp8 round trip as well (scaled_fp8_quant with layer._q_scale, :806-811)
-            query = ops.fp8_round(query.contiguous(), float(getattr(layer, "_q_scale_float", 1.0)))
+            # queries take the fp8 round trip as well (scaled_fp8_quant with layer._q_scale, :806-811), and so do keys and
+            # values that a prompt attends to in flight (:853-869); with the append in one launch, below
+            rounds = [(query.contiguous(), float(getattr(layer, "_q_scale_float", 1.0)))]
+            append = None
         byte_kv = int8_kv or fp8_kv
         fuse_append = (kv_cache.numel() > 0 and key is not None and value is not None and not byte_kv
                        and attn_metadata.num_prefill_tokens == 0 and attn_metadata.num_decode_tokens > 0
@@ -535,8 +542,7 @@ class MetaAttentionImpl:
             if fp8_kv and key_cache.dtype not in (torch.uint8, torch.float8_e4m3fn):
                 raise ValueError(f"an fp8 kv-cache must be a uint8 or float8_e4m3fn tensor, got {key_cache.dtype}")
             if key is not None and value is not None and fp8_kv:
-                ops.kv_append_fp8(key, value, key_cache, value_cache, _flat(attn_metadata.slot_mapping),
-                                  k_scale_f, v_scale_f)
+                append = (key, value, key_cache, value_cache, _flat(attn_metadata.slot_mapping), k_scale_f, v_scale_f)
             elif key is not None and value is not None and int8_kv:
                 # rows are quantised on their way in: 128 code bytes + one scale per (token, kv head)
                 ops.kv_append_int8(key, value, key_cache, value_cache, scales["k_scale"], scales["v_scale"],
@@ -547,6 +553,12 @@ class MetaAttentionImpl:
 
         num_prefill_query_tokens = attn_metadata.num_prefill_tokens
         num_decode_query_tokens = attn_metadata.num_decode_tokens
+        if fp8_kv:
+            prompts = attn_metadata.prefill_metadata
+            if prompts and key is not None and _in_flight(kv_cache, prompts):
+                rounds += [(_rows_of(key, 0, num_prefill_query_tokens).contiguous(), k_scale_f),
+                           (_rows_of(value, 0, num_prefill_query_tokens).contiguous(), v_scale_f)]
+            query, *fp8_prompt = ops.fp8_step(append, rounds)
         num_meta_prefill_tokens = num_prefill_query_tokens
         if query2 is not None:
             query2 = query2.view(-1, self.num_heads, self.head_size)
@@ -590,13 +602,14 @@ class MetaAttentionImpl:
         assert decode_query.shape[0] == num_decode_query_tokens
 
         if prefill_meta := attn_metadata.prefill_metadata:
-            if kv_cache.numel() == 0 or prefill_meta.block_tables is None or prefill_meta.block_tables.numel() == 0:
+            if _in_flight(kv_cache, prefill_meta):
                 # plain prompt run: keys and values are the in-flight tensors (:835-884)
-                pk, pv = _rows_of(key, 0, num_prefill_query_tokens), _rows_of(value, 0, num_prefill_query_tokens)
+                if not fp8_kv:
+                    pk, pv = _rows_of(key, 0, num_prefill_query_tokens), _rows_of(value, 0, num_prefill_query_tokens)
                 if int8_kv:   # attend to what the cache will hold: the rows as quantize_sym returns them
                     pk, pv = ops.quantize_sym(pk), ops.quantize_sym(pv)
-                elif fp8_kv:  # scaled_fp8_quant of the prompt's keys and values (:853-869)
-                    pk, pv = ops.fp8_round(pk.contiguous(), k_scale_f), ops.fp8_round(pv.contiguous(), v_scale_f)
+                elif fp8_kv:  # the prompt's keys and values after their round trip
+                    pk, pv = fp8_prompt
                 self._varlen_inflight(query, pk, pv, prefill_meta, prefill_output, window_left, meta_kv=prefill_kv)
             else:
                 # prefix hit / chunked prefill: keys and values come from the paged cache (:885-919)

@@ -420,10 +420,8 @@ def kv_append_int8(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor
     N.check(N.lib().sb_kv_append_int8(C.byref(a)), "kv_append_int8")
 
 
-def kv_append_fp8(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
-                  slot_mapping: torch.Tensor, k_scale: float = 1.0, v_scale: float = 1.0) -> None:
-    """Store this step's K/V rows as fp8 (e4m3fn) codes of x / scale (saturating at +-448) at their slots;
-    slots < 0 are skipped. Caches float8_e4m3fn or uint8 [nb, bs, Hkv, 128]."""
+def _append_fp8_args(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+                     slot_mapping: torch.Tensor, k_scale: float, v_scale: float):
     dev = N.require_gpu(key, value, k_cache, v_cache, slot_mapping)
     if key.dim() != 3 or value.shape != key.shape or value.dtype != key.dtype:
         raise ValueError("key and value must be [tokens, num_kv_heads, head_size] of one dtype")
@@ -438,13 +436,20 @@ def kv_append_fp8(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
     _inner_contiguous(value, "value")
     if slot_mapping.dtype != torch.int64 or not slot_mapping.is_contiguous() or slot_mapping.numel() < T:
         raise ValueError("slot_mapping must be a contiguous int64 vector with one entry per token")
-    a = N.KvAppendFp8Args(
+    return N.KvAppendFp8Args(
         key=N.ptr(key), value=N.ptr(value), k_cache=N.ptr(k_cache), v_cache=N.ptr(v_cache),
         slot_mapping=N.ptr(slot_mapping), num_tokens=T, num_kv_heads=Hkv, head_size=D, block_size=k_cache.shape[1],
         dtype=N.dtype_code(key.dtype), key_stride_token=key.stride(0), key_stride_head=key.stride(1),
         value_stride_token=value.stride(0), value_stride_head=value.stride(1),
         cache_stride_block=k_cache.stride(0), cache_stride_row=k_cache.stride(1), cache_stride_head=k_cache.stride(2),
         k_scale=float(k_scale), v_scale=float(v_scale), stream=N.stream_ptr(dev))
+
+
+def kv_append_fp8(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+                  slot_mapping: torch.Tensor, k_scale: float = 1.0, v_scale: float = 1.0) -> None:
+    """Store this step's K/V rows as fp8 (e4m3fn) codes of x / scale (saturating at +-448) at their slots;
+    slots < 0 are skipped. Caches float8_e4m3fn or uint8 [nb, bs, Hkv, 128]."""
+    a = _append_fp8_args(key, value, k_cache, v_cache, slot_mapping, k_scale, v_scale)
     N.check(N.lib().sb_kv_append_fp8(C.byref(a)), "kv_append_fp8")
 
 
@@ -465,6 +470,25 @@ def fp8_round(x: torch.Tensor, scale: float = 1.0, out: Optional[torch.Tensor] =
     N.check(N.lib().sb_fp8_round(N.ptr(x), N.ptr(out), x2.shape[0], x2.shape[1], x2.stride(0), x2.stride(0),
                                  N.dtype_code(x.dtype), float(scale), N.stream_ptr(dev)), "fp8_round")
     return out
+
+
+def fp8_step(append: Optional[tuple], rounds) -> list:
+    """The append (arguments of kv_append_fp8, or None) and the fp8 round trip of up to three contiguous tensors,
+    rounds = [(x, scale), ...], in one launch where all are of one dtype; returns the rounded tensors."""
+    a = None if append is None else _append_fp8_args(*append)
+    outs = []
+    jobs = (N.Fp8RoundArgs * max(1, len(rounds)))()
+    dev = N.require_gpu(*([x for x, _ in rounds] + ([append[0]] if append else [])))
+    for job, (x, scale) in zip(jobs, rounds):
+        if x.dim() < 1 or x.shape[-1] % 8 != 0 or not x.is_contiguous():
+            raise ValueError("x must be contiguous, with a last dimension that is a multiple of 8")
+        out = torch.empty_like(x)
+        outs.append(out)
+        job.in_, job.out, job.dtype, job.scale = N.ptr(x), N.ptr(out), N.dtype_code(x.dtype), float(scale)
+        job.row_elems = job.in_stride_row = job.out_stride_row = x.shape[-1]
+        job.rows = x.numel() // x.shape[-1] if x.shape[-1] else 0
+    N.check(N.lib().sb_fp8_step(None if a is None else C.byref(a), jobs, len(rounds), N.stream_ptr(dev)), "fp8_step")
+    return outs
 
 
 def quantize_sym(x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
