@@ -355,7 +355,8 @@ int sb_gla_recurrent(const sb_gla_recurrent_args *args);
  * idle otherwise). sb_gla_prompt_segments: how many segments the library would cut this call's longest prompt into
  * (1 = not at all); sb_gla_prompt_workspace_bytes: scratch memory that takes (device, 16-byte aligned, contents
  * irrelevant before and after; calls whose scratch memory overlaps must be ordered); sb_gla_prompt_segmented: the
- * call, cut into at most n_segments pieces. args->seq_len bounds the prompts' lengths as in sb_gla_recurrent. A
+ * call, cut into at most n_segments pieces. args->seq_len bounds the prompts' lengths as in sb_gla_recurrent (what lies
+ * beyond it falls to the last piece). A
  * segment starts from a state that was formed in fp32 from its predecessors' contributions, so results agree with
  * the uncut call within fp32 rounding of the state. n_segments < 2: sb_gla_recurrent. */
 int32_t sb_gla_prompt_segments(const sb_gla_recurrent_args *args);

@@ -145,8 +145,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   bool last_segment = true;
   if constexpr (kSeg) {
     const int64_t t0 = (int64_t)seg * p.seg_tokens;
-    last_segment = T <= t0 + p.seg_tokens;
-    T = (int)min((int64_t)p.seg_tokens, T - t0);
+    // (the last segment there is takes what is left, also of a prompt longer than the call's bound said)
+    last_segment = seg + 1 == p.n_seg || T <= t0 + p.seg_tokens;
+    T = last_segment ? (int)(T - t0) : p.seg_tokens;
     qo += t0 * p.q_st; ko += t0 * p.k_st; vo += t0 * p.v_st; go += t0 * p.g_st; oo += t0 * p.o_st;
   }
   if (T <= 0) return;
@@ -604,7 +605,7 @@ __global__ __launch_bounds__(256) void gla_segment_scan_kernel(const GlaChunkPar
   const int64_t slot = p.slot_idx ? (int64_t)p.slot_idx[b] : (int64_t)b;
   if (slot < 0) return;
   const int T = p.cu ? p.cu[b + 1] - p.cu[b] : p.T;
-  const int n = (T + p.seg_tokens - 1) / p.seg_tokens;   // segments of this prompt
+  const int n = min((T + p.seg_tokens - 1) / p.seg_tokens, p.n_seg);   // segments of this prompt
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, c = lane & 15;
   const int rt = blockIdx.y >> 1, nt = blockIdx.y & 1;
   const int row = 32 * (rt >> 1) + 8 * g + 4 * (rt & 1);
@@ -673,8 +674,9 @@ __global__ __launch_bounds__(256) void gla_chunk_group_kernel(const GlaChunkPara
   bool last_segment = true;
   if constexpr (kSeg) {
     const int64_t t0 = (int64_t)seg * p.seg_tokens;
-    last_segment = T <= t0 + p.seg_tokens;
-    T = (int)min((int64_t)p.seg_tokens, T - t0);
+    // (the last segment there is takes what is left, also of a prompt longer than the call's bound said)
+    last_segment = seg + 1 == p.n_seg || T <= t0 + p.seg_tokens;
+    T = last_segment ? (int)(T - t0) : p.seg_tokens;
     qo += t0 * p.q_st; ko += t0 * p.k_st; vo += t0 * p.v_st; go += t0 * p.g_st; oo += t0 * p.o_st;
   }
   if (T <= 0) return;

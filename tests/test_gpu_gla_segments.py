@@ -91,3 +91,22 @@ def test_batched_prompt_cut_into_segments(sb, dev, cuts, H, Hk):
     assert np.abs(s.double().cpu().numpy() - ref_s[:, ::n]).max() <= 1e-4 * np.abs(ref_s).max()
     got = o.float().cpu().numpy()
     assert (np.abs(got - ref_o) <= 2e-2 + 2.0 ** -8 * np.abs(ref_o) + 2.0 ** -9 * np.abs(ref_o).max()).all()
+
+
+@pytest.mark.parametrize("H,Hk", [(2, 2), (8, 2)])
+def test_prompt_longer_than_the_stated_bound(sb, dev, cuts, H, Hk):
+    """The bound only sizes the cut: the last segment takes what is left, and nothing outside the workspace is touched."""
+    lens = [900, 40]
+    g = torch.Generator().manual_seed(1)
+    q = torch.randn(sum(lens), H, D, generator=g).bfloat16().relu().to(dev)
+    k, v = (torch.randn(sum(lens), Hk, D, generator=g).bfloat16().relu().to(dev) for _ in range(2))
+    gate = (F.logsigmoid(torch.randn(sum(lens), Hk, D, generator=g)) / 16).to(dev)
+    state = (torch.randn(2, Hk, D, D, generator=g) * 0.02).to(dev)
+    cu = torch.tensor([0, 900, 940], dtype=torch.int32, device=dev)
+    st, st1 = state.clone(), state.clone()
+    o = sb.ops.gla_recurrent_packed(q, k, v, gate, st, cu, None, max_seq_len=512)
+    o1 = sb.ops.gla_recurrent_packed(q, k, v, gate, st1, cu, None, max_seq_len=900, per_head=True)
+    assert cuts[0] > 1 and cuts[1] == 1
+    assert (st - st1).abs().max() <= 1e-4 * st1.abs().max()
+    d, ref = (o.float() - o1.float()).abs(), o1.float().abs()
+    assert (d <= 2.0 ** -7 * ref + 2.0 ** -8 * ref.max()).all()      # each rounds the same sums, and its operands, to bf16
