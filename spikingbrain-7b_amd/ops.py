@@ -530,6 +530,7 @@ def plan_decode_split(num_rows: int, num_kv_heads: int, max_seq_len: int, window
     return prefer_balanced_split(host_seq_lens, window_left, n_split)
 
 
+INT32_MAX = 2**31 - 1
 PREFILL_TILE = 64  # query tokens per workgroup of the prefill kernel
 PREFILL_CONTIGUOUS_TILES = 1024  # lists of this many tiles keep sequence order
 
@@ -554,6 +555,8 @@ class PrefillPlan:
             raise ValueError(f"sequence {s}: {lq[s]} queries need at least as many keys, got {lk[s]}")
         S = len(query_lens)
         cu = np.concatenate([[0], np.cumsum(lq)])
+        if max(int(cu[-1]), max(seq_lens_k, default=0)) > INT32_MAX:
+            raise RuntimeError("the kernel counts keys and packed query rows in 32 bits: lengths cannot be converted without overflow")
         n = -(-lq // PREFILL_TILE)
         T = int(n.sum())
         tile_seq = np.repeat(np.arange(S), n)
