@@ -1045,8 +1045,8 @@ def dense_rows(batch: int, num_queries: int, num_keys: int, kv_step: int, device
     buf = torch.empty(batch + (3 * R + 1) // 2, dtype=torch.int64, device=device)
     rows = buf[batch:].view(torch.int32)
     kv_start, seq_lens, row_seq, key_lo = buf[:batch], rows[:R], rows[R:2 * R], rows[2 * R:3 * R]
-    a = N.DenseRowsArgs(
-        mask=N.ptr(mask), seq_lens=N.ptr(seq_lens), row_seq=N.ptr(row_seq),
+    a = N.DenseRowsArgs(   # (a mask without columns has no address, and null means no mask: any other pointer, nothing is read)
+        mask=None if mask is None else N.ptr(mask) or N.ptr(buf), seq_lens=N.ptr(seq_lens), row_seq=N.ptr(row_seq),
         key_lo=None if mask is None else N.ptr(key_lo), kv_start=N.ptr(kv_start), batch=batch, num_queries=num_queries,
         num_keys=num_keys, kv_step=kv_step, mask_cols=0 if mask is None else mask.shape[1],
         mask_stride_row=0 if mask is None else mask.stride(0), mask_stride_col=0 if mask is None else mask.stride(1),

@@ -37,6 +37,14 @@ def test_dense_rows_without_mask_and_many_queries(sb, dev):
         sb.ops.dense_rows(2, 1, 4, 0, dev, torch.ones(1, 4, device=dev))
 
 
+def test_mask_without_columns_hides_every_key(sb, dev):
+    """An empty tensor has no address, which is not the same as no mask."""
+    empty = torch.ones(2, 0, dtype=torch.int64, device=dev)
+    assert sb.ops.dense_rows(2, 3, 4, 0, dev, empty)[2].tolist() == [4] * 6
+    q, k = torch.randn(2, 4, 1, 64, device=dev), torch.randn(2, 2, 1, 64, device=dev)
+    assert bool((sb.sliding_window_attention(q, k, k, 8, attention_mask=empty) == 0).all())
+
+
 @pytest.mark.parametrize("v_keep", [5, 3])   # the same rows in both (one launch), and not (two)
 def test_window_shift_pair(sb, dev, v_keep):
     gen = torch.Generator().manual_seed(0)
