@@ -670,9 +670,14 @@ __global__ __launch_bounds__(256) void swa_prefill_merge_kernel(const PrefillPar
     float4 a[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
+      const bool there = s0 + u < parts;   // (past the last part: nothing, not that part again times 0: it may hold an infinity)
       const int s = min(s0 + u, parts - 1);
       x[u] = ml[s];
       a[u] = acc[s * 32];
+      if (!there) {
+        x[u] = make_float2(kNegInf, 0.f);
+        a[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+      }
     }
     float Mn = M;
 #pragma unroll
@@ -683,12 +688,12 @@ __global__ __launch_bounds__(256) void swa_prefill_merge_kernel(const PrefillPar
     L *= keep;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const float f = fast_exp2((s0 + u < parts ? x[u].x : kNegInf) - ref);
+      const float f = fast_exp2(x[u].x - ref);
       tot.x = fmaf(a[u].x, f, tot.x);
       tot.y = fmaf(a[u].y, f, tot.y);
       tot.z = fmaf(a[u].z, f, tot.z);
       tot.w = fmaf(a[u].w, f, tot.w);
-      L = fmaf(x[u].y, f, L);  // (past the last part: the last one again, times 0)
+      L = fmaf(x[u].y, f, L);
     }
     M = Mn;
   }

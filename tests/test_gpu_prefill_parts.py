@@ -108,3 +108,17 @@ def test_parted_call_under_capture(sb, dev):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
+
+
+@pytest.mark.parametrize("parts", [2, 3, 5, 8])
+def test_infinite_value_in_the_last_part(sb, dev, parts):
+    """An infinite value that all queries see makes the output infinite, cut or not: the merge fills the rest of a trip
+    to memory with the last part again, which must not count (infinity times 0 is a NaN)."""
+    g = torch.Generator().manual_seed(parts)
+    n, ctx = 40, 600
+    q, k, v = (torch.randn(m, h, D, generator=g).bfloat16() for m, h in ((n, 4), (n + ctx, 2), (n + ctx, 2)))
+    v[ctx - 5, :, 7] = float("inf")
+    kw = dict(query_lens=[n], seq_lens_k=[n + ctx], kv_start=torch.zeros(1, dtype=torch.int64, device=dev), window_left=-1)
+    whole, cut = (sb.ops.swa_prefill_attention(q.to(dev), k.to(dev), v.to(dev), n_parts=m, **kw).float().cpu() for m in (1, parts))
+    assert torch.isposinf(whole[:, :, 7]).all() and torch.isposinf(cut[:, :, 7]).all()
+    assert torch.equal(torch.isfinite(whole), torch.isfinite(cut))
