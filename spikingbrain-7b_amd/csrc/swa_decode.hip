@@ -413,8 +413,9 @@ __global__ __launch_bounds__(256) void swa_decode_merge_kernel(const DecodeParam
           L *= keep;
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            const float f = (s0 + j >= p.n_split || ms[j0 + j] == kNegInf) ? 0.f : fast_exp2(ms[j0 + j] - Mn);
-            tot = fmaf(av[j0 + j], f, tot);
+            const bool there = s0 + j < p.n_split;  // (else the last one again: it may hold an infinity, which f = 0 does not undo)
+            const float f = (!there || ms[j0 + j] == kNegInf) ? 0.f : fast_exp2(ms[j0 + j] - Mn);
+            tot = fmaf(there ? av[j0 + j] : 0.f, f, tot);
             L = fmaf(ls[j0 + j], f, L);
           }
         }
@@ -495,8 +496,9 @@ __global__ __launch_bounds__(128) void swa_decode_merge_balanced_kernel(const De
         }
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          const float f = (w + j > w_hi || ms[j] == kNegInf) ? 0.f : fast_exp2(ms[j] - M);
-          tot = fmaf(av[j], f, tot);
+          const bool there = w + j <= w_hi;  // as in the merge above
+          const float f = (!there || ms[j] == kNegInf) ? 0.f : fast_exp2(ms[j] - M);
+          tot = fmaf(there ? av[j] : 0.f, f, tot);
           L = fmaf(ls[j], f, L);
         }
       }
@@ -540,8 +542,9 @@ __global__ __launch_bounds__(128) void swa_decode_merge_rows_kernel(const Decode
         L *= keep;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          const float f = (w + j > w_hi || ms[j] == kNegInf) ? 0.f : fast_exp2(ms[j] - Mn);
-          tot = fmaf(av[j], f, tot);
+          const bool there = w + j <= w_hi;  // as in the merge above
+          const float f = (!there || ms[j] == kNegInf) ? 0.f : fast_exp2(ms[j] - Mn);
+          tot = fmaf(there ? av[j] : 0.f, f, tot);
           L = fmaf(ls[j], f, L);
         }
       }

@@ -510,7 +510,8 @@ __device__ __forceinline__ void split_segment(const DecodeParams &p, const int32
         L *= keep;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const float f = (s0 + j >= p.n_split || ms[j] == kNegInf) ? 0.f : fast_exp2(ms[j] - Mn);
+          if (s0 + j >= p.n_split) break;  // (the last one again: it may hold an infinity, which 0 does not undo)
+          const float f = ms[j] == kNegInf ? 0.f : fast_exp2(ms[j] - Mn);
 #pragma unroll
           for (int q4 = 0; q4 < 8; ++q4) {
             tot[4 * q4 + 0] = fmaf(__uint_as_float(av[j][q4].x), f, tot[4 * q4 + 0]);

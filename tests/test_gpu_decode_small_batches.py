@@ -53,3 +53,22 @@ def test_chosen_split_matches_unsplit_rows(sb, dev, rows, length):
     one, auto = (sb.ops.swa_decode_attention(q, kv[0], kv[1], sl, block_table=tables, window_left=1024, n_split=n, balanced=False)
                  for n in (1, 0))
     assert ((auto.float() - one.float()).abs() <= 2 ** -7 * one.float().abs() + 2 ** -9 * one.float().abs().max()).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("how", [dict(n_split=n, balanced=False) for n in (2, 3, 5, 9)] + [
+    dict(n_split=3, merge_in_kernel=True, balanced=False), dict(n_split=3, balanced=True), dict(n_split=3, balanced=True, per_segment=True)])
+def test_infinite_value_in_the_last_partial(sb, dev, dtype, how):
+    """A visible key whose value is infinite makes the output infinite however the row is cut: the merges fill the
+    rest of a trip to memory with the last partial again, which must not count (infinity times 0 is a NaN)."""
+    if dtype == torch.float32 and (how["balanced"] or "merge_in_kernel" in how):
+        pytest.skip("matrix-core kernels only")
+    lens = [320, 320]
+    q, kv, tables, sl = _problem(dev, dtype, lens, 4)
+    kv[1, tables[0, 19], 15, :, 5] = float("inf")     # the newest key of row 0
+    kvd = kv.to(dev)
+    run = lambda **kw: sb.ops.swa_decode_attention(q.to(dev), kvd[0], kvd[1], sl.to(dev), block_table=tables.to(dev),
+                                                   window_left=1024, **kw).float().cpu()
+    whole, cut = run(n_split=1, balanced=False), run(**how)
+    assert torch.isposinf(whole[0, :, 5]).all() and torch.isposinf(cut[0, :, 5]).all()
+    assert torch.equal(torch.isfinite(whole), torch.isfinite(cut))
