@@ -87,6 +87,15 @@ __device__ __forceinline__ float row16_allreduce_sum(float v) {
 // exp2 with the hardware instruction (inputs here are <= 0 or -inf).
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// Block that holds 16-key tile t of a paged sequence: t / tiles_per_block by multiplication with magic =
+// ceil(2^31 / tiles_per_block). The product exceeds the quotient by t * e / (2^31 * tiles_per_block), e = magic * tiles_per_block -
+// 2^31 < tiles_per_block: less than one for every 32-bit t, but enough to reach the next block from t = 2^31 / e on
+// (741 thousand keys in one block of 46410 tiles), hence the correction.
+__device__ __forceinline__ int tile_block(int t, int tiles_per_block, uint32_t magic) {
+  const int b = (int)__umulhi((uint32_t)t << 1, magic);
+  return b - (b * tiles_per_block > t);
+}
+
 // The two score options flash-attn takes from the backend (vllm_hymeta/attention/meta_attention.py:665-690:
 // alibi_slopes, logits_soft_cap). A raw dot product s becomes, in the units the kernels keep their scores in,
 //   (cap * tanh(s * mult / cap) + slope * dist) / mult,     mult = softmax scale (times a cache's K scale),

@@ -115,8 +115,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // Where a chunk's two tiles are: block-table entry and first row inside the block. Looked up one chunk ahead of its
   // loads (the lookup inside them kept every chunk's loads waiting for a table entry, and its block a division; with
   // the edge tests out of the interior chunks and nothing read twice at a run's end: 100 ragged rows 83.5 -> 81.0 us a call).
-  // block of 16-key tile t: t / tiles_per_block by multiplication (exact while t < 2^31 / tiles_per_block)
-  const uint32_t tiles_per_block = (uint32_t)p.block_size >> 4;
+  const int tiles_per_block = p.block_size >> 4;
   const uint32_t tpb_magic = (0x80000000u + tiles_per_block - 1) / tiles_per_block;
   const int32_t *const table_row = p.block_table + seq * p.bt_stride;
   struct Where {
@@ -126,8 +125,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int tile = min(max(2 * cc + t, first_tile), last_tile);  // resident, uniform over the wavefront
-      const int bi = (int)__umulhi((uint32_t)tile << 1, tpb_magic);
-      at.row[t] = (tile - bi * (int)tiles_per_block) << 4;
+      const int bi = tile_block(tile, tiles_per_block, tpb_magic);
+      at.row[t] = (tile - bi * tiles_per_block) << 4;
       at.blk[t] = table_row[bi];
     }
   };

@@ -72,7 +72,7 @@ struct PrefillParams {
   int bucket, head_groups;    // order of an XCD's workgroups (see the kernel)
   int block_size, window_left;
   int tiles_per_block;        // block_size / 16
-  uint32_t tpb_magic;         // ceil(2^31 / tiles_per_block): tile -> block by one multiplication
+  uint32_t tpb_magic;         // ceil(2^31 / tiles_per_block), see tile_block
   float scale_log2;
   int64_t q_sr, q_sh, o_sr, o_sh;  // elements
   int64_t kv_sb, kv_sr, kv_sh;     // bytes
@@ -286,8 +286,7 @@ void swa_prefill_kernel(const PrefillParams p) {
     auto walk_tile = [&](int x) __attribute__((always_inline)) {  // (past the end of the walk: the last tile again)
       return min(max(2 * (ch_begin + x) + tsel, first_tile), last_tile);
     };
-    // block of 16-key tile t: t / tiles_per_block by multiplication (exact while t < 2^31 / tiles_per_block)
-    auto block_of = [&](int t) __attribute__((always_inline)) { return (int)__umulhi((uint32_t)t << 1, p.tpb_magic); };
+    auto block_of = [&](int t) __attribute__((always_inline)) { return tile_block(t, p.tiles_per_block, p.tpb_magic); };
     int next_blk = 0;  // table entry of the tile the next fetch takes
     if constexpr (PAGED) next_blk = table_row[block_of(walk_tile(0))];
     int fx = 0;        // walk index the next fetch takes
