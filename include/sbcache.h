@@ -234,7 +234,9 @@ typedef struct sb_swa_decode_args {
 } sb_swa_decode_args;
 
 /* Split count the auto rule (n_split = 0) would use for these shapes: the one with the lowest estimated
- * duration, counting the rounds in which rows x splits workgroups pass over the CUs (one at a time per CU). */
+ * duration, counting the rounds in which rows x splits workgroups pass over the CUs (one at a time per CU). A call
+ * that leaves the choice to the library takes fewer where the workspace does not hold this many partials, down to runs
+ * of eight 32-key chunks per split; with less memory than that takes, it is rejected with SB_ERR_WORKSPACE. */
 int32_t sb_swa_decode_auto_split(int64_t num_rows, int32_t num_kv_heads, int32_t max_seq_len,
                                  int32_t window_left);
 /* 1 if SB_DECODE_BALANCED is expected to be faster than the fixed split into n_split (>= 1) parts for rows
@@ -257,8 +259,8 @@ int sb_swa_decode(const sb_swa_decode_args *args);
  * `workspace_bytes` are ignored: the split-K partial results live in a device array of
  * SB_SWA_DECODE_STATIC_SCRATCH_BYTES that is part of the library image (every GPU the library runs
  * on holds its own copy from module load until the process ends). A call whose partials need more
- * (sb_swa_decode_workspace_bytes for its rows, heads and split count) is rejected with
- * SB_ERR_WORKSPACE before anything is launched. The call makes no hipMalloc / hipFree and calls no
+ * (sb_swa_decode_workspace_bytes for its rows, heads and split count; n_split = 0 follows the array as it would a
+ * workspace of that size) is rejected with SB_ERR_WORKSPACE before anything is launched. The call makes no hipMalloc / hipFree and calls no
  * allocating routine; the first call on a device looks the array's address up once
  * (hipGetSymbolAddress; make that call outside stream capture, with the device of the tensors
  * current on the calling thread).

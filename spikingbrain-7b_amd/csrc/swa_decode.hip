@@ -666,39 +666,64 @@ static double one_round_us(int64_t wgs, int64_t n, int64_t chunks, int64_t cus) 
 // Windows of at most this many chunks are left whole.
 constexpr int64_t kWholeChunks = 11;
 
-extern "C" int32_t sb_swa_decode_auto_split(int64_t num_rows, int32_t num_kv_heads,
-                                            int32_t max_seq_len, int32_t window_left) {
-  if (num_rows <= 0 || num_kv_heads <= 0 || max_seq_len <= 0) return 1;
+// Workgroups of a launch (per split), and the chunks of a row.
+struct SplitShape {
+  int64_t wgs, chunks, run, cus;
+};
+static SplitShape split_shape(int64_t num_rows, int32_t num_kv_heads, int32_t max_seq_len, int32_t window_left) {
   int64_t keys = max_seq_len;
   if (window_left >= 0 && keys > (int64_t)window_left + 1) keys = (int64_t)window_left + 1;
-  const int64_t chunks = (keys + 31) / 32 + 1;  // +1: an unaligned window touches one more chunk
-  // A split is one workgroup per (row, group of up to 4 kv heads). Where rows x splits takes more than one round
-  // over the CUs: the split count with the lowest estimated duration (just above a multiple of the CU count costs a
-  // whole extra round), leaving every workgroup at least 8 chunks; ties go to more splits (more CUs streaming).
-  const int64_t wgs = num_rows * ((num_kv_heads + 3) / 4);
-  const int64_t cus = device_cu_count();
-  int64_t cap = chunks / 8;
+  SplitShape s;
+  s.chunks = (keys + 31) / 32 + 1;  // +1: an unaligned window touches one more chunk
+  s.run = keys < max_seq_len ? s.chunks : s.chunks - 1;  // (a window that starts at the first key is aligned)
+  s.wgs = num_rows * ((num_kv_heads + 3) / 4);  // one workgroup per (row, group of up to 4 kv heads)
+  s.cus = device_cu_count();
+  return s;
+}
+
+// The split of runs of at least 8 chunks: where rows x splits takes more than one round over the CUs, the split count with
+// the lowest estimated duration (just above a multiple of the CU count costs a whole extra round); ties go to more
+// splits (more CUs streaming).
+static int64_t long_run_split(const SplitShape &s) {
+  int64_t cap = s.chunks / 8;
   if (cap > 64) cap = 64;
   if (cap < 1) cap = 1;
   int64_t best = 1;
-  double best_cost = split_cost(wgs, 1, chunks, cus);
+  double best_cost = split_cost(s.wgs, 1, s.chunks, s.cus);
   for (int64_t n = 2; n <= cap; ++n) {
-    const double c = split_cost(wgs, n, chunks, cus);
+    const double c = split_cost(s.wgs, n, s.chunks, s.cus);
     if (c <= best_cost) { best = n; best_cost = c; }
   }
-  if (wgs * best > cus || chunks <= kWholeChunks) return (int32_t)best;
+  return best;
+}
+
+extern "C" int32_t sb_swa_decode_auto_split(int64_t num_rows, int32_t num_kv_heads,
+                                            int32_t max_seq_len, int32_t window_left) {
+  if (num_rows <= 0 || num_kv_heads <= 0 || max_seq_len <= 0) return 1;
+  const SplitShape s = split_shape(num_rows, num_kv_heads, max_seq_len, window_left);
+  int64_t best = long_run_split(s);
+  if (s.wgs * best > s.cus || s.chunks <= kWholeChunks) return (int32_t)best;
   // One round: the CUs that 8 chunks a workgroup would leave idle are worth more than the partials they add. Measured
   // with 8 chunks or more each -> without that bound (us per call): 1 row x 4097 keys 24.1 -> 17.1 (15 -> 43 splits),
   // 8 x 4097 27.5 -> 22.3 (15 -> 26), 1 x 2000 21.1 -> 12.9 (8 -> 32), 16 x 1000 22.5 -> 14.7 (4 -> 16),
   // 64 x 600 28.3 -> 21.6 (2 -> 4); INT8 8 x 4097 21.3 -> 18.1.
-  const int64_t run = keys < max_seq_len ? chunks : chunks - 1;  // (a window that starts at the first key is aligned)
   best = 1;
-  best_cost = one_round_us(wgs, 1, run, cus);
-  for (int64_t n = 2; n <= 64 && n <= run && wgs * n <= cus; ++n) {
-    const double c = one_round_us(wgs, n, run, cus);
+  double best_cost = one_round_us(s.wgs, 1, s.run, s.cus);
+  for (int64_t n = 2; n <= 64 && n <= s.run && s.wgs * n <= s.cus; ++n) {
+    const double c = one_round_us(s.wgs, n, s.run, s.cus);
     if (c <= best_cost) { best = n; best_cost = c; }
   }
   return (int32_t)best;
+}
+
+// The split of a call that leaves it to the library: what the rule says, with no more partials than `bytes` hold, down
+// to the split of long runs (memory that takes less than that one's partials is refused).
+static int32_t chosen_split(const sb_swa_decode_args *a, size_t bytes) {
+  int32_t n = sb_swa_decode_auto_split(a->num_rows, a->num_kv_heads, a->max_seq_len, a->window_left);
+  if (n < 2 || sb_swa_decode_workspace_bytes(a->num_rows, a->num_q_heads, a->head_size, n) <= bytes) return n;
+  const int64_t least = long_run_split(split_shape(a->num_rows, a->num_kv_heads, a->max_seq_len, a->window_left));
+  while (n > least && sb_swa_decode_workspace_bytes(a->num_rows, a->num_q_heads, a->head_size, n) > bytes) --n;
+  return n;
 }
 
 // Rows up to which the balanced split is used (every wavefront sums over all rows' lengths).
@@ -822,8 +847,7 @@ extern "C" int sb_swa_decode(const sb_swa_decode_args *a) {
 
   int n_split = a->n_split;
   if (n_split < 0) return fail(SB_ERR_INVALID, "sb_swa_decode: negative n_split");
-  if (n_split == 0)
-    n_split = sb_swa_decode_auto_split(a->num_rows, a->num_kv_heads, a->max_seq_len, a->window_left);
+  if (n_split == 0) n_split = chosen_split(a, a->workspace ? a->workspace_bytes : 0);
   if (n_split > 65535) return fail(SB_ERR_UNSUPPORTED, "sb_swa_decode: n_split > 65535");
   const size_t need = sb_swa_decode_workspace_bytes(a->num_rows, a->num_q_heads, a->head_size, n_split);
   if (need > 0 && (!a->workspace || a->workspace_bytes < need))
@@ -1041,12 +1065,7 @@ extern "C" int sb_swa_decode_static(const sb_swa_decode_args *a) {
   if (a->num_rows == 0) return SB_OK;
   int n_split = a->n_split;
   if (n_split < 0) return fail(SB_ERR_INVALID, "sb_swa_decode_static: negative n_split");
-  if (n_split == 0)
-    n_split = sb_swa_decode_auto_split(a->num_rows, a->num_kv_heads, a->max_seq_len, a->window_left);
-  // (chosen here: never more partials than the library's scratch holds)
-  while (a->n_split == 0 && n_split > 1 && sb_swa_decode_workspace_bytes(a->num_rows, a->num_q_heads, a->head_size, n_split) >
-                                               (size_t)SB_SWA_DECODE_STATIC_SCRATCH_BYTES)
-    --n_split;
+  if (n_split == 0) n_split = chosen_split(a, (size_t)SB_SWA_DECODE_STATIC_SCRATCH_BYTES);
   const size_t need = sb_swa_decode_workspace_bytes(a->num_rows, a->num_q_heads, a->head_size, n_split);
   if (need > (size_t)SB_SWA_DECODE_STATIC_SCRATCH_BYTES)
     return fail(SB_ERR_WORKSPACE,

@@ -80,3 +80,26 @@ def test_static_scratch_rejects_oversized_call(sb, dev):
               -1, n_split, 0, None)
     assert L.sb_swa_decode_static(C.byref(a)) == N.SB_ERR_WORKSPACE
     assert "scratch" in N.last_error()
+
+
+@pytest.mark.parametrize("length,fits", [(4097, 15), (4097, 20), (400, 1), (400, 3), (400, 64)])
+def test_chosen_split_follows_the_workspace(sb, dev, length, fits):
+    """n_split = 0: the library never chooses more partials than the caller's workspace holds, down to runs of eight
+    chunks each (15 splits of 4097 keys, 1 of 400); below that the call is refused, as an explicit split is."""
+    N = sb._native
+    L = N.lib()
+    kv, tables = _problem([length], 16, 4, 128, 6)
+    kv, tables = kv.to(dev), tables.to(dev)
+    q = torch.randn(1, 28, 128, generator=torch.Generator().manual_seed(7)).bfloat16().to(dev)
+    lens = torch.tensor([length], dtype=torch.int32, device=dev)
+    need = L.sb_swa_decode_workspace_bytes(1, 28, 128, fits)
+    ws = torch.zeros(need, dtype=torch.uint8, device=dev) if need else None
+    outs = []
+    for n_split, w in ((0, ws), (1, None)):
+        out = torch.full((1, 28, 128), float("nan"), dtype=torch.bfloat16, device=dev)
+        assert L.sb_swa_decode(C.byref(_args(N, q, kv, tables, lens, out, None, 4200, n_split, 0, w))) == 0, N.last_error()
+        outs.append(out.float())
+    assert (outs[0] - outs[1]).abs().max() <= 2 ** -7 * outs[1].abs().max()     # each rounds fp32 results to bf16
+    if length == 4097:
+        small = torch.zeros(L.sb_swa_decode_workspace_bytes(1, 28, 128, 14), dtype=torch.uint8, device=dev)
+        assert L.sb_swa_decode(C.byref(_args(N, q, kv, tables, lens, out, None, 4200, 0, 0, small))) == N.SB_ERR_WORKSPACE
