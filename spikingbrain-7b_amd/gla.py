@@ -101,10 +101,11 @@ def gla_prefill_packed(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gk: to
                        state_indices_tensor: torch.Tensor, query_start_loc: torch.Tensor, num_prefills: int,
                        max_query_len: Optional[int] = None) -> torch.Tensor:
     """The prefill half of `_prefill_and_mix_infer` (vllm_hymeta/model_for_7B/gla_attention.py:179-214)
-    as ONE launch: q, k, v, gk [num_tokens, H, D] with the prefill tokens first; prompt i owns tokens
+    as ONE call: q, k, v, gk [num_tokens, H, D] with the prefill tokens first; prompt i owns tokens
     query_start_loc[i] .. query_start_loc[i+1]-1, starts from the state in kv_cache[slot_i] (the
     runner zeroes the slots of new prompts, `clear_prefill_slots`) and leaves its final state there,
-    with no per-request Python loop, slice copies or state copy. Returns o for the prefill tokens
+    with no per-request Python loop, slice copies or state copy. max_query_len: an upper bound of the prompts'
+    lengths, by which long prompts of a few requests are cut into segments that run side by side. Returns o for the prefill tokens
     [num_prefill_tokens, H, D] (before g_norm)."""
     n = int(num_prefills)
     cu = query_start_loc[:n + 1].to(torch.int32).contiguous()

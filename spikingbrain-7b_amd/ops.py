@@ -909,8 +909,11 @@ def gla_recurrent_packed(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: t
                          check_gates: bool = False, per_head: Optional[bool] = None) -> torch.Tensor:
     """The same recurrence over packed prompts: q, k, v, g [total_tokens, H, D] (token/head strides
     free, contiguous D), sequence b owning tokens cu_seqlens[b] .. cu_seqlens[b+1]-1 (int32 device
-    vector [B+1]); its state is state[slot_idx[b]] (default b), advanced in place. One launch for
-    all sequences. Returns o [total_tokens, H, D]. Shared states as in gla_recurrent: k, v, g
+    vector [B+1]); its state is state[slot_idx[b]] (default b), advanced in place. One call for all
+    sequences; long prompts of a few sequences are cut into segments that run side by side (see gla_recurrent), as
+    max_seq_len, an upper bound of their lengths, says (default: the mean length, which some sequence reaches: eight
+    prompts of 100 tokens are not cut like one of 800, of whose segments the first would hold all there is; what lies
+    beyond falls to a prompt's last segment). Returns o [total_tokens, H, D]. Shared states as in gla_recurrent: k, v, g
     [total_tokens, Hkv, D] with state [slots, Hkv, D, D]."""
     dev = N.require_gpu(q, k, v, g, state, cu_seqlens, slot_idx, out)
     if q.dim() != 3 or k.dim() != 3 or v.shape != k.shape or g.shape != k.shape or \
@@ -942,7 +945,7 @@ def gla_recurrent_packed(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: t
         return out
     a = N.GlaRecurrentArgs(
         q=N.ptr(q), k=N.ptr(k), v=N.ptr(v), g=N.ptr(g), state=N.ptr(state), out=N.ptr(out),
-        slot_idx=N.ptr(slot_idx), batch=B, num_heads=H, seq_len=int(max_seq_len or Tt), head_dim=D,
+        slot_idx=N.ptr(slot_idx), batch=B, num_heads=H, seq_len=int(max_seq_len or -(-Tt // B)), head_dim=D,
         dtype=N.dtype_code(q.dtype), g_dtype=N.dtype_code(g.dtype), state_dtype=N.dtype_code(state.dtype),
         scale=float(scale),
         q_stride_b=0, q_stride_h=q.stride(1), q_stride_t=q.stride(0),

@@ -110,3 +110,23 @@ def test_prompt_longer_than_the_stated_bound(sb, dev, cuts, H, Hk):
     assert (st - st1).abs().max() <= 1e-4 * st1.abs().max()
     d, ref = (o.float() - o1.float()).abs(), o1.float().abs()
     assert (d <= 2.0 ** -7 * ref + 2.0 ** -8 * ref.max()).all()      # each rounds the same sums, and its operands, to bf16
+
+
+@pytest.mark.parametrize("B,T,bound,cut", [(8, 100, None, False), (8, 100, 100, False), (1, 800, None, True), (2, 800, None, True),
+                                           (2, 800, 800, True)])
+def test_prompts_of_unstated_length(sb, dev, cuts, B, T, bound, cut):
+    """Without max_seq_len only the total of all prompts is known: many short prompts must not be cut as one long one
+    (every segment but the first would be empty, behind two more launches)."""
+    g = torch.Generator().manual_seed(B)
+    q = torch.randn(B * T, 28, D, generator=g).bfloat16().relu().to(dev)
+    k, v = (torch.randn(B * T, 4, D, generator=g).bfloat16().relu().to(dev) for _ in range(2))
+    gate = (F.logsigmoid(torch.randn(B * T, 4, D, generator=g)) / 16).to(dev)
+    state = torch.zeros(B, 4, D, D, device=dev)
+    cu = (torch.arange(B + 1, dtype=torch.int32) * T).to(dev)
+    o = sb.gla_prefill_packed(q, k, v, gate, state, torch.arange(B, device=dev), cu, B, max_query_len=bound)
+    assert any(n > 1 for n in cuts) == cut
+    state1 = torch.zeros_like(state)
+    o1 = sb.ops.gla_recurrent_packed(q, k, v, gate, state1, cu, per_head=True)      # (never cut)
+    assert (state - state1).abs().max() <= 1e-4 * state1.abs().max()
+    d, ref = (o.float() - o1.float()).abs(), o1.float().abs()
+    assert (d <= 2.0 ** -7 * ref + 2.0 ** -8 * ref.max()).all()
