@@ -507,6 +507,13 @@ typedef struct sb_swa_prefill_args {
 
 int sb_swa_prefill(const sb_swa_prefill_args *args);
 
+/* The index arrays of such a call from HOST lengths (no device access): `plan` [2 * num_seqs + 1 + 2 * num_tiles] receives
+ * cu_seqlens_q, seq_lens_k, tile_seq and tile_q0, one behind the other, for the caller to upload. num_tiles: the sum of
+ * ceil(query_lens[s] / 64). The tiles are listed in the order the kernel likes best; any other order, and plans of the caller's
+ * own, give the same results. */
+int sb_swa_prefill_plan(const int32_t *query_lens, const int32_t *seq_lens_k, int64_t num_seqs, int64_t num_tiles,
+                        int32_t *plan);
+
 /* The same call with the keys of a tile cut into parts that run side by side (a few tiles leave most of the GPU idle
  * otherwise: a chunk of 200 prompt tokens behind a full window is 4 tiles). sb_swa_prefill_parts: how many parts the
  * library would cut this call's longest walk into (1 = not at all); max_keys bounds seq_lens_k.

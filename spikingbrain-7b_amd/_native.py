@@ -201,6 +201,7 @@ EXPORTS = {
     "sb_window_shift_pair": (C.c_int, [C.POINTER(WindowShiftArgs), C.POINTER(WindowShiftArgs)]),
     "sb_dense_rows": (C.c_int, [C.POINTER(DenseRowsArgs)]),
     "sb_swa_prefill": (C.c_int, [C.POINTER(SwaPrefillArgs)]),
+    "sb_swa_prefill_plan": (C.c_int, [C.POINTER(i32), C.POINTER(i32), i64, i64, vp]),
     "sb_swa_prefill_parts": (i32, [C.POINTER(SwaPrefillArgs), i64]),
     "sb_swa_prefill_workspace_bytes": (sz, [C.POINTER(SwaPrefillArgs), i64, i32]),
     "sb_swa_prefill_parted": (C.c_int, [C.POINTER(SwaPrefillArgs), i64, i64, i32, vp, sz]),

@@ -6,7 +6,6 @@ from __future__ import annotations
 import ctypes as C
 from typing import Dict, Optional, Tuple
 
-import numpy as np
 import torch
 
 from . import _native as N
@@ -532,7 +531,6 @@ def plan_decode_split(num_rows: int, num_kv_heads: int, max_seq_len: int, window
 
 INT32_MAX = 2**31 - 1
 PREFILL_TILE = 64  # query tokens per workgroup of the prefill kernel
-PREFILL_CONTIGUOUS_TILES = 1024  # lists of this many tiles keep sequence order
 
 
 class PrefillPlan:
@@ -548,37 +546,23 @@ class PrefillPlan:
         seq_lens_k = query_lens if seq_lens_k is None else [int(x) for x in seq_lens_k]
         if len(seq_lens_k) != len(query_lens):
             raise ValueError("query_lens and seq_lens_k must have one entry per sequence")
-        lq, lk = np.asarray(query_lens, dtype=np.int64), np.asarray(seq_lens_k, dtype=np.int64)
-        bad = np.nonzero((lq < 0) | (lk < lq))[0]
-        if bad.size:
-            s = int(bad[0])
-            raise ValueError(f"sequence {s}: {lq[s]} queries need at least as many keys, got {lk[s]}")
-        S = len(query_lens)
-        cu = np.concatenate([[0], np.cumsum(lq)])
-        if max(int(cu[-1]), max(seq_lens_k, default=0)) > INT32_MAX:
+        for s, (lq, lk) in enumerate(zip(query_lens, seq_lens_k)):
+            if not 0 <= lq <= lk:
+                raise ValueError(f"sequence {s}: {lq} queries need at least as many keys, got {lk}")
+        S, total_q = len(query_lens), sum(query_lens)
+        self.max_k, self.total_k = max(seq_lens_k, default=0), sum(seq_lens_k)
+        if total_q > INT32_MAX or self.max_k > INT32_MAX:
             raise RuntimeError("the kernel counts keys and packed query rows in 32 bits: lengths cannot be converted without overflow")
-        n = -(-lq // PREFILL_TILE)
-        T = int(n.sum())
-        tile_seq = np.repeat(np.arange(S), n)
-        tile_q0 = (np.arange(T) - np.repeat(np.cumsum(n) - n, n)) * PREFILL_TILE
-        if 0 < T < PREFILL_CONTIGUOUS_TILES:
-            # The kernel gives XCD x the x-th contiguous eighth of the list. Tiles late in a long sequence see the
-            # most keys: they are dealt out in turn, latest first, so that the XCDs get equal shares and the
-            # longest workgroups start first. (Long lists stay in sequence order: an XCD's neighbouring tiles
-            # then share their keys in its L2, and there are enough of them to even out.)
-            order = np.argsort(-(tile_q0 + (lk - lq)[tile_seq]), kind="stable")
-            per_xcd = -(-T // 8)
-            k = np.arange(8 * per_xcd)
-            at = (k % 8) * per_xcd + k // 8
-            at = at[at < T]
-            tile_seq[at], tile_q0[at] = tile_seq[order], tile_q0[order]
-        packed = torch.from_numpy(np.concatenate([cu, lk, tile_seq, tile_q0]).astype(np.int32)).to(device, non_blocking=False)
+        T = sum([(n + PREFILL_TILE - 1) // PREFILL_TILE for n in query_lens])
+        packed = torch.empty(2 * S + 1 + 2 * T, dtype=torch.int32)
+        ints = C.c_int32 * S
+        N.check(N.lib().sb_swa_prefill_plan(ints(*query_lens), ints(*seq_lens_k), S, T, packed.data_ptr()), "prefill plan")
+        packed = packed.to(device, non_blocking=False)
         self.cu_seqlens_q = packed[:S + 1]
         self.seq_lens_k = packed[S + 1:2 * S + 1]
         self.tile_seq = packed[2 * S + 1:2 * S + 1 + T]
         self.tile_q0 = packed[2 * S + 1 + T:]
-        self.num_tiles, self.total_q, self.num_seqs = T, int(cu[-1]), S
-        self.max_k, self.total_k = max(seq_lens_k, default=0), sum(seq_lens_k)
+        self.num_tiles, self.total_q, self.num_seqs = T, total_q, S
 
 
 def swa_prefill_attention(
