@@ -27,7 +27,7 @@
 extern "C" {
 #endif
 
-#define SB_ABI_VERSION 4
+#define SB_ABI_VERSION 5
 
 enum sb_dtype { SB_BF16 = 0, SB_F16 = 1, SB_F32 = 2 };
 
@@ -503,6 +503,10 @@ typedef struct sb_swa_prefill_args {
   int64_t meta_bias_row0, meta_bias_rows;
   /* kv_start as 32-bit values (the step metadata's seq_start_loc as it is); read where kv_start is NULL. */
   const int32_t *kv_start32;
+  /* HOST array or NULL: the keys up to the end of every tile, longest first [num_tiles], as sb_swa_prefill_plan fills it.
+   * Only the choice of how the call is spread over the GPU reads it (before the call returns); NULL: as if all tiles
+   * walked as many keys as the longest. */
+  const int32_t *tile_keys;
 } sb_swa_prefill_args;
 
 int sb_swa_prefill(const sb_swa_prefill_args *args);
@@ -510,9 +514,10 @@ int sb_swa_prefill(const sb_swa_prefill_args *args);
 /* The index arrays of such a call from HOST lengths (no device access): `plan` [2 * num_seqs + 1 + 2 * num_tiles] receives
  * cu_seqlens_q, seq_lens_k, tile_seq and tile_q0, one behind the other, for the caller to upload. num_tiles: the sum of
  * ceil(query_lens[s] / 64). The tiles are listed in the order the kernel likes best; any other order, and plans of the caller's
- * own, give the same results. */
+ * own, give the same results. tile_keys [num_tiles] (may be NULL) stays on the host, for the field of that name; it is filled
+ * for fewer than 1024 tiles, more have no use for it. */
 int sb_swa_prefill_plan(const int32_t *query_lens, const int32_t *seq_lens_k, int64_t num_seqs, int64_t num_tiles,
-                        int32_t *plan);
+                        int32_t *plan, int32_t *tile_keys);
 
 /* The same call with the keys of a tile cut into parts that run side by side (a few tiles leave most of the GPU idle
  * otherwise: a chunk of 200 prompt tokens behind a full window is 4 tiles). sb_swa_prefill_parts: how many parts the
@@ -521,8 +526,9 @@ int sb_swa_prefill_plan(const int32_t *query_lens, const int32_t *seq_lens_k, in
  * after; calls whose scratch memory overlaps must be ordered), total_q being the packed query rows (cu_seqlens_q's last
  * entry). sb_swa_prefill_parted: the call. Every part keeps its softmax in fp32 and the parts are put together in fp32.
  * n_parts < 2: sb_swa_prefill with max_keys known (workspace unused). A walk longer than max_keys allows is still
- * walked whole. */
+ * walked whole. sb_swa_prefill_group_heads: how many query heads a workgroup of that call takes at most, 4 or 2 (same bits). */
 int32_t sb_swa_prefill_parts(const sb_swa_prefill_args *args, int64_t max_keys);
+int32_t sb_swa_prefill_group_heads(const sb_swa_prefill_args *args, int64_t max_keys, int32_t n_parts);
 size_t sb_swa_prefill_workspace_bytes(const sb_swa_prefill_args *args, int64_t total_q, int32_t n_parts);
 int sb_swa_prefill_parted(const sb_swa_prefill_args *args, int64_t total_q, int64_t max_keys, int32_t n_parts,
                           void *workspace, size_t workspace_bytes);

@@ -27,7 +27,7 @@ SB_GLA_PER_HEAD = 4
 SB_GLA_GROUP_PASS = 8
 SB_GLA_ZERO_SKIPPED = 16
 SB_SWA_DECODE_STATIC_SCRATCH_BYTES = 8 << 20
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 _DTYPES = {torch.bfloat16: SB_BF16, torch.float16: SB_F16, torch.float32: SB_F32}
 
@@ -120,7 +120,7 @@ class SwaPrefillArgs(C.Structure):
         ("k_scale_tensor", f32), ("v_scale_tensor", f32),
         ("meta_k", vp), ("meta_v", vp), ("meta_len", i32), ("meta_stride_row", i64), ("meta_stride_head", i64),
         ("softcap", f32), ("alibi_slopes", vp), ("meta_bias_row0", i64), ("meta_bias_rows", i64),
-        ("kv_start32", vp),
+        ("kv_start32", vp), ("tile_keys", vp),
     ]
 
 
@@ -201,8 +201,9 @@ EXPORTS = {
     "sb_window_shift_pair": (C.c_int, [C.POINTER(WindowShiftArgs), C.POINTER(WindowShiftArgs)]),
     "sb_dense_rows": (C.c_int, [C.POINTER(DenseRowsArgs)]),
     "sb_swa_prefill": (C.c_int, [C.POINTER(SwaPrefillArgs)]),
-    "sb_swa_prefill_plan": (C.c_int, [C.POINTER(i32), C.POINTER(i32), i64, i64, vp]),
+    "sb_swa_prefill_plan": (C.c_int, [C.POINTER(i32), C.POINTER(i32), i64, i64, vp, vp]),
     "sb_swa_prefill_parts": (i32, [C.POINTER(SwaPrefillArgs), i64]),
+    "sb_swa_prefill_group_heads": (i32, [C.POINTER(SwaPrefillArgs), i64, i32]),
     "sb_swa_prefill_workspace_bytes": (sz, [C.POINTER(SwaPrefillArgs), i64, i32]),
     "sb_swa_prefill_parted": (C.c_int, [C.POINTER(SwaPrefillArgs), i64, i64, i32, vp, sz]),
     "sb_window_advance": (C.c_int, [C.POINTER(WindowAdvanceArgs)]),

@@ -732,11 +732,16 @@ constexpr int64_t kCUs = 256;
 
 // How a call is spread over the GPU: with groups of four heads a workgroup of eight wavefronts fills a CU, and a call
 // of `wgs` of them takes as long as its longest walk while wgs <= 256. Two ways to shorten that:
-//  * pairs: workgroups of two heads and four wavefronts, two to a CU. A CU that holds one runs its chunks at 0.69 us
-//    instead of 0.9, and in whole prompts a long walk shares its CU with a short one (1 x 300 / 700 / 1000 / 1517 /
-//    2560 / 3000 tokens: 16.6 / 28.3 / 35.8 / 50.7 / 80.7 / 92.8 -> 13.1 / 21.9 / 28.2 / 42.3 / 69 / 87 us). With walks of
-//    equal length (prompt chunks behind a context) only while every CU gets one (1024 tokens behind 4200: 125 -> 97;
-//    1500: 126 -> 136), and beyond 1.5 x 256 workgroups of four heads they lose (1 x 6000: 256 -> 271);
+//  * pairs: workgroups of two heads and four wavefronts, two to a CU. Measured, with L the longest walk in chunks and L' the
+//    walk of the longest workgroup that has to share its CU (in whole prompts a long walk shares with a short one; behind a
+//    context all are as long): groups of four 8.4 + 0.94 L us, pairs 6.3 + 0.72 L + 0.35 L'. So they always pay while every
+//    CU gets one, and up to 256 workgroups of four where L' < 6 + 0.63 L (28 : 4 heads, us of groups of four -> pairs):
+//      whole prompts, window 4096   300 / 700 / 1000 / 1517 / 2560 tokens 16.6 / 28.3 / 35.8 / 50.7 / 80.7 -> 13.1 / 21.9 / 28.2 / 42.3 / 69
+//      behind 4200                  window 512: 1075 / 2035 28.8 / 29.9 -> 29.2 / 30.1, 1024: 42.4 / 43.7 -> 44.5 / 45.3, 4096: 124 / 129 -> 136 / 142
+//      between                      1200 behind 300 49.6 -> 41.7, 2000 behind 800 85.5 -> 74.7; 2035, window 512 28.1 -> 28.7 (not taken)
+//    From 256 to 384 workgroups of four (a second round that leaves most CUs idle) they pay unless the walks are many chunks
+//    long: 3059 tokens, window 4096 92.8 -> 88.8; behind 4200, windows 512 / 1024 / 2048 / 4096 52.4 / 77.1 / 127 / 228 -> 47 / 72.9 / 124 /
+//    230; beyond that they lose (1 x 6000: 256 -> 271).
 //  * parts: the keys of a walk cut into parts of 8 chunks or more side by side, at the price of fp32 partials and
 //    a merge (64 / 200 / 512 / 1024 tokens behind 4200: 123 -> 24 (16 parts) / 33 (8) / 49 (4) / 80 (2) us).
 struct Spread {
@@ -748,9 +753,13 @@ int64_t quad_workgroups(const sb_swa_prefill_args *a) {
 }
 bool pairs_pay(const sb_swa_prefill_args *a, int64_t chunks, int64_t parts) {
   const int64_t wgs = quad_workgroups(a) * parts;
-  // (whole prompts walk two chunks per tile at most; a longer walk means a context in front of the queries)
-  const bool whole = chunks <= 2 * a->num_tiles + 2;
-  return whole && parts == 1 ? 2 * wgs <= 3 * kCUs : 2 * wgs <= kCUs;
+  if (2 * wgs <= kCUs) return true;
+  if (parts > 1 || 2 * wgs > 3 * kCUs) return false;
+  if (wgs > kCUs) return chunks <= 2 * a->num_tiles + 2;
+  if (!a->tile_keys) return false;   // (unknown: as if all walks were equal)
+  const int64_t pairs_per_tile = (int64_t)a->num_kv_heads * ((a->num_q_heads / a->num_kv_heads + 1) / 2);
+  const int64_t sharing = kCUs / pairs_per_tile;   // tiles in front of the first one that shares
+  return sharing >= a->num_tiles || (double)most_chunks(a, a->tile_keys[sharing]) < 6.0 + 0.63 * (double)chunks;
 }
 Spread spread_of(const sb_swa_prefill_args *a, int64_t max_keys) {
   const int64_t chunks = most_chunks(a, max_keys), wgs = quad_workgroups(a);
@@ -909,7 +918,7 @@ constexpr int kTileTokens = 64;
 // Native because every new prompt pays it in front of its first layer: the whole plan of 64 / 1517 / 8192 / 16 x 8192 tokens in
 // numpy took 39 / 39 / 43 / 37 us of host time, in Python loops without the dealing 13 / 17 / 35 / 370; here 13 / 13 / 14 / 21.
 extern "C" int sb_swa_prefill_plan(const int32_t *query_lens, const int32_t *seq_lens_k, int64_t num_seqs, int64_t num_tiles,
-                                   int32_t *plan) {
+                                   int32_t *plan, int32_t *tile_keys) {
   using namespace sb_host;
   if (num_seqs < 0 || num_tiles < 0 || !plan || (num_seqs > 0 && (!query_lens || !seq_lens_k)))
     return fail(SB_ERR_INVALID, "sb_swa_prefill_plan: negative size or null pointer");
@@ -943,6 +952,7 @@ extern "C" int sb_swa_prefill_plan(const int32_t *query_lens, const int32_t *seq
   for (int64_t k = 0; k < 8 * per_xcd; ++k) {
     const int64_t slot = (k % 8) * per_xcd + k / 8;
     if (slot >= tiles) continue;
+    if (tile_keys) tile_keys[next] = (int32_t)std::min<int64_t>((order[next] >> 12) + kTileTokens, INT32_MAX);
     const int64_t t = kDealtTiles - 1 - (order[next++] & 0xfff);
     at_seq[slot] = seq[t];
     at_q0[slot] = q0[t];
@@ -955,8 +965,13 @@ extern "C" int sb_swa_prefill_plan(const int32_t *query_lens, const int32_t *seq
 extern "C" int sb_swa_prefill(const sb_swa_prefill_args *a) { return prefill(a, INT32_MAX, 1, nullptr, nullptr); }
 
 extern "C" int32_t sb_swa_prefill_parts(const sb_swa_prefill_args *a, int64_t max_keys) {
-  if (!a || a->num_tiles <= 0 || a->num_kv_heads <= 0 || a->num_q_heads <= 0 || max_keys <= 0) return 1;
+  if (!a || a->num_tiles <= 0 || a->num_kv_heads <= 0 || a->num_q_heads < a->num_kv_heads || max_keys <= 0) return 1;
   return spread_of(a, max_keys < INT32_MAX ? max_keys : INT32_MAX).parts;
+}
+
+extern "C" int32_t sb_swa_prefill_group_heads(const sb_swa_prefill_args *a, int64_t max_keys, int32_t n_parts) {
+  if (!a || a->num_tiles <= 0 || a->num_kv_heads <= 0 || a->num_q_heads < a->num_kv_heads || max_keys <= 0) return 4;
+  return pairs_pay(a, most_chunks(a, max_keys < INT32_MAX ? max_keys : INT32_MAX), n_parts < 1 ? 1 : n_parts) ? 2 : 4;
 }
 
 extern "C" size_t sb_swa_prefill_workspace_bytes(const sb_swa_prefill_args *a, int64_t total_q, int32_t n_parts) {

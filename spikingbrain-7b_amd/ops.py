@@ -531,6 +531,7 @@ def plan_decode_split(num_rows: int, num_kv_heads: int, max_seq_len: int, window
 
 INT32_MAX = 2**31 - 1
 PREFILL_TILE = 64  # query tokens per workgroup of the prefill kernel
+PREFILL_DEALT_TILES = 1024  # shorter tile lists are dealt to the XCDs longest walk first
 
 
 class PrefillPlan:
@@ -539,7 +540,7 @@ class PrefillPlan:
     (which the scheduler already has as Python ints), uploaded with one copy."""
 
     __slots__ = ("cu_seqlens_q", "seq_lens_k", "tile_seq", "tile_q0", "num_tiles", "total_q", "num_seqs", "max_k",
-                 "total_k")
+                 "total_k", "_host", "tile_keys_ptr")
 
     def __init__(self, query_lens, seq_lens_k, device):
         query_lens = [int(x) for x in query_lens]
@@ -554,14 +555,15 @@ class PrefillPlan:
         if total_q > INT32_MAX or self.max_k > INT32_MAX:
             raise RuntimeError("the kernel counts keys and packed query rows in 32 bits: lengths cannot be converted without overflow")
         T = sum([(n + PREFILL_TILE - 1) // PREFILL_TILE for n in query_lens])
-        packed = torch.empty(2 * S + 1 + 2 * T, dtype=torch.int32)
-        ints = C.c_int32 * S
-        N.check(N.lib().sb_swa_prefill_plan(ints(*query_lens), ints(*seq_lens_k), S, T, packed.data_ptr()), "prefill plan")
-        packed = packed.to(device, non_blocking=False)
+        self._host = torch.empty(2 * S + 1 + 3 * T, dtype=torch.int32)
+        host_ptr, ints = self._host.data_ptr(), C.c_int32 * S
+        self.tile_keys_ptr = host_ptr + 4 * (2 * S + 1 + 2 * T) if 0 < T < PREFILL_DEALT_TILES else None   # (read on the host)
+        N.check(N.lib().sb_swa_prefill_plan(ints(*query_lens), ints(*seq_lens_k), S, T, host_ptr, self.tile_keys_ptr), "prefill plan")
+        packed = self._host.to(device, non_blocking=False)
         self.cu_seqlens_q = packed[:S + 1]
         self.seq_lens_k = packed[S + 1:2 * S + 1]
         self.tile_seq = packed[2 * S + 1:2 * S + 1 + T]
-        self.tile_q0 = packed[2 * S + 1 + T:]
+        self.tile_q0 = packed[2 * S + 1 + T:2 * S + 1 + 2 * T]
         self.num_tiles, self.total_q, self.num_seqs = T, total_q, S
 
 
@@ -724,7 +726,7 @@ def swa_prefill_attention(
         softcap=float(softcap), alibi_slopes=N.ptr(_slopes(alibi_slopes, Hq, dev)),
         meta_bias_row0=int(meta_bias[0]) if meta_bias else 0,
         meta_bias_rows=int(meta_bias[1]) if meta_bias else int(q.shape[0]),
-        kv_start32=N.ptr(kv_start32) if block_table is None else None, **meta)
+        kv_start32=N.ptr(kv_start32) if block_table is None else None, tile_keys=plan.tile_keys_ptr, **meta)
     L = N.lib()
     if n_parts == 0:
         n_parts = L.sb_swa_prefill_parts(C.byref(a), plan.max_k)

@@ -46,11 +46,11 @@ def test_long_lists_keep_sequence_order(sb):
 def test_native_plan_refuses_what_does_not_fit(sb):
     L, ints = sb._native.lib(), ctypes.c_int32 * 2
     plan = (ctypes.c_int32 * 64)()
-    run = lambda q, k, tiles: L.sb_swa_prefill_plan(ints(*q), ints(*k), 2, tiles, ctypes.addressof(plan))
+    run = lambda q, k, tiles: L.sb_swa_prefill_plan(ints(*q), ints(*k), 2, tiles, ctypes.addressof(plan), None)
     assert run((64, 65), (64, 65), 3) == 0 and list(plan[:5]) == [0, 64, 129, 64, 65]
     for q, k, tiles in (((64, 65), (64, 65), 2), ((64, 65), (64, 65), 4), ((64, 65), (64, 64), 3), ((-1, 65), (64, 65), 2)):
         assert run(q, k, tiles) == sb._native.SB_ERR_INVALID
-    assert L.sb_swa_prefill_plan(None, None, 1, 1, ctypes.addressof(plan)) == sb._native.SB_ERR_INVALID
+    assert L.sb_swa_prefill_plan(None, None, 1, 1, ctypes.addressof(plan), None) == sb._native.SB_ERR_INVALID
 
 
 @pytest.mark.parametrize("lens", [[64], [1517, 3, 900], [100] * 128, [100] * 129, [8192] * 2, [8192] * 16])
@@ -61,3 +61,35 @@ def test_plan_covers_every_tile_once(sb, lens):
     assert plan.cu_seqlens_q.tolist() == [sum(lens[:i]) for i in range(len(lens) + 1)]
     assert plan.seq_lens_k.tolist() == [n + 7 for n in lens] and plan.total_k == sum(lens) + 7 * len(lens)
     assert all(t.dtype == plan.cu_seqlens_q.dtype for t in (plan.seq_lens_k, plan.tile_seq, plan.tile_q0))
+
+
+def _heads(sb, lens, context, window, known=True):
+    """Query heads per workgroup of an uncut call of 28 : 4 heads (256 CUs where the device cannot be asked)."""
+    keys = [n + context for n in lens]
+    plan = sb.ops.PrefillPlan(lens, keys, "cpu")
+    a = sb._native.SwaPrefillArgs(num_tiles=plan.num_tiles, num_q_heads=28, num_kv_heads=4, window_left=window,
+                                  tile_keys=plan.tile_keys_ptr if known else None)
+    return sb._native.lib().sb_swa_prefill_group_heads(ctypes.byref(a), plan.max_k, 1)
+
+
+@pytest.mark.parametrize("lens,context,window,heads", [
+    ([563], 4200, 4096, 2), ([1024], 4200, 4096, 2),                            # a workgroup of two heads for every CU
+    ([1075], 4200, 512, 4), ([1523], 4200, 1024, 4), ([2035], 4200, 1024, 4), ([2035], 4200, 4096, 4), ([1000, 300, 600], 4200, 2048, 4),
+    ([1075], 0, 512, 2), ([1523], 0, 512, 2), ([2035], 0, 512, 4),              # whole prompts, more and more walks of a full window
+    ([1523], 0, 1024, 2), ([2035], 0, 4096, 2), ([1200], 300, 4096, 2), ([2000], 800, 4096, 2),
+    ([3059], 4200, 1024, 2), ([3059], 4200, 4096, 4), ([3059], 0, 4096, 2), ([700] * 3, 0, 512, 2), ([6000], 0, 4096, 4)])
+def test_heads_per_workgroup(sb, lens, context, window, heads):
+    """Prompt chunks behind a context walk equally many keys per tile, whatever the window: above one workgroup of two heads
+    per CU they take groups of four."""
+    assert _heads(sb, lens, context, window) == heads
+    tiles = sum(-(-n // 64) for n in lens)
+    if 16 < tiles <= 32:
+        assert _heads(sb, lens, context, window, known=False) == 4
+
+
+def test_keys_of_the_tiles(sb):
+    lens, keys = [100, 0, 64, 200], [100, 7, 3064, 250]
+    plan = sb.ops.PrefillPlan(lens, keys, "cpu")
+    got = plan._host[-plan.num_tiles:].tolist()
+    assert got == sorted((64 + at + k - n for n, k in zip(lens, keys) for at in range(0, n, 64)), reverse=True)
+    assert sb.ops.PrefillPlan([64 * 1024], None, "cpu").tile_keys_ptr is None
