@@ -239,6 +239,10 @@ typedef struct sb_swa_decode_args {
  * of eight 32-key chunks per split; with less memory than that takes, it is rejected with SB_ERR_WORKSPACE. */
 int32_t sb_swa_decode_auto_split(int64_t num_rows, int32_t num_kv_heads, int32_t max_seq_len,
                                  int32_t window_left);
+/* The same for calls that run on the vector ALUs (fp32 queries, SB_DECODE_FORCE_VALU, head sizes other than 128, more than
+ * 16 query heads per kv head), whose workgroups are smaller and more. */
+int32_t sb_swa_decode_auto_split_vector(int64_t num_rows, int32_t num_q_heads, int32_t num_kv_heads, int32_t max_seq_len,
+                                        int32_t window_left);
 /* 1 if SB_DECODE_BALANCED is expected to be faster than the fixed split into n_split (>= 1) parts for rows
  * with these lengths, else 0. host_seq_lens: the step's seq_lens as a HOST array (the scheduler has them;
  * a caller without them can pass max_seq_len for every row: the balanced split adapts to the real lengths

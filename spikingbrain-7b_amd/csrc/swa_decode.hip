@@ -697,29 +697,66 @@ static int64_t long_run_split(const SplitShape &s) {
   return best;
 }
 
-extern "C" int32_t sb_swa_decode_auto_split(int64_t num_rows, int32_t num_kv_heads,
-                                            int32_t max_seq_len, int32_t window_left) {
-  if (num_rows <= 0 || num_kv_heads <= 0 || max_seq_len <= 0) return 1;
-  const SplitShape s = split_shape(num_rows, num_kv_heads, max_seq_len, window_left);
-  int64_t best = long_run_split(s);
-  if (s.wgs * best > s.cus || s.chunks <= kWholeChunks) return (int32_t)best;
-  // One round: the CUs that 8 chunks a workgroup would leave idle are worth more than the partials they add. Measured
-  // with 8 chunks or more each -> without that bound (us per call): 1 row x 4097 keys 24.1 -> 17.1 (15 -> 43 splits),
-  // 8 x 4097 27.5 -> 22.3 (15 -> 26), 1 x 2000 21.1 -> 12.9 (8 -> 32), 16 x 1000 22.5 -> 14.7 (4 -> 16),
-  // 64 x 600 28.3 -> 21.6 (2 -> 4); INT8 8 x 4097 21.3 -> 18.1.
-  best = 1;
-  double best_cost = one_round_us(s.wgs, 1, s.run, s.cus);
-  for (int64_t n = 2; n <= 64 && n <= s.run && s.wgs * n <= s.cus; ++n) {
+// The split into at least `least` parts with the lowest estimated duration whose workgroups all run at once.
+static int32_t one_round_split(const SplitShape &s, int64_t least) {
+  int64_t best = least;
+  double best_cost = one_round_us(s.wgs, best, s.run, s.cus);
+  for (int64_t n = least + 1; n <= 64 && n <= s.run && s.wgs * n <= s.cus; ++n) {
     const double c = one_round_us(s.wgs, n, s.run, s.cus);
     if (c <= best_cost) { best = n; best_cost = c; }
   }
   return (int32_t)best;
 }
 
+extern "C" int32_t sb_swa_decode_auto_split(int64_t num_rows, int32_t num_kv_heads,
+                                            int32_t max_seq_len, int32_t window_left) {
+  if (num_rows <= 0 || num_kv_heads <= 0 || max_seq_len <= 0) return 1;
+  const SplitShape s = split_shape(num_rows, num_kv_heads, max_seq_len, window_left);
+  const int64_t best = long_run_split(s);
+  if (s.wgs * best > s.cus || s.chunks <= kWholeChunks) return (int32_t)best;
+  // One round: the CUs that 8 chunks a workgroup would leave idle are worth more than the partials they add. Measured
+  // with 8 chunks or more each -> without that bound (us per call): 1 row x 4097 keys 24.1 -> 17.1 (15 -> 43 splits),
+  // 8 x 4097 27.5 -> 22.3 (15 -> 26), 1 x 2000 21.1 -> 12.9 (8 -> 32), 16 x 1000 22.5 -> 14.7 (4 -> 16),
+  // 64 x 600 28.3 -> 21.6 (2 -> 4); INT8 8 x 4097 21.3 -> 18.1.
+  return one_round_split(s, 1);
+}
+
+// The vector kernel is built for 1, 2, 4, 7 and 8 query heads per workgroup; any other group size is cut
+// into parts of the largest of these that divides it (the parts read the same K/V rows).
+static int vector_heads(int G) {
+  for (int cand : {8, 7, 4, 2})
+    if (G % cand == 0) return cand;
+  return 1;
+}
+
+// bf16/fp16 at head size 128 run on the matrix cores (up to 16 query heads per kv head); everything else on the vector ALUs
+static bool on_matrix_cores(const sb_swa_decode_args *a) {
+  return a->dtype != SB_F32 && !(a->flags & SB_DECODE_FORCE_VALU) && a->head_size == 128 &&
+         a->num_q_heads <= 16 * (int64_t)a->num_kv_heads;
+}
+
+// The vector kernel has a workgroup per (row, kv head, part of the group), four and more times as many as the other kernels,
+// and fills the CUs with less of a split: finer splits pay only while those workgroups fit the CUs. Measured (us per call, fp32, 28 : 4
+// heads, split of long runs -> this -> the rule above): 1 row x 400 / 4097 keys 20.4 / 20.9 -> 11.0 / 18.6 (the same 13 / 43 splits),
+// 4 x 4097 27.2 -> 27.2 -> 32.9, 8 x 2000 25.4 -> 25.4 -> 29.9, 16 x 400 21.0 -> 15.9 -> 22.2, 64 x 400 30.0 -> 30.0 -> 34.9; bf16, head size 64,
+// 16 x 1000 17.1 -> 17.1 -> 22.4, 40 x 400 18.2 -> 18.2 -> 24.1.
+extern "C" int32_t sb_swa_decode_auto_split_vector(int64_t num_rows, int32_t num_q_heads, int32_t num_kv_heads,
+                                                   int32_t max_seq_len, int32_t window_left) {
+  if (num_rows <= 0 || num_kv_heads <= 0 || num_q_heads < num_kv_heads || max_seq_len <= 0) return 1;
+  SplitShape s = split_shape(num_rows, num_kv_heads, max_seq_len, window_left);
+  const int64_t best = long_run_split(s);
+  const int G = num_q_heads / num_kv_heads;
+  s.wgs = num_rows * num_kv_heads * (G / vector_heads(G));
+  if (s.wgs * best > s.cus || s.chunks <= kWholeChunks) return (int32_t)best;
+  return one_round_split(s, best);
+}
+
 // The split of a call that leaves it to the library: what the rule says, with no more partials than `bytes` hold, down
 // to the split of long runs (memory that takes less than that one's partials is refused).
 static int32_t chosen_split(const sb_swa_decode_args *a, size_t bytes) {
-  int32_t n = sb_swa_decode_auto_split(a->num_rows, a->num_kv_heads, a->max_seq_len, a->window_left);
+  int32_t n = on_matrix_cores(a)
+                  ? sb_swa_decode_auto_split(a->num_rows, a->num_kv_heads, a->max_seq_len, a->window_left)
+                  : sb_swa_decode_auto_split_vector(a->num_rows, a->num_q_heads, a->num_kv_heads, a->max_seq_len, a->window_left);
   if (n < 2 || sb_swa_decode_workspace_bytes(a->num_rows, a->num_q_heads, a->head_size, n) <= bytes) return n;
   const int64_t least = long_run_split(split_shape(a->num_rows, a->num_kv_heads, a->max_seq_len, a->window_left));
   while (n > least && sb_swa_decode_workspace_bytes(a->num_rows, a->num_q_heads, a->head_size, n) > bytes) --n;
@@ -890,16 +927,11 @@ extern "C" int sb_swa_decode(const sb_swa_decode_args *a) {
   hipStream_t st = (hipStream_t)a->stream;
   int rc = 0;
   if (a->phases < 0 || a->phases > 2) return fail(SB_ERR_INVALID, "sb_swa_decode: phases must be 0, 1 or 2");
-  // bf16/fp16 at head size 128 run on the matrix cores (up to 16 query heads per kv head); everything else on the vector ALUs
-  const bool mfma = (a->dtype != SB_F32) && !(a->flags & SB_DECODE_FORCE_VALU) && a->head_size == 128 && G <= 16;
+  const bool mfma = on_matrix_cores(a);
   if (int8_kv && G > 16)
     return fail(SB_ERR_UNSUPPORTED, "sb_swa_decode: GQA group size %d over a byte-code cache (the matrix-core kernels take up to 16 query heads per kv head)", G);
   if (a->num_q_heads > 65535) return fail(SB_ERR_UNSUPPORTED, "sb_swa_decode: grid too large");
-  // The vector kernel is built for 1, 2, 4, 7 and 8 query heads per workgroup; any other group size is cut
-  // into parts of the largest of these that divides it (the parts read the same K/V rows).
-  int vec_g = 1;
-  for (int cand : {8, 7, 4, 2})
-    if (G % cand == 0) { vec_g = cand; break; }
+  const int vec_g = vector_heads(G);
   p.group_parts = mfma ? 1 : G / vec_g;
   if (mfma && (a->kv_stride_row <= 0 || a->kv_stride_row * kv_esz * 16 >= (1LL << 31)))
     return fail(SB_ERR_UNSUPPORTED, "sb_swa_decode: kv row stride %lld does not fit the kernel's 32-bit in-tile offsets",

@@ -304,7 +304,10 @@ def swa_decode_attention(
     L = N.lib()
     auto_balance = balanced is None
     if n_split == 0:
-        n_split = L.sb_swa_decode_auto_split(R, Hkv, int(max_seq_len), int(window_left))
+        if q.dtype != torch.float32 and not force_valu and D == 128 and Hq <= 16 * Hkv:
+            n_split = L.sb_swa_decode_auto_split(R, Hkv, int(max_seq_len), int(window_left))
+        else:   # the vector kernel
+            n_split = L.sb_swa_decode_auto_split_vector(R, Hq, Hkv, int(max_seq_len), int(window_left))
     can_balance = (q.dtype in (torch.bfloat16, torch.float16) and not int8_kv and not force_valu and R <= 1024
                    and "meta_k" not in fused)
     if auto_balance:

@@ -128,3 +128,15 @@ def test_auto_split_of_one_round(sb):
             if rows <= 64:
                 assert rows * n <= 256
                 assert L.sb_swa_decode_workspace_bytes(rows, 28, 128, n) <= sb._native.SB_SWA_DECODE_STATIC_SCRATCH_BYTES
+
+
+@pytest.mark.parametrize("rows,q_heads,kv_heads,keys,split", [
+    (1, 28, 4, 400, 13), (1, 28, 4, 4097, 43), (4, 28, 4, 4097, 15), (8, 28, 4, 2000, 8), (16, 28, 4, 400, 4), (16, 28, 4, 1000, 4),
+    (40, 28, 4, 400, 1), (64, 28, 4, 400, 1), (100, 16, 4, 400, 1), (8, 28, 1, 2000, 8), (64, 28, 1, 400, 1), (1, 8, 8, 4097, 26),
+    (8, 8, 8, 1000, 4)])
+def test_auto_split_of_the_vector_kernel(sb, rows, q_heads, kv_heads, keys, split):
+    """Its workgroups, one per (row, kv head, part of the group) and split, exceed the CUs (256 where the device cannot be
+    asked) only with runs of eight chunks or more each; a group of 28 heads is cut into four parts of 7."""
+    n = sb._native.lib().sb_swa_decode_auto_split_vector(rows, q_heads, kv_heads, keys, 4096)
+    parts = {7: 1, 28: 4, 1: 1, 4: 1}[q_heads // kv_heads]
+    assert n == split and (rows * kv_heads * parts * n <= 256 or keys // n >= 8 * 32)
