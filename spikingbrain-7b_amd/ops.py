@@ -871,12 +871,19 @@ def gla_recurrent(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
     return out
 
 
-def _launch_gla(a, dev: torch.device) -> None:
+def _launch_gla(a, dev: torch.device, total: int = 0) -> None:
     """Enqueue the recurrence; long prompts of a few sequences are cut into segments that run side by side, with
-    scratch memory from torch's allocator (stream-ordered, and part of the graph under capture)."""
+    scratch memory from torch's allocator (stream-ordered, and part of the graph under capture). total: the tokens of
+    all prompts, where seq_len is only their mean length."""
     L = N.lib()
     n = L.sb_gla_prompt_segments(C.byref(a)) if a.seq_len > 1 else 1
     if n > 1:
+        if total:
+            # segments as for prompts of the mean length, and enough of them for one of four times that (1000 + 100 + 100
+            # tokens on 4 states 165 us uncut, 173 with 8 segments for 400 tokens, 39 with 19)
+            tokens = (-(-a.seq_len // n) + 31) // 32 * 32
+            a.seq_len = min(total, 4 * a.seq_len)
+            n = -(-a.seq_len // tokens)
         ws = torch.empty(L.sb_gla_prompt_workspace_bytes(C.byref(a), n), dtype=torch.uint8, device=dev)
         N.check(L.sb_gla_prompt_segmented(C.byref(a), n, ws.data_ptr(), ws.numel()), "gla_recurrent")
     else:
@@ -900,9 +907,8 @@ def gla_recurrent_packed(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: t
     free, contiguous D), sequence b owning tokens cu_seqlens[b] .. cu_seqlens[b+1]-1 (int32 device
     vector [B+1]); its state is state[slot_idx[b]] (default b), advanced in place. One call for all
     sequences; long prompts of a few sequences are cut into segments that run side by side (see gla_recurrent), as
-    max_seq_len, an upper bound of their lengths, says (default: the mean length, which some sequence reaches: eight
-    prompts of 100 tokens are not cut like one of 800, of whose segments the first would hold all there is; what lies
-    beyond falls to a prompt's last segment). Returns o [total_tokens, H, D]. Shared states as in gla_recurrent: k, v, g
+    max_seq_len, an upper bound of their lengths, says (default: by the mean length, which some sequence reaches: eight
+    prompts of 100 tokens are not cut like one of 800, of whose segments the first would hold all there is). Returns o [total_tokens, H, D]. Shared states as in gla_recurrent: k, v, g
     [total_tokens, Hkv, D] with state [slots, Hkv, D, D]."""
     dev = N.require_gpu(q, k, v, g, state, cu_seqlens, slot_idx, out)
     if q.dim() != 3 or k.dim() != 3 or v.shape != k.shape or g.shape != k.shape or \
@@ -947,7 +953,7 @@ def gla_recurrent_packed(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: t
         flags=(N.SB_GLA_VECTOR_ONLY if vector_only else 0) | (N.SB_GLA_CHECK_GATES if check_gates else 0)
         | (0 if per_head is None else (N.SB_GLA_PER_HEAD if per_head else N.SB_GLA_GROUP_PASS)),
         q_heads_per_state=H // Hk)
-    _launch_gla(a, dev)
+    _launch_gla(a, dev, 0 if max_seq_len or B == 1 else Tt)
     return out
 
 

@@ -112,17 +112,18 @@ def test_prompt_longer_than_the_stated_bound(sb, dev, cuts, H, Hk):
     assert (d <= 2.0 ** -7 * ref + 2.0 ** -8 * ref.max()).all()      # each rounds the same sums, and its operands, to bf16
 
 
-@pytest.mark.parametrize("B,T,bound,cut", [(8, 100, None, False), (8, 100, 100, False), (1, 800, None, True), (2, 800, None, True),
-                                           (2, 800, 800, True)])
-def test_prompts_of_unstated_length(sb, dev, cuts, B, T, bound, cut):
+@pytest.mark.parametrize("lens,bound,cut", [([100] * 8, None, False), ([100] * 8, 100, False), ([800], None, True), ([800] * 2, None, True),
+                                            ([800] * 2, 800, True), ([1000, 100, 100], None, True), ([10, 0, 0, 0, 0, 2000], None, True)])
+def test_prompts_of_unstated_length(sb, dev, cuts, lens, bound, cut):
     """Without max_seq_len only the total of all prompts is known: many short prompts must not be cut as one long one
     (every segment but the first would be empty, behind two more launches)."""
+    B, T = len(lens), sum(lens)
     g = torch.Generator().manual_seed(B)
-    q = torch.randn(B * T, 28, D, generator=g).bfloat16().relu().to(dev)
-    k, v = (torch.randn(B * T, 4, D, generator=g).bfloat16().relu().to(dev) for _ in range(2))
-    gate = (F.logsigmoid(torch.randn(B * T, 4, D, generator=g)) / 16).to(dev)
+    q = torch.randn(T, 28, D, generator=g).bfloat16().relu().to(dev)
+    k, v = (torch.randn(T, 4, D, generator=g).bfloat16().relu().to(dev) for _ in range(2))
+    gate = (F.logsigmoid(torch.randn(T, 4, D, generator=g)) / 16).to(dev)
     state = torch.zeros(B, 4, D, D, device=dev)
-    cu = (torch.arange(B + 1, dtype=torch.int32) * T).to(dev)
+    cu = torch.tensor([0] + lens).cumsum(0).int().to(dev)
     o = sb.gla_prefill_packed(q, k, v, gate, state, torch.arange(B, device=dev), cu, B, max_query_len=bound)
     assert any(n > 1 for n in cuts) == cut
     state1 = torch.zeros_like(state)
