@@ -380,7 +380,15 @@ __global__ __launch_bounds__(256) void swa_decode_split_kernel(const DecodeParam
 // kBatch splits per trip to memory, every load of a trip issued before any is used: the kernel is latency and little
 // else, so the host takes the batch that covers the split count in one or two trips. The arithmetic goes four
 // splits at a time in the same order whatever the batch (same bits); from four to four the running sums are
-// rescaled to the new maximum.
+// rescaled to the new maximum. A trip's loads past the last partial are out of their buffer's range and give zeros:
+// that partial again, times 0, would be a NaN where it holds an infinity (and a select on the loaded value makes the
+// compiler wait for each load in a branch of its own: 19 -> 21 us a call at 4 rows and 43 splits).
+__device__ __forceinline__ float load_partial(__amdgpu_buffer_rsrc_t partials, int float_index) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(partials, float_index * 4, 0, 0));
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t partials_from(float *first, int64_t floats) {
+  return __builtin_amdgcn_make_buffer_rsrc(first, 0, (int)(floats * 4), 0x00020000);
+}
 template <typename E, int kBatch>
 __global__ __launch_bounds__(256) void swa_decode_merge_kernel(const DecodeParams p) {
   const int64_t rh = blockIdx.x;  // r*Hq + hq
@@ -388,7 +396,7 @@ __global__ __launch_bounds__(256) void swa_decode_merge_kernel(const DecodeParam
   const int hq = (int)(rh - r * p.Hq);
   const int d = threadIdx.x;
   const float *ml = p.ws_ml + rh * p.n_split * 2;
-  const float *acc = p.ws_acc + rh * p.n_split * p.D + d;
+  const __amdgpu_buffer_rsrc_t acc = partials_from(p.ws_acc + rh * p.n_split * p.D, p.n_split * p.D);
   float tot = 0.f, L = 0.f, M = kNegInf;
   for (int b0 = 0; b0 < p.n_split; b0 += kBatch) {
     float ms[kBatch], ls[kBatch], av[kBatch];
@@ -397,7 +405,7 @@ __global__ __launch_bounds__(256) void swa_decode_merge_kernel(const DecodeParam
       const int s = min(b0 + j, p.n_split - 1);
       ms[j] = ml[2 * s];
       ls[j] = ml[2 * s + 1];
-      av[j] = acc[(int64_t)s * p.D];
+      av[j] = load_partial(acc, (b0 + j) * p.D + d);
     }
 #pragma unroll
     for (int j0 = 0; j0 < kBatch; j0 += 4) {
@@ -413,9 +421,8 @@ __global__ __launch_bounds__(256) void swa_decode_merge_kernel(const DecodeParam
           L *= keep;
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            const bool there = s0 + j < p.n_split;  // (else the last one again: it may hold an infinity, which f = 0 does not undo)
-            const float f = (!there || ms[j0 + j] == kNegInf) ? 0.f : fast_exp2(ms[j0 + j] - Mn);
-            tot = fmaf(there ? av[j0 + j] : 0.f, f, tot);
+            const float f = (s0 + j >= p.n_split || ms[j0 + j] == kNegInf) ? 0.f : fast_exp2(ms[j0 + j] - Mn);
+            tot = fmaf(av[j0 + j], f, tot);
             L = fmaf(ls[j0 + j], f, L);
           }
         }
@@ -433,6 +440,11 @@ void launch_merge(dim3 grid, dim3 block, hipStream_t st, const DecodeParams &p) 
   else if (p.n_split <= 8) hipLaunchKernelGGL((swa_decode_merge_kernel<E, 8>), grid, block, 0, st, p);
   else if (p.n_split <= 16) hipLaunchKernelGGL((swa_decode_merge_kernel<E, 16>), grid, block, 0, st, p);
   else hipLaunchKernelGGL((swa_decode_merge_kernel<E, 32>), grid, block, 0, st, p);
+}
+
+// Balanced split: the partials of (row r, head hq) from number w up to w_hi or eight of them, in steps of Hq x 128 floats.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_partials(const DecodeParams &p, int r, int hq, int w, int w_hi) {
+  return partials_from(p.ws_acc + ((int64_t)(w + r) * p.Hq + hq) * 128, (int64_t)min(w_hi - w, 7) * p.Hq * 128 + 128);
 }
 
 // Merge for the balanced split: the partials of row r are numbers w + r for the workgroups w whose
@@ -475,7 +487,7 @@ __global__ __launch_bounds__(128) void swa_decode_merge_balanced_kernel(const De
   if (n_r > 0) {
     const int per = (total + p.n_wg - 1) / p.n_wg;
     const int own = before + kBalancedRowStartChunks;          // the row's own chunks start behind its virtual ones
-    const int w_lo = own / per, w_hi = (own + n_r - 1) / per;
+    const int w_lo = __builtin_amdgcn_readfirstlane(own / per), w_hi = __builtin_amdgcn_readfirstlane((own + n_r - 1) / per);
     // a long row among short ones can have hundreds of partials: loads go out eight at a time
     for (int w = w_lo; w <= w_hi; w += 8) {
       float ms[8];
@@ -487,18 +499,18 @@ __global__ __launch_bounds__(128) void swa_decode_merge_balanced_kernel(const De
     if (M != kNegInf) {
       for (int w = w_lo; w <= w_hi; w += 8) {
         float ms[8], ls[8], av[8];
+        const __amdgpu_buffer_rsrc_t acc = row_partials(p, r, hq, w, w_hi);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const int64_t part = (int64_t)(min(w + j, w_hi) + r) * p.Hq + hq;
           ms[j] = p.ws_ml[part * 2];
           ls[j] = p.ws_ml[part * 2 + 1];
-          av[j] = p.ws_acc[part * 128 + d];
+          av[j] = load_partial(acc, j * p.Hq * 128 + d);
         }
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          const bool there = w + j <= w_hi;  // as in the merge above
-          const float f = (!there || ms[j] == kNegInf) ? 0.f : fast_exp2(ms[j] - M);
-          tot = fmaf(there ? av[j] : 0.f, f, tot);
+          const float f = (w + j > w_hi || ms[j] == kNegInf) ? 0.f : fast_exp2(ms[j] - M);
+          tot = fmaf(av[j], f, tot);
           L = fmaf(ls[j], f, L);
         }
       }
@@ -526,12 +538,13 @@ __global__ __launch_bounds__(128) void swa_decode_merge_rows_kernel(const Decode
     // than eight runs goes round again and rescales what it has): one trip for almost every row
     for (int w = w_lo; w <= w_hi; w += 8) {
       float ms[8], ls[8], av[8];
+      const __amdgpu_buffer_rsrc_t acc = row_partials(p, r, hq, w, w_hi);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const int64_t part = (int64_t)(min(w + j, w_hi) + r) * p.Hq + hq;
         ms[j] = p.ws_ml[part * 2];
         ls[j] = p.ws_ml[part * 2 + 1];
-        av[j] = p.ws_acc[part * 128 + d];
+        av[j] = load_partial(acc, j * p.Hq * 128 + d);
       }
       float Mn = M;
 #pragma unroll
@@ -542,9 +555,8 @@ __global__ __launch_bounds__(128) void swa_decode_merge_rows_kernel(const Decode
         L *= keep;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          const bool there = w + j <= w_hi;  // as in the merge above
-          const float f = (!there || ms[j] == kNegInf) ? 0.f : fast_exp2(ms[j] - Mn);
-          tot = fmaf(there ? av[j] : 0.f, f, tot);
+          const float f = (w + j > w_hi || ms[j] == kNegInf) ? 0.f : fast_exp2(ms[j] - Mn);
+          tot = fmaf(av[j], f, tot);
           L = fmaf(ls[j], f, L);
         }
       }

@@ -492,12 +492,13 @@ __device__ __forceinline__ void split_segment(const DecodeParams &p, const int32
       u32x4_t av[4][8];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
+        const bool there = s0 + j < p.n_split;  // (else: zeros, from an offset out of range; see the merge kernel)
         const int64_t part = part0 + min(s0 + j, p.n_split - 1);
         ms[j] = __hip_atomic_load(p.ws_ml + part * 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         ls[j] = __hip_atomic_load(p.ws_ml + part * 2 + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
         for (int q4 = 0; q4 < 8; ++q4)
-          av[j][q4] = __builtin_amdgcn_raw_buffer_load_b128(acc_rsrc, (int)((part * 128 + 32 * g + 4 * q4) * 4), 0, 1 << 4);
+          av[j][q4] = __builtin_amdgcn_raw_buffer_load_b128(acc_rsrc, there ? (int)((part * 128 + 32 * g + 4 * q4) * 4) : -16, 0, 1 << 4);
       }
       float Mn = M;
 #pragma unroll
@@ -510,8 +511,7 @@ __device__ __forceinline__ void split_segment(const DecodeParams &p, const int32
         L *= keep;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          if (s0 + j >= p.n_split) break;  // (the last one again: it may hold an infinity, which 0 does not undo)
-          const float f = ms[j] == kNegInf ? 0.f : fast_exp2(ms[j] - Mn);
+          const float f = (s0 + j >= p.n_split || ms[j] == kNegInf) ? 0.f : fast_exp2(ms[j] - Mn);
 #pragma unroll
           for (int q4 = 0; q4 < 8; ++q4) {
             tot[4 * q4 + 0] = fmaf(__uint_as_float(av[j][q4].x), f, tot[4 * q4 + 0]);
