@@ -243,7 +243,10 @@ int32_t sb_swa_decode_auto_split(int64_t num_rows, int32_t num_kv_heads, int32_t
  * 16 query heads per kv head), whose workgroups are smaller and more. */
 int32_t sb_swa_decode_auto_split_vector(int64_t num_rows, int32_t num_q_heads, int32_t num_kv_heads, int32_t max_seq_len,
                                         int32_t window_left);
-/* 1 if SB_DECODE_BALANCED is expected to be faster than the fixed split into n_split (>= 1) parts for rows
+/* The split count to give a call with SB_DECODE_BALANCED (what n_split = 0 does): its number of workgroups goes by it, and finer
+ * splits than runs of eight chunks only make more partials of a long row. */
+int32_t sb_swa_decode_balanced_split(int64_t num_rows, int32_t num_kv_heads, int32_t max_seq_len, int32_t window_left);
+/* 1 if SB_DECODE_BALANCED (with that split) is expected to be faster than the fixed split into n_split (>= 1) parts for rows
  * with these lengths, else 0. host_seq_lens: the step's seq_lens as a HOST array (the scheduler has them;
  * a caller without them can pass max_seq_len for every row: the balanced split adapts to the real lengths
  * on the device); no device access. */

@@ -186,6 +186,7 @@ EXPORTS = {
     "sb_abi_version": (C.c_int, []),
     "sb_last_error": (C.c_char_p, []),
     "sb_kv_append": (C.c_int, [C.POINTER(KvAppendArgs)]),
+    "sb_swa_decode_balanced_split": (i32, [i64, i32, i32, i32]),
     "sb_swa_decode_auto_split_vector": (C.c_int32, [i64, i32, i32, i32, i32]),
     "sb_swa_decode_auto_split": (i32, [i64, i32, i32, i32]),
     "sb_swa_decode_workspace_bytes": (sz, [i64, i32, i32, i32]),

@@ -678,6 +678,9 @@ static double one_round_us(int64_t wgs, int64_t n, int64_t chunks, int64_t cus) 
 // Windows of at most this many chunks are left whole.
 constexpr int64_t kWholeChunks = 11;
 
+// Rows up to which the balanced split is used (every wavefront sums over all rows' lengths).
+constexpr int64_t kBalancedMaxRows = 1024;
+
 // Workgroups of a launch (per split), and the chunks of a row.
 struct SplitShape {
   int64_t wgs, chunks, run, cus;
@@ -763,9 +766,16 @@ extern "C" int32_t sb_swa_decode_auto_split_vector(int64_t num_rows, int32_t num
   return one_round_split(s, best);
 }
 
+extern "C" int32_t sb_swa_decode_balanced_split(int64_t num_rows, int32_t num_kv_heads, int32_t max_seq_len, int32_t window_left) {
+  if (num_rows <= 0 || num_kv_heads <= 0 || max_seq_len <= 0) return 1;
+  return (int32_t)long_run_split(split_shape(num_rows, num_kv_heads, max_seq_len, window_left));
+}
+
 // The split of a call that leaves it to the library: what the rule says, with no more partials than `bytes` hold, down
 // to the split of long runs (memory that takes less than that one's partials is refused).
 static int32_t chosen_split(const sb_swa_decode_args *a, size_t bytes) {
+  if ((a->flags & SB_DECODE_BALANCED) && on_matrix_cores(a) && a->kv_quant == SB_KV_NONE && a->num_rows <= kBalancedMaxRows)
+    return sb_swa_decode_balanced_split(a->num_rows, a->num_kv_heads, a->max_seq_len, a->window_left);
   int32_t n = on_matrix_cores(a)
                   ? sb_swa_decode_auto_split(a->num_rows, a->num_kv_heads, a->max_seq_len, a->window_left)
                   : sb_swa_decode_auto_split_vector(a->num_rows, a->num_q_heads, a->num_kv_heads, a->max_seq_len, a->window_left);
@@ -774,9 +784,6 @@ static int32_t chosen_split(const sb_swa_decode_args *a, size_t bytes) {
   while (n > least && sb_swa_decode_workspace_bytes(a->num_rows, a->num_q_heads, a->head_size, n) > bytes) --n;
   return n;
 }
-
-// Rows up to which the balanced split is used (every wavefront sums over all rows' lengths).
-constexpr int64_t kBalancedMaxRows = 1024;
 
 // Workgroups per kv-head group of the balanced split: one per CU (a CU holds one at a time), fewer only
 // when the fixed split would have launched less than half as many (very little work).
@@ -799,12 +806,33 @@ extern "C" int32_t sb_swa_decode_prefer_balanced(const int32_t *host_seq_lens, i
   if (!host_seq_lens || num_rows <= 0 || num_rows > kBalancedMaxRows || n_split < 1) return 0;
   const int64_t cus = device_cu_count();
   std::vector<int64_t> chunks((size_t)num_rows);
-  int64_t total = 0;
+  int64_t total = 0, longest = 0, longest_row = 0;
   for (int64_t r = 0; r < num_rows; ++r) {
     const int64_t hi = host_seq_lens[r];
     const int64_t lo = (window_left >= 0 && hi - 1 - window_left > 0) ? hi - 1 - window_left : 0;
     chunks[r] = hi > lo ? ((hi - 1) >> 5) - (lo >> 5) + 1 : 0;
     total += chunks[r];
+    longest = std::max(longest, chunks[r]);
+    longest_row = std::max(longest_row, hi);
+  }
+  // A fixed split finer than runs of 8 chunks, all at once: against one_round_us of the workgroups there are, the estimate for
+  // the balanced split into its own number of workgroups, fitted to 355 launches of 2 .. 128 rows of 60 .. 6000 keys (rms
+  // 6.5 %; what a long row among short ones costs is the merge of its many partials). Measured, us, fixed -> balanced: 3 rows of 60,
+  // 60, 6000 keys 17.1 -> 18.8; 4 uneven ones of up to 6000 18.9 -> 21.7; 64 / 100 uneven ones of up to 600 / 400 18.3 / 21.5 -> 16.4 /
+  // 17.6. Chosen so, the 200 shapes measured take 0.99 of what the model below made of them on average, and none more than 1.08.
+  const int64_t runs = long_run_split(split_shape(num_rows, 4, (int32_t)longest_row, window_left));
+  if (total > 0 && num_rows * n_split <= cus && n_split > runs) {
+    int64_t most = 0, active = 0;
+    for (int64_t r = 0; r < num_rows; ++r) {
+      const int64_t cps = (chunks[r] + n_split - 1) / n_split;
+      most = std::max(most, cps);
+      if (cps) active += (chunks[r] + cps - 1) / cps;
+    }
+    const int64_t per = (total + balanced_workgroups(num_rows, runs < 2 ? 2 : runs) - 1) / balanced_workgroups(num_rows, runs < 2 ? 2 : runs);
+    const double fill = (double)active / (double)cus, fill_b = (double)((total + per - 1) / per) / (double)cus;
+    const double fixed_us = 5.7 + (double)most * (1.82 + 0.84 * fill * fill) + 0.14 * (double)n_split;
+    const double balanced_us = 7.05 + (double)per * (2.0 + 0.74 * fill_b * fill_b) + 0.109 * (double)longest / (double)per + 0.045 * (double)num_rows;
+    return balanced_us < fixed_us ? 1 : 0;
   }
   // Fixed split: its workgroups (split-major, rows fastest: the dispatch order) handed to the CUs as
   // these fall free, one workgroup per CU at a time; each costs its chunks plus the fixed part.

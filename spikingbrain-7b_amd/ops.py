@@ -302,8 +302,8 @@ def swa_decode_attention(
     if window_left >= 0:
         max_seq_len = max(1, max_seq_len)
     L = N.lib()
-    auto_balance = balanced is None
-    if n_split == 0:
+    auto_balance, auto_split = balanced is None, n_split == 0
+    if auto_split:
         if q.dtype != torch.float32 and not force_valu and D == 128 and Hq <= 16 * Hkv:
             n_split = L.sb_swa_decode_auto_split(R, Hkv, int(max_seq_len), int(window_left))
         else:   # the vector kernel
@@ -324,6 +324,8 @@ def swa_decode_attention(
                 if len(_SHAPE_POLICY) >= 4096:   # lengths that grow step by step would fill it without end
                     _SHAPE_POLICY.clear()
                 balanced = _SHAPE_POLICY[key] = prefer_balanced_split([int(max_seq_len)] * R, window_left, n_split)
+    if balanced and can_balance and auto_split:
+        n_split = L.sb_swa_decode_balanced_split(R, Hkv, int(max_seq_len), int(window_left))
     if balanced and can_balance and n_split < 2:
         n_split = 2  # the balanced split always goes through partial results and the merge
     ws_bytes = L.sb_swa_decode_workspace_bytes(R, Hq, D, n_split)

@@ -140,3 +140,16 @@ def test_auto_split_of_the_vector_kernel(sb, rows, q_heads, kv_heads, keys, spli
     n = sb._native.lib().sb_swa_decode_auto_split_vector(rows, q_heads, kv_heads, keys, 4096)
     parts = {7: 1, 28: 4, 1: 1, 4: 1}[q_heads // kv_heads]
     assert n == split and (rows * kv_heads * parts * n <= 256 or keys // n >= 8 * 32)
+
+
+def test_balanced_or_fixed_split_of_small_batches(sb):
+    """One long row among a few short ones is cut finely (its partials would be merged one by one otherwise); many
+    short rows of uneven lengths run balanced; and the balanced split keeps runs of eight chunks whatever the fixed one does."""
+    L, prefer = sb._native.lib(), sb.ops.prefer_balanced_split
+    auto = lambda lens: L.sb_swa_decode_auto_split(len(lens), 4, max(lens), 4096)
+    uneven = lambda rows, longest: [max(1, int(longest * (i / rows) ** 2)) for i in range(1, rows + 1)]
+    for lens, balanced in (([60, 60, 6000], False), ([60] * 7 + [6000], False), (uneven(4, 6000), False), ([6000] * 8, False), ([400] * 100, False),
+                           (uneven(100, 400), True), (uneven(128, 400), True), (uneven(64, 600), True)):
+        assert prefer(lens, 4096, auto(lens)) is balanced, lens
+    assert [L.sb_swa_decode_balanced_split(rows, 4, keys, 4096) for rows, keys in ((4, 6000), (64, 400), (0, 400), (64, 20000))] == [15, 1, 1, 4]
+    assert not prefer([0, 0], 4096, 4)
