@@ -2,6 +2,8 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <atomic>
+
 #include "common.h"
 
 namespace {
@@ -30,6 +32,17 @@ int check_launch(const char *what) {
   if (e == hipSuccess) return SB_OK;
   set_error("%s: launch failed: %s", what, hipGetErrorString(e));
   return (int)e;
+}
+
+int device_cu_count() {
+  static std::atomic<int> known[64];  // per device; a device's count does not change
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 256;
+  const bool keep = dev >= 0 && dev < 64;
+  if (keep && (cus = known[dev].load(std::memory_order_relaxed)) > 0) return cus;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) return 256;
+  if (keep) known[dev].store(cus, std::memory_order_relaxed);
+  return cus;
 }
 
 }  // namespace sb_host

@@ -122,4 +122,5 @@ namespace sb_host {
 void set_error(const char *fmt, ...);
 int fail(int code, const char *fmt, ...);
 int check_launch(const char *what);
+int device_cu_count();  // compute units of the current device (256 on MI355X); 256 if the query fails
 }  // namespace sb_host

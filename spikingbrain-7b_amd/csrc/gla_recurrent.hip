@@ -579,12 +579,13 @@ extern "C" int32_t sb_gla_prompt_segments(const sb_gla_recurrent_args *a) {
   const int G = a->q_heads_per_state > 1 ? a->q_heads_per_state : 1;
   const int64_t chains = a->batch * (int64_t)(a->num_heads / G);
   if (chains == 0) return 1;
+  const int64_t cus = sb_host::device_cu_count();
   int64_t n;
   if (G > 1) {
-    n = 256 / chains < a->seq_len / 48 ? 256 / chains : a->seq_len / 48;
+    n = cus / chains < a->seq_len / 48 ? cus / chains : a->seq_len / 48;
     if (n < 2) return 1;
   } else {
-    n = 512 / chains < a->seq_len / 64 ? 512 / chains : a->seq_len / 64;
+    n = 2 * cus / chains < a->seq_len / 64 ? 2 * cus / chains : a->seq_len / 64;
     if (n < 4 || a->seq_len < (n < 8 ? 1024 : 512)) return 1;
   }
   const int seg = segment_tokens(a->seq_len, (int)n);

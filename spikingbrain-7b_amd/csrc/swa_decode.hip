@@ -634,15 +634,6 @@ inline int64_t round_up(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 
 }  // namespace
 
-// Number of compute units of the current device (256 on MI355X); 256 if the query fails.
-static int device_cu_count() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    return 256;
-  return cus;
-}
-
 // Cost model of a split launch, in units of one 32-key chunk streamed by one workgroup while every CU is
 // busy (about 2.5 us), fitted to launches of 16 .. 384 window-saturated rows of the 7B shape:
 //   fixed split    : rounds of workgroups over the CUs (one workgroup fits a CU at a time), each round
@@ -692,7 +683,7 @@ static SplitShape split_shape(int64_t num_rows, int32_t num_kv_heads, int32_t ma
   s.chunks = (keys + 31) / 32 + 1;  // +1: an unaligned window touches one more chunk
   s.run = keys < max_seq_len ? s.chunks : s.chunks - 1;  // (a window that starts at the first key is aligned)
   s.wgs = num_rows * ((num_kv_heads + 3) / 4);  // one workgroup per (row, group of up to 4 kv heads)
-  s.cus = device_cu_count();
+  s.cus = sb_host::device_cu_count();
   return s;
 }
 
@@ -788,7 +779,7 @@ static int32_t chosen_split(const sb_swa_decode_args *a, size_t bytes) {
 // Workgroups per kv-head group of the balanced split: one per CU (a CU holds one at a time), fewer only
 // when the fixed split would have launched less than half as many (very little work).
 static int64_t balanced_workgroups(int64_t num_rows, int64_t n_split) {
-  const int64_t fixed = num_rows * n_split, cus = device_cu_count();
+  const int64_t fixed = num_rows * n_split, cus = sb_host::device_cu_count();
   return fixed * 2 >= cus ? cus : fixed;
 }
 
@@ -804,7 +795,7 @@ static int64_t partial_slots(int64_t num_rows, int64_t n_split) {
 extern "C" int32_t sb_swa_decode_prefer_balanced(const int32_t *host_seq_lens, int64_t num_rows,
                                                  int32_t window_left, int32_t n_split) {
   if (!host_seq_lens || num_rows <= 0 || num_rows > kBalancedMaxRows || n_split < 1) return 0;
-  const int64_t cus = device_cu_count();
+  const int64_t cus = sb_host::device_cu_count();
   std::vector<int64_t> chunks((size_t)num_rows);
   int64_t total = 0, longest = 0, longest_row = 0;
   for (int64_t r = 0; r < num_rows; ++r) {

@@ -728,8 +728,6 @@ int64_t most_chunks(const sb_swa_prefill_args *a, int64_t max_keys) {
   return (span + 30) / 32 + 1;
 }
 
-constexpr int64_t kCUs = 256;
-
 // How a call is spread over the GPU: with groups of four heads a workgroup of eight wavefronts fills a CU, and a call
 // of `wgs` of them takes as long as its longest walk while wgs <= 256. Two ways to shorten that:
 //  * pairs: workgroups of two heads and four wavefronts, two to a CU. Measured, with L the longest walk in chunks and L' the
@@ -752,22 +750,22 @@ int64_t quad_workgroups(const sb_swa_prefill_args *a) {
   return a->num_tiles * a->num_kv_heads * ((a->num_q_heads / a->num_kv_heads + 3) / 4);
 }
 bool pairs_pay(const sb_swa_prefill_args *a, int64_t chunks, int64_t parts) {
-  const int64_t wgs = quad_workgroups(a) * parts;
-  if (2 * wgs <= kCUs) return true;
-  if (parts > 1 || 2 * wgs > 3 * kCUs) return false;
-  if (wgs > kCUs) return chunks <= 2 * a->num_tiles + 2;
+  const int64_t wgs = quad_workgroups(a) * parts, cus = sb_host::device_cu_count();
+  if (2 * wgs <= cus) return true;
+  if (parts > 1 || 2 * wgs > 3 * cus) return false;
+  if (wgs > cus) return chunks <= 2 * a->num_tiles + 2;
   if (!a->tile_keys) return false;   // (unknown: as if all walks were equal)
   const int64_t pairs_per_tile = (int64_t)a->num_kv_heads * ((a->num_q_heads / a->num_kv_heads + 1) / 2);
-  const int64_t sharing = kCUs / pairs_per_tile;   // tiles in front of the first one that shares
+  const int64_t sharing = cus / pairs_per_tile;   // tiles in front of the first one that shares
   return sharing >= a->num_tiles || (double)most_chunks(a, a->tile_keys[sharing]) < 6.0 + 0.63 * (double)chunks;
 }
 Spread spread_of(const sb_swa_prefill_args *a, int64_t max_keys) {
-  const int64_t chunks = most_chunks(a, max_keys), wgs = quad_workgroups(a);
+  const int64_t chunks = most_chunks(a, max_keys), wgs = quad_workgroups(a), cus = sb_host::device_cu_count();
   Spread best{1, pairs_pay(a, chunks, 1)};
   double best_us = 5.0 + (best.pairs ? 0.69 : 0.9) * (double)chunks;
-  for (int64_t n = 2; n * wgs <= kCUs && 8 * n <= chunks; ++n) {
+  for (int64_t n = 2; n * wgs <= cus && 8 * n <= chunks; ++n) {
     const bool pairs = pairs_pay(a, chunks, n);
-    const double us = 13.5 + 0.28 * (double)n + 8.0 * (double)(n * wgs) / (double)kCUs +
+    const double us = 13.5 + 0.28 * (double)n + 8.0 * (double)(n * wgs) / (double)cus +
                       (pairs ? 0.69 : 0.86) * (double)((chunks + n - 1) / n);
     if (us < best_us) {
       best = Spread{(int)n, pairs};
