@@ -1,12 +1,14 @@
 """Prompt attention with the keys of a tile cut into parts (fp32 partials and a merge) and with workgroups of two heads:
-against float64 attention. Element outputs are rounded to bf16 from fp32 and the probabilities to bf16 on the way: 1e-2 of
-the 2-norm, the same bound as for uncut calls; cut against uncut the same, with the log-sum-exp (fp32 throughout) within
-2e-5 + the two's rounding of scores."""
+against float64 attention, over dense keys and over paged element and byte-code caches, in bf16 and fp16. Outputs are rounded
+from fp32 and the probabilities on the way: 1e-2 (bf16) or 1.25e-3 (fp16, three more bits) of the 2-norm, the same bound for cut
+and uncut calls and between the two. Their log-sum-exps come from the same fp32 scores, summed in another order: terms of up to
+1100 keys, each within 2^-24 of itself, move the logarithm by 6.6e-5 at most, and a value below 16 has places of 1e-6: 1e-4."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 D = 128
+BOUND = {torch.bfloat16: 1e-2, torch.float16: 1.25e-3}
 
 
 def _reference(q, k, v, lens, ctx, window, key_lo, G):
@@ -28,11 +30,11 @@ def _reference(q, k, v, lens, ctx, window, key_lo, G):
 
 @pytest.mark.parametrize("G", [1, 2, 3, 4, 5, 7, 8])
 @pytest.mark.parametrize("lens,ctx,window", [([1], 0, -1), ([65], 300, -1), ([64, 3], 257, 100), ([130, 1, 70], 0, 4096), ([40], 1000, 511)])
-@pytest.mark.parametrize("n_parts", [0, 1, 2, 3, 7, 40])
-def test_parts_and_pairs(sb, dev, G, lens, ctx, window, n_parts):
+@pytest.mark.parametrize("n_parts,dtype", [(n, torch.bfloat16) for n in (0, 1, 2, 3, 7, 40)] + [(3, torch.float16)])
+def test_parts_and_pairs(sb, dev, G, lens, ctx, window, n_parts, dtype):
     g = torch.Generator().manual_seed(G * 100 + n_parts)
     Hkv, T, Lk = 2, sum(lens), sum(lens) + ctx * len(lens)
-    q, k, v = torch.randn(T, Hkv * G, D, generator=g).bfloat16(), torch.randn(Lk, Hkv, D, generator=g).bfloat16(), torch.randn(Lk, Hkv, D, generator=g).bfloat16()
+    q, k, v = (torch.randn(n, h, D, generator=g).to(dtype) for n, h in ((T, Hkv * G), (Lk, Hkv), (Lk, Hkv)))
     key_lo = [(7 * s) % (n + ctx + 2) for s, n in enumerate(lens)]      # some rows see nothing: zeros
     kv_start = torch.tensor([0] + [n + ctx for n in lens]).cumsum(0)[:-1].to(dev)
     run = lambda parts: sb.ops.swa_prefill_attention(
@@ -40,8 +42,11 @@ def test_parts_and_pairs(sb, dev, G, lens, ctx, window, n_parts):
         key_lo=torch.tensor(key_lo, dtype=torch.int32, device=dev), window_left=window, return_lse=True, n_parts=parts)
     out, lse = run(n_parts)
     ref = _reference(q, k, v, lens, ctx, window, key_lo, G)
-    assert (out.cpu().double() - ref).norm() <= 1e-2 * ref.norm()
+    assert (out.cpu().double() - ref).norm() <= BOUND[dtype] * ref.norm()
+    if n_parts == 1:
+        return
     out1, lse1 = run(1)
+    assert (out.double() - out1.double()).norm() <= BOUND[dtype] * out1.double().norm()
     assert torch.equal(torch.isneginf(lse), torch.isneginf(lse1))
     ok = ~torch.isneginf(lse)
     assert (lse[ok] - lse1[ok]).abs().max() <= 1e-4
@@ -62,7 +67,9 @@ def test_starts_as_32_bit_values(sb, dev):
 
 @pytest.mark.parametrize("kv", ["bf16", "int8", "fp8"])
 def test_paged_parts_with_meta_rows_and_options(sb, dev, kv):
-    """The parts over a paged cache (element and byte codes), with meta rows (walked by the first part) and score options."""
+    """The parts over a paged cache (element and byte codes), with meta rows (walked by the first part) and score options,
+    against float64 attention over the dequantised rows (the soft cap's exp2 and reciprocal are of the hardware's precision,
+    2^-22 of a score of at most 20: 5e-6 more)."""
     g = torch.Generator().manual_seed(5)
     Hkv, G, bs, n, ctx = 2, 4, 16, 50, 500
     L = n + ctx
@@ -83,9 +90,25 @@ def test_paged_parts_with_meta_rows_and_options(sb, dev, kv):
     kw.update(meta_k=meta[0], meta_v=meta[1], softcap=20.0, alibi_slopes=torch.linspace(0.01, 0.3, Hkv * G, device=dev))
     run = lambda parts: sb.ops.swa_prefill_attention(q, cache[0], cache[1], query_lens=[n], seq_lens_k=[L], block_table=table,
                                                      window_left=400, return_lse=True, n_parts=parts, **kw)
+    order = table[0].long().cpu()
+    rows = cache.cpu().float()[:, order].flatten(1, 2)[:, :L]                       # as the kernel takes them: rounded to bf16
+    if kv == "int8":
+        rows = (rows * sc.cpu()[:, order].permute(0, 1, 3, 2).flatten(1, 2)[:, :L, :, None]).bfloat16()
+    elif kv == "fp8":
+        rows = (rows * torch.tensor([0.5, 2.0])[:, None, None, None]).bfloat16()
+    keys, values = (torch.cat([m.cpu().double(), r.double()]).repeat_interleave(G, 1) for m, r in zip(meta, rows))
+    score = torch.einsum("nhd,khd->hnk", q.cpu().double(), keys) * D ** -0.5
+    slope = torch.linspace(0.01, 0.3, Hkv * G).double()[:, None, None]
+    pos, key, m = torch.arange(n)[:, None], torch.arange(L)[None], torch.arange(37)[None]
+    dist = torch.cat([(pos + 37 - n - m).abs(), pos + ctx - key], 1)                # meta rows: one stacked sequence of n queries
+    score = 20 * torch.tanh(score / 20) - slope * dist
+    score.masked_fill_(torch.cat([torch.zeros(n, 37, dtype=torch.bool), (key > pos + ctx) | (key < pos + ctx - 400)], 1), float("-inf"))
+    ref, ref_lse = torch.einsum("hnk,khd->nhd", torch.softmax(score, -1), values), torch.logsumexp(score, -1).t()
     one, lse1 = run(1)
-    for parts in (2, 5):
+    for parts in (1, 2, 5):
         out, lse = run(parts)
+        assert (out.cpu().double() - ref).norm() <= BOUND[torch.bfloat16] * ref.norm()
+        assert (lse.cpu().double() - ref_lse).abs().max() <= 1e-4
         assert (out.float() - one.float()).norm() <= 5e-3 * one.float().norm()   # both round the same sums to bf16
         assert (lse - lse1).abs().max() <= 1e-4
 
