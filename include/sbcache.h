@@ -299,8 +299,8 @@ int sb_swa_decode_static(const sb_swa_decode_args *args);
 #define SB_GLA_VECTOR_ONLY 1
 #define SB_GLA_CHECK_GATES 2 /* matrix-core block form: count gates beyond its range (see flags, sb_gla_gate_range_hits) */
 #define SB_GLA_PER_HEAD 4 /* shared states, matrix-core block form: one workgroup per query head (two launches), whatever the batch */
-#define SB_GLA_ZERO_SKIPPED 16 /* calls of one step: the outputs of rows whose slot is negative are set to zero (else left as they are) */
 #define SB_GLA_GROUP_PASS 8 /* ... one workgroup per group of query heads (one launch), whatever the batch; default: by batch size */
+#define SB_GLA_ZERO_SKIPPED 16 /* calls of one step: the outputs of rows whose slot is negative are set to zero (else left as they are) */
 
 typedef struct sb_gla_recurrent_args {
   const void *q, *k, *v, *g;

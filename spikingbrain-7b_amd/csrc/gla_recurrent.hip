@@ -564,14 +564,15 @@ bool block_form(const sb_gla_recurrent_args *a) {
 int segment_tokens(int seq_len, int n) { return ((seq_len + n - 1) / n + 31) / 32 * 32; }
 }  // namespace
 
-// Where the line lies (28 : 28 and 28 : 4 heads, fp32 state and gate, us per call uncut -> cut into n, measured):
-// * one state per head: two workgroups fit a CU and a cut prompt does 1.6 x the work, so it pays while 512
-//   workgroups allow four segments (18 at one prompt), of 64 tokens or more: 1 x 512 46 -> 28 (8), 1 x 3001 233 -> 63
-//   (16), 1 x 8192 691 -> 148, 2 x 2048 161 -> 75, 4 x 4096 358 -> 300; six prompts 371 -> 402 (3). The two extra
-//   launches cost about 15 us: 4 x 600 54 -> 57;
+// Where the line lies (28 : 28 and 28 : 4 heads, fp32 state and gate, us per call uncut -> cut into the n this rule takes,
+// from graph replays):
+// * one state per head: two workgroups fit a CU and a cut prompt does 1.6 x the work, so it pays while two workgroups
+//   per CU allow four segments (18 at one prompt), of 64 tokens or more: 1 x 512 47 -> 29 (8), 1 x 3001 260 -> 73 (16), 1 x 8192
+//   694 -> 162 (18), 2 x 2048 183 -> 92 (8), 4 x 4096 363 -> 304 (4); six prompts in 3 371 -> 402. The two extra launches cost
+//   about 15 us: 4 x 600 in 2 61 -> 66;
 // * shared states: the one-pass kernel per group fills a CU by itself and beats a workgroup per query head as soon as
-//   there are enough of them: 1 x 512 87 -> 27 (16), 1 x 8192 1250 -> 72 (64), 4 x 4096 684 -> 121, 16 x 8192 1738 -> 786
-//   (4), 26 x 4096 1230 -> 766 (2).
+//   there are enough of them: 1 x 512 90 -> 35 (8), 1 x 8192 1348 -> 79 (64), 4 x 4096 696 -> 124 (16), 16 x 8192 1736 -> 784
+//   (4), 26 x 4096 1252 -> 769 (2). (Chosen by hand, 1 x 512 in 16 segments of 32 tokens takes 29.)
 extern "C" int32_t sb_gla_prompt_segments(const sb_gla_recurrent_args *a) {
   if (!a || a->batch <= 0 || a->num_heads <= 0 || a->seq_len < 256 || !block_form(a) ||
       (a->flags & (SB_GLA_CHECK_GATES | SB_GLA_PER_HEAD | SB_GLA_GROUP_PASS)))

@@ -8,10 +8,10 @@
 // Work decomposition
 //   grid = (query tiles of 64 tokens, kv heads, groups of 4 or 3 query heads of the kv head, or of 2 and 1 in small
 //   calls; parts of the tile's keys); a workgroup covers one of those groups (7 = 4 + 3 = 2 + 2 + 2 + 1; behind groups of
-//   four a last group of 1 or 2 heads takes a launch of its own). Every wavefront owns two "column blocks" of
-//   16 tokens x 1 head (32 score columns, no padding): a pair of heads is served by 4 wavefronts (one
-//   per 16-token sub-tile), an odd last head by 2 wavefronts (two sub-tiles each) - 8 wavefronts for 4
-//   heads, 6 for 3. At 256 registers per wavefront two of them share a SIMD.
+//   four a last group of 1 or 2 heads takes a launch of its own). A wavefront owns "column blocks" of 16 tokens x 1
+//   head (no padding): a pair of heads is served by 4 wavefronts (one per 16-token sub-tile, a block of each head),
+//   an odd last head by 4 wavefronts of one block each - 8 wavefronts for 4 heads and for 3. At 256 registers per
+//   wavefront two of them share a SIMD.
 //   The workgroup walks the union of its tokens' windows in chunks of 32 keys. Each chunk of K and V
 //   (32 rows x 256 B each) is fetched from global memory ONCE per workgroup (every wavefront of an
 //   8-wavefront workgroup fetches 4 rows with whole-row 16-byte lanes, else the first four fetch 8) into a
@@ -133,11 +133,9 @@ __device__ __forceinline__ uint2 load_transposed(const char *row) {
 constexpr float kNegInf = kNegInfF;
 constexpr float kRaise = 8.f;
 
-// NHEADS query heads of one kv head per workgroup; wavefronts own two column blocks each
-// (a column block = 16 tokens x 1 head): head pairs are served by 4 wavefronts (one per 16-token
-// sub-tile, both heads of the pair), an odd last head by 2 wavefronts (two sub-tiles each).
-// NHEADS = 4 also serves 3 heads (the last four wavefronts then own one column block each) and NHEADS = 2 one, so that
-// all groups of a GQA group of 7 are one launch either way.
+// NHEADS query heads of one kv head per workgroup: head pairs are served by 4 wavefronts of two column blocks (one
+// 16-token sub-tile, both heads of the pair), an odd last head by 4 of one. NHEADS = 4 also serves 3 heads and NHEADS = 2
+// one, so that all groups of a GQA group of 7 are one launch either way.
 template <int NHEADS>
 struct Shape {
   static constexpr int kWaves = 4 * (NHEADS / 2) + 4 * (NHEADS % 2);
@@ -741,7 +739,8 @@ int64_t most_chunks(const sb_swa_prefill_args *a, int64_t max_keys) {
 //    long: 3059 tokens, window 4096 92.8 -> 88.8; behind 4200, windows 512 / 1024 / 2048 / 4096 52.4 / 77.1 / 127 / 228 -> 47 / 72.9 / 124 /
 //    230; beyond that they lose (1 x 6000: 256 -> 271).
 //  * parts: the keys of a walk cut into parts of 8 chunks or more side by side, at the price of fp32 partials and
-//    a merge (64 / 200 / 512 / 1024 tokens behind 4200: 123 -> 24 (16 parts) / 33 (8) / 49 (4) / 80 (2) us).
+//    a merge (64 / 200 / 512 / 1024 tokens behind 4200: 100 with pairs, 123 with groups of four -> 27.5 (12 parts) / 37 (8) /
+//    54 (4) / 85 (2) us; 64 tokens in 8 parts 25.7, which the estimate below does not find).
 struct Spread {
   int parts;
   bool pairs;
