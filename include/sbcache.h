@@ -129,7 +129,7 @@ int sb_kv_append(const sb_kv_append_args *args);
 /* bf16/fp16 fixed split, phases 0, no meta tokens: merge the partial results inside the split kernel instead
  * of in a kernel of its own. The splits of a row run on one XCD (the launch sees to that), so the last of
  * its wavefronts to finish can pick the others' partials up from the shared L2 without any cache write-back;
- * same arithmetic and order as the merge kernel, same bits. Measured NOT faster on MI355X at 16..128 rows
+ * same arithmetic and order as the merge kernel of fewer than 12 splits, same bits as there. Measured NOT faster on MI355X at 16..128 rows
  * (the hand-over chain at the end of the kernel costs what the second launch costs), hence opt-in. Needs the
  * workspace's first 64 KiB zeroed before its first use (see below). */
 #define SB_DECODE_MERGE_IN_KERNEL 4

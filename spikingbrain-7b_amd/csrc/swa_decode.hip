@@ -378,7 +378,7 @@ __global__ __launch_bounds__(256) void swa_decode_split_kernel(const DecodeParam
 
 // One workgroup of head_size threads per (query row, query head): log-sum-exp merge of the splits.
 // kBatch splits per trip to memory, every load of a trip issued before any is used: the kernel is latency and little
-// else, so the host takes the batch that covers the split count in one or two trips. The arithmetic goes four
+// else, so the host takes the batch that covers the split count in one trip. The arithmetic goes four
 // splits at a time in the same order whatever the batch (same bits); from four to four the running sums are
 // rescaled to the new maximum. A trip's loads past the last partial are out of their buffer's range and give zeros:
 // that partial again, times 0, would be a NaN where it holds an infinity (and a select on the loaded value makes the
@@ -434,12 +434,78 @@ __global__ __launch_bounds__(256) void swa_decode_merge_kernel(const DecodeParam
   if (d == 0 && p.lse) p.lse[rh] = L > 0.f ? (M + log2f(L)) * kLn2 : kNegInf;
 }
 
+// The same merge of many partials: four groups of head_size threads take every fourth partial, kBatch of them per trip, and the
+// four sums are put together through LDS. One thread per (row, head, dim) goes through its partials one behind the other
+// (7 us at 43, and empty ones count: a step captured for full windows merges all its splits over any context). Split + merge, us,
+// narrow -> wide: 1 row x 4097 keys in 43 splits 17.0 -> 12.8, 8 x 4097 in 26 21.6 -> 19.6, 4 rows of 300 keys in 33 13.0 -> 9.6, 8 of 366 in
+// 26 12.3 -> 10.3; 16 x 1000 in 12 14.9 -> 14.6, 1 x 400 in 8 9.5 -> 9.1 but 32 x 600 in 8 15.6 -> 16.2, 64 x 4097 in 4 85.9 -> 87.8.
+template <typename E, int kBatch>
+__global__ __launch_bounds__(1024) void swa_decode_merge_wide_kernel(const DecodeParams p) {
+  constexpr int kGroups = 4;
+  const int64_t rh = blockIdx.x;  // r*Hq + hq
+  const int64_t r = rh / p.Hq;
+  const int hq = (int)(rh - r * p.Hq);
+  const int d = threadIdx.x, group = threadIdx.y;
+  const __amdgpu_buffer_rsrc_t ml = partials_from(p.ws_ml + rh * p.n_split * 2, p.n_split * 2);
+  const __amdgpu_buffer_rsrc_t acc = partials_from(p.ws_acc + rh * p.n_split * p.D, p.n_split * p.D);
+  float tot = 0.f, L = 0.f, M = kNegInf;
+  for (int b0 = group; b0 < p.n_split; b0 += kGroups * kBatch) {
+    float ms[kBatch], ls[kBatch], av[kBatch];
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      const int s = b0 + kGroups * j;
+      ms[j] = load_partial(ml, 2 * s);
+      ls[j] = load_partial(ml, 2 * s + 1);
+      av[j] = load_partial(acc, s * p.D + d);
+    }
+    float Mn = M;
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j)
+      if (b0 + kGroups * j < p.n_split) Mn = fmaxf(Mn, ms[j]);
+    if (Mn != kNegInf) {
+      const float keep = (M == kNegInf) ? 0.f : fast_exp2(M - Mn);
+      tot *= keep;
+      L *= keep;
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j) {
+        const float f = (b0 + kGroups * j >= p.n_split || ms[j] == kNegInf) ? 0.f : fast_exp2(ms[j] - Mn);
+        tot = fmaf(av[j], f, tot);
+        L = fmaf(ls[j], f, L);
+      }
+    }
+    M = Mn;
+  }
+  __shared__ float s_tot[kGroups][256], s_ml[kGroups][2];
+  s_tot[group][d] = tot;
+  if (d == 0) {
+    s_ml[group][0] = M;
+    s_ml[group][1] = L;
+  }
+  __syncthreads();
+  if (group != 0) return;
+  M = fmaxf(fmaxf(s_ml[0][0], s_ml[1][0]), fmaxf(s_ml[2][0], s_ml[3][0]));
+  tot = L = 0.f;
+#pragma unroll
+  for (int g = 0; g < kGroups; ++g) {
+    const float f = s_ml[g][0] == kNegInf ? 0.f : fast_exp2(s_ml[g][0] - M);
+    tot = fmaf(s_tot[g][d], f, tot);
+    L = fmaf(s_ml[g][1], f, L);
+  }
+  store_out<E>(p.out, r * p.o_sr + (int64_t)hq * p.o_sh + d, L > 0.f ? tot / L : 0.f);
+  if (d == 0 && p.lse) p.lse[rh] = L > 0.f ? (M + log2f(L)) * kLn2 : kNegInf;
+}
+
+constexpr int kWideMergeSplits = 12;
 template <typename E>
 void launch_merge(dim3 grid, dim3 block, hipStream_t st, const DecodeParams &p) {
+  const dim3 wide(block.x, 4);
   if (p.n_split <= 4) hipLaunchKernelGGL((swa_decode_merge_kernel<E, 4>), grid, block, 0, st, p);
   else if (p.n_split <= 8) hipLaunchKernelGGL((swa_decode_merge_kernel<E, 8>), grid, block, 0, st, p);
-  else if (p.n_split <= 16) hipLaunchKernelGGL((swa_decode_merge_kernel<E, 16>), grid, block, 0, st, p);
-  else hipLaunchKernelGGL((swa_decode_merge_kernel<E, 32>), grid, block, 0, st, p);
+  else if (p.n_split < kWideMergeSplits) hipLaunchKernelGGL((swa_decode_merge_kernel<E, 16>), grid, block, 0, st, p);
+  else if (p.n_split <= 16) hipLaunchKernelGGL((swa_decode_merge_wide_kernel<E, 4>), grid, wide, 0, st, p);
+  else if (p.n_split <= 32) hipLaunchKernelGGL((swa_decode_merge_wide_kernel<E, 8>), grid, wide, 0, st, p);
+  else if (p.n_split <= 48) hipLaunchKernelGGL((swa_decode_merge_wide_kernel<E, 12>), grid, wide, 0, st, p);
+  else hipLaunchKernelGGL((swa_decode_merge_wide_kernel<E, 16>), grid, wide, 0, st, p);
 }
 
 // Balanced split: the partials of (row r, head hq) from number w up to w_hi or eight of them, in steps of Hq x 128 floats.

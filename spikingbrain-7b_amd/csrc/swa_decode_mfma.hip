@@ -451,7 +451,7 @@ __device__ __forceinline__ void split_segment(const DecodeParams &p, const int32
   // partials from one wavefront to another takes no cache write-back: a wavefront waits until its own
   // partial stores have been acknowledged by the L2, then bumps the pair's counter (an atomic executed in
   // that L2); whoever sees n_split - 1 knows that every partial of the pair is in the L2, reads them with
-  // loads that skip its CU's L1 (sc1), merges exactly as swa_decode_merge_kernel does (same order, same
+  // loads that skip its CU's L1 (sc1), merges exactly as swa_decode_merge_kernel does (the merge of fewer than 12 splits: same order, same
   // arithmetic: the same bits) and zeroes the counter for the next launch. Nobody waits for anybody.
   // (Across XCDs the same hand-over needs the dirty L2 lines written back to memory and the reader's L2
   // invalidated: with agent-scope fences that made the whole step 1.5x slower.)

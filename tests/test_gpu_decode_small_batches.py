@@ -1,5 +1,5 @@
-"""Small decode batches: split counts at the edges of the merge kernel's batches (4, 8, 16, 32 partials per trip), in fp32
-against float64 attention (2e-6 of the largest value: 32-bit sums over at most 700 keys), and the bf16 stream kernel at
+"""Small decode batches: split counts at the edges of the merge kernels' batches (4, 8 and, below 12, 16 partials per trip;
+from 12 on 16, 32, 48 and 64 by four groups of threads), in fp32 against float64 attention (2e-6 of the largest value: 32-bit sums over at most 700 keys), and the bf16 stream kernel at
 the split the library chooses against the same rows unsplit (both round fp32 results to bf16: one last place, 2^-7)."""
 import pytest
 import torch
@@ -32,7 +32,7 @@ def _reference(q, kv, tables, lens, window):
     return torch.stack(out)
 
 
-@pytest.mark.parametrize("n_split", [2, 4, 5, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 65])
+@pytest.mark.parametrize("n_split", [2, 4, 5, 8, 9, 11, 12, 13, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 130])
 def test_merge_of_many_partials(sb, dev, n_split):
     lens = [700, 33, 1, 512, 97]          # rows with fewer chunks than splits leave empty partials
     q, kv, tables, sl = _problem(dev, torch.float32, lens, n_split)
@@ -56,7 +56,7 @@ def test_chosen_split_matches_unsplit_rows(sb, dev, rows, length):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("how", [dict(n_split=n, balanced=False) for n in (2, 3, 5, 9)] + [
+@pytest.mark.parametrize("how", [dict(n_split=n, balanced=False) for n in (2, 3, 5, 9, 10, 13)] + [
     dict(n_split=3, merge_in_kernel=True, balanced=False), dict(n_split=3, balanced=True), dict(n_split=3, balanced=True, per_segment=True)])
 def test_infinite_value_in_the_last_partial(sb, dev, dtype, how):
     """A visible key whose value is infinite makes the output infinite however the row is cut: the merges fill the
