@@ -87,13 +87,19 @@ __device__ __forceinline__ float row16_allreduce_sum(float v) {
 // exp2 with the hardware instruction (inputs here are <= 0 or -inf).
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// Block that holds 16-key tile t of a paged sequence: t / tiles_per_block by multiplication with magic =
-// ceil(2^31 / tiles_per_block). The product exceeds the quotient by t * e / (2^31 * tiles_per_block), e = magic * tiles_per_block -
-// 2^31 < tiles_per_block: less than one for every 32-bit t, but enough to reach the next block from t = 2^31 / e on
-// (741 thousand keys in one block of 46410 tiles), hence the correction.
-__device__ __forceinline__ int tile_block(int t, int tiles_per_block, uint32_t magic) {
-  const int b = (int)__umulhi((uint32_t)t << 1, magic);
-  return b - (b * tiles_per_block > t);
+// Block that holds 16-key tile t (t < 2^27: a sequence has 32-bit keys) of a paged sequence: t / d by a multiplication that is
+// exact there. With l = ceil(log2 d) and m = ceil(2^(27 + l) / d), m d - 2^(27 + l) < d <= 2^l, so t m / 2^(27 + l) exceeds t / d
+// by less than 1 / d.
+struct TileDivision {
+  uint32_t magic, shift;
+};
+__host__ __device__ __forceinline__ TileDivision tile_division(uint32_t tiles_per_block) {
+  uint32_t l = 0;
+  while ((1ull << l) < tiles_per_block) ++l;
+  return TileDivision{(uint32_t)(((1ull << (27 + l)) + tiles_per_block - 1) / tiles_per_block), l};
+}
+__host__ __device__ __forceinline__ int tile_block(int t, const TileDivision &by) {
+  return (int)((uint32_t)(((uint64_t)((uint32_t)t << 5) * by.magic) >> 32) >> by.shift);
 }
 
 // The two score options flash-attn takes from the backend (vllm_hymeta/attention/meta_attention.py:665-690:

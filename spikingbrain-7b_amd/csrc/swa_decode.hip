@@ -1005,6 +1005,7 @@ extern "C" int sb_swa_decode(const sb_swa_decode_args *a) {
   p.ws_rows = need ? (int32_t *)((char *)a->workspace + kMergeCounterBytes + round_up(parts * a->head_size * 4, 256) +
                                  round_up(parts * 2 * 4, 256)) : nullptr;
   p.Hq = a->num_q_heads; p.block_size = a->block_size > 0 ? a->block_size : 16;
+  p.tile_div = tile_division((uint32_t)p.block_size >> 4);
   p.window_left = a->window_left; p.n_split = n_split;
   p.rows = (int)a->num_rows; p.n_wg = 0;
   p.scale_log2 = a->scale * sb::kLog2e;

@@ -118,7 +118,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // the code grew by 1100 instructions for it, which shows in the shortest fp8 runs: 100 rows of 200 keys 12.4 -> 13.0 us, of
   // 6000 80.0 -> 77.8; INT8 14.8 -> 13.5, 82.7 -> 80.4).
   const int tiles_per_block = p.block_size >> 4;
-  const uint32_t tpb_magic = (0x80000000u + tiles_per_block - 1) / tiles_per_block;
   const int32_t *const table_row = p.block_table + seq * p.bt_stride;
   struct Where {
     int blk[2], row[2];
@@ -127,7 +126,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int tile = min(max(2 * cc + t, first_tile), last_tile);  // resident, uniform over the wavefront
-      const int bi = tile_block(tile, tiles_per_block, tpb_magic);
+      const int bi = tile_block(tile, p.tile_div);
       at.row[t] = (tile - bi * tiles_per_block) << 4;
       at.blk[t] = table_row[bi];
     }

@@ -75,7 +75,7 @@ struct PrefillParams {
   int bucket, head_groups;    // order of an XCD's workgroups (see the kernel)
   int block_size, window_left;
   int tiles_per_block;        // block_size / 16
-  uint32_t tpb_magic;         // ceil(2^31 / tiles_per_block), see tile_block
+  TileDivision tile_div;      // by tiles_per_block
   float scale_log2;
   int64_t q_sr, q_sh, o_sr, o_sh;  // elements
   int64_t kv_sb, kv_sr, kv_sh;     // bytes
@@ -287,7 +287,7 @@ void swa_prefill_kernel(const PrefillParams p) {
     auto walk_tile = [&](int x) __attribute__((always_inline)) {  // (past the end of the walk: the last tile again)
       return min(max(2 * (ch_begin + x) + tsel, first_tile), last_tile);
     };
-    auto block_of = [&](int t) __attribute__((always_inline)) { return tile_block(t, p.tiles_per_block, p.tpb_magic); };
+    auto block_of = [&](int t) __attribute__((always_inline)) { return tile_block(t, p.tile_div); };
     int next_blk = 0;  // table entry of the tile the next fetch takes
     if constexpr (PAGED) next_blk = table_row[block_of(walk_tile(0))];
     int fx = 0;        // walk index the next fetch takes
@@ -824,7 +824,7 @@ int prefill(const sb_swa_prefill_args *a, int64_t max_keys, int n_parts, float *
   p.G = a->num_q_heads / a->num_kv_heads; p.head_begin = 0;
   p.block_size = a->block_size > 0 ? a->block_size : 16; p.window_left = a->window_left;
   p.tiles_per_block = p.block_size / 16;
-  p.tpb_magic = (uint32_t)(((1ull << 31) + p.tiles_per_block - 1) / p.tiles_per_block);
+  p.tile_div = tile_division((uint32_t)p.tiles_per_block);
   p.scale_log2 = a->scale * sb::kLog2e;
   p.q_sr = a->q_stride_row; p.q_sh = a->q_stride_head; p.o_sr = a->out_stride_row; p.o_sh = a->out_stride_head;
   p.kv_sb = a->kv_stride_block * kv_esz; p.kv_sr = a->kv_stride_row * kv_esz; p.kv_sh = a->kv_stride_head * kv_esz;
