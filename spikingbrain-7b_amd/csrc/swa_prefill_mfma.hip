@@ -174,7 +174,9 @@ __device__ __forceinline__ uint4 dequant8(uint2 w, float s) {
                     Mma<E>::pack(code_value<Q, 2>(w.y) * s, code_value<Q, 3>(w.y) * s));
 }
 
-template <typename E, int NHEADS, int KVQ, bool PAGED>
+// ODD: the last group of heads may have one less (3 of 4, 1 of 2): a build of its own, because the second path costs
+// the kernel of two heads 5 % (16 : 8 heads, 2000 tokens behind 3000 95 -> 100 us).
+template <typename E, int NHEADS, int KVQ, bool PAGED, bool ODD>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * Shape<NHEADS>::kWaves, 64 * Shape<NHEADS>::kWaves),
                           amdgpu_waves_per_eu(2, 2)))
 void swa_prefill_kernel(const PrefillParams p) {
@@ -197,7 +199,7 @@ void swa_prefill_kernel(const PrefillParams p) {
   if (tile >= p.num_tiles) return;
   const int head_group = pair / p.Hkv, kvh = pair - head_group * p.Hkv;
   const int head_begin = p.head_begin + NHEADS * head_group;
-  const int nheads = min(NHEADS, p.G - head_begin);
+  const int nheads = ODD ? min(NHEADS, p.G - head_begin) : NHEADS;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
@@ -640,6 +642,8 @@ void swa_prefill_kernel(const PrefillParams p) {
   };
   if constexpr (NHEADS == 1) {
     run(std::integral_constant<int, 1>{});
+  } else if constexpr (!ODD) {
+    run(std::integral_constant<int, 2>{});
   } else if constexpr (NHEADS == 2) {
     if (nheads == 1) run(std::integral_constant<int, 1>{});
     else run(std::integral_constant<int, 2>{});
@@ -704,19 +708,20 @@ __global__ __launch_bounds__(256) void swa_prefill_merge_kernel(const PrefillPar
 }
 
 template <typename E, int KVQ, bool PAGED>
-void launch_prefill_q(int nh, dim3 grid, hipStream_t st, const PrefillParams &p) {
-  switch (nh) {
-    case 1: hipLaunchKernelGGL((swa_prefill_kernel<E, 1, KVQ, PAGED>), grid, dim3(64 * Shape<1>::kWaves), 0, st, p); break;
-    case 2: hipLaunchKernelGGL((swa_prefill_kernel<E, 2, KVQ, PAGED>), grid, dim3(64 * Shape<2>::kWaves), 0, st, p); break;
-    default: hipLaunchKernelGGL((swa_prefill_kernel<E, 4, KVQ, PAGED>), grid, dim3(64 * Shape<4>::kWaves), 0, st, p); break;
-  }
+void launch_prefill_q(int nh, bool odd, dim3 grid, hipStream_t st, const PrefillParams &p) {
+  const dim3 b1(64 * Shape<1>::kWaves), b2(64 * Shape<2>::kWaves), b4(64 * Shape<4>::kWaves);
+  if (nh == 1) hipLaunchKernelGGL((swa_prefill_kernel<E, 1, KVQ, PAGED, false>), grid, b1, 0, st, p);
+  else if (nh == 2 && odd) hipLaunchKernelGGL((swa_prefill_kernel<E, 2, KVQ, PAGED, true>), grid, b2, 0, st, p);
+  else if (nh == 2) hipLaunchKernelGGL((swa_prefill_kernel<E, 2, KVQ, PAGED, false>), grid, b2, 0, st, p);
+  else if (odd) hipLaunchKernelGGL((swa_prefill_kernel<E, 4, KVQ, PAGED, true>), grid, b4, 0, st, p);
+  else hipLaunchKernelGGL((swa_prefill_kernel<E, 4, KVQ, PAGED, false>), grid, b4, 0, st, p);
 }
 template <typename E>
-void launch_prefill(int kv_quant, int nh, dim3 grid, hipStream_t st, const PrefillParams &p) {
-  if (kv_quant == SB_KV_INT8) launch_prefill_q<E, SB_KV_INT8, true>(nh, grid, st, p);
-  else if (kv_quant == SB_KV_FP8) launch_prefill_q<E, SB_KV_FP8, true>(nh, grid, st, p);
-  else if (p.block_table) launch_prefill_q<E, SB_KV_NONE, true>(nh, grid, st, p);
-  else launch_prefill_q<E, SB_KV_NONE, false>(nh, grid, st, p);
+void launch_prefill(int kv_quant, int nh, bool odd, dim3 grid, hipStream_t st, const PrefillParams &p) {
+  if (kv_quant == SB_KV_INT8) launch_prefill_q<E, SB_KV_INT8, true>(nh, odd, grid, st, p);
+  else if (kv_quant == SB_KV_FP8) launch_prefill_q<E, SB_KV_FP8, true>(nh, odd, grid, st, p);
+  else if (p.block_table) launch_prefill_q<E, SB_KV_NONE, true>(nh, odd, grid, st, p);
+  else launch_prefill_q<E, SB_KV_NONE, false>(nh, odd, grid, st, p);
 }
 
 // Most 32-key chunks a tile of 64 queries walks when no sequence has more than max_keys keys.
@@ -885,12 +890,13 @@ int prefill(const sb_swa_prefill_args *a, int64_t max_keys, int n_parts, float *
     const int left = p.G - h0;
     const int groups = pairs ? (left + 1) / 2 : (left >= 3 ? left / 4 + (left % 4 == 3) : 1);
     const int nh = pairs ? 2 : (left >= 3 ? 4 : left);
+    const bool odd = nh * groups > left;   // (the last group has one head less)
     p.head_begin = h0;
     h0 += nh * groups;
     p.head_groups = groups;
     const dim3 grid((unsigned)(per_xcd * 8 * a->num_kv_heads * groups), (unsigned)n_parts);
-    if (a->dtype == SB_BF16) launch_prefill<BF16>(a->kv_quant, nh, grid, (hipStream_t)a->stream, p);
-    else launch_prefill<F16>(a->kv_quant, nh, grid, (hipStream_t)a->stream, p);
+    if (a->dtype == SB_BF16) launch_prefill<BF16>(a->kv_quant, nh, odd, grid, (hipStream_t)a->stream, p);
+    else launch_prefill<F16>(a->kv_quant, nh, odd, grid, (hipStream_t)a->stream, p);
     const int rc = check_launch("swa_prefill_kernel");
     if (rc != SB_OK) return rc;
   }
