@@ -665,8 +665,12 @@ __global__ __launch_bounds__(256) void swa_prefill_merge_kernel(const PrefillPar
   const int j = q0 + 8 * blockIdx.z + (threadIdx.x >> 5), d4 = threadIdx.x & 31;
   if (parts < 2 || j >= Lq) return;
   const int64_t rh = (int64_t)(qrow0 + j) * p.Hq + head;
-  const float2 *ml = reinterpret_cast<const float2 *>(p.ws_ml) + rh * p.n_parts;
-  const float4 *acc = reinterpret_cast<const float4 *>(p.ws_acc) + rh * p.n_parts * 32 + d4;
+  // from the first of the workgroup's rows on; past the last part an offset out of range, which gives zeros: that part again, times 0,
+  // would be a NaN where it holds an infinity
+  const int64_t rec0 = ((int64_t)(qrow0 + q0 + 8 * blockIdx.z) * p.Hq + head) * p.n_parts;
+  const int rec = (int)(threadIdx.x >> 5) * p.Hq * p.n_parts;
+  const __amdgpu_buffer_rsrc_t ml = __builtin_amdgcn_make_buffer_rsrc(p.ws_ml + rec0 * 2, 0, 0x7fffffff, 0x00020000);
+  const __amdgpu_buffer_rsrc_t acc = __builtin_amdgcn_make_buffer_rsrc(p.ws_acc + rec0 * 128, 0, 0x7fffffff, 0x00020000);
   float4 tot = make_float4(0.f, 0.f, 0.f, 0.f);
   float L = 0.f, M = kNegInf;
   for (int s0 = 0; s0 < parts; s0 += 4) {  // four parts per trip to memory
@@ -674,18 +678,16 @@ __global__ __launch_bounds__(256) void swa_prefill_merge_kernel(const PrefillPar
     float4 a[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const bool there = s0 + u < parts;   // (past the last part: nothing, not that part again times 0: it may hold an infinity)
-      const int s = min(s0 + u, parts - 1);
-      x[u] = ml[s];
-      a[u] = acc[s * 32];
-      if (!there) {
-        x[u] = make_float2(kNegInf, 0.f);
-        a[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-      }
+      const bool there = s0 + u < parts;
+      x[u] = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(ml, there ? (rec + s0 + u) * 8 : -16, 0, 0));
+      a[u] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(acc, there ? (rec + s0 + u) * 512 + 16 * d4 : -16, 0, 0));
     }
     float Mn = M;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) Mn = fmaxf(Mn, x[u].x);
+    for (int u = 0; u < 4; ++u) {
+      if (s0 + u >= parts) x[u].x = kNegInf;
+      Mn = fmaxf(Mn, x[u].x);
+    }
     const float ref = Mn == kNegInf ? 0.f : Mn;  // (nothing visible so far: every factor is 0, and a NaN stays one)
     const float keep = fast_exp2(M - ref);
     tot.x *= keep; tot.y *= keep; tot.z *= keep; tot.w *= keep;
@@ -995,6 +997,9 @@ extern "C" int sb_swa_prefill_parted(const sb_swa_prefill_args *a, int64_t total
       workspace_bytes < sb_swa_prefill_workspace_bytes(a, total_q, n_parts))
     return fail(SB_ERR_WORKSPACE, "sb_swa_prefill_parted: workspace of %zu bytes (16-byte aligned) needed, got %zu",
                 sb_swa_prefill_workspace_bytes(a, total_q, n_parts), workspace ? workspace_bytes : (size_t)0);
+  // (the merge addresses eight rows of a head with 32 bits; fewer parts are always right)
+  if (a->num_q_heads > 0)
+    n_parts = (int32_t)std::max<int64_t>(1, std::min<int64_t>(n_parts, INT32_MAX / ((int64_t)8 * 512 * a->num_q_heads)));
   float *acc = static_cast<float *>(workspace);
   return prefill(a, max_keys, n_parts, acc, acc + total_q * a->num_q_heads * n_parts * 128);
 }
