@@ -545,7 +545,7 @@ class PrefillPlan:
     (which the scheduler already has as Python ints), uploaded with one copy."""
 
     __slots__ = ("cu_seqlens_q", "seq_lens_k", "tile_seq", "tile_q0", "num_tiles", "total_q", "num_seqs", "max_k",
-                 "total_k", "_host", "tile_keys_ptr")
+                 "total_k", "_host", "_packed")
 
     def __init__(self, query_lens, seq_lens_k, device):
         query_lens = [int(x) for x in query_lens]
@@ -562,14 +562,25 @@ class PrefillPlan:
         T = sum([(n + PREFILL_TILE - 1) // PREFILL_TILE for n in query_lens])
         self._host = torch.empty(2 * S + 1 + 3 * T, dtype=torch.int32)
         host_ptr, ints = self._host.data_ptr(), C.c_int32 * S
-        self.tile_keys_ptr = host_ptr + 4 * (2 * S + 1 + 2 * T) if 0 < T < PREFILL_DEALT_TILES else None   # (read on the host)
-        N.check(N.lib().sb_swa_prefill_plan(ints(*query_lens), ints(*seq_lens_k), S, T, host_ptr, self.tile_keys_ptr), "prefill plan")
-        packed = self._host.to(device, non_blocking=False)
+        N.check(N.lib().sb_swa_prefill_plan(ints(*query_lens), ints(*seq_lens_k), S, T, host_ptr, host_ptr + 4 * (2 * S + 1 + 2 * T)),
+                "prefill plan")
+        self._packed = packed = self._host.to(device, non_blocking=False)
         self.cu_seqlens_q = packed[:S + 1]
         self.seq_lens_k = packed[S + 1:2 * S + 1]
         self.tile_seq = packed[2 * S + 1:2 * S + 1 + T]
         self.tile_q0 = packed[2 * S + 1 + T:2 * S + 1 + 2 * T]
         self.num_tiles, self.total_q, self.num_seqs = T, total_q, S
+
+    @property
+    def tile_keys_ptr(self):
+        """Address of the keys that the tiles walk, which the call reads on the host: None for lists too long to need them, and
+        for a plan whose lists are not those made here (a copy's are: no address is kept)."""
+        T, at = self.num_tiles, 2 * self.num_seqs + 1
+        first = self._packed.data_ptr() + 4 * at
+        if (not 0 < T < PREFILL_DEALT_TILES or self._host.numel() != at + 3 * T or
+                self.tile_seq.data_ptr() != first or self.tile_q0.data_ptr() != first + 4 * T):
+            return None
+        return self._host.data_ptr() + 4 * (at + 2 * T)
 
 
 def swa_prefill_attention(

@@ -1,5 +1,7 @@
 """Tile plans of the prompt kernel (host only)."""
+import copy
 import ctypes
+import pickle
 import random
 
 import pytest
@@ -93,3 +95,28 @@ def test_keys_of_the_tiles(sb):
     got = plan._host[-plan.num_tiles:].tolist()
     assert got == sorted((64 + at + k - n for n, k in zip(lens, keys) for at in range(0, n, 64)), reverse=True)
     assert sb.ops.PrefillPlan([64 * 1024], None, "cpu").tile_keys_ptr is None
+
+
+@pytest.mark.parametrize("again", [copy.copy, copy.deepcopy, lambda plan: pickle.loads(pickle.dumps(plan))])
+def test_copies_do_not_read_the_original(sb, again):
+    """A copied or saved plan outlives the one it was made of, and the call reads the tiles' keys on the host: from the
+    copy's own memory, or not at all."""
+    plan = sb.ops.PrefillPlan([100, 7, 640], [300, 7, 641], "cpu")
+    host, keys = plan._host.data_ptr(), plan._host[-plan.num_tiles:].tolist()
+    kept = again(plan)
+    at = kept.tile_keys_ptr
+    assert at is None or list((ctypes.c_int32 * kept.num_tiles).from_address(at)) == keys
+    assert at is None or at == kept._host.data_ptr() + 4 * (kept._host.numel() - kept.num_tiles)
+    if again is not copy.copy:
+        assert kept._host.data_ptr() != host
+    assert kept.tile_seq.tolist() == plan.tile_seq.tolist() and kept.tile_q0.tolist() == plan.tile_q0.tolist()
+
+
+def test_lists_of_the_callers_own_have_no_known_keys(sb):
+    plan = sb.ops.PrefillPlan([100, 7, 640], None, "cpu")
+    assert plan.tile_keys_ptr is not None
+    plan.num_tiles += 1
+    assert plan.tile_keys_ptr is None
+    plan.num_tiles -= 1
+    plan.tile_q0 = plan.tile_q0.clone()
+    assert plan.tile_keys_ptr is None
