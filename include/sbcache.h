@@ -514,15 +514,20 @@ typedef struct sb_swa_prefill_args {
    * Only the choice of how the call is spread over the GPU reads it (before the call returns); NULL: as if all tiles
    * walked as many keys as the longest. */
   const int32_t *tile_keys;
+  /* The tiles of tile_seq / tile_q0 in sequence order (device, both or neither): what the call takes where the walks are as good as
+   * equal (tile_keys). */
+  const int32_t *ordered_tile_seq;
+  const int32_t *ordered_tile_q0;
 } sb_swa_prefill_args;
 
 int sb_swa_prefill(const sb_swa_prefill_args *args);
 
-/* The index arrays of such a call from HOST lengths (no device access): `plan` [2 * num_seqs + 1 + 2 * num_tiles] receives
- * cu_seqlens_q, seq_lens_k, tile_seq and tile_q0, one behind the other, for the caller to upload. num_tiles: the sum of
- * ceil(query_lens[s] / 64). The tiles are listed in the order the kernel likes best; any other order, and plans of the caller's
- * own, give the same results. tile_keys [num_tiles] (may be NULL) stays on the host, for the field of that name; it is filled
- * for fewer than 1024 tiles, more have no use for it. */
+/* The index arrays of such a call from HOST lengths (no device access): `plan` receives cu_seqlens_q [num_seqs + 1], seq_lens_k
+ * [num_seqs], tile_seq and tile_q0 [num_tiles], and for fewer than 1024 tiles ordered_tile_seq and ordered_tile_q0 [num_tiles], one
+ * behind the other, for the caller to upload. num_tiles: the sum of ceil(query_lens[s] / 64). The tiles of tile_seq are listed in
+ * the order that suits walks of different lengths; any other order, and plans of the caller's own, give the same results.
+ * tile_keys [num_tiles] (may be NULL) stays on the host, for the field of that name; it is filled for fewer than 1024 tiles, more
+ * have no use for it. */
 int sb_swa_prefill_plan(const int32_t *query_lens, const int32_t *seq_lens_k, int64_t num_seqs, int64_t num_tiles,
                         int32_t *plan, int32_t *tile_keys);
 

@@ -120,7 +120,7 @@ class SwaPrefillArgs(C.Structure):
         ("k_scale_tensor", f32), ("v_scale_tensor", f32),
         ("meta_k", vp), ("meta_v", vp), ("meta_len", i32), ("meta_stride_row", i64), ("meta_stride_head", i64),
         ("softcap", f32), ("alibi_slopes", vp), ("meta_bias_row0", i64), ("meta_bias_rows", i64),
-        ("kv_start32", vp), ("tile_keys", vp),
+        ("kv_start32", vp), ("tile_keys", vp), ("ordered_tile_seq", vp), ("ordered_tile_q0", vp),
     ]
 
 

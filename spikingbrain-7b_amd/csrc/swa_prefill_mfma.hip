@@ -726,6 +726,8 @@ void launch_prefill(int kv_quant, int nh, bool odd, dim3 grid, hipStream_t st, c
   else launch_prefill_q<E, SB_KV_NONE, false>(nh, odd, grid, st, p);
 }
 
+constexpr int64_t kDealtTiles = 1024;   // shorter tile lists come dealt to the XCDs, see sb_swa_prefill_plan
+
 // Most 32-key chunks a tile of 64 queries walks when no sequence has more than max_keys keys.
 int64_t most_chunks(const sb_swa_prefill_args *a, int64_t max_keys) {
   int64_t span = max_keys;
@@ -755,8 +757,8 @@ struct Spread {
 int64_t quad_workgroups(const sb_swa_prefill_args *a) {
   return a->num_tiles * a->num_kv_heads * ((a->num_q_heads / a->num_kv_heads + 3) / 4);
 }
-bool pairs_pay(const sb_swa_prefill_args *a, int64_t chunks, int64_t parts) {
-  const int64_t wgs = quad_workgroups(a) * parts, cus = sb_host::device_cu_count();
+bool pairs_pay(const sb_swa_prefill_args *a, int64_t chunks, int64_t parts, int64_t cus) {
+  const int64_t wgs = quad_workgroups(a) * parts;
   if (2 * wgs <= cus) return true;
   if (parts > 1 || 2 * wgs > 3 * cus) return false;
   if (wgs > cus) return chunks <= 2 * a->num_tiles + 2;
@@ -765,12 +767,35 @@ bool pairs_pay(const sb_swa_prefill_args *a, int64_t chunks, int64_t parts) {
   const int64_t sharing = cus / pairs_per_tile;   // tiles in front of the first one that shares
   return sharing >= a->num_tiles || (double)most_chunks(a, a->tile_keys[sharing]) < 6.0 + 0.63 * (double)chunks;
 }
+// Order of a short list's tiles. Dealt to the XCDs longest walk first, in tile-major order, evens out the work of walks of
+// different lengths; in sequence order, kv heads outermost, the tiles that run on an XCD at a time are neighbours of one head and
+// share its keys in the L2. Where the walks are as good as equal there is nothing to even out, and the fewer query heads share
+// a kv head (the less a workgroup does per byte), the more the L2 counts. us, dealt -> in sequence order (mean walk / longest walk):
+//   28 : 4   6000 / 20000 behind 12000 381 / 1246 -> 359 / 1162 (1.0); 2500 x 4 behind 3000 574 -> 589 (0.94); 6000 whole 253 -> 348 (0.66)
+//   12 : 4   6000 behind 3000 231 -> 205 (0.98); 16 : 8 6000 with a window of 1024 79.7 -> 72.6 (0.92), 800 x 6 behind 3000 183 -> 196 (0.90)
+//   16 : 16  6000 / 20000 behind 12000 461 / 1489 -> 287 / 908 (1.0), 20000 whole 1300 -> 870 (0.90), 800 x 6 behind 800 115 -> 96 (0.77);
+//            below, dealt with kv heads outermost where that is many workgroups: 6000 whole 268 -> 243 (0.66; in sequence order 265), 40 : 40,
+//            2500 x 4 behind 800 915 -> 650 (0.63; 761), but 3000 whole 71 -> 101 (0.52; 106)
+//   20 : 4, 24 : 4 and 16 : 8  20000 whole 967 -> 863, 1018 -> 978, 695 -> 657 (0.90)
+enum class Order { kDealt, kDealtByHead, kSequence };
+Order tile_order(const sb_swa_prefill_args *a, int64_t max_keys, int64_t chunks, int64_t cus) {
+  if (a->num_tiles >= kDealtTiles || !a->tile_keys || !a->ordered_tile_seq || !a->ordered_tile_q0) return Order::kDealt;
+  int64_t total = 0;
+  for (int64_t t = 0; t < a->num_tiles; ++t) total += most_chunks(a, a->tile_keys[t] < max_keys ? a->tile_keys[t] : max_keys);
+  const int G = a->num_q_heads / a->num_kv_heads;
+  const double even = (double)total / (double)(a->num_tiles * chunks);
+  // (a last launch of one or two heads reads as much per head as G <= 2 does; over many rounds it decides)
+  const bool thin = G <= 3 || G % 4 == 1 || G % 4 == 2, rounds6 = quad_workgroups(a) >= 6 * cus;
+  if (even >= (G == 1 ? 0.75 : thin && rounds6 ? 0.88 : G <= 3 ? 0.92 : 0.97)) return Order::kSequence;
+  return G == 1 && 2 * a->num_tiles * a->num_kv_heads >= 7 * cus ? Order::kDealtByHead : Order::kDealt;
+}
+
 Spread spread_of(const sb_swa_prefill_args *a, int64_t max_keys) {
   const int64_t chunks = most_chunks(a, max_keys), wgs = quad_workgroups(a), cus = sb_host::device_cu_count();
-  Spread best{1, pairs_pay(a, chunks, 1)};
+  Spread best{1, pairs_pay(a, chunks, 1, cus)};
   double best_us = 5.0 + (best.pairs ? 0.69 : 0.9) * (double)chunks;
   for (int64_t n = 2; n * wgs <= cus && 8 * n <= chunks; ++n) {
-    const bool pairs = pairs_pay(a, chunks, n);
+    const bool pairs = pairs_pay(a, chunks, n, cus);
     const double us = 13.5 + 0.28 * (double)n + 8.0 * (double)(n * wgs) / (double)cus +
                       (pairs ? 0.69 : 0.86) * (double)((chunks + n - 1) / n);
     if (us < best_us) {
@@ -840,6 +865,12 @@ int prefill(const sb_swa_prefill_args *a, int64_t max_keys, int n_parts, float *
   p.bt_stride = a->block_table_stride;
   p.num_tiles = (int)a->num_tiles;
   const int64_t chunks = most_chunks(a, max_keys);
+  const int64_t cus = sb_host::device_cu_count();
+  const Order order = n_parts == 1 ? tile_order(a, max_keys, chunks, cus) : Order::kDealt;
+  if (order == Order::kSequence) {
+    p.tile_seq = a->ordered_tile_seq;
+    p.tile_q0 = a->ordered_tile_q0;
+  }
   p.n_parts = n_parts; p.part_chunks = (int)((chunks + n_parts - 1) / n_parts);
   p.ws_acc = ws_acc; p.ws_ml = ws_ml;
   p.meta_k = p.meta_v = nullptr;
@@ -885,8 +916,10 @@ int prefill(const sb_swa_prefill_args *a, int64_t max_keys, int n_parts, float *
   // 1 x 8192 388 / 398 / 411 / 458 / 448 us (tile lists sorted longest first: what starts last should be short whatever
   // its heads); 16 x 8192 in sequence order 6.34 ms at 1 against 6.04 at 4, 6.08 at 16 and 6.13 at all (four tiles and one
   // kv head at a time keep their keys in the XCD's L2).
-  p.bucket = a->num_tiles < 1024 ? 1 : 4;
-  const bool pairs = p.G > 1 && pairs_pay(a, chunks, n_parts);
+  // Up to four query heads per kv head that is 1 to 10 % slower than all (16 : 16 3194 / 2951 us, 16 : 8 2270 / 2222, 32 : 8 4407 / 4356
+  // for 10 x 8192). Shorter lists: see tile_order.
+  p.bucket = a->num_tiles >= kDealtTiles ? (p.G <= 4 ? (int)per_xcd : 4) : order == Order::kDealt ? 1 : (int)per_xcd;
+  const bool pairs = p.G > 1 && pairs_pay(a, chunks, n_parts, cus);
   if (per_xcd * 8 * a->num_kv_heads * p.G > 0x7fffffffLL) return fail(SB_ERR_UNSUPPORTED, "sb_swa_prefill: grid too large");
   for (int h0 = 0; h0 < p.G;) {
     const int left = p.G - h0;
@@ -915,9 +948,8 @@ int prefill(const sb_swa_prefill_args *a, int64_t max_keys, int n_parts, float *
 
 // The kernel gives XCD x the x-th contiguous eighth of the tile list. In lists of less than this many tiles those late in a
 // long sequence, which see the most keys, are dealt out in turn, latest first, so that the XCDs get equal shares and the longest
-// workgroups start first. Longer lists stay in sequence order: an XCD's neighbouring tiles then share their keys in its
-// L2, and there are enough of them to even out.
-constexpr int64_t kDealtTiles = 1024;
+// workgroups start first (unless the call finds sequence order better, tile_order above). Longer lists stay in sequence
+// order: an XCD's neighbouring tiles then share their keys in its L2, and there are enough of them to even out.
 constexpr int kTileTokens = 64;
 
 // Native because every new prompt pays it in front of its first layer: the whole plan of 64 / 1517 / 8192 / 16 x 8192 tokens in
@@ -927,8 +959,10 @@ extern "C" int sb_swa_prefill_plan(const int32_t *query_lens, const int32_t *seq
   using namespace sb_host;
   if (num_seqs < 0 || num_tiles < 0 || !plan || (num_seqs > 0 && (!query_lens || !seq_lens_k)))
     return fail(SB_ERR_INVALID, "sb_swa_prefill_plan: negative size or null pointer");
-  int32_t *const cu = plan, *const keys = plan + num_seqs + 1, *const seq = keys + num_seqs, *const q0 = seq + num_tiles;
   const bool dealt = num_tiles < kDealtTiles;
+  // (in sequence order: behind the dealt lists, or in their place)
+  int32_t *const cu = plan, *const keys = plan + num_seqs + 1, *const dealt_seq = keys + num_seqs, *const dealt_q0 = dealt_seq + num_tiles;
+  int32_t *const seq = dealt ? dealt_q0 + num_tiles : dealt_seq, *const q0 = seq + num_tiles;
   int64_t order[kDealtTiles];   // dealt: (position of the tile in the keys, earlier tiles of the list first) of every tile
   int64_t total = 0, tiles = 0;
   for (int64_t s = 0; s < num_seqs; ++s) {
@@ -952,18 +986,15 @@ extern "C" int sb_swa_prefill_plan(const int32_t *query_lens, const int32_t *seq
   if (!dealt) return SB_OK;
   std::sort(order, order + tiles, std::greater<int64_t>());
   const int64_t per_xcd = (tiles + 7) / 8;
-  int32_t at_seq[kDealtTiles], at_q0[kDealtTiles];
   int64_t next = 0;
   for (int64_t k = 0; k < 8 * per_xcd; ++k) {
     const int64_t slot = (k % 8) * per_xcd + k / 8;
     if (slot >= tiles) continue;
     if (tile_keys) tile_keys[next] = (int32_t)std::min<int64_t>((order[next] >> 12) + kTileTokens, INT32_MAX);
     const int64_t t = kDealtTiles - 1 - (order[next++] & 0xfff);
-    at_seq[slot] = seq[t];
-    at_q0[slot] = q0[t];
+    dealt_seq[slot] = seq[t];
+    dealt_q0[slot] = q0[t];
   }
-  std::copy(at_seq, at_seq + tiles, seq);
-  std::copy(at_q0, at_q0 + tiles, q0);
   return SB_OK;
 }
 
@@ -976,7 +1007,7 @@ extern "C" int32_t sb_swa_prefill_parts(const sb_swa_prefill_args *a, int64_t ma
 
 extern "C" int32_t sb_swa_prefill_group_heads(const sb_swa_prefill_args *a, int64_t max_keys, int32_t n_parts) {
   if (!a || a->num_tiles <= 0 || a->num_kv_heads <= 0 || a->num_q_heads < a->num_kv_heads || max_keys <= 0) return 4;
-  return pairs_pay(a, most_chunks(a, max_keys < INT32_MAX ? max_keys : INT32_MAX), n_parts < 1 ? 1 : n_parts) ? 2 : 4;
+  return pairs_pay(a, most_chunks(a, max_keys < INT32_MAX ? max_keys : INT32_MAX), n_parts < 1 ? 1 : n_parts, sb_host::device_cu_count()) ? 2 : 4;
 }
 
 extern "C" size_t sb_swa_prefill_workspace_bytes(const sb_swa_prefill_args *a, int64_t total_q, int32_t n_parts) {

@@ -560,27 +560,31 @@ class PrefillPlan:
         if total_q > INT32_MAX or self.max_k > INT32_MAX:
             raise RuntimeError("the kernel counts keys and packed query rows in 32 bits: lengths cannot be converted without overflow")
         T = sum([(n + PREFILL_TILE - 1) // PREFILL_TILE for n in query_lens])
-        self._host = torch.empty(2 * S + 1 + 3 * T, dtype=torch.int32)
+        at = 2 * S + 1
+        self._host = torch.empty(at + (5 if T < PREFILL_DEALT_TILES else 2) * T, dtype=torch.int32)
         host_ptr, ints = self._host.data_ptr(), C.c_int32 * S
-        N.check(N.lib().sb_swa_prefill_plan(ints(*query_lens), ints(*seq_lens_k), S, T, host_ptr, host_ptr + 4 * (2 * S + 1 + 2 * T)),
+        N.check(N.lib().sb_swa_prefill_plan(ints(*query_lens), ints(*seq_lens_k), S, T, host_ptr, host_ptr + 4 * (at + 4 * T)),
                 "prefill plan")
         self._packed = packed = self._host.to(device, non_blocking=False)
         self.cu_seqlens_q = packed[:S + 1]
         self.seq_lens_k = packed[S + 1:2 * S + 1]
-        self.tile_seq = packed[2 * S + 1:2 * S + 1 + T]
-        self.tile_q0 = packed[2 * S + 1 + T:2 * S + 1 + 2 * T]
+        self.tile_seq = packed[at:at + T]
+        self.tile_q0 = packed[at + T:at + 2 * T]
         self.num_tiles, self.total_q, self.num_seqs = T, total_q, S
+
+    def list_ptrs(self):
+        """Addresses of the keys that the tiles walk (read on the host, at the call) and of the tiles in sequence order: None
+        for lists too long to need them, and for a plan whose lists are not those made here (a copy's are: no address is kept)."""
+        T, at = self.num_tiles, 2 * self.num_seqs + 1
+        first = self._packed.data_ptr() + 4 * at
+        if (not 0 < T < PREFILL_DEALT_TILES or self._host.numel() != at + 5 * T or
+                self.tile_seq.data_ptr() != first or self.tile_q0.data_ptr() != first + 4 * T):
+            return None, None, None
+        return self._host.data_ptr() + 4 * (at + 4 * T), first + 8 * T, first + 12 * T
 
     @property
     def tile_keys_ptr(self):
-        """Address of the keys that the tiles walk, which the call reads on the host: None for lists too long to need them, and
-        for a plan whose lists are not those made here (a copy's are: no address is kept)."""
-        T, at = self.num_tiles, 2 * self.num_seqs + 1
-        first = self._packed.data_ptr() + 4 * at
-        if (not 0 < T < PREFILL_DEALT_TILES or self._host.numel() != at + 3 * T or
-                self.tile_seq.data_ptr() != first or self.tile_q0.data_ptr() != first + 4 * T):
-            return None
-        return self._host.data_ptr() + 4 * (at + 2 * T)
+        return self.list_ptrs()[0]
 
 
 def swa_prefill_attention(
@@ -725,6 +729,7 @@ def swa_prefill_attention(
         if meta_k.shape[0] > 0:
             meta = dict(meta_k=N.ptr(meta_k), meta_v=N.ptr(meta_v), meta_len=meta_k.shape[0],
                         meta_stride_row=meta_k.stride(0), meta_stride_head=meta_k.stride(1))
+    tile_keys, ordered_seq, ordered_q0 = plan.list_ptrs()
     a = N.SwaPrefillArgs(
         q=N.ptr(q), k=N.ptr(k), v=N.ptr(v), out=N.ptr(out),
         block_table=N.ptr(block_table), kv_start=N.ptr(kv_start) if block_table is None else None,
@@ -742,7 +747,8 @@ def swa_prefill_attention(
         softcap=float(softcap), alibi_slopes=N.ptr(_slopes(alibi_slopes, Hq, dev)),
         meta_bias_row0=int(meta_bias[0]) if meta_bias else 0,
         meta_bias_rows=int(meta_bias[1]) if meta_bias else int(q.shape[0]),
-        kv_start32=N.ptr(kv_start32) if block_table is None else None, tile_keys=plan.tile_keys_ptr, **meta)
+        kv_start32=N.ptr(kv_start32) if block_table is None else None,
+        tile_keys=tile_keys, ordered_tile_seq=ordered_seq, ordered_tile_q0=ordered_q0, **meta)
     L = N.lib()
     if n_parts == 0:
         n_parts = L.sb_swa_prefill_parts(C.byref(a), plan.max_k)

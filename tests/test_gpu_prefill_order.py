@@ -24,3 +24,21 @@ def test_long_list_equals_short_lists(sb, dev, G, Hkv, extra):
     for a, b, part in ((0, at, lens[:cut]), (at, T, lens[cut:])):
         got = sb.ops.swa_prefill_attention(q[a:b], k[a:b], v[a:b], query_lens=part, window_left=wl)
         assert torch.equal(got, whole[a:b])
+
+
+@pytest.mark.parametrize("HQ,Hkv", [(6, 6), (8, 4), (6, 2), (7, 1)])
+@pytest.mark.parametrize("lens,ctx,window", [([1500], 700, 300), ([700, 64, 333], 900, 4096), ([2100], 0, 4096), ([65, 1, 700] * 4, 40, 4096)])
+def test_short_lists_in_either_order(sb, dev, HQ, Hkv, lens, ctx, window):
+    """Which of a plan's two lists a call takes, and in what order its workgroups take the heads, goes by the walks and
+    the group size; the bits do not: against the same call with the dealt list alone, and with lists of the caller's own."""
+    g = torch.Generator(device=dev).manual_seed(HQ)
+    keys = [n + ctx for n in lens]
+    q = torch.randn(sum(lens), HQ, 128, device=dev, generator=g).bfloat16()
+    k, v = (torch.randn(sum(keys), Hkv, 128, device=dev, generator=g).bfloat16() for _ in range(2))
+    start = torch.tensor([0] + keys, device=dev).cumsum(0)[:-1].contiguous()
+    plan, dealt, own = (sb.ops.PrefillPlan(lens, keys, dev) for _ in range(3))
+    dealt.tile_seq = dealt.tile_seq.clone()   # (no longer the plan's own: the call knows neither its keys nor the other list)
+    turn = torch.randperm(own.num_tiles, generator=torch.Generator().manual_seed(1)).to(dev)
+    own.tile_seq, own.tile_q0 = own.tile_seq[turn].contiguous(), own.tile_q0[turn].contiguous()
+    a, b, c = (sb.ops.swa_prefill_attention(q, k, v, plan=p, kv_start=start, window_left=window, n_parts=1) for p in (plan, dealt, own))
+    assert torch.equal(a, b) and torch.equal(a, c)

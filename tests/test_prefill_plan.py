@@ -36,12 +36,17 @@ def test_dealt_lists(sb):
         keys = [n + rng.choice([0, 0, rng.randint(0, 6000)]) for n in lens]
         plan = sb.ops.PrefillPlan(lens, keys, "cpu")
         assert list(zip(plan.tile_seq.tolist(), plan.tile_q0.tolist())) == _lists(lens, keys), (lens, keys)
+        T, at = plan.num_tiles, 2 * len(lens) + 1
+        ordered = plan._host[at + 2 * T:at + 4 * T].tolist()
+        assert list(zip(ordered[:T], ordered[T:])) == [(s, q0) for s, n in enumerate(lens) for q0 in range(0, n, 64)]
+        first = plan._host.data_ptr() + 4 * at
+        assert plan.list_ptrs() == ((first + 16 * T, first + 8 * T, first + 12 * T) if T else (None, None, None))
 
 
 def test_long_lists_keep_sequence_order(sb):
     lens = [64 * 700, 1, 64 * 323]
     plan = sb.ops.PrefillPlan(lens, None, "cpu")
-    assert plan.num_tiles == 1024
+    assert plan.num_tiles == 1024 and plan.list_ptrs() == (None, None, None)
     assert list(zip(plan.tile_seq.tolist(), plan.tile_q0.tolist())) == [(s, at) for s, n in enumerate(lens) for at in range(0, n, 64)]
 
 
