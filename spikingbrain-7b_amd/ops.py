@@ -545,7 +545,7 @@ class PrefillPlan:
     (which the scheduler already has as Python ints), uploaded with one copy."""
 
     __slots__ = ("cu_seqlens_q", "seq_lens_k", "tile_seq", "tile_q0", "num_tiles", "total_q", "num_seqs", "max_k",
-                 "total_k", "_host", "_packed")
+                 "total_k", "_host", "_packed", "_made")
 
     def __init__(self, query_lens, seq_lens_k, device):
         query_lens = [int(x) for x in query_lens]
@@ -571,16 +571,18 @@ class PrefillPlan:
         self.tile_seq = packed[at:at + T]
         self.tile_q0 = packed[at + T:at + 2 * T]
         self.num_tiles, self.total_q, self.num_seqs = T, total_q, S
+        self._made = (T if T < PREFILL_DEALT_TILES else 0, 4 * at)   # (tiles listed in both orders, bytes in front of the lists)
 
     def list_ptrs(self):
         """Addresses of the keys that the tiles walk (read on the host, at the call) and of the tiles in sequence order: None
-        for lists too long to need them, and for a plan whose lists are not those made here (a copy's are: no address is kept)."""
-        T, at = self.num_tiles, 2 * self.num_seqs + 1
-        first = self._packed.data_ptr() + 4 * at
-        if (not 0 < T < PREFILL_DEALT_TILES or self._host.numel() != at + 5 * T or
-                self.tile_seq.data_ptr() != first or self.tile_q0.data_ptr() != first + 4 * T):
+        for lists too long or too short to need them, and for a plan whose lists are not those made here (a copy's are: no address is kept)."""
+        T, at = self._made
+        if T < 2 or self.num_tiles != T:
             return None, None, None
-        return self._host.data_ptr() + 4 * (at + 4 * T), first + 8 * T, first + 12 * T
+        first = self._packed.data_ptr() + at
+        if self.tile_seq.data_ptr() != first or self.tile_q0.data_ptr() != first + 4 * T:
+            return None, None, None
+        return self._host.data_ptr() + at + 16 * T, first + 8 * T, first + 12 * T
 
     @property
     def tile_keys_ptr(self):

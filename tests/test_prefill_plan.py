@@ -40,7 +40,7 @@ def test_dealt_lists(sb):
         ordered = plan._host[at + 2 * T:at + 4 * T].tolist()
         assert list(zip(ordered[:T], ordered[T:])) == [(s, q0) for s, n in enumerate(lens) for q0 in range(0, n, 64)]
         first = plan._host.data_ptr() + 4 * at
-        assert plan.list_ptrs() == ((first + 16 * T, first + 8 * T, first + 12 * T) if T else (None, None, None))
+        assert plan.list_ptrs() == ((first + 16 * T, first + 8 * T, first + 12 * T) if T > 1 else (None, None, None))
 
 
 def test_long_lists_keep_sequence_order(sb):
