@@ -772,10 +772,12 @@ bool pairs_pay(const sb_swa_prefill_args *a, int64_t chunks, int64_t parts, int6
 // share its keys in the L2. Where the walks are as good as equal there is nothing to even out, and the fewer query heads share
 // a kv head (the less a workgroup does per byte), the more the L2 counts. us, dealt -> in sequence order (mean walk / longest walk):
 //   28 : 4   6000 / 20000 behind 12000 381 / 1246 -> 359 / 1162 (1.0); 2500 x 4 behind 3000 574 -> 589 (0.94); 6000 whole 253 -> 348 (0.66)
-//   12 : 4   6000 behind 3000 231 -> 205 (0.98); 16 : 8 6000 with a window of 1024 79.7 -> 72.6 (0.92), 800 x 6 behind 3000 183 -> 196 (0.90)
+//   12 : 4   6000 behind 3000 231 -> 205 (0.98), 2500 x 4 behind 3000 284 -> 311 (0.94)
+//   16 : 8   6000 with a window of 1024 79.7 -> 72.6 (0.92), 800 x 6 behind 3000 183 -> 196 (0.90)
 //   16 : 16  6000 / 20000 behind 12000 461 / 1489 -> 287 / 908 (1.0), 20000 whole 1300 -> 870 (0.90), 800 x 6 behind 800 115 -> 96 (0.77);
-//            below, dealt with kv heads outermost where that is many workgroups: 6000 whole 268 -> 243 (0.66; in sequence order 265), 40 : 40,
-//            2500 x 4 behind 800 915 -> 650 (0.63; 761), but 3000 whole 71 -> 101 (0.52; 106)
+//            below, dealt with kv heads outermost where that is many workgroups for how uneven the walks are (tiles * kv heads per
+//            CU): 6000 whole 268 -> 243 (0.66, 5.9), 40 : 40, 2500 x 4 behind 800 915 -> 650 (0.63, 25), but 3000 whole 71 -> 101 (0.52,
+//            2.9), 2500 x 4 whole 163 -> 192 (0.52, 10) and 40 : 40, 2000 whole 108 -> 118 (0.52, 5)
 //   20 : 4, 24 : 4 and 16 : 8  20000 whole 967 -> 863, 1018 -> 978, 695 -> 657 (0.90)
 enum class Order { kDealt, kDealtByHead, kSequence };
 Order tile_order(const sb_swa_prefill_args *a, int64_t max_keys, int64_t chunks, int64_t cus) {
@@ -786,8 +788,8 @@ Order tile_order(const sb_swa_prefill_args *a, int64_t max_keys, int64_t chunks,
   const double even = (double)total / (double)(a->num_tiles * chunks);
   // (a last launch of one or two heads reads as much per head as G <= 2 does; over many rounds it decides)
   const bool thin = G <= 3 || G % 4 == 1 || G % 4 == 2, rounds6 = quad_workgroups(a) >= 6 * cus;
-  if (even >= (G == 1 ? 0.75 : thin && rounds6 ? 0.88 : G <= 3 ? 0.92 : 0.97)) return Order::kSequence;
-  return G == 1 && 2 * a->num_tiles * a->num_kv_heads >= 7 * cus ? Order::kDealtByHead : Order::kDealt;
+  if (even >= (G == 1 ? 0.75 : thin && rounds6 ? 0.88 : G == 2 ? 0.92 : 0.97)) return Order::kSequence;
+  return G == 1 && 2 * a->num_tiles * a->num_kv_heads >= (even >= 0.65 ? 7 : 22) * cus ? Order::kDealtByHead : Order::kDealt;
 }
 
 Spread spread_of(const sb_swa_prefill_args *a, int64_t max_keys) {
