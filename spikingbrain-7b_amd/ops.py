@@ -571,17 +571,16 @@ class PrefillPlan:
         self.tile_seq = packed[at:at + T]
         self.tile_q0 = packed[at + T:at + 2 * T]
         self.num_tiles, self.total_q, self.num_seqs = T, total_q, S
-        self._made = (T if T < PREFILL_DEALT_TILES else 0, 4 * at)   # (tiles listed in both orders, bytes in front of the lists)
+        # (tiles listed in both orders, bytes in front of the lists, and the lists themselves: a caller may put others in their place)
+        self._made = (T if T < PREFILL_DEALT_TILES else 0, 4 * at, self.tile_seq, self.tile_q0)
 
     def list_ptrs(self):
         """Addresses of the keys that the tiles walk (read on the host, at the call) and of the tiles in sequence order: None
         for lists too long or too short to need them, and for a plan whose lists are not those made here (a copy's are: no address is kept)."""
-        T, at = self._made
-        if T < 2 or self.num_tiles != T:
+        T, at, tile_seq, tile_q0 = self._made
+        if T < 2 or self.num_tiles != T or self.tile_seq is not tile_seq or self.tile_q0 is not tile_q0:
             return None, None, None
         first = self._packed.data_ptr() + at
-        if self.tile_seq.data_ptr() != first or self.tile_q0.data_ptr() != first + 4 * T:
-            return None, None, None
         return self._host.data_ptr() + at + 16 * T, first + 8 * T, first + 12 * T
 
     @property
@@ -732,6 +731,8 @@ def swa_prefill_attention(
             meta = dict(meta_k=N.ptr(meta_k), meta_v=N.ptr(meta_v), meta_len=meta_k.shape[0],
                         meta_stride_row=meta_k.stride(0), meta_stride_head=meta_k.stride(1))
     tile_keys, ordered_seq, ordered_q0 = plan.list_ptrs()
+    if tile_keys is not None:
+        meta.update(tile_keys=tile_keys, ordered_tile_seq=ordered_seq, ordered_tile_q0=ordered_q0)
     a = N.SwaPrefillArgs(
         q=N.ptr(q), k=N.ptr(k), v=N.ptr(v), out=N.ptr(out),
         block_table=N.ptr(block_table), kv_start=N.ptr(kv_start) if block_table is None else None,
@@ -749,8 +750,7 @@ def swa_prefill_attention(
         softcap=float(softcap), alibi_slopes=N.ptr(_slopes(alibi_slopes, Hq, dev)),
         meta_bias_row0=int(meta_bias[0]) if meta_bias else 0,
         meta_bias_rows=int(meta_bias[1]) if meta_bias else int(q.shape[0]),
-        kv_start32=N.ptr(kv_start32) if block_table is None else None,
-        tile_keys=tile_keys, ordered_tile_seq=ordered_seq, ordered_tile_q0=ordered_q0, **meta)
+        kv_start32=N.ptr(kv_start32) if block_table is None else None, **meta)
     L = N.lib()
     if n_parts == 0:
         n_parts = L.sb_swa_prefill_parts(C.byref(a), plan.max_k)
