@@ -145,3 +145,13 @@ def test_infinite_value_in_the_last_part(sb, dev, parts):
     whole, cut = (sb.ops.swa_prefill_attention(q.to(dev), k.to(dev), v.to(dev), n_parts=m, **kw).float().cpu() for m in (1, parts))
     assert torch.isposinf(whole[:, :, 7]).all() and torch.isposinf(cut[:, :, 7]).all()
     assert torch.equal(torch.isfinite(whole), torch.isfinite(cut))
+
+
+def test_more_parts_than_the_merge_addresses(sb, dev):
+    """Eight rows of a head's partials are addressed with 32 bits: 511 parts at 1024 heads. A call that asks for more gets fewer,
+    and from as many parts as the walk has chunks on the cut is the same: the same bits."""
+    g = torch.Generator().manual_seed(4)
+    q, k, v = (torch.randn(n, h, D, generator=g).bfloat16().to(dev) for n, h in ((1, 1024), (300, 64), (300, 64)))
+    run = lambda n: sb.ops.swa_prefill_attention(q, k, v, query_lens=[1], seq_lens_k=[300], kv_start=torch.zeros(1, dtype=torch.int64, device=dev),
+                                                 window_left=4096, n_parts=n)
+    assert torch.equal(run(1024), run(40))
