@@ -271,7 +271,7 @@ def bench_gla_step(sb, dev, B3=64, H3=28, iters=100):
 def bench_gla_prompt(sb, dev, S=16, L=8192, H=28, iters=3):
     """The GLA layers' share of BASELINE config 4 (16 prompts x 8192 tokens): one packed launch
     over token-major [tokens, H, D] projections, states read from and left in the slot cache.
-    bf16 prompts run the recurrence 16 tokens at a time on the matrix cores; the step-by-step fp32
+    bf16 prompts run the recurrence 32 tokens at a time on the matrix cores; the step-by-step fp32
     vector kernel is timed beside it. Bytes: q, k, v, out in bf16 and the fp32 gate, once each."""
     g = torch.Generator().manual_seed(0)
     tokens = S * L

@@ -326,10 +326,10 @@ typedef struct sb_gla_recurrent_args {
    * fields are the token strides, and seq_len is only an upper bound of the row lengths. */
   const int32_t *cu_seqlens;
   /* SB_GLA_* bits. Calls of 32 steps or more, and every packed call, with bf16 q/k/v run the
-   * recurrence 16 tokens at a time on the matrix cores (its exact block form; fp32 state, gate
+   * recurrence 32 tokens at a time on the matrix cores (its exact block form; fp32 state, gate
    * scan and accumulation; bf16 operand rounding on the output path as in any bf16 GEMM).
    * SB_GLA_VECTOR_ONLY keeps such calls on the step-by-step fp32 kernel.
-   * Gate range of the block form: inside a pair of blocks it forms exp(-(g_1 + .. + g_s)) per key dim, with
+   * Gate range of the block form: inside a block it forms exp(-(g_1 + .. + g_s)) per key dim, with
    * the exponent clamped at 80, so it is exact only while the gates of any 32 consecutive tokens sum to
    * more than -80 per key dim (|g| up to 2.5 per token, sustained; the model's log-sigmoid(x) / 16 gates
    * reach that only for x < -40). Beyond it near-diagonal q.k terms are under-weighted; the call itself
@@ -374,7 +374,7 @@ int sb_gla_prompt_segmented(const sb_gla_recurrent_args *args, int32_t n_segment
 
 /* Gate range check of the block form above. No counterpart in the reference (fla's kernel gives no such
  * signal). *hits = number of times the matrix-core GLA launches made with SB_GLA_CHECK_GATES on the current
- * device met gates beyond the range stated at `flags` (one per prompt, head, 32 key dims and pair of 16-token blocks concerned), since
+ * device met gates beyond the range stated at `flags` (one per prompt, head, 32 key dims and block of 32 tokens concerned), since
  * the counter was last cleared; reset != 0 clears it. Waits for the device (a blocking copy): call it where a synchronisation is
  * acceptable, e.g. once after the prompts of a batch, not under stream capture. 0 hits = every block-form
  * result so far is exact in the sense stated there. */

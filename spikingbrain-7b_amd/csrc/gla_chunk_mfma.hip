@@ -1,47 +1,51 @@
 // GLA over prompts on the matrix cores: the recurrence S <- diag(exp g) S + k^T v, o = (q*scale) S
-// advanced 16 tokens at a time in its exact block form. With B_t = g_1 + .. + g_t (per key dim,
+// advanced 32 tokens at a time in its exact block form. With B_t = g_1 + .. + g_t (per key dim,
 // inside the block) and S_0 the state before the block,
 //   o_t  = (q_t * exp(B_t)) S_0 + sum_{s<=t} [(q_t * exp(B_t)) . (k_s * exp(-B_s))] v_s
-//   S_16 = diag(exp(B_16)) S_0 + sum_s (k_s * exp(B_16 - B_s))^T v_s
-// i.e. per block one [16x16] score product, two products into o and a rank-16 update of the state,
-// all v_mfma_f32_16x16x32_bf16 with fp32 accumulation.
-// The decay of the state is applied every SECOND block: in between the registers hold S' = diag(exp(-L)) S,
-// L = the log-decay of the block just done, and the operands of the next block carry L in their exponents,
-//   o_t = (q_t * exp(B_t + L)) S' + intra-block term,   S' <- S' + (k_s * exp(-(B_s + L)))^T v_s,
-// after which S = diag(exp(L + B_16)) S' is formed. This halves the multiplies on the 64 state registers,
-// and k * exp(-(B_s + L)) serves both as the score operand and, transposed, as the state-update operand. The reference computes prompts with fla's
+//   S_32 = diag(exp(B_32)) (S_0 + sum_s (k_s * exp(-B_s))^T v_s)
+// i.e. per block three [16x16] score products (the fourth lies above the diagonal), two products into o and a
+// rank-32 update of the state, all v_mfma_f32_16x16x32_bf16 with fp32 accumulation; k * exp(-B_s) serves both as the
+// score operand and, transposed, as the state-update operand. The reference computes prompts with fla's
 // fused_chunk_gla (vllm_hymeta/model_for_7B/gla_attention.py:207-208), the same block mathematics.
 //
 // One workgroup per (sequence, head), four wavefronts; wavefront w keeps the state columns
 // [32w, 32w+32) as 16 accumulator tiles (64 registers) for the whole prompt: the state crosses HBM
-// once each way. Per block: thread (dim group r = tid / 16, token t = tid % 16) loads 8 consecutive dims of
-// its token's q, k, v (16 bytes each) and gate, five or four 16-byte loads instead of 48 two- and
-// four-byte ones (the vector memory pipe takes a wave's load at a fixed rate whatever its width); the
-// 16 tokens of a dim sit in the 16 lanes of a DPP row, so the gate scan over tokens is four row-shift
-// adds per dim. The threads turn their pieces into the four LDS operands, one barrier, then each
-// wavefront runs its 30 matrix instructions. LDS is double-buffered, so one barrier per block is
-// enough, and a wavefront prepares block n + 1 in the same stretch of code as it multiplies block n.
+// once each way. Per block a thread turns 8 dims of two neighbouring tokens of q, k, v and gate into LDS operands, and each
+// wavefront runs 66 matrix instructions on them. A block has two stretches of code between barriers:
+//   1. the gates of block n + 1 are summed over the tokens (see scan_gates), next to the outputs of block n;
+//   2. the operands of block n + 1 are formed, next to the state's update with block n.
+// k and v operands are double-buffered, q's (read in the first stretch, written in the second) are not.
 //
-// Precision: 16 tokens fill half of the instruction's K = 32, and the other half carries a second
-// bf16 term: the state update uses k * exp(B_16 - B_s) as hi + lo, so the state keeps fp32-level
+// What bounds it is memory, and there the pattern: heads of a token lie side by side, so a workgroup reads pieces of 256
+// bytes (512 of the fp32 gates) and a wavefront's share of a row is what one of its loads finds together. A loop of the
+// same loads and stores that computes nothing takes, for 16 x 8192 tokens x 28 heads (5.64 GB), 1340 us where a
+// wavefront's load covers 64 bytes of 16 rows and its store 32, 1258 with 64 bytes per store, 1172 with 128 bytes of 8 rows
+// per load as here, 1158 with whole rows (which would cut the sum over the tokens into four wavefronts).
+// Measured (us per call, blocks of 16 tokens read in 64-byte pieces -> this form): 16 x 8192 tokens 1400 -> 1240 (4.5 TB/s),
+// 8 x 4096 368 -> 283, 16 x 500 82 -> 66, 4 x 900 75 -> 68; shared states 16 x 8192 777 -> 659.
+//
+// Precision: the state update uses k * exp(-B_s) as hi + lo, two bf16 terms, so the state keeps fp32-level
 // accuracy (decay and accumulation are fp32; v is bf16 as given), and the scores enter o = A v as
-// hi + lo as well (their 16 signed products per row do not average out a 2^-9 rounding). The rest of
+// hi + lo as well (their signed products per row do not average out a 2^-9 rounding). The rest of
 // the output path rounds its operands (q*exp(B), k*exp(-B), S_0) to bf16 like any bf16 GEMM.
-// exp(-(B_s + L)) grows with the gates of at most two blocks: 32 * max|g| stays far below the fp32/bf16
+// exp(-B_s) grows with the gates of one block: 32 * max|g| stays far below the fp32/bf16
 // exponent range for any log-sigmoid gate (|g| up to 2.5 per token, sustained); the exponent is clamped at
-// 80 as a guard. A wavefront whose gates reach the clamp in a pair of blocks (results then under-weight
-// near-diagonal terms) adds one to a device counter that sb_gla_gate_range_hits reads.
+// 80 as a guard. Gates that reach the clamp in a block (results then under-weight near-diagonal terms) are counted, per 32
+// key dims, in a device counter that sb_gla_gate_range_hits reads.
 //
 // Tile row order: accumulator tile rt of the state holds rows 32*(rt/2) + 8*(m/4) + 4*(rt%2) + m%4
 // (m = tile row), so that the 8 consecutive rows a lane needs as the B operand of q S_0 are exactly
 // the rows it already holds in tiles 2*st and 2*st+1: no cross-lane movement between the update
 // and the next block's read of the state.
+//
+// Token order of a contraction over tokens: a lane's k index 8g + j stands for token 4g + j for j < 4 and
+// token 16 + 4g + j - 4 above, which is where the accumulator tiles of the two 16-token halves leave the scores.
 #include <mutex>
 
 #include "common.h"
 #include "mfma_util.h"
 
-// Events of gla_chunk_kernel meeting gates beyond the block form's range (one per wavefront and pair of blocks
+// Events of gla_chunk_kernel meeting gates beyond the block form's range (one per 32 key dims and block
 // concerned) since the counter was last cleared; one copy per GPU (the name is only the host's handle for
 // hipGetSymbolAddress).
 static __device__ unsigned int gla_range_hits;
@@ -65,7 +69,7 @@ struct GlaChunkParams {
   // stands for state head hh / jn and query head (hh / jn) * G + j0 + hh % jn; write_state: store the
   // final state. One state per head: G = jn = 1, j0 = 0, write_state = 1.
   int G, jn, j0, write_state;
-  unsigned int *range_hits;  // device counter of (wavefront, pair of blocks) events whose gates reached the exponent clamp
+  unsigned int *range_hits;  // device counter of (32 key dims, block) events whose gates reached the exponent clamp
   // Prompts cut into segments (0: not cut): seg_tokens tokens each, n_seg of them for the longest prompt. ws holds
   // per (row, state head, segment) the state in register order, 16384 floats, and behind all of those the
   // segments' total log-decays, 128 floats each (log2 units).
@@ -73,24 +77,33 @@ struct GlaChunkParams {
   float *ws;
 };
 
-constexpr int kCB = 16;      // tokens per block
-#ifndef SB_GLA_ROW
-#define SB_GLA_ROW 152
-#endif
-constexpr int kRow = SB_GLA_ROW;    // elements per row of the [16 tokens][128] LDS operands (304 B = 76 dwords: the 16-byte
-                             // stores and loads of 16 rows and the transposing loads of 4 rows spread over the banks)
+constexpr int kCB = 32;      // tokens per block
 constexpr float kMaxExp = 80.f;
 
 // All operands are stored token-major, one 16-byte store per thread each. The state update and the output
 // product contract over tokens and need [dim][token] operands: those are read with the transposing LDS load
 // (ds_read_b64_tr_b16), no transposed copy is ever written.
-struct Stage {
-  uint16_t qs[kCB][kRow];  // q * exp(B_t + L) * scale
-  uint16_t ks[kCB][kRow];  // k * exp(-(B_t + L)) rounded to bf16: score operand, and high part of the state-update operand
-  uint16_t kl[kCB][kRow];  // what the rounding left: low part of the state-update operand
-  uint16_t vs[kCB][kRow];  // v as loaded
-  float dec[128];          // exp(L + B_16) (second block of a pair), L + B_16 in log2 units (first block)
+typedef uint16_t Operand[kCB * 128];   // [token][dim], the 16-byte pieces of a row permuted: see piece_at
+
+struct KvStage {
+  Operand ks;      // k * exp(-B_t) rounded to bf16: score operand, and high part of the state-update operand
+  Operand kl;      // what the rounding left: low part of the state-update operand
+  Operand vs;      // v as loaded
+  float dec[128];  // exp(B_32)
 };
+// Gate sums of the block's first 16 tokens, for the wavefronts that hold the second 16; those of the first half read zeros.
+// Stores that are not wanted go to `spare`: no branches in that code.
+struct Carry {
+  float first[128], zero[128], spare[4];
+};
+
+// Rows are 256 bytes = all 64 banks, so piece p of row t lies at place p ^ f(t), with f such that the 16-byte accesses of 8
+// consecutive rows (matrix operands), of rows 0, 2, 4, 6 and two pieces (the stores) and the transposing loads of four rows
+// by four pieces all spread over the banks: the low two bits of t in front (a transposing load takes pieces 4 P .. 4 P + 3 of
+// rows 4 j .. 4 j + 3), bits 2 and 3 behind them. (Rows padded to 304 bytes instead spent half of the LDS cycles on conflicts.)
+__device__ __forceinline__ int piece_at(int t, int piece) {
+  return t * 128 + ((piece ^ ((t & 3) << 2 | (t >> 1 & 2) | (t >> 3 & 1))) << 3);
+}
 
 // ds_read_b64_tr_b16: in every group of 16 lanes, lane i names 8 bytes (4 elements) of LDS, "row i"; lane l
 // receives element l % 4 of rows l / 4, l / 4 + 4, l / 4 + 8, l / 4 + 12 (checked on the GPU). With row
@@ -119,6 +132,258 @@ __device__ __forceinline__ float row_shr(float x) {
 
 __device__ __forceinline__ float bf16_to_f32(uint16_t x) { return __uint_as_float((uint32_t)x << 16); }
 __device__ __forceinline__ uint16_t f32_to_bf16(float x) { return __builtin_bit_cast(uint16_t, (__bf16)x); }  // v_cvt_pk_bf16_f32
+
+// ---- pieces of a block that the kernels below share (same operations in the same order in all of them, so their
+// states and outputs are the same bits) ----------------------------------------------------------------------------
+template <int GDT>
+constexpr int kGateBytes = GDT == SB_F32 ? 4 : 2;
+
+// What thread `lane` of wavefront w loads and prepares: dims 8 piece .. 8 piece + 7 of tokens tok and tok + 1. A wavefront has
+// half of the dims of half of the tokens, so that its loads find 128 bytes of a row together; two pieces by eight token pairs
+// sit in the 16 lanes of a DPP row, the pairs two lanes apart.
+struct Share {
+  int piece, tok;
+  bool last_pair;   // of its half of the block
+  __device__ __forceinline__ Share(int w, int lane)
+      : piece(8 * (w & 1) + 2 * (lane >> 4) + (lane & 1)), tok(16 * (w >> 1) + (lane & 14)), last_pair((lane & 14) == 14) {}
+};
+template <int GDT>
+struct GateIn {
+  uint4 g[2][kGateBytes<GDT> / 2];  // fp32: dims 0..3, 4..7 of the piece; 16-bit: all 8
+};
+struct KvIn {
+  uint4 k[2], v[2];
+};
+
+// Where a thread's two rows lie behind a block's first row, in bytes. Tokens past the end of the prompt lie outside the
+// descriptors: such a load gives zeros, and a token with g = 0, q = k = v = 0 changes nothing.
+struct RowOffsets {
+  uint32_t at[2];
+  __device__ __forceinline__ RowOffsets(const Share &me, int piece_bytes, int64_t row_bytes) {
+    at[0] = me.tok * (int)row_bytes + me.piece * piece_bytes;
+    at[1] = at[0] + (int)row_bytes;
+  }
+  __device__ __forceinline__ void cut(const Share &me, int valid) {   // only tokens 0 .. valid - 1 of the block exist
+    if (me.tok >= valid) at[0] = 0x80000000u;
+    if (me.tok + 1 >= valid) at[1] = 0x80000000u;
+  }
+};
+
+template <int GDT>
+__device__ __forceinline__ float gate_at(const uint4 *g, int i) {
+  if constexpr (GDT == SB_F32) return __uint_as_float(word(g[i >> 2], i & 3));
+  else if constexpr (GDT == SB_BF16) return (i & 1) ? bf16_hi(word(g[0], i >> 1)) : bf16_lo(word(g[0], i >> 1));
+  else return (i & 1) ? f16_hi(word(g[0], i >> 1)) : f16_lo(word(g[0], i >> 1));
+}
+
+// Gates of the thread's two tokens summed from the start of its half of the block on, per dim, in log2 units (bare v_exp
+// afterwards); the first half's totals go to LDS. One add inside the pair, three row-shift adds over the pairs, one more for
+// the first token (two separate tokens would take eight).
+template <int GDT>
+__device__ __forceinline__ void scan_gates(const GateIn<GDT> &in, const Share &me, int w, Carry &carry, float (&b0)[8], float (&b1)[8]) {
+#pragma clang fp contract(off)   // (the last sum as a multiply-add would need its shifted operand moved first)
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float x0 = gate_at<GDT>(in.g[0], i) * kLog2e;
+    float x = x0 + gate_at<GDT>(in.g[1], i) * kLog2e;
+    x += row_shr<2>(x);
+    x += row_shr<4>(x);
+    x += row_shr<8>(x);
+    b1[i] = x;
+    b0[i] = x0 + row_shr<2>(x);
+  }
+  const bool keep = w < 2 && me.last_pair;
+  float *d = keep ? &carry.first[8 * me.piece] : carry.spare;
+  *reinterpret_cast<float4 *>(d) = make_float4(b1[0], b1[1], b1[2], b1[3]);
+  *reinterpret_cast<float4 *>(keep ? d + 4 : d) = make_float4(b1[4], b1[5], b1[6], b1[7]);
+}
+// ... and from the start of the block on, behind the barrier that follows
+__device__ __forceinline__ void add_carry(const Carry &carry, const Share &me, int w, float (&b0)[8], float (&b1)[8]) {
+  const float *first = (w < 2 ? carry.zero : carry.first) + 8 * me.piece;
+  const f32x4_t x[2] = {*reinterpret_cast<const f32x4_t *>(first), *reinterpret_cast<const f32x4_t *>(first + 4)};
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    b0[i] += x[i >> 2][i & 3];
+    b1[i] += x[i >> 2][i & 3];
+  }
+}
+
+// k-hat of the thread's two tokens as hi + lo, and v, into their rows
+__device__ __forceinline__ void store_kv(KvStage &st, const Share &me, const KvIn &in, const float (&b0)[8], const float (&b1)[8]) {
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const float(&b)[8] = u ? b1 : b0;
+    uint32_t ks[4], kl[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float x0 = bf16_lo(word(in.k[u], i)) * fast_exp2(fminf(-b[2 * i], kMaxExp * kLog2e));
+      const float x1 = bf16_hi(word(in.k[u], i)) * fast_exp2(fminf(-b[2 * i + 1], kMaxExp * kLog2e));
+      // the rounded value is the score operand and the high part of the state-update operand
+      ks[i] = Mma<BF16>::pack(x0, x1);
+      kl[i] = Mma<BF16>::pack(x0 - __uint_as_float(ks[i] << 16), x1 - __uint_as_float(ks[i] & 0xffff0000u));
+    }
+    const int at = piece_at(me.tok + u, me.piece);
+    *reinterpret_cast<uint4 *>(&st.ks[at]) = make_uint4(ks[0], ks[1], ks[2], ks[3]);
+    *reinterpret_cast<uint4 *>(&st.kl[at]) = make_uint4(kl[0], kl[1], kl[2], kl[3]);
+    *reinterpret_cast<uint4 *>(&st.vs[at]) = in.v[u];
+  }
+}
+// q * scale * exp(B) of the two tokens; e: exp(B)
+__device__ __forceinline__ void store_q(Operand &qs, const Share &me, const uint4 (&q)[2], const float (&e0)[8], const float (&e1)[8],
+                                        float scale) {
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const float(&e)[8] = u ? e1 : e0;
+    uint32_t x[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      x[i] = Mma<BF16>::pack(bf16_lo(word(q[u], i)) * scale * e[2 * i], bf16_hi(word(q[u], i)) * scale * e[2 * i + 1]);
+    *reinterpret_cast<uint4 *>(&qs[piece_at(me.tok + u, me.piece)]) = make_uint4(x[0], x[1], x[2], x[3]);
+  }
+}
+// The block's decay: exp(B_32) of the last token
+__device__ __forceinline__ void store_decay(KvStage &st, Carry &carry, const Share &me, int w, const float (&e1)[8]) {
+  const bool keep = w >= 2 && me.last_pair;
+  float *d = keep ? &st.dec[8 * me.piece] : carry.spare;
+  *reinterpret_cast<float4 *>(d) = make_float4(e1[0], e1[1], e1[2], e1[3]);
+  *reinterpret_cast<float4 *>(keep ? d + 4 : d) = make_float4(e1[4], e1[5], e1[6], e1[7]);
+}
+
+// The lane's place in a matrix tile, for code behind the block loop: worked out again there, or the addresses that the loop
+// keeps for its operands would have copies of their own live across it (34 spilled registers).
+struct TileLane {
+  int g, c;
+  __device__ __forceinline__ explicit TileLane(int lane) {
+    asm volatile("" : "+v"(lane));
+    g = lane >> 4;
+    c = lane & 15;
+  }
+};
+
+// 16-byte matrix operand: dims 32 s4 + 8g .. + 7 of token c of a half
+__device__ __forceinline__ uint4 row_operand(const Operand &x, int half, int g, int c, int s4) {
+  return *reinterpret_cast<const uint4 *>(&x[piece_at(c, 4 * s4 + g) + half * 16 * 128]);
+}
+// Operand of a product that contracts over the block's tokens: dims f(j) = 32 block + 8 j + 4 part, j = c / 4, element c % 4
+__device__ __forceinline__ uint4 column_operand(const Operand &x, int g, int c, int block, int part) {
+  const int at = piece_at(4 * g + (c >> 2), 4 * block + (c & 3)) + 4 * part;
+  const uint2 lo = load_transposed(&x[at]), hi = load_transposed(&x[at + 16 * 128]);
+  return make_uint4(lo.x, lo.y, hi.x, hi.y);
+}
+
+// The state of one (slot, head): 16 tiles of this wavefront's 32 columns; column n = c of tile nt is column
+// 32w + 8 (c / 4) + 4 nt + c % 4, so that a lane has 8 neighbouring columns of its tokens' outputs in its two tiles (one
+// 16-byte store). A lane's elements lie at one offset of its own
+// plus constants (scalar offsets of the buffer loads: no address registers per element).
+typedef f32x4_t StateTiles[8][2];
+__device__ __forceinline__ int state_offset(int rt, int nt, int i) { return (32 * (rt >> 1) + 4 * (rt & 1) + i) * 128 + 4 * nt; }
+template <bool kF32>
+__device__ __forceinline__ void load_state(StateTiles &S, const char *base, int g, int c, int w) {
+  const __amdgpu_buffer_rsrc_t rows = rows_from(base);
+  const int at = (8 * g * 128 + 32 * w + 8 * (c >> 2) + (c & 3)) * (kF32 ? 4 : 2);
+#pragma unroll
+  for (int rt = 0; rt < 8; ++rt)
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        S[rt][nt][i] = kF32 ? __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rows, at, state_offset(rt, nt, i) * 4, 0))
+                            : bf16_to_f32(__builtin_amdgcn_raw_buffer_load_b16(rows, at, state_offset(rt, nt, i) * 2, 0));
+}
+template <bool kF32>
+__device__ __forceinline__ void store_state(const StateTiles &S, char *base, int g, int c, int w) {
+  const __amdgpu_buffer_rsrc_t rows = rows_from(base);
+  const int at = (8 * g * 128 + 32 * w + 8 * (c >> 2) + (c & 3)) * (kF32 ? 4 : 2);
+#pragma unroll
+  for (int rt = 0; rt < 8; ++rt)
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if constexpr (kF32) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(S[rt][nt][i]), rows, at, state_offset(rt, nt, i) * 4, 0);
+        else __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16(S[rt][nt][i]), rows, at, state_offset(rt, nt, i) * 2, 0);
+      }
+}
+
+// Scores x (rows s = 4g + i of a half, column t = c) as two bf16 terms
+__device__ __forceinline__ void split_scores(const f32x4_t &x, uint2 &hi, uint2 &lo) {
+  hi.x = Mma<BF16>::pack(x[0], x[1]);
+  hi.y = Mma<BF16>::pack(x[2], x[3]);
+  lo.x = Mma<BF16>::pack(x[0] - __uint_as_float(hi.x << 16), x[1] - __uint_as_float(hi.x & 0xffff0000u));
+  lo.y = Mma<BF16>::pack(x[2] - __uint_as_float(hi.y << 16), x[3] - __uint_as_float(hi.y & 0xffff0000u));
+}
+__device__ __forceinline__ void mask_diagonal(f32x4_t &x, int g, int c) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (4 * g + i > c) x[i] = 0.f;
+}
+
+// Rows 32 s4 + 8g .. + 7 of the state, rounded, as operand of q S_0
+__device__ __forceinline__ uint4 state_operand(const StateTiles &S, int s4, int nt) {
+  const f32x4_t &a = S[2 * s4][nt], &b = S[2 * s4 + 1][nt];
+  return make_uint4(Mma<BF16>::pack(a[0], a[1]), Mma<BF16>::pack(a[2], a[3]), Mma<BF16>::pack(b[0], b[1]), Mma<BF16>::pack(b[2], b[3]));
+}
+
+// Scores of one head and block, and what they contribute to its outputs, o[half][tile]: o^T = v^T A^T, lane (g, c) has token c
+// of a half and 4 of the tile's columns (the operand registers are the same either way round: a lane holds
+// index c of the tile's outer dimension and 8g..8g+7 of the contraction in both operands).
+__device__ __forceinline__ void output_scores(const uint4 (&ka)[2][4], const uint4 (&qa)[2][4], const uint4 (&vb)[2], int g, int c,
+                                              f32x4_t (&o)[2][2]) {
+  // (transposed) a[s half][t half], element i = A[t = c][s = 4g + i], zero above the diagonal
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4_t a00 = zero, a01 = zero, a11 = zero;
+#pragma unroll
+  for (int s4 = 0; s4 < 4; ++s4) {
+    a00 = Mma<BF16>::run(ka[0][s4], qa[0][s4], a00);
+    a01 = Mma<BF16>::run(ka[0][s4], qa[1][s4], a01);
+    a11 = Mma<BF16>::run(ka[1][s4], qa[1][s4], a11);
+  }
+  mask_diagonal(a00, g, c);
+  mask_diagonal(a11, g, c);
+  uint2 h00, l00, h01, l01, h11, l11;
+  split_scores(a00, h00, l00);
+  split_scores(a01, h01, l01);
+  split_scores(a11, h11, l11);
+  // the first half's scores fill half of the contraction: their low terms take the other, against v repeated
+#pragma unroll
+  for (int nt = 0; nt < 2; ++nt) {
+    o[0][nt] = Mma<BF16>::run(make_uint4(vb[nt].x, vb[nt].y, vb[nt].x, vb[nt].y), make_uint4(h00.x, h00.y, l00.x, l00.y), zero);
+    o[1][nt] = Mma<BF16>::run(vb[nt], make_uint4(l01.x, l01.y, l11.x, l11.y), zero);
+    o[1][nt] = Mma<BF16>::run(vb[nt], make_uint4(h01.x, h01.y, h11.x, h11.y), o[1][nt]);
+  }
+}
+
+// S <- diag(dec) (S + k-hat^T v); a tile pair is decayed behind the matrix instructions of the next one
+__device__ __forceinline__ void update_state(StateTiles &S, const KvStage &st, int g, int c, const uint4 (&vb)[2]) {
+  auto decay = [&](int rt) {
+    const float4 dc = *reinterpret_cast<const float4 *>(&st.dec[32 * (rt >> 1) + 8 * g + 4 * (rt & 1)]);
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+      S[rt][nt][0] *= dc.x; S[rt][nt][1] *= dc.y; S[rt][nt][2] *= dc.z; S[rt][nt][3] *= dc.w;
+    }
+  };
+#pragma unroll
+  for (int rt = 0; rt < 8; ++rt) {
+    // this lane's operand row is state row 32 (rt / 2) + 8 (c / 4) + 4 (rt % 2) + c % 4
+    const uint4 kh = column_operand(st.ks, g, c, rt >> 1, rt & 1), kl = column_operand(st.kl, g, c, rt >> 1, rt & 1);
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) S[rt][nt] = Mma<BF16>::run(kh, vb[nt], S[rt][nt]);
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) S[rt][nt] = Mma<BF16>::run(kl, vb[nt], S[rt][nt]);
+    if (rt > 0) decay(rt - 1);
+  }
+  decay(7);
+}
+
+// 8 columns of one token's output; rows past the end of the prompt fall outside the descriptor and are dropped
+__device__ __forceinline__ void store_out(__amdgpu_buffer_rsrc_t rows, uint32_t off, const f32x4_t &a, const f32x4_t &b) {
+  u32x4_t val;
+  val.x = Mma<BF16>::pack(a[0], a[1]);
+  val.y = Mma<BF16>::pack(a[2], a[3]);
+  val.z = Mma<BF16>::pack(b[0], b[1]);
+  val.w = Mma<BF16>::pack(b[2], b[3]);
+  __builtin_amdgcn_raw_buffer_store_b128(val, rows, off, 0, 0);
+}
 
 // kCheck: report gates beyond the block form's range (SB_GLA_CHECK_GATES); a build of its own, because even this
 // little extra work shifts the register allocation of a kernel that runs at the edge of its budget (0-4 % slower).
@@ -157,16 +422,94 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int g = lane >> 4, c = lane & 15;
-  const int r = tid >> 4;          // dims 8r .. 8r+7 of token c: this thread's piece of a block's inputs
+  const Share me(w, lane);
 
-  __shared__ __attribute__((aligned(16))) Stage stage[2];
+  __shared__ __attribute__((aligned(16))) KvStage stage[2];
+  __shared__ __attribute__((aligned(16))) Operand qs;   // q * exp(B_t) * scale
+  __shared__ __attribute__((aligned(16))) Carry carry;
 
   // ---- state: 8 row tiles x 2 column tiles of this wavefront's 32 columns -------------------------
   char *sbase = reinterpret_cast<char *>(p.state) + (slot * p.s_slot + (int64_t)hk * p.s_head) * (kStateF32 ? 4 : 2);
-  f32x4_t S[8][2];
-  auto state_index = [&](int rt, int nt, int i) {
-    return (32 * (rt >> 1) + 8 * g + 4 * (rt & 1) + i) * 128 + 32 * w + 16 * nt + c;
+  StateTiles S;
+
+  // ---- block inputs in registers -------------------------------------------------------------------------
+  constexpr int GB = kGateBytes<GDT>;
+  const char *gb = reinterpret_cast<const char *>(p.g) + go * GB;
+  const char *qb = reinterpret_cast<const char *>(p.q + qo), *kb = reinterpret_cast<const char *>(p.k + ko),
+             *vb_ = reinterpret_cast<const char *>(p.v + vo);
+  const int64_t g_row = p.g_st * GB, q_row = p.q_st * 2, k_row = p.k_st * 2, v_row = p.v_st * 2, o_row = p.o_st * 2;
+  RowOffsets q_at(me, 16, q_row), k_at(me, 16, k_row), v_at(me, 16, v_row), g_at(me, 8 * GB, g_row);
+  const int last = (T - 1) / kCB;   // (only this block can have rows past the end, and it is fetched last)
+  GateIn<GDT> gates;
+  KvIn kv;
+  uint4 q[2];
+  auto fetch_gates = [&](int n) {
+    if ((n + 1) * kCB > T) g_at.cut(me, T - n * kCB);
+    const __amdgpu_buffer_rsrc_t gr = rows_from(gb + n * kCB * g_row);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int j = 0; j < GB / 2; ++j) gates.g[u][j] = load16(gr, g_at.at[u] + 16 * j);
   };
+  auto fetch = [&](int n) {
+    if ((n + 1) * kCB > T) { q_at.cut(me, T - n * kCB); k_at.cut(me, T - n * kCB); v_at.cut(me, T - n * kCB); }
+    const __amdgpu_buffer_rsrc_t qr = rows_from(qb + n * kCB * q_row), kr = rows_from(kb + n * kCB * k_row),
+                                 vr = rows_from(vb_ + n * kCB * v_row);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      kv.k[u] = load16(kr, k_at.at[u]);
+      q[u] = load16(qr, q_at.at[u]);
+      kv.v[u] = load16(vr, v_at.at[u]);
+    }
+  };
+
+  // ---- the LDS operands of one block -----------------------------------------------------------------------
+  float b0[8], b1[8];   // gate sums of the thread's two tokens
+  auto prepare = [&](KvStage &st, [[maybe_unused]] bool real) {
+    add_carry(carry, me, w, b0, b1);
+    // Gate range: the largest exponent formed in a block is minus its total log-decay; one event per 32 dims = half of the
+    // wavefronts that hold the last token, reported on the spot
+    if constexpr (kCheck) {
+      const float worst = fminf(fminf(fminf(b1[0], b1[1]), fminf(b1[2], b1[3])), fminf(fminf(b1[4], b1[5]), fminf(b1[6], b1[7])));
+      const uint64_t hit = __builtin_amdgcn_ballot_w64(real && w >= 2 && me.last_pair && worst < -kMaxExp * kLog2e);
+      if (hit != 0 && lane == 0) atomicAdd(p.range_hits, ((uint32_t)hit != 0) + ((uint32_t)(hit >> 32) != 0));
+    }
+    store_kv(st, me, kv, b0, b1);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) { b0[i] = fast_exp2(b0[i]); b1[i] = fast_exp2(b1[i]); }
+    store_q(qs, me, q, b0, b1, p.scale);
+    store_decay(st, carry, me, w, b1);
+  };
+
+  // ---- the outputs of one block on this wavefront's 32 state columns ----------------------------------------
+  uint4 vb[2];
+  auto outputs = [&](int n, const KvStage &st) {
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) vb[nt] = column_operand(st.vs, g, c, w, nt);
+    uint4 qa[2][4], ka[2][4];
+#pragma unroll
+    for (int s4 = 0; s4 < 4; ++s4)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) { ka[u][s4] = row_operand(st.ks, u, g, c, s4); qa[u][s4] = row_operand(qs, u, g, c, s4); }
+    f32x4_t o[2][2];
+    output_scores(ka, qa, vb, g, c, o);
+#pragma unroll
+    for (int s4 = 0; s4 < 4; ++s4)
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) {
+        const uint4 sb16 = state_operand(S, s4, nt);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) o[u][nt] = Mma<BF16>::run(sb16, qa[u][s4], o[u][nt]);
+      }
+    const __amdgpu_buffer_rsrc_t orows = __builtin_amdgcn_make_buffer_rsrc(
+        reinterpret_cast<char *>(p.out + oo) + n * kCB * o_row, 0, min(kCB, T - n * kCB) * (int)o_row, 0x00020000);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) store_out(orows, (16 * u + c) * (int)o_row + (32 * w + 8 * g) * 2, o[u][0], o[u][1]);
+  };
+
+  // ---- block loop. Loads are issued as soon as their registers are free: the gates of block n + 2 in the first stretch of
+  // block n, its q, k and v in the second.
+  // (behind the first block's loads, which are waited for first)
   if constexpr (kSeg) {
     const int Hk = p.H / p.jn;
     const f32x4_t *src = reinterpret_cast<const f32x4_t *>(p.ws + (((int64_t)b * Hk + hk) * p.n_seg + seg) * 16384) + tid;
@@ -175,271 +518,43 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
       for (int nt = 0; nt < 2; ++nt) S[rt][nt] = src[(2 * rt + nt) * 256];
   } else {
-#pragma unroll
-    for (int rt = 0; rt < 8; ++rt)
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int idx = state_index(rt, nt, i);
-          S[rt][nt][i] = kStateF32 ? reinterpret_cast<const float *>(sbase)[idx]
-                                   : bf16_to_f32(reinterpret_cast<const uint16_t *>(sbase)[idx]);
-        }
+    load_state<kStateF32>(S, sbase, g, c, w);
   }
-
-  // ---- block inputs in registers: 8 dims of one token's q, k, v (bf16) and gate ---------------------------
-  constexpr int kGateBytes = GDT == SB_F32 ? 4 : 2;
-  const char *gb = reinterpret_cast<const char *>(p.g) + go * kGateBytes;
-  const char *qb = reinterpret_cast<const char *>(p.q + qo), *kb = reinterpret_cast<const char *>(p.k + ko),
-             *vb_ = reinterpret_cast<const char *>(p.v + vo);
-  const int64_t g_row = p.g_st * kGateBytes, q_row = p.q_st * 2, k_row = p.k_st * 2, v_row = p.v_st * 2, o_row = p.o_st * 2;
-  struct BlockIn {
-    uint4 q, k, v;
-    uint4 g[kGateBytes / 2];  // fp32: dims 8r..8r+3, 8r+4..8r+7; 16-bit: all 8
-  };
-  auto fetch = [&](int t0, BlockIn &in) {
-    const int tok = min(c, T - 1 - t0);  // rows past the end re-read the last token; prepare() zeroes them
-    in.q = load16(rows_from(qb + t0 * q_row), tok * (int)q_row + r * 16);
-    in.k = load16(rows_from(kb + t0 * k_row), tok * (int)k_row + r * 16);
-    in.v = load16(rows_from(vb_ + t0 * v_row), tok * (int)v_row + r * 16);
-    const __amdgpu_buffer_rsrc_t gr = rows_from(gb + t0 * g_row);
-#pragma unroll
-    for (int j = 0; j < kGateBytes / 2; ++j) in.g[j] = load16(gr, tok * (int)g_row + r * 8 * kGateBytes + 16 * j);
-  };
-
-  // ---- the four LDS operands of one block. Gates in log2 units (bare v_exp afterwards); a token past the
-  // end of the prompt is a token with g = 0, q = k = v = 0 ------------------------------------------------
-  auto fix_tail = [&](BlockIn &in, int t0) {
-    if (t0 + kCB > T && t0 + c >= T) {
-      in.q = in.k = in.v = make_uint4(0u, 0u, 0u, 0u);
-#pragma unroll
-      for (int j = 0; j < kGateBytes / 2; ++j) in.g[j] = make_uint4(0u, 0u, 0u, 0u);
-    }
-  };
-  // kSecond = false: first block of a pair (state undecayed on entry: L = 0); leaves L = its total log-decay
-  // in `carry` and, for the case that the prompt ends here, in st.dec (log2 units).
-  // kSecond = true: exponents carry L; st.dec = exp(L + B_16), the decay multiply() applies afterwards.
-  float carry[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) carry[i] = 0.f;
-  auto prepare = [&](const BlockIn &in, Stage &st, auto second_tag) {
-    constexpr bool kSecond = decltype(second_tag)::value;
-    const uint4 rq = in.q, rk = in.k, rv = in.v;
-    float B[8], tot[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      float x;
-      if constexpr (GDT == SB_F32) x = __uint_as_float(word(in.g[i >> 2], i & 3));
-      else if constexpr (GDT == SB_BF16) x = (i & 1) ? bf16_hi(word(in.g[0], i >> 1)) : bf16_lo(word(in.g[0], i >> 1));
-      else x = (i & 1) ? f16_hi(word(in.g[0], i >> 1)) : f16_lo(word(in.g[0], i >> 1));
-      x *= kLog2e;
-      // inclusive scan over the 16 tokens = the 16 lanes of this row
-      x += row_shr<1>(x);
-      x += row_shr<2>(x);
-      x += row_shr<4>(x);
-      x += row_shr<8>(x);
-      if constexpr (kSecond) x += carry[i];
-      B[i] = x;
-      tot[i] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane | 15) << 2, __builtin_bit_cast(int, x)));
-    }
-    // Gate range: the largest exponent formed inside a pair of blocks is minus its total log-decay. Checked where
-    // the pair ends, and reported on the spot (a flag carried through the loop costs this kernel 6 %: it runs at
-    // the edge of its register budget).
-    if constexpr (kSecond && kCheck) {
-      const float worst = fminf(fminf(fminf(tot[0], tot[1]), fminf(tot[2], tot[3])), fminf(fminf(tot[4], tot[5]), fminf(tot[6], tot[7])));
-      if (__builtin_amdgcn_ballot_w64(worst < -kMaxExp * kLog2e) != 0 && lane == 0) atomicAdd(p.range_hits, 1u);
-    }
-    float qf[8], kf[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      qf[2 * i] = bf16_lo(word(rq, i));
-      qf[2 * i + 1] = bf16_hi(word(rq, i));
-      kf[2 * i] = bf16_lo(word(rk, i));
-      kf[2 * i + 1] = bf16_hi(word(rk, i));
-    }
-    uint32_t qs[4], ks[4], kl[4];
-#pragma unroll
-    for (int i = 0; i < 8; i += 2) {
-      qs[i / 2] = Mma<BF16>::pack(qf[i] * p.scale * fast_exp2(B[i]), qf[i + 1] * p.scale * fast_exp2(B[i + 1]));
-      const float x0 = kf[i] * fast_exp2(fminf(-B[i], kMaxExp * kLog2e)), x1 = kf[i + 1] * fast_exp2(fminf(-B[i + 1], kMaxExp * kLog2e));
-      // the rounded value is the score operand and the high part of the state-update operand
-      const uint32_t h = Mma<BF16>::pack(x0, x1);
-      const uint32_t l = Mma<BF16>::pack(x0 - __uint_as_float(h << 16), x1 - __uint_as_float(h & 0xffff0000u));
-      ks[i / 2] = h;
-      kl[i / 2] = l;
-    }
-    *reinterpret_cast<uint4 *>(&st.qs[c][8 * r]) = make_uint4(qs[0], qs[1], qs[2], qs[3]);
-    *reinterpret_cast<uint4 *>(&st.ks[c][8 * r]) = make_uint4(ks[0], ks[1], ks[2], ks[3]);
-    *reinterpret_cast<uint4 *>(&st.kl[c][8 * r]) = make_uint4(kl[0], kl[1], kl[2], kl[3]);
-    *reinterpret_cast<uint4 *>(&st.vs[c][8 * r]) = rv;
-    // (every lane of the row holds the same totals and stores them to the same address: no branch here)
-    if constexpr (kSecond) {
-      *reinterpret_cast<float4 *>(&st.dec[8 * r]) = make_float4(fast_exp2(tot[0]), fast_exp2(tot[1]), fast_exp2(tot[2]), fast_exp2(tot[3]));
-      *reinterpret_cast<float4 *>(&st.dec[8 * r + 4]) = make_float4(fast_exp2(tot[4]), fast_exp2(tot[5]), fast_exp2(tot[6]), fast_exp2(tot[7]));
-    } else {
-      *reinterpret_cast<float4 *>(&st.dec[8 * r]) = make_float4(tot[0], tot[1], tot[2], tot[3]);
-      *reinterpret_cast<float4 *>(&st.dec[8 * r + 4]) = make_float4(tot[4], tot[5], tot[6], tot[7]);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) carry[i] = tot[i];
-    }
-  };
-
-  // ---- the 30 matrix instructions of one block on this wavefront's 32 state columns ---------------------
-  auto multiply = [&](int t0, const Stage &st, auto second_tag) {
-    constexpr bool kSecond = decltype(second_tag)::value;
-    // scores (transposed): at[i] = A[t = c][s = 4g + i], zero above the diagonal
-    uint4 qa[4];
-    f32x4_t at = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s4 = 0; s4 < 4; ++s4) {
-      qa[s4] = *reinterpret_cast<const uint4 *>(&st.qs[c][32 * s4 + 8 * g]);
-      const uint4 ka = *reinterpret_cast<const uint4 *>(&st.ks[c][32 * s4 + 8 * g]);
-      at = Mma<BF16>::run(ka, qa[s4], at);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (4 * g + i > c) at[i] = 0.f;
-    // as the A operand of o = A v: row t = c, k index 8g + j <-> s = 4g + j for j < 4; the scores go in
-    // as two bf16 terms (hi in k index 0..3, lo in 4..7, against v repeated), so that the 16 signed
-    // products of a row are summed from scores good to 16 bits
-    const uint32_t h01 = Mma<BF16>::pack(at[0], at[1]), h23 = Mma<BF16>::pack(at[2], at[3]);
-    const uint4 pa = make_uint4(h01, h23,
-                                Mma<BF16>::pack(at[0] - __uint_as_float(h01 << 16), at[1] - __uint_as_float(h01 & 0xffff0000u)),
-                                Mma<BF16>::pack(at[2] - __uint_as_float(h23 << 16), at[3] - __uint_as_float(h23 & 0xffff0000u)));
-
-    // v as the B operand of both products: v[s = 4g + j][col] at k index j and again at 4 + j, so
-    // that the A operands can carry a high term in k index 0..3 and a low term in 4..7 (16 tokens
-    // fill only half of the instruction's K = 32)
-    uint4 vb[2];
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      const uint2 x = load_transposed(&st.vs[4 * g + (c >> 2)][32 * w + 16 * nt + 4 * (c & 3)]);
-      vb[nt] = make_uint4(x.x, x.y, x.x, x.y);
-    }
-
-    // o^T = v^T A^T + S_0^T (q exp B)^T: lane (g, c) ends up with token c, columns 4g..4g+3 of each tile:
-    // one 8-byte store per tile (the operand registers are the same either way round: a lane holds
-    // index c of the tile's outer dimension and 8g..8g+7 of the contraction in both operands)
-    f32x4_t o[2];
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      o[nt] = Mma<BF16>::run(vb[nt], pa, f32x4_t{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-      for (int s4 = 0; s4 < 4; ++s4) {
-        const f32x4_t &a = S[2 * s4][nt], &bb = S[2 * s4 + 1][nt];  // rows 32 s4 + 8g + {0..3}, {4..7}
-        const uint4 sb16 = make_uint4(Mma<BF16>::pack(a[0], a[1]), Mma<BF16>::pack(a[2], a[3]),
-                                      Mma<BF16>::pack(bb[0], bb[1]), Mma<BF16>::pack(bb[2], bb[3]));
-        o[nt] = Mma<BF16>::run(sb16, qa[s4], o[nt]);
-      }
-    }
-    {  // rows past the end of the prompt fall outside the descriptor and are dropped: no branch in this code
-      const __amdgpu_buffer_rsrc_t orows = __builtin_amdgcn_make_buffer_rsrc(
-          reinterpret_cast<char *>(p.out + oo) + t0 * o_row, 0, min(kCB, T - t0) * (int)o_row, 0x00020000);
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt) {
-        typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
-        u32x2_t val;
-        val.x = Mma<BF16>::pack(o[nt][0], o[nt][1]);
-        val.y = Mma<BF16>::pack(o[nt][2], o[nt][3]);
-        __builtin_amdgcn_raw_buffer_store_b64(val, orows, c * (int)o_row + (32 * w + 16 * nt + 4 * g) * 2, 0, 0);
-      }
-    }
-
-    // S' <- S' + k-hat^T v, and after the second block of a pair S <- diag(exp(L + B_16)) S'
-#pragma unroll
-    for (int rt = 0; rt < 8; ++rt) {
-      // this lane's operand row is state row 32 (rt / 2) + 8 (c / 4) + 4 (rt % 2) + c % 4: f(j) = 32 (rt / 2) + 8 j + 4 (rt % 2)
-      const int tok = 4 * g + (c >> 2), dims = 32 * (rt >> 1) + 8 * (c & 3) + 4 * (rt & 1);
-      const uint2 h2 = load_transposed(&st.ks[tok][dims]);
-      const uint2 l2 = load_transposed(&st.kl[tok][dims]);
-      const uint4 ka = make_uint4(h2.x, h2.y, l2.x, l2.y);
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt) S[rt][nt] = Mma<BF16>::run(ka, vb[nt], S[rt][nt]);
-      if constexpr (kSecond) {
-        const float4 dc = *reinterpret_cast<const float4 *>(&st.dec[32 * (rt >> 1) + 8 * g + 4 * (rt & 1)]);
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt) {
-          S[rt][nt][0] *= dc.x; S[rt][nt][1] *= dc.y; S[rt][nt][2] *= dc.z; S[rt][nt][3] *= dc.w;
-        }
-      }
-    }
-  };
-
-  // ---- block loop. An iteration runs the matrix instructions of block blk and turns the inputs of block
-  // blk + 1 into the other LDS stage, then fetches the inputs of block blk + 2 into the registers just used; a
-  // fetch past the last block re-reads it, and the block after the last is prepared as 16 dead tokens (never
-  // multiplied). One barrier per block: what an iteration writes was last read one iteration before the
-  // barrier it follows. Blocks go in pairs (first, second); a prompt that ends on a first block leaves
-  // S' = diag(exp(-L)) S in the registers, put right after the loop.
-  const int n_blocks = (T + kCB - 1) / kCB;
-  const std::false_type kFirst{};
-  const std::true_type kSecond{};
-  BlockIn in;
-  fetch(0, in);
-  fix_tail(in, 0);
-  prepare(in, stage[0], kFirst);
-  fetch(min(1, n_blocks - 1) * kCB, in);
-  int blk = 0;
-  for (; blk + 1 < n_blocks; blk += 2) {
+  if (tid < 128) carry.zero[tid] = 0.f;
+  fetch_gates(0);
+  fetch(0);
+  scan_gates<GDT>(gates, me, w, carry, b0, b1);
+  fetch_gates(min(1, last));
+  __syncthreads();
+  prepare(stage[0], true);
+  fetch(min(1, last));
+  // (one body for all blocks: the last one forms operands that nothing multiplies, 0.5 us; a copy of the body without them
+  // behind the loop costs registers that the loop needs, 8 x 4096 tokens 283 -> 288-328 us)
+  for (int n = 0; n <= last; ++n) {
+    const KvStage &now = stage[n & 1];
     __syncthreads();
-    fix_tail(in, (blk + 1) * kCB);
-    multiply(blk * kCB, stage[0], kFirst);
-    prepare(in, stage[1], kSecond);
-    fetch(min(blk + 2, n_blocks - 1) * kCB, in);
-    __syncthreads();
-    fix_tail(in, (blk + 2) * kCB);
-    multiply((blk + 1) * kCB, stage[1], kSecond);
-    prepare(in, stage[0], kFirst);
-    fetch(min(blk + 3, n_blocks - 1) * kCB, in);
-  }
-  if (blk < n_blocks) {
-    __syncthreads();
-    multiply(blk * kCB, stage[0], kFirst);
-    float worst = 0.f;  // (a last block without a partner: its own total is the exponent range it used)
-#pragma unroll
-    for (int rt = 0; rt < 8; ++rt) {
-      const float4 dc = *reinterpret_cast<const float4 *>(&stage[0].dec[32 * (rt >> 1) + 8 * g + 4 * (rt & 1)]);
-      if constexpr (kCheck) worst = fminf(worst, fminf(fminf(dc.x, dc.y), fminf(dc.z, dc.w)));
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt) {
-        S[rt][nt][0] *= fast_exp2(dc.x); S[rt][nt][1] *= fast_exp2(dc.y);
-        S[rt][nt][2] *= fast_exp2(dc.z); S[rt][nt][3] *= fast_exp2(dc.w);
-      }
-    }
-    if constexpr (kCheck)
-      if (__builtin_amdgcn_ballot_w64(worst < -kMaxExp * kLog2e) != 0 && tid == 0) atomicAdd(p.range_hits, 1u);
+    scan_gates<GDT>(gates, me, w, carry, b0, b1);
+    fetch_gates(min(n + 2, last));
+    outputs(n, now);
+    __syncthreads();   // the first half's gate sums are there, and every wavefront has read this block's q
+    prepare(stage[(n & 1) ^ 1], n < last);
+    fetch(min(n + 2, last));
+    update_state(S, now, g, c, vb);
   }
 
   if (kSeg ? (!last_segment || hh % p.jn != 0) : !p.write_state) return;
-#pragma unroll
-  for (int rt = 0; rt < 8; ++rt)
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int idx = state_index(rt, nt, i);
-        if (kStateF32) reinterpret_cast<float *>(sbase)[idx] = S[rt][nt][i];
-        else reinterpret_cast<uint16_t *>(sbase)[idx] = f32_to_bf16(S[rt][nt][i]);
-      }
+  store_state<kStateF32>(S, sbase, g, c, w);
 }
-
 
 // ---- prompts cut into segments -----------------------------------------------------------------------------------
 // Few chains (one prompt: 28 of them) leave most CUs idle, so long prompts are cut: the segments' own contributions
 // to the state (from a zero start) and total decays are formed side by side (gla_segment_state_kernel), a scan over
 // the segments turns them into the state each one starts from (gla_segment_scan_kernel), and gla_chunk_kernel<kSeg>
-// then runs all segments at once. Segments are whole pairs of blocks, so the operands of a pair are those of the
-// uncut prompt. k, v and the gate are read twice; what is bought is n_seg times as many workgroups.
+// then runs all segments at once. Segments are whole blocks, so the operands of a block are those of the uncut prompt. k, v and the gate are read twice; what is bought is n_seg times as many workgroups.
 
 // One workgroup per (row, state head, segment but the last): S_loc = sum over the segment's tokens of
-// (k_s exp(B_end - B_s))^T v_s, with the operand arithmetic, the tiles and the pairing of gla_chunk_kernel but
-// without its outputs (16 matrix instructions per wavefront and block instead of 30, no q).
-struct StateStage {
-  uint16_t ks[kCB][kRow];
-  uint16_t kl[kCB][kRow];
-  uint16_t vs[kCB][kRow];
-  float dec[128];
-};
+// (k_s exp(B_end - B_s))^T v_s, with the operand arithmetic and the tiles of gla_chunk_kernel but
+// without its outputs (32 matrix instructions per wavefront and block instead of 66, no q).
 
 template <int GDT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gla_segment_state_kernel(const GlaChunkParams p) {
@@ -465,130 +580,88 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int g = lane >> 4, c = lane & 15;
-  const int r = tid >> 4;
+  const Share me(w, lane);
 
-  __shared__ __attribute__((aligned(16))) StateStage stage[2];
+  __shared__ __attribute__((aligned(16))) KvStage stage[2];
+  __shared__ __attribute__((aligned(16))) Carry carry;
 
-  f32x4_t S[8][2];
+  StateTiles S;
 #pragma unroll
   for (int rt = 0; rt < 8; ++rt)
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) S[rt][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  constexpr int kGateBytes = GDT == SB_F32 ? 4 : 2;
-  const char *gb = reinterpret_cast<const char *>(p.g) + go * kGateBytes;
+  constexpr int GB = kGateBytes<GDT>;
+  const char *gb = reinterpret_cast<const char *>(p.g) + go * GB;
   const char *kb = reinterpret_cast<const char *>(p.k + ko), *vb_ = reinterpret_cast<const char *>(p.v + vo);
-  const int64_t g_row = p.g_st * kGateBytes, k_row = p.k_st * 2, v_row = p.v_st * 2;
-  struct BlockIn {
-    uint4 k, v;
-    uint4 g[kGateBytes / 2];
+  const int64_t g_row = p.g_st * GB, k_row = p.k_st * 2, v_row = p.v_st * 2;
+  const RowOffsets k_at(me, 16, k_row), v_at(me, 16, v_row), g_at(me, 8 * GB, g_row);   // (every block of such a segment is whole)
+  const int last = p.seg_tokens / kCB - 1;
+  GateIn<GDT> gates;
+  KvIn kv;
+  auto fetch_gates = [&](int n) {
+    const __amdgpu_buffer_rsrc_t gr = rows_from(gb + n * kCB * g_row);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int j = 0; j < GB / 2; ++j) gates.g[u][j] = load16(gr, g_at.at[u] + 16 * j);
   };
-  auto fetch = [&](int t0, BlockIn &in) {   // (every block of such a segment is whole)
-    in.k = load16(rows_from(kb + t0 * k_row), c * (int)k_row + r * 16);
-    in.v = load16(rows_from(vb_ + t0 * v_row), c * (int)v_row + r * 16);
-    const __amdgpu_buffer_rsrc_t gr = rows_from(gb + t0 * g_row);
+  auto fetch = [&](int n) {
+    const __amdgpu_buffer_rsrc_t kr = rows_from(kb + n * kCB * k_row), vr = rows_from(vb_ + n * kCB * v_row);
 #pragma unroll
-    for (int j = 0; j < kGateBytes / 2; ++j) in.g[j] = load16(gr, c * (int)g_row + r * 8 * kGateBytes + 16 * j);
-  };
-  float carry[8], total[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) carry[i] = total[i] = 0.f;
-  auto prepare = [&](const BlockIn &in, StateStage &st, auto second_tag) {
-    constexpr bool kSecond = decltype(second_tag)::value;
-    float B[8], tot[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      float x;
-      if constexpr (GDT == SB_F32) x = __uint_as_float(word(in.g[i >> 2], i & 3));
-      else if constexpr (GDT == SB_BF16) x = (i & 1) ? bf16_hi(word(in.g[0], i >> 1)) : bf16_lo(word(in.g[0], i >> 1));
-      else x = (i & 1) ? f16_hi(word(in.g[0], i >> 1)) : f16_lo(word(in.g[0], i >> 1));
-      x *= kLog2e;
-      x += row_shr<1>(x);
-      x += row_shr<2>(x);
-      x += row_shr<4>(x);
-      x += row_shr<8>(x);
-      if constexpr (kSecond) x += carry[i];
-      B[i] = x;
-      tot[i] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane | 15) << 2, __builtin_bit_cast(int, x)));
-    }
-    float kf[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      kf[2 * i] = bf16_lo(word(in.k, i));
-      kf[2 * i + 1] = bf16_hi(word(in.k, i));
-    }
-    uint32_t ks[4], kl[4];
-#pragma unroll
-    for (int i = 0; i < 8; i += 2) {
-      const float x0 = kf[i] * fast_exp2(fminf(-B[i], kMaxExp * kLog2e)), x1 = kf[i + 1] * fast_exp2(fminf(-B[i + 1], kMaxExp * kLog2e));
-      const uint32_t h = Mma<BF16>::pack(x0, x1);
-      ks[i / 2] = h;
-      kl[i / 2] = Mma<BF16>::pack(x0 - __uint_as_float(h << 16), x1 - __uint_as_float(h & 0xffff0000u));
-    }
-    *reinterpret_cast<uint4 *>(&st.ks[c][8 * r]) = make_uint4(ks[0], ks[1], ks[2], ks[3]);
-    *reinterpret_cast<uint4 *>(&st.kl[c][8 * r]) = make_uint4(kl[0], kl[1], kl[2], kl[3]);
-    *reinterpret_cast<uint4 *>(&st.vs[c][8 * r]) = in.v;
-    if constexpr (kSecond) {
-      *reinterpret_cast<float4 *>(&st.dec[8 * r]) = make_float4(fast_exp2(tot[0]), fast_exp2(tot[1]), fast_exp2(tot[2]), fast_exp2(tot[3]));
-      *reinterpret_cast<float4 *>(&st.dec[8 * r + 4]) = make_float4(fast_exp2(tot[4]), fast_exp2(tot[5]), fast_exp2(tot[6]), fast_exp2(tot[7]));
-#pragma unroll
-      for (int i = 0; i < 8; ++i) total[i] += tot[i];
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) carry[i] = tot[i];
+    for (int u = 0; u < 2; ++u) {
+      kv.k[u] = load16(kr, k_at.at[u]);
+      kv.v[u] = load16(vr, v_at.at[u]);
     }
   };
-  auto multiply = [&](const StateStage &st, auto second_tag) {
-    constexpr bool kSecond = decltype(second_tag)::value;
-    uint4 vb[2];
+  float b0[8], b1[8], total[8];   // total: of the segment, in the lanes that hold the last token of a block
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      const uint2 x = load_transposed(&st.vs[4 * g + (c >> 2)][32 * w + 16 * nt + 4 * (c & 3)]);
-      vb[nt] = make_uint4(x.x, x.y, x.x, x.y);
-    }
+  for (int i = 0; i < 8; ++i) total[i] = 0.f;
+  auto prepare = [&](KvStage &st) {
+    add_carry(carry, me, w, b0, b1);
+    store_kv(st, me, kv, b0, b1);
 #pragma unroll
-    for (int rt = 0; rt < 8; ++rt) {
-      const int tok = 4 * g + (c >> 2), dims = 32 * (rt >> 1) + 8 * (c & 3) + 4 * (rt & 1);
-      const uint2 h2 = load_transposed(&st.ks[tok][dims]);
-      const uint2 l2 = load_transposed(&st.kl[tok][dims]);
-      const uint4 ka = make_uint4(h2.x, h2.y, l2.x, l2.y);
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt) S[rt][nt] = Mma<BF16>::run(ka, vb[nt], S[rt][nt]);
-      if constexpr (kSecond) {
-        const float4 dc = *reinterpret_cast<const float4 *>(&st.dec[32 * (rt >> 1) + 8 * g + 4 * (rt & 1)]);
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt) {
-          S[rt][nt][0] *= dc.x; S[rt][nt][1] *= dc.y; S[rt][nt][2] *= dc.z; S[rt][nt][3] *= dc.w;
-        }
-      }
-    }
+    for (int i = 0; i < 8; ++i) { total[i] += b1[i]; b1[i] = fast_exp2(b1[i]); }
+    store_decay(st, carry, me, w, b1);
   };
 
-  const int n_blocks = p.seg_tokens / kCB;   // a whole number of pairs
-  const std::false_type kFirst{};
-  const std::true_type kSecond{};
-  BlockIn in;
-  fetch(0, in);
-  prepare(in, stage[0], kFirst);
-  fetch(kCB, in);
-  for (int blk = 0; blk < n_blocks; blk += 2) {
+  if (tid < 128) carry.zero[tid] = 0.f;
+  fetch_gates(0);
+  fetch(0);
+  scan_gates<GDT>(gates, me, w, carry, b0, b1);
+  fetch_gates(min(1, last));
+  __syncthreads();
+  prepare(stage[0]);
+  fetch(min(1, last));
+  int n = 0;
+  uint4 vb[2];
+  auto v_operands = [&](const KvStage &st, int g, int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) vb[nt] = column_operand(st.vs, g, c, w, nt);
+  };
+  for (; n < last; ++n) {
+    const KvStage &now = stage[n & 1];
     __syncthreads();
-    multiply(stage[0], kFirst);
-    prepare(in, stage[1], kSecond);
-    fetch(min(blk + 2, n_blocks - 1) * kCB, in);
+    scan_gates<GDT>(gates, me, w, carry, b0, b1);
+    fetch_gates(min(n + 2, last));
+    v_operands(now, g, c);
     __syncthreads();
-    multiply(stage[1], kSecond);
-    prepare(in, stage[0], kFirst);
-    fetch(min(blk + 3, n_blocks - 1) * kCB, in);
+    prepare(stage[(n & 1) ^ 1]);
+    fetch(min(n + 2, last));
+    update_state(S, now, g, c, vb);
   }
+  __syncthreads();
+  const TileLane end(lane);
+  v_operands(stage[n & 1], end.g, end.c);
+  update_state(S, stage[n & 1], end.g, end.c, vb);
   const int64_t at = ((int64_t)b * Hk + hk) * p.n_seg + seg;
   f32x4_t *dst = reinterpret_cast<f32x4_t *>(p.ws + at * 16384) + tid;
 #pragma unroll
   for (int rt = 0; rt < 8; ++rt)
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) dst[(2 * rt + nt) * 256] = S[rt][nt];
-  if (c == 0) {   // every lane of the row holds the totals of its 8 dims
-    float4 *d = reinterpret_cast<float4 *>(p.ws + (int64_t)gridDim.x * p.n_seg * 16384 + at * 128 + 8 * r);
+  if (w >= 2 && me.last_pair) {
+    float4 *d = reinterpret_cast<float4 *>(p.ws + (int64_t)gridDim.x * p.n_seg * 16384 + at * 128 + 8 * me.piece);
     d[0] = make_float4(total[0], total[1], total[2], total[3]);
     d[1] = make_float4(total[4], total[5], total[6], total[7]);
   }
@@ -613,7 +686,7 @@ __global__ __launch_bounds__(256) void gla_segment_scan_kernel(const GlaChunkPar
   f32x4_t S;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int idx = (row + i) * 128 + 32 * w + 16 * nt + c;
+    const int idx = (row + i) * 128 + 32 * w + 8 * (c >> 2) + 4 * nt + (c & 3);
     S[i] = kStateF32 ? reinterpret_cast<const float *>(sbase)[idx] : bf16_to_f32(reinterpret_cast<const uint16_t *>(sbase)[idx]);
   }
   const int64_t at0 = (int64_t)blockIdx.x * p.n_seg;
@@ -647,11 +720,9 @@ __global__ __launch_bounds__(256) void gla_segment_scan_kernel(const GlaChunkPar
 constexpr int kMaxGroup = 8;
 
 struct GroupStage {
-  uint16_t qs[kMaxGroup][kCB][kRow];
-  uint16_t ks[kCB][kRow];
-  uint16_t kl[kCB][kRow];
-  uint16_t vs[kCB][kRow];
-  float dec[128];
+  KvStage kv[2];
+  Operand qs[kMaxGroup];
+  Carry carry;
 };
 
 template <bool kStateF32, int GDT, bool kSeg>
@@ -686,16 +757,96 @@ __global__ __launch_bounds__(256) void gla_chunk_group_kernel(const GlaChunkPara
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int g = lane >> 4, c = lane & 15;
-  const int r = tid >> 4;
+  const Share me(w, lane);
 
   extern __shared__ __attribute__((aligned(16))) char group_smem[];
-  GroupStage *const stage = reinterpret_cast<GroupStage *>(group_smem);
+  GroupStage &stage = *reinterpret_cast<GroupStage *>(group_smem);
 
   char *sbase = reinterpret_cast<char *>(p.state) + (slot * p.s_slot + (int64_t)hk * p.s_head) * (kStateF32 ? 4 : 2);
-  f32x4_t S[8][2];
-  auto state_index = [&](int rt, int nt, int i) {
-    return (32 * (rt >> 1) + 8 * g + 4 * (rt & 1) + i) * 128 + 32 * w + 16 * nt + c;
+  StateTiles S;
+  constexpr int GB = kGateBytes<GDT>;
+  const char *gb = reinterpret_cast<const char *>(p.g) + go * GB;
+  const char *qb = reinterpret_cast<const char *>(p.q + qo), *kb = reinterpret_cast<const char *>(p.k + ko),
+             *vb_ = reinterpret_cast<const char *>(p.v + vo);
+  const int64_t g_row = p.g_st * GB, q_row = p.q_st * 2, k_row = p.k_st * 2, v_row = p.v_st * 2, o_row = p.o_st * 2;
+  const int64_t q_head = p.q_sh * 2, o_head = p.o_sh * 2;  // bytes between the group's heads
+  RowOffsets q_at(me, 16, q_row), k_at(me, 16, k_row), v_at(me, 16, v_row), g_at(me, 8 * GB, g_row);
+  const int last = (T - 1) / kCB;   // (only this block can have rows past the end, and it is fetched last)
+  GateIn<GDT> gates;
+  KvIn kv;
+  uint4 q[kMaxGroup][2];
+  auto fetch_gates = [&](int n) {
+    if ((n + 1) * kCB > T) g_at.cut(me, T - n * kCB);
+    const __amdgpu_buffer_rsrc_t gr = rows_from(gb + n * kCB * g_row);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int j = 0; j < GB / 2; ++j) gates.g[u][j] = load16(gr, g_at.at[u] + 16 * j);
   };
+  auto fetch = [&](int n) {
+    if ((n + 1) * kCB > T) { q_at.cut(me, T - n * kCB); k_at.cut(me, T - n * kCB); v_at.cut(me, T - n * kCB); }
+    const __amdgpu_buffer_rsrc_t kr = rows_from(kb + n * kCB * k_row), vr = rows_from(vb_ + n * kCB * v_row);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      kv.k[u] = load16(kr, k_at.at[u]);
+      kv.v[u] = load16(vr, v_at.at[u]);
+    }
+#pragma unroll
+    for (int h = 0; h < kMaxGroup; ++h)
+      if (h < G) {
+        const __amdgpu_buffer_rsrc_t qr = rows_from(qb + n * kCB * q_row + h * q_head);
+        q[h][0] = load16(qr, q_at.at[0]);
+        q[h][1] = load16(qr, q_at.at[1]);
+      }
+  };
+  float b0[8], b1[8];   // gate sums of the thread's two tokens
+  auto prepare = [&](KvStage &st) {
+    add_carry(stage.carry, me, w, b0, b1);
+    store_kv(st, me, kv, b0, b1);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) { b0[i] = fast_exp2(b0[i]); b1[i] = fast_exp2(b1[i]); }
+#pragma unroll
+    for (int h = 0; h < kMaxGroup; ++h)
+      if (h < G) store_q(stage.qs[h], me, q[h], b0, b1, p.scale);
+    store_decay(st, stage.carry, me, w, b1);
+  };
+
+  uint4 vb[2];
+  auto outputs = [&](int n, const KvStage &st, int g, int c) __attribute__((always_inline)) {
+    // what every head of the group shares: k-hat as the score operand, v, and the state before the block as
+    // the operand of q S_0
+    uint4 ka[2][4], sb16[4][2];
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) vb[nt] = column_operand(st.vs, g, c, w, nt);
+#pragma unroll
+    for (int s4 = 0; s4 < 4; ++s4)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) { ka[u][s4] = row_operand(st.ks, u, g, c, s4); sb16[s4][u] = state_operand(S, s4, u); }
+    for (int h = 0; h < G; ++h) {
+      uint4 qa[2][4];
+#pragma unroll
+      for (int s4 = 0; s4 < 4; ++s4)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) qa[u][s4] = row_operand(stage.qs[h], u, g, c, s4);
+      f32x4_t o[2][2];
+      output_scores(ka, qa, vb, g, c, o);
+#pragma unroll
+      for (int s4 = 0; s4 < 4; ++s4)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) o[u][nt] = Mma<BF16>::run(sb16[s4][nt], qa[u][s4], o[u][nt]);
+      // (a descriptor per head: its bound drops the rows past the end of the prompt, whatever the head stride)
+      const __amdgpu_buffer_rsrc_t orows = __builtin_amdgcn_make_buffer_rsrc(
+          reinterpret_cast<char *>(p.out + oo) + n * kCB * o_row + h * o_head, 0, min(kCB, T - n * kCB) * (int)o_row, 0x00020000);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) store_out(orows, (16 * u + c) * (int)o_row + (32 * w + 8 * g) * 2, o[u][0], o[u][1]);
+    }
+  };
+
+  if (tid < 128) stage.carry.zero[tid] = 0.f;
+  fetch_gates(0);
+  fetch(0);
   if constexpr (kSeg) {
     const f32x4_t *src = reinterpret_cast<const f32x4_t *>(p.ws + ((int64_t)blockIdx.x * p.n_seg + seg) * 16384) + tid;
 #pragma unroll
@@ -703,256 +854,38 @@ __global__ __launch_bounds__(256) void gla_chunk_group_kernel(const GlaChunkPara
 #pragma unroll
       for (int nt = 0; nt < 2; ++nt) S[rt][nt] = src[(2 * rt + nt) * 256];
   } else {
-#pragma unroll
-    for (int rt = 0; rt < 8; ++rt)
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int idx = state_index(rt, nt, i);
-          S[rt][nt][i] = kStateF32 ? reinterpret_cast<const float *>(sbase)[idx]
-                                   : bf16_to_f32(reinterpret_cast<const uint16_t *>(sbase)[idx]);
-        }
+    load_state<kStateF32>(S, sbase, g, c, w);
   }
-
-  constexpr int kGateBytes = GDT == SB_F32 ? 4 : 2;
-  const char *gb = reinterpret_cast<const char *>(p.g) + go * kGateBytes;
-  const char *qb = reinterpret_cast<const char *>(p.q + qo), *kb = reinterpret_cast<const char *>(p.k + ko),
-             *vb_ = reinterpret_cast<const char *>(p.v + vo);
-  const int64_t g_row = p.g_st * kGateBytes, q_row = p.q_st * 2, k_row = p.k_st * 2, v_row = p.v_st * 2, o_row = p.o_st * 2;
-  const int q_head = (int)(p.q_sh * 2), o_head = (int)(p.o_sh * 2);  // bytes between the group's heads (host-checked to fit)
-  struct BlockIn {
-    uint4 q[kMaxGroup], k, v;
-    uint4 g[kGateBytes / 2];
-  };
-  auto fetch = [&](int t0, BlockIn &in) {
-    const int tok = min(c, T - 1 - t0);
-    const __amdgpu_buffer_rsrc_t qr = rows_from(qb + t0 * q_row);
-#pragma unroll
-    for (int h = 0; h < kMaxGroup; ++h)
-      if (h < G) in.q[h] = load16(qr, tok * (int)q_row + h * q_head + r * 16);
-    in.k = load16(rows_from(kb + t0 * k_row), tok * (int)k_row + r * 16);
-    in.v = load16(rows_from(vb_ + t0 * v_row), tok * (int)v_row + r * 16);
-    const __amdgpu_buffer_rsrc_t gr = rows_from(gb + t0 * g_row);
-#pragma unroll
-    for (int j = 0; j < kGateBytes / 2; ++j) in.g[j] = load16(gr, tok * (int)g_row + r * 8 * kGateBytes + 16 * j);
-  };
-  auto fix_tail = [&](BlockIn &in, int t0) {
-    if (t0 + kCB > T && t0 + c >= T) {
-#pragma unroll
-      for (int h = 0; h < kMaxGroup; ++h) in.q[h] = make_uint4(0u, 0u, 0u, 0u);
-      in.k = in.v = make_uint4(0u, 0u, 0u, 0u);
-#pragma unroll
-      for (int j = 0; j < kGateBytes / 2; ++j) in.g[j] = make_uint4(0u, 0u, 0u, 0u);
-    }
-  };
-  float carry[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) carry[i] = 0.f;
-  auto prepare = [&](const BlockIn &in, GroupStage &st, auto second_tag) {
-    constexpr bool kSecond = decltype(second_tag)::value;
-    const uint4 rk = in.k, rv = in.v;
-    float B[8], tot[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      float x;
-      if constexpr (GDT == SB_F32) x = __uint_as_float(word(in.g[i >> 2], i & 3));
-      else if constexpr (GDT == SB_BF16) x = (i & 1) ? bf16_hi(word(in.g[0], i >> 1)) : bf16_lo(word(in.g[0], i >> 1));
-      else x = (i & 1) ? f16_hi(word(in.g[0], i >> 1)) : f16_lo(word(in.g[0], i >> 1));
-      x *= kLog2e;
-      x += row_shr<1>(x);
-      x += row_shr<2>(x);
-      x += row_shr<4>(x);
-      x += row_shr<8>(x);
-      if constexpr (kSecond) x += carry[i];
-      B[i] = x;
-      tot[i] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane | 15) << 2, __builtin_bit_cast(int, x)));
-    }
-    float eq[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) eq[i] = fast_exp2(B[i]);
-#pragma unroll
-    for (int h = 0; h < kMaxGroup; ++h)
-      if (h < G) {
-        const uint4 rq = in.q[h];
-        uint32_t qs[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          qs[i] = Mma<BF16>::pack(bf16_lo(word(rq, i)) * p.scale * eq[2 * i], bf16_hi(word(rq, i)) * p.scale * eq[2 * i + 1]);
-        *reinterpret_cast<uint4 *>(&st.qs[h][c][8 * r]) = make_uint4(qs[0], qs[1], qs[2], qs[3]);
-      }
-    float kf[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      kf[2 * i] = bf16_lo(word(rk, i));
-      kf[2 * i + 1] = bf16_hi(word(rk, i));
-    }
-    uint32_t ks[4], kl[4];
-#pragma unroll
-    for (int i = 0; i < 8; i += 2) {
-      const float x0 = kf[i] * fast_exp2(fminf(-B[i], kMaxExp * kLog2e)), x1 = kf[i + 1] * fast_exp2(fminf(-B[i + 1], kMaxExp * kLog2e));
-      const uint32_t h = Mma<BF16>::pack(x0, x1);
-      const uint32_t l = Mma<BF16>::pack(x0 - __uint_as_float(h << 16), x1 - __uint_as_float(h & 0xffff0000u));
-      ks[i / 2] = h;
-      kl[i / 2] = l;
-    }
-    *reinterpret_cast<uint4 *>(&st.ks[c][8 * r]) = make_uint4(ks[0], ks[1], ks[2], ks[3]);
-    *reinterpret_cast<uint4 *>(&st.kl[c][8 * r]) = make_uint4(kl[0], kl[1], kl[2], kl[3]);
-    *reinterpret_cast<uint4 *>(&st.vs[c][8 * r]) = rv;
-    if constexpr (kSecond) {
-      *reinterpret_cast<float4 *>(&st.dec[8 * r]) = make_float4(fast_exp2(tot[0]), fast_exp2(tot[1]), fast_exp2(tot[2]), fast_exp2(tot[3]));
-      *reinterpret_cast<float4 *>(&st.dec[8 * r + 4]) = make_float4(fast_exp2(tot[4]), fast_exp2(tot[5]), fast_exp2(tot[6]), fast_exp2(tot[7]));
-    } else {
-      *reinterpret_cast<float4 *>(&st.dec[8 * r]) = make_float4(tot[0], tot[1], tot[2], tot[3]);
-      *reinterpret_cast<float4 *>(&st.dec[8 * r + 4]) = make_float4(tot[4], tot[5], tot[6], tot[7]);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) carry[i] = tot[i];
-    }
-  };
-
-  auto multiply = [&](int t0, const GroupStage &st, auto second_tag) {
-    constexpr bool kSecond = decltype(second_tag)::value;
-    // what every head of the group shares: k-hat as the score operand, v, and the state before the block as
-    // the operand of q S_0
-    uint4 ka[4];
-#pragma unroll
-    for (int s4 = 0; s4 < 4; ++s4) ka[s4] = *reinterpret_cast<const uint4 *>(&st.ks[c][32 * s4 + 8 * g]);
-    uint4 vb[2];
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      const uint2 x = load_transposed(&st.vs[4 * g + (c >> 2)][32 * w + 16 * nt + 4 * (c & 3)]);
-      vb[nt] = make_uint4(x.x, x.y, x.x, x.y);
-    }
-    uint4 sb16[4][2];
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-      for (int s4 = 0; s4 < 4; ++s4) {
-        const f32x4_t &a = S[2 * s4][nt], &bb = S[2 * s4 + 1][nt];
-        sb16[s4][nt] = make_uint4(Mma<BF16>::pack(a[0], a[1]), Mma<BF16>::pack(a[2], a[3]),
-                                  Mma<BF16>::pack(bb[0], bb[1]), Mma<BF16>::pack(bb[2], bb[3]));
-      }
-    // NP heads at a time, their chains of dependent matrix instructions taken in turn (a head alone is one
-    // chain: four instructions for its scores, then five per output tile)
-    auto heads = [&](int h0, auto np_tag) __attribute__((always_inline)) {
-      constexpr int NP = decltype(np_tag)::value;
-      uint4 qa[NP][4];
-      f32x4_t at[NP];
-#pragma unroll
-      for (int u = 0; u < NP; ++u) at[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int s4 = 0; s4 < 4; ++s4)
-#pragma unroll
-        for (int u = 0; u < NP; ++u) {
-          qa[u][s4] = *reinterpret_cast<const uint4 *>(&st.qs[h0 + u][c][32 * s4 + 8 * g]);
-          at[u] = Mma<BF16>::run(ka[s4], qa[u][s4], at[u]);
-        }
-      uint4 pa[NP];
-#pragma unroll
-      for (int u = 0; u < NP; ++u) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (4 * g + i > c) at[u][i] = 0.f;
-        const uint32_t h01 = Mma<BF16>::pack(at[u][0], at[u][1]), h23 = Mma<BF16>::pack(at[u][2], at[u][3]);
-        pa[u] = make_uint4(h01, h23,
-                           Mma<BF16>::pack(at[u][0] - __uint_as_float(h01 << 16), at[u][1] - __uint_as_float(h01 & 0xffff0000u)),
-                           Mma<BF16>::pack(at[u][2] - __uint_as_float(h23 << 16), at[u][3] - __uint_as_float(h23 & 0xffff0000u)));
-      }
-      f32x4_t o[NP][2];
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-        for (int u = 0; u < NP; ++u) o[u][nt] = Mma<BF16>::run(vb[nt], pa[u], f32x4_t{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-      for (int s4 = 0; s4 < 4; ++s4)
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-          for (int u = 0; u < NP; ++u) o[u][nt] = Mma<BF16>::run(sb16[s4][nt], qa[u][s4], o[u][nt]);
-#pragma unroll
-      for (int u = 0; u < NP; ++u) {
-        // (a descriptor per head: its bound drops the rows past the end of the prompt, whatever the head stride)
-        const __amdgpu_buffer_rsrc_t orows = __builtin_amdgcn_make_buffer_rsrc(
-            reinterpret_cast<char *>(p.out + oo) + t0 * o_row + (int64_t)(h0 + u) * o_head, 0, min(kCB, T - t0) * (int)o_row,
-            0x00020000);
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt) {
-          typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
-          u32x2_t val;
-          val.x = Mma<BF16>::pack(o[u][nt][0], o[u][nt][1]);
-          val.y = Mma<BF16>::pack(o[u][nt][2], o[u][nt][3]);
-          __builtin_amdgcn_raw_buffer_store_b64(val, orows, c * (int)o_row + (32 * w + 16 * nt + 4 * g) * 2, 0, 0);
-        }
-      }
-    };
-    {
-      int h = 0;
-      for (; h + 2 <= G; h += 2) heads(h, std::integral_constant<int, 2>{});
-      if (h < G) heads(h, std::integral_constant<int, 1>{});
-    }
-#pragma unroll
-    for (int rt = 0; rt < 8; ++rt) {
-      const int tok = 4 * g + (c >> 2), dims = 32 * (rt >> 1) + 8 * (c & 3) + 4 * (rt & 1);
-      const uint2 h2 = load_transposed(&st.ks[tok][dims]);
-      const uint2 l2 = load_transposed(&st.kl[tok][dims]);
-      const uint4 kt = make_uint4(h2.x, h2.y, l2.x, l2.y);
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt) S[rt][nt] = Mma<BF16>::run(kt, vb[nt], S[rt][nt]);
-      if constexpr (kSecond) {
-        const float4 dc = *reinterpret_cast<const float4 *>(&st.dec[32 * (rt >> 1) + 8 * g + 4 * (rt & 1)]);
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt) {
-          S[rt][nt][0] *= dc.x; S[rt][nt][1] *= dc.y; S[rt][nt][2] *= dc.z; S[rt][nt][3] *= dc.w;
-        }
-      }
-    }
-  };
-
-  const int n_blocks = (T + kCB - 1) / kCB;
-  const std::false_type kFirst{};
-  const std::true_type kSecond{};
-  BlockIn in;
-  fetch(0, in);
-  fix_tail(in, 0);
-  prepare(in, stage[0], kFirst);
-  fetch(min(1, n_blocks - 1) * kCB, in);
-  int blk = 0;
-  for (; blk + 1 < n_blocks; blk += 2) {
+  scan_gates<GDT>(gates, me, w, stage.carry, b0, b1);
+  fetch_gates(min(1, last));
+  __syncthreads();
+  prepare(stage.kv[0]);
+  fetch(min(1, last));
+  auto finish = [&](int n) __attribute__((always_inline)) {
+    const TileLane end(lane);
     __syncthreads();
-    fix_tail(in, (blk + 1) * kCB);
-    multiply(blk * kCB, stage[0], kFirst);
-    prepare(in, stage[1], kSecond);
-    fetch(min(blk + 2, n_blocks - 1) * kCB, in);
-    __syncthreads();
-    fix_tail(in, (blk + 2) * kCB);
-    multiply((blk + 1) * kCB, stage[1], kSecond);
-    prepare(in, stage[0], kFirst);
-    fetch(min(blk + 3, n_blocks - 1) * kCB, in);
+    outputs(n, stage.kv[n & 1], end.g, end.c);
+    if (!last_segment) return;
+    update_state(S, stage.kv[n & 1], end.g, end.c, vb);
+    store_state<kStateF32>(S, sbase, end.g, end.c, w);
+  };
+  if (last == 0) {
+    finish(0);
+    return;
   }
-  if (blk < n_blocks) {
+  int n = 0;
+  do {
+    const KvStage &now = stage.kv[n & 1];
     __syncthreads();
-    multiply(blk * kCB, stage[0], kFirst);
-#pragma unroll
-    for (int rt = 0; rt < 8; ++rt) {
-      const float4 dc = *reinterpret_cast<const float4 *>(&stage[0].dec[32 * (rt >> 1) + 8 * g + 4 * (rt & 1)]);
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt) {
-        S[rt][nt][0] *= fast_exp2(dc.x); S[rt][nt][1] *= fast_exp2(dc.y);
-        S[rt][nt][2] *= fast_exp2(dc.z); S[rt][nt][3] *= fast_exp2(dc.w);
-      }
-    }
-  }
-  if (!last_segment) return;
-#pragma unroll
-  for (int rt = 0; rt < 8; ++rt)
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int idx = state_index(rt, nt, i);
-        if (kStateF32) reinterpret_cast<float *>(sbase)[idx] = S[rt][nt][i];
-        else reinterpret_cast<uint16_t *>(sbase)[idx] = f32_to_bf16(S[rt][nt][i]);
-      }
+    scan_gates<GDT>(gates, me, w, stage.carry, b0, b1);
+    fetch_gates(min(n + 2, last));
+    outputs(n, now, g, c);
+    __syncthreads();
+    prepare(stage.kv[(n & 1) ^ 1]);
+    fetch(min(n + 2, last));
+    update_state(S, now, g, c, vb);
+  } while (++n < last);
+  finish(n);
 }
 
 }  // namespace
@@ -1056,7 +989,7 @@ template <bool kSeg>
 static int launch_group_kernel(const sb_gla_recurrent_args *a, const GlaChunkParams &p, dim3 grid) {
   const dim3 block(256);
   hipStream_t st = (hipStream_t)a->stream;
-  constexpr int kLds = 2 * (int)sizeof(GroupStage);
+  constexpr int kLds = (int)sizeof(GroupStage);
 #define SB_LAUNCH(F32S, GDT)                                                                                     \
   do {                                                                                                           \
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gla_chunk_group_kernel<F32S, GDT, kSeg>), \
@@ -1077,7 +1010,7 @@ static int launch_group_kernel(const sb_gla_recurrent_args *a, const GlaChunkPar
   return SB_OK;
 }
 
-// Prompts cut into n_seg segments of seg_tokens tokens (a multiple of 2 blocks); ws: see GlaChunkParams. With shared
+// Prompts cut into n_seg segments of seg_tokens tokens (whole blocks); ws: see GlaChunkParams. With shared
 // states the segments fill the machine, so the one-pass kernel per group runs them (it does 0.4 x the work; per query
 // head where its strides do not fit, again in one launch: no head reads the state cache the last segments store into).
 int launch_gla_chunk_segments(const sb_gla_recurrent_args *a, int G, int n_seg, int seg_tokens, float *ws) {

@@ -549,10 +549,12 @@ static int check_args(const sb_gla_recurrent_args *a) {
 
 namespace {
 // Whether a call runs on the matrix cores in block form: bf16, 32 steps or more or packed, and q, k, v, g movable as
-// 16-byte pieces and out as 8-byte pieces.
+// 16-byte pieces with rows less than 64 MiB apart.
 bool block_form(const sb_gla_recurrent_args *a) {
+  // (the 32 rows of a block are addressed with 32-bit offsets)
   auto pieces = [](const void *ptr, int64_t per16, int64_t sb_, int64_t sh, int64_t st) {
-    return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0 && sb_ % per16 == 0 && sh % per16 == 0 && st % per16 == 0;
+    return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0 && sb_ % per16 == 0 && sh % per16 == 0 && st % per16 == 0 && st >= 0 &&
+           st / per16 < (1LL << 31) / (32 * 16);
   };
   return a->dtype == SB_BF16 && !(a->flags & SB_GLA_VECTOR_ONLY) && (a->cu_seqlens || a->seq_len >= kChunkKernelMinSteps) &&
          pieces(a->q, 8, a->q_stride_b, a->q_stride_h, a->q_stride_t) && pieces(a->k, 8, a->k_stride_b, a->k_stride_h, a->k_stride_t) &&
@@ -560,7 +562,7 @@ bool block_form(const sb_gla_recurrent_args *a) {
          pieces(a->g, a->g_dtype == SB_F32 ? 4 : 8, a->g_stride_b, a->g_stride_h, a->g_stride_t) &&
          pieces(a->out, 8, a->out_stride_b, a->out_stride_h, a->out_stride_t);
 }
-// Tokens per segment of a prompt cut into n segments: whole pairs of 16-token blocks.
+// Tokens per segment of a prompt cut into n segments: whole blocks of 32 tokens.
 int segment_tokens(int seq_len, int n) { return ((seq_len + n - 1) / n + 31) / 32 * 32; }
 }  // namespace
 

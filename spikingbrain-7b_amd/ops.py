@@ -816,9 +816,9 @@ def meta_token_attention(q: torch.Tensor, k2: torch.Tensor, v2: torch.Tensor, sc
 
 def gla_gate_range_hits(reset: bool = False) -> int:
     """How often the matrix-core GLA launches made with check_gates=True on the current device met gates beyond the block form's range (a
-    pair of 16-token blocks whose log-gates sum below -80 for some key dim: results there under-weight
+    block of 32 tokens whose log-gates sum below -80 for some key dim: results there under-weight
     near-diagonal terms; `vector_only=True` has no such limit) since the counter was last cleared: one count per
-    prompt, head, 32 key dims and pair of blocks concerned. Waits for the device."""
+    prompt, head, 32 key dims and block concerned. Waits for the device."""
     hits = C.c_int64(0)
     N.check(N.lib().sb_gla_gate_range_hits(C.byref(hits), 1 if reset else 0), "gla_gate_range_hits")
     return int(hits.value)
@@ -832,7 +832,7 @@ def gla_recurrent(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
     """q, k, v, g [B, H, T, D] (any batch/head/time strides, contiguous D); state
     [slots, H, D, D] fp32 or bf16, updated in place; returns o [B, H, T, D] in q's dtype.
     Rows with slot_idx == -1 are skipped (state and output untouched; zero_skipped=True, one step only: output zero).
-    Calls of 32 steps or more with bf16 q/k/v run 16 tokens at a time on the matrix cores (state, gates
+    Calls of 32 steps or more with bf16 q/k/v run 32 tokens at a time on the matrix cores (state, gates
     and accumulation in fp32, bf16 operand rounding on the output path); vector_only=True keeps them on
     the step-by-step fp32 kernel. check_gates=True: the block form counts gates beyond its range (see
     gla_gate_range_hits). per_head (shared states, block form): True = one workgroup per query head, False = one
