@@ -71,9 +71,11 @@ struct GlaChunkParams {
   int G, jn, j0, write_state;
   unsigned int *range_hits;  // device counter of (32 key dims, block) events whose gates reached the exponent clamp
   // Prompts cut into segments (0: not cut): seg_tokens tokens each, n_seg of them for the longest prompt. ws holds
-  // per (row, state head, segment) the state in register order, 16384 floats, and behind all of those the
-  // segments' total log-decays, 128 floats each (log2 units).
-  int seg_tokens, n_seg;
+  // per (row, state head) n_seg states in register order, 16384 floats each, and behind all of those (chains of them) the decays of
+  // the segments, 128 factors each. State 0 is the one the prompt starts from, state 1 the one behind its first segment, state i > 1
+  // what segment i - 1 adds; scanned: gla_segment_scan_kernel has turned them into the states that the segments start from.
+  int seg_tokens, n_seg, scanned;
+  int64_t chains;
   float *ws;
 };
 
@@ -385,9 +387,51 @@ __device__ __forceinline__ void store_out(__amdgpu_buffer_rsrc_t rows, uint32_t 
   __builtin_amdgcn_raw_buffer_store_b128(val, rows, off, 0, 0);
 }
 
+// The state that segment `seg` of a prompt starts from: that behind the first segment, decayed and added to by those in between, or
+// the one the scan left. A few additions are requested together. lds: room for kFoldMax segments' decays.
+// Up to this many segments each one adds up what the segments before it hand on; from there on a scan over them, a launch of its own, is
+// faster (us per call, added up / scanned: a workgroup per head, 2 x 2048 tokens in 9 72.1 / 77.8, 4 x 2048 in 4 120.5 / 127.7,
+// 1 x 1024 in 9 40.1 / 40.2 and in 16 47.9 / 46.7, 16 heads 1 x 1000 in 16 37.5 / 33.8; a workgroup per group, 16 x 200 in 4
+// 39.2 / 43.8, 4 x 200 in 6 31.6 / 32.2, 4 x 512 in 8 39.9 / 38.5).
+constexpr int kFoldMax = 9, kFoldMaxGroup = 6;
+__device__ __forceinline__ void segment_start(StateTiles &S, const GlaChunkParams &p, int64_t chain, int seg, int tid, int g, float *lds) {
+  const int first = p.scanned ? seg : min(seg, 1), steps = seg - first;
+  const f32x4_t *const entry = reinterpret_cast<const f32x4_t *>(p.ws + (chain * p.n_seg + first) * 16384) + tid;
+#pragma unroll
+  for (int rt = 0; rt < 8; ++rt)
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) S[rt][nt] = entry[(2 * rt + nt) * 256];
+  if (steps == 0) return;
+  const f32x4_t *const decay = reinterpret_cast<const f32x4_t *>(p.ws + ((p.chains * 128 + chain) * p.n_seg + 1) * 128);
+  for (int i = tid; i < steps * 32; i += 256) reinterpret_cast<f32x4_t *>(lds)[i] = decay[i];
+  __syncthreads();
+  constexpr int kAhead = 3;
+#pragma unroll
+  for (int half = 0; half < 2; ++half)
+    for (int i0 = 0; i0 < steps; i0 += kAhead) {
+      f32x4_t add[kAhead][4][2];
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j)
+#pragma unroll
+        for (int x = 0; x < 8; ++x) add[j][x >> 1][x & 1] = entry[(int64_t)(min(i0 + j, steps - 1) + 1) * 4096 + (8 * half + x) * 256];
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j)
+        if (i0 + j < steps)
+#pragma unroll
+          for (int r4 = 0; r4 < 4; ++r4) {
+            const int rt = 4 * half + r4;
+            const f32x4_t d = *reinterpret_cast<const f32x4_t *>(lds + (i0 + j) * 128 + 32 * (rt >> 1) + 8 * g + 4 * (rt & 1));
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) S[rt][nt][i] = fmaf(d[i], S[rt][nt][i], add[j][r4][nt][i]);
+          }
+    }
+}
+
 // kCheck: report gates beyond the block form's range (SB_GLA_CHECK_GATES); a build of its own, because even this
 // little extra work shifts the register allocation of a kernel that runs at the edge of its budget (0-4 % slower).
-// kSeg: the workgroup runs one segment of its prompt, from the state gla_segment_scan_kernel left in the workspace
+// kSeg: the workgroup runs one segment of its prompt, from the state that segment_start finds in the workspace
 // for it; the workgroup of a prompt's last segment stores the final state.
 template <bool kStateF32, int GDT, bool kCheck, bool kSeg>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gla_chunk_kernel(const GlaChunkParams p) {
@@ -509,20 +553,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   // ---- block loop. Loads are issued as soon as their registers are free: the gates of block n + 2 in the first stretch of
   // block n, its q, k and v in the second.
-  // (behind the first block's loads, which are waited for first)
-  if constexpr (kSeg) {
-    const int Hk = p.H / p.jn;
-    const f32x4_t *src = reinterpret_cast<const f32x4_t *>(p.ws + (((int64_t)b * Hk + hk) * p.n_seg + seg) * 16384) + tid;
-#pragma unroll
-    for (int rt = 0; rt < 8; ++rt)
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt) S[rt][nt] = src[(2 * rt + nt) * 256];
-  } else {
-    load_state<kStateF32>(S, sbase, g, c, w);
-  }
   if (tid < 128) carry.zero[tid] = 0.f;
   fetch_gates(0);
   fetch(0);
+  if constexpr (kSeg) segment_start(S, p, b * (int64_t)(p.H / p.jn) + hk, seg, tid, g, reinterpret_cast<float *>(&stage[1]));
+  else load_state<kStateF32>(S, sbase, g, c, w);   // (behind the first block's loads, which are waited for first)
   scan_gates<GDT>(gates, me, w, carry, b0, b1);
   fetch_gates(min(1, last));
   __syncthreads();
@@ -548,21 +583,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
 // ---- prompts cut into segments -----------------------------------------------------------------------------------
 // Few chains (one prompt: 28 of them) leave most CUs idle, so long prompts are cut: the segments' own contributions
-// to the state (from a zero start) and total decays are formed side by side (gla_segment_state_kernel), a scan over
-// the segments turns them into the state each one starts from (gla_segment_scan_kernel), and gla_chunk_kernel<kSeg>
-// then runs all segments at once. Segments are whole blocks, so the operands of a block are those of the uncut prompt. k, v and the gate are read twice; what is bought is n_seg times as many workgroups.
+// to the state (from a zero start) and total decays are formed side by side (gla_segment_state_kernel), and the prompt kernels
+// then run all segments at once, each from the state that the segments before it add up to (segment_start; with many segments
+// a scan, gla_segment_scan_kernel, adds up once for all). Segments are whole blocks, so the operands of a block are those of the
+// uncut prompt. k, v and the gate are read twice; what is bought is n_seg times as many workgroups.
 
 // One workgroup per (row, state head, segment but the last): S_loc = sum over the segment's tokens of
-// (k_s exp(B_end - B_s))^T v_s, with the operand arithmetic and the tiles of gla_chunk_kernel but
+// (k_s exp(B_end - B_s))^T v_s (the first one starts from the prompt's state instead of zero), with the operand arithmetic and the tiles of gla_chunk_kernel but
 // without its outputs (32 matrix instructions per wavefront and block instead of 66, no q).
 
-template <int GDT>
+template <bool kStateF32, int GDT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gla_segment_state_kernel(const GlaChunkParams p) {
   const int seg = blockIdx.y;
   const int Hk = p.H;   // state heads here
   const int b = blockIdx.x / Hk;
   const int hk = blockIdx.x - b * Hk;
-  if (p.slot_idx && p.slot_idx[b] < 0) return;
+  const int64_t slot = p.slot_idx ? (int64_t)p.slot_idx[b] : (int64_t)b;
+  if (slot < 0) return;
+  const int tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const int g = lane >> 4, c = lane & 15;
+  const int64_t chain = blockIdx.x;
+  StateTiles S;
+  auto hand_on = [&](int entry) __attribute__((always_inline)) {
+    f32x4_t *dst = reinterpret_cast<f32x4_t *>(p.ws + (chain * p.n_seg + entry) * 16384) + tid;
+#pragma unroll
+    for (int rt = 0; rt < 8; ++rt)
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) dst[(2 * rt + nt) * 256] = S[rt][nt];
+  };
   int T = p.T;
   int64_t ko, vo, go;
   if (p.cu) {
@@ -573,23 +623,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     ko = b * p.k_sb; vo = b * p.v_sb; go = b * p.g_sb;
   }
   const int64_t s0 = (int64_t)seg * p.seg_tokens;
-  if (T <= s0 + p.seg_tokens) return;   // a prompt's last segment hands nothing on
+  const char *const sbase = reinterpret_cast<const char *>(p.state) + (slot * p.s_slot + (int64_t)hk * p.s_head) * (kStateF32 ? 4 : 2);
+  if (T <= s0 + p.seg_tokens) {   // a prompt's last segment hands nothing on
+    if (seg == 0) {
+      load_state<kStateF32>(S, sbase, g, c, w);
+      hand_on(0);
+    }
+    return;
+  }
   ko += s0 * p.k_st + hk * p.k_sh; vo += s0 * p.v_st + hk * p.v_sh; go += s0 * p.g_st + hk * p.g_sh;
 
-  const int tid = threadIdx.x;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lane = tid & 63;
-  const int g = lane >> 4, c = lane & 15;
   const Share me(w, lane);
 
   __shared__ __attribute__((aligned(16))) KvStage stage[2];
   __shared__ __attribute__((aligned(16))) Carry carry;
-
-  StateTiles S;
-#pragma unroll
-  for (int rt = 0; rt < 8; ++rt)
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) S[rt][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   constexpr int GB = kGateBytes<GDT>;
   const char *gb = reinterpret_cast<const char *>(p.g) + go * GB;
@@ -628,10 +675,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if (tid < 128) carry.zero[tid] = 0.f;
   fetch_gates(0);
   fetch(0);
+  if (seg == 0) load_state<kStateF32>(S, sbase, g, c, w);
+  else
+#pragma unroll
+    for (int rt = 0; rt < 8; ++rt)
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) S[rt][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   scan_gates<GDT>(gates, me, w, carry, b0, b1);
   fetch_gates(min(1, last));
   __syncthreads();
   prepare(stage[0]);
+  // the prompt's state is also passed on as it is: the segments of the next launch read it while the last of them stores the final
+  // one into the cache
+  if (seg == 0) hand_on(0);
   fetch(min(1, last));
   int n = 0;
   uint4 vb[2];
@@ -654,59 +710,47 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const TileLane end(lane);
   v_operands(stage[n & 1], end.g, end.c);
   update_state(S, stage[n & 1], end.g, end.c, vb);
-  const int64_t at = ((int64_t)b * Hk + hk) * p.n_seg + seg;
-  f32x4_t *dst = reinterpret_cast<f32x4_t *>(p.ws + at * 16384) + tid;
-#pragma unroll
-  for (int rt = 0; rt < 8; ++rt)
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) dst[(2 * rt + nt) * 256] = S[rt][nt];
+  hand_on(seg + 1);
   if (w >= 2 && me.last_pair) {
-    float4 *d = reinterpret_cast<float4 *>(p.ws + (int64_t)gridDim.x * p.n_seg * 16384 + at * 128 + 8 * me.piece);
+    float4 *d = reinterpret_cast<float4 *>(p.ws + ((p.chains * 128 + chain) * p.n_seg + seg) * 128 + 8 * me.piece);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) total[i] = fast_exp2(total[i]);
     d[0] = make_float4(total[0], total[1], total[2], total[3]);
     d[1] = make_float4(total[4], total[5], total[6], total[7]);
   }
 }
 
 // Grid (rows x state heads, 16 accumulator tiles): thread tid of workgroup (., tile) owns the four state elements
-// that thread tid of the other two kernels holds in that tile. In place: S_loc of a segment becomes the state the
-// segment starts from. A few segments' contributions are requested together, ahead of the chain over them.
-template <bool kStateF32>
+// that thread tid of the other kernels holds in that tile. In place: what segment i - 1 adds becomes the state that segment i
+// starts from, with the operations of segment_start. A few segments' contributions are requested together, ahead of the
+// chain over them.
 __global__ __launch_bounds__(256) void gla_segment_scan_kernel(const GlaChunkParams p) {
-  const int Hk = p.H;
-  const int b = blockIdx.x / Hk;
-  const int hk = blockIdx.x - b * Hk;
-  const int64_t slot = p.slot_idx ? (int64_t)p.slot_idx[b] : (int64_t)b;
-  if (slot < 0) return;
+  const int b = blockIdx.x / p.H;
+  if (p.slot_idx && p.slot_idx[b] < 0) return;
   const int T = p.cu ? p.cu[b + 1] - p.cu[b] : p.T;
   const int n = min((T + p.seg_tokens - 1) / p.seg_tokens, p.n_seg);   // segments of this prompt
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, c = lane & 15;
-  const int rt = blockIdx.y >> 1, nt = blockIdx.y & 1;
-  const int row = 32 * (rt >> 1) + 8 * g + 4 * (rt & 1);
-  const char *sbase = reinterpret_cast<const char *>(p.state) + (slot * p.s_slot + (int64_t)hk * p.s_head) * (kStateF32 ? 4 : 2);
-  f32x4_t S;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int idx = (row + i) * 128 + 32 * w + 8 * (c >> 2) + 4 * nt + (c & 3);
-    S[i] = kStateF32 ? reinterpret_cast<const float *>(sbase)[idx] : bf16_to_f32(reinterpret_cast<const uint16_t *>(sbase)[idx]);
-  }
-  const int64_t at0 = (int64_t)blockIdx.x * p.n_seg;
-  f32x4_t *const ws = reinterpret_cast<f32x4_t *>(p.ws + at0 * 16384) + blockIdx.y * 256 + tid;
-  const float *const decay = p.ws + (int64_t)gridDim.x * p.n_seg * 16384 + at0 * 128 + row;
+  const int tid = threadIdx.x, g = (tid & 63) >> 4;
+  const int rt = blockIdx.y >> 1;
+  const int64_t chain = blockIdx.x;
+  f32x4_t *const ws = reinterpret_cast<f32x4_t *>(p.ws + chain * p.n_seg * 16384) + blockIdx.y * 256 + tid;
+  const float *const decay = p.ws + (p.chains * 128 + chain) * p.n_seg * 128 + 32 * (rt >> 1) + 8 * g + 4 * (rt & 1);
+  if (n < 3) return;
+  f32x4_t S = ws[4096];
   constexpr int kAhead = 4;
-  for (int s0 = 0; s0 < n; s0 += kAhead) {
-    f32x4_t loc[kAhead], d[kAhead];
+  for (int s0 = 2; s0 < n; s0 += kAhead) {
+    f32x4_t add[kAhead], d[kAhead];
 #pragma unroll
     for (int j = 0; j < kAhead; ++j) {
-      const int s = min(s0 + j, n - 1);   // (the last segment's entry is not used: it hands nothing on)
-      loc[j] = ws[(int64_t)s * 4096];
-      d[j] = *reinterpret_cast<const f32x4_t *>(decay + s * 128);
+      const int s = min(s0 + j, n - 1);
+      add[j] = ws[(int64_t)s * 4096];
+      d[j] = *reinterpret_cast<const f32x4_t *>(decay + (s - 1) * 128);
     }
 #pragma unroll
     for (int j = 0; j < kAhead; ++j)
       if (s0 + j < n) {
-        ws[(int64_t)(s0 + j) * 4096] = S;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) S[i] = fmaf(fast_exp2(d[j][i]), S[i], loc[j][i]);
+        for (int i = 0; i < 4; ++i) S[i] = fmaf(d[j][i], S[i], add[j][i]);
+        ws[(int64_t)(s0 + j) * 4096] = S;
       }
   }
 }
@@ -847,15 +891,8 @@ __global__ __launch_bounds__(256) void gla_chunk_group_kernel(const GlaChunkPara
   if (tid < 128) stage.carry.zero[tid] = 0.f;
   fetch_gates(0);
   fetch(0);
-  if constexpr (kSeg) {
-    const f32x4_t *src = reinterpret_cast<const f32x4_t *>(p.ws + ((int64_t)blockIdx.x * p.n_seg + seg) * 16384) + tid;
-#pragma unroll
-    for (int rt = 0; rt < 8; ++rt)
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt) S[rt][nt] = src[(2 * rt + nt) * 256];
-  } else {
-    load_state<kStateF32>(S, sbase, g, c, w);
-  }
+  if constexpr (kSeg) segment_start(S, p, blockIdx.x, seg, tid, g, reinterpret_cast<float *>(&stage.kv[1]));
+  else load_state<kStateF32>(S, sbase, g, c, w);
   scan_gates<GDT>(gates, me, w, stage.carry, b0, b1);
   fetch_gates(min(1, last));
   __syncthreads();
@@ -948,7 +985,8 @@ static GlaChunkParams fill(const sb_gla_recurrent_args *a, int heads, int G, int
   p.o_sb = a->out_stride_b; p.o_sh = a->out_stride_h; p.o_st = a->out_stride_t;
   p.s_slot = a->state_stride_slot; p.s_head = a->state_stride_head;
   p.range_hits = nullptr;
-  p.seg_tokens = p.n_seg = 0;
+  p.seg_tokens = p.n_seg = p.scanned = 0;
+  p.chains = 0;
   p.ws = nullptr;
   return p;
 }
@@ -1017,18 +1055,30 @@ int launch_gla_chunk_segments(const sb_gla_recurrent_args *a, int G, int n_seg, 
   const int Hk = a->num_heads / G;
   GlaChunkParams p = fill(a, Hk, G, G, 0, 1);
   p.seg_tokens = seg_tokens; p.n_seg = n_seg; p.ws = ws;
+  p.chains = a->batch * (int64_t)Hk;
+  const bool grouped = group_fits(a, G) && !(a->flags & SB_GLA_PER_HEAD);
+  p.scanned = n_seg > (grouped ? kFoldMaxGroup : kFoldMax);
   const dim3 block(256);
-  const unsigned chains = (unsigned)(a->batch * (int64_t)Hk);
+  const unsigned chains = (unsigned)p.chains;
   hipStream_t st = (hipStream_t)a->stream;
   const dim3 sgrid(chains, (unsigned)(n_seg - 1));
-  if (a->g_dtype == SB_F32) hipLaunchKernelGGL((gla_segment_state_kernel<SB_F32>), sgrid, block, 0, st, p);
-  else if (a->g_dtype == SB_BF16) hipLaunchKernelGGL((gla_segment_state_kernel<SB_BF16>), sgrid, block, 0, st, p);
-  else hipLaunchKernelGGL((gla_segment_state_kernel<SB_F16>), sgrid, block, 0, st, p);
+#define SB_LAUNCH(F32S, GDT) hipLaunchKernelGGL((gla_segment_state_kernel<F32S, GDT>), sgrid, block, 0, st, p)
+  if (a->state_dtype == SB_F32) {
+    if (a->g_dtype == SB_F32) SB_LAUNCH(true, SB_F32);
+    else if (a->g_dtype == SB_BF16) SB_LAUNCH(true, SB_BF16);
+    else SB_LAUNCH(true, SB_F16);
+  } else {
+    if (a->g_dtype == SB_F32) SB_LAUNCH(false, SB_F32);
+    else if (a->g_dtype == SB_BF16) SB_LAUNCH(false, SB_BF16);
+    else SB_LAUNCH(false, SB_F16);
+  }
+#undef SB_LAUNCH
   if (int rc = check_launch("gla_segment_state_kernel")) return rc;
-  if (a->state_dtype == SB_F32) hipLaunchKernelGGL((gla_segment_scan_kernel<true>), dim3(chains, 16), block, 0, st, p);
-  else hipLaunchKernelGGL((gla_segment_scan_kernel<false>), dim3(chains, 16), block, 0, st, p);
-  if (int rc = check_launch("gla_segment_scan_kernel")) return rc;
-  if (group_fits(a, G) && !(a->flags & SB_GLA_PER_HEAD)) {
+  if (p.scanned) {
+    hipLaunchKernelGGL(gla_segment_scan_kernel, dim3(chains, 16), block, 0, st, p);
+    if (int rc = check_launch("gla_segment_scan_kernel")) return rc;
+  }
+  if (grouped) {
     const int rc = launch_group_kernel<true>(a, p, dim3(chains, (unsigned)n_seg));
     return rc ? rc : check_launch("gla_chunk_group_kernel");
   }

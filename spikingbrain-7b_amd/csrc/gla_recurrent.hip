@@ -568,28 +568,35 @@ int segment_tokens(int seq_len, int n) { return ((seq_len + n - 1) / n + 31) / 3
 
 // Where the line lies (28 : 28 and 28 : 4 heads, fp32 state and gate, us per call uncut -> cut into the n this rule takes,
 // from graph replays):
-// * one state per head: two workgroups fit a CU and a cut prompt does 1.6 x the work, so it pays while two workgroups
-//   per CU allow four segments (18 at one prompt), of 64 tokens or more: 1 x 512 47 -> 29 (8), 1 x 3001 260 -> 73 (16), 1 x 8192
-//   694 -> 162 (18), 2 x 2048 183 -> 92 (8), 4 x 4096 363 -> 304 (4); six prompts in 3 371 -> 402. The two extra launches cost
-//   about 15 us: 4 x 600 in 2 61 -> 66;
+// * one state per head: a cut prompt does 1.6 x the work and pays about 10 us for the launch in front, so it wants segments of 64
+//   tokens or more, and one workgroup per CU: 1 x 300 32.5 -> 30.2 (4), 1 x 1024 80 -> 40 (9; two per CU, 16: 47), 1 x 3001 272 -> 66
+//   (9; 16: 69), 3 x 600 53.5 -> 48.4 (3), 2 x 600 52 -> 39 (4; 9: 41). Where that gives fewer than eight segments, long prompts
+//   fill the CUs twice: 2 x 2048 148 -> 72 (9; 4: 82), 2 x 1024 80 -> 52 (either), 4 x 4096 288 -> 259 (4; 2: 274). Two segments
+//   are never worth it (4 x 2048 150 -> 141, 4 x 1024 80.8 -> 80.2) nor are short prompts (1 x 200 26.2 -> 27.8, 3 x 300
+//   33.7 -> 36.9), nor three segments with two workgroups per CU (5 x 4000 282 -> 316);
 // * shared states: the one-pass kernel per group fills a CU by itself and beats a workgroup per query head as soon as
-//   there are enough of them: 1 x 512 90 -> 35 (8), 1 x 8192 1348 -> 79 (64), 4 x 4096 696 -> 124 (16), 16 x 8192 1736 -> 784
-//   (4), 26 x 4096 1252 -> 769 (2). (Chosen by hand, 1 x 512 in 16 segments of 32 tokens takes 29.)
+//   there are enough of them: 1 x 100 31.8 -> 23.6 (4), 1 x 512 90 -> 28 (16), 1 x 3001 520 -> 50 (47), 4 x 4096 700 -> 110 (16),
+//   16 x 512 107 -> 61 (4), 16 x 8192 1417 -> 662 (4). A single prompt, whose length the call states, goes down to segments of one
+//   block (1 x 512 in 8 of 64 tokens: 34.2); of several the shorter ones leave such segments empty, so they keep 64.
 extern "C" int32_t sb_gla_prompt_segments(const sb_gla_recurrent_args *a) {
-  if (!a || a->batch <= 0 || a->num_heads <= 0 || a->seq_len < 256 || !block_form(a) ||
+  if (!a || a->batch <= 0 || a->num_heads <= 0 || a->seq_len <= 64 || !block_form(a) ||
       (a->flags & (SB_GLA_CHECK_GATES | SB_GLA_PER_HEAD | SB_GLA_GROUP_PASS)))
     return 1;
   const int G = a->q_heads_per_state > 1 ? a->q_heads_per_state : 1;
   const int64_t chains = a->batch * (int64_t)(a->num_heads / G);
   if (chains == 0) return 1;
-  const int64_t cus = sb_host::device_cu_count();
+  const int64_t cus = sb_host::device_cu_count(), T = a->seq_len;
+  auto least = [](int64_t x, int64_t y) { return x < y ? x : y; };
   int64_t n;
   if (G > 1) {
-    n = cus / chains < a->seq_len / 48 ? cus / chains : a->seq_len / 48;
+    if (a->batch > 1 && T < 256) return 1;
+    n = least(cus / chains, a->batch > 1 ? T / 48 : (T + 31) / 32);
     if (n < 2) return 1;
   } else {
-    n = 2 * cus / chains < a->seq_len / 64 ? 2 * cus / chains : a->seq_len / 64;
-    if (n < 4 || a->seq_len < (n < 8 ? 1024 : 512)) return 1;
+    n = cus / chains;
+    if (n < 8 && T >= 1024 && 2 * cus / chains >= 4) n = 2 * cus / chains;
+    n = least(n, T / 64);
+    if (T < (n < 4 ? 512 : 256) || n < 3) return 1;
   }
   const int seg = segment_tokens(a->seq_len, (int)n);
   return (a->seq_len + seg - 1) / seg;

@@ -60,3 +60,24 @@ def test_rows_too_far_apart_for_the_block_form(sb, dev):
     cu = torch.tensor([0, T], dtype=torch.int32, device=dev)
     o = sb.ops.gla_recurrent_packed(apart(q), k.to(dev), v.to(dev), gate.to(dev), state, cu)
     _check(o.transpose(0, 1), ref_o[0], state[0], ref_S[0])
+
+
+@pytest.mark.parametrize("H,Hk,lens", [(14, 2, [300, 257, 64, 1] + [65] * 28),   # 64 groups: 4 segments, each adds up those before it
+                                       (2, 2, [1100]),                           # 17 segments: a scan adds up
+                                       (28, 28, [600, 500]),                     # 4 segments per head, added up
+                                       (8, 2, [97])])                            # a single prompt in segments of one block
+def test_segments_start_from_what_those_before_them_add_up_to(sb, dev, H, Hk, lens):
+    """Cut calls against the uncut one: the same blocks, a state rounded once more per segment (fp32: 1e-4 of the largest entry)."""
+    n, T = len(lens), sum(lens)
+    g = torch.Generator().manual_seed(T)
+    q = torch.randn(T, H, D, generator=g).bfloat16().relu().to(dev)
+    k, v = (torch.randn(T, Hk, D, generator=g).bfloat16().relu().to(dev) for _ in range(2))
+    gate = (F.logsigmoid(torch.randn(T, Hk, D, generator=g)) / 16).to(dev)
+    S0 = (torch.randn(n, Hk, D, D, generator=g) * 0.1).to(dev)
+    cu = torch.tensor([0] + lens).cumsum(0).int().to(dev)
+    st, st1 = S0.clone(), S0.clone()
+    o = sb.ops.gla_recurrent_packed(q, k, v, gate, st, cu, None, max_seq_len=max(lens))
+    o1 = sb.ops.gla_recurrent_packed(q, k, v, gate, st1, cu, None, max_seq_len=max(lens), per_head=True)   # (never cut)
+    assert (st - st1).abs().max() <= 1e-4 * st1.abs().max()
+    d, ref = (o.float() - o1.float()).abs(), o1.float().abs()
+    assert (d <= 2.0 ** -7 * ref + 2.0 ** -8 * ref.max()).all()      # each rounds the same sums, and its operands, to bf16
