@@ -72,7 +72,7 @@ struct PrefillParams {
   int G, head_begin;          // query heads per kv head; first of them handled by this launch
   int Hq;
   int num_tiles;
-  int bucket, head_groups;    // order of an XCD's workgroups (see the kernel)
+  int bucket, head_groups;    // order of an XCD's workgroups (see the kernel); bucket 0: not by XCD
   int block_size, window_left;
   int tiles_per_block;        // block_size / 16
   TileDivision tile_div;      // by tiles_per_block
@@ -130,16 +130,21 @@ __device__ __forceinline__ uint2 load_transposed(const char *row) {
   const v4s v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4s __attribute__((address_space(3))) *)row);
   return __builtin_bit_cast(uint2, v);
 }
+constexpr int kHandOver = 2048 * 4 + 1024;   // bytes of one wavefront's block between the halves of a walk: sums, reference points and denominators
+static_assert(8 * kHandOver <= 6 * kStage, "hand-over of two sets of four wavefronts");
 constexpr float kNegInf = kNegInfF;
 constexpr float kRaise = 8.f;
 
 // NHEADS query heads of one kv head per workgroup: head pairs are served by 4 wavefronts of two column blocks (one
 // 16-token sub-tile, both heads of the pair), an odd last head by 4 of one. NHEADS = 4 also serves 3 heads and NHEADS = 2
 // one, so that all groups of a GQA group of 7 are one launch either way.
-template <int NHEADS>
+// HALVES: the workgroup holds that set of wavefronts twice, and each takes half of the walk through a ring of its own; at the
+// end they put their sums together in LDS.
+template <int NHEADS, bool HALVES>
 struct Shape {
-  static constexpr int kWaves = 4 * (NHEADS / 2) + 4 * (NHEADS % 2);
-  static constexpr int kFetchWaves = kWaves == 8 ? 8 : (kWaves < 4 ? kWaves : 4);   // wavefronts that move K/V into LDS
+  static constexpr int kSetWaves = 4 * (NHEADS / 2) + 4 * (NHEADS % 2);
+  static constexpr int kWaves = kSetWaves * (HALVES ? 2 : 1);
+  static constexpr int kFetchWaves = kSetWaves == 8 ? 8 : 4;    // wavefronts (of a set) that move K/V into LDS
   static constexpr int kLoads = 8 / kFetchWaves;                // 4-row loads per fetching lane, per K and per V
 };
 
@@ -176,12 +181,12 @@ __device__ __forceinline__ uint4 dequant8(uint2 w, float s) {
 
 // ODD: the last group of heads may have one less (3 of 4, 1 of 2): a build of its own, because the second path costs
 // the kernel of two heads 5 % (16 : 8 heads, 2000 tokens behind 3000 95 -> 100 us).
-template <typename E, int NHEADS, int KVQ, bool PAGED, bool ODD>
-__global__ __attribute__((amdgpu_flat_work_group_size(64 * Shape<NHEADS>::kWaves, 64 * Shape<NHEADS>::kWaves),
+template <typename E, int NHEADS, int KVQ, bool PAGED, bool ODD, bool HALVES>
+__global__ __attribute__((amdgpu_flat_work_group_size(64 * Shape<NHEADS, HALVES>::kWaves, 64 * Shape<NHEADS, HALVES>::kWaves),
                           amdgpu_waves_per_eu(2, 2)))
 void swa_prefill_kernel(const PrefillParams p) {
-  using S = Shape<NHEADS>;
-  __shared__ __attribute__((aligned(16))) char smem[3 * kStage];  // ring of three chunks, each [K|V]
+  using S = Shape<NHEADS, HALVES>;
+  __shared__ __attribute__((aligned(16))) char smem_all[(HALVES ? 6 : 3) * kStage];  // ring(s) of three chunks, each [K|V]
 
   // Workgroups are handed to the 8 XCDs round-robin by index, and each XCD has its own L2. Give XCD x
   // the x-th contiguous eighth of the tiles, so that the workgroups resident on one XCD at a time are
@@ -189,19 +194,31 @@ void swa_prefill_kernel(const PrefillParams p) {
   // Inside an XCD's list the order is: buckets of p.bucket tiles, in a bucket the head groups, in those the kv heads,
   // in those the tiles.
   const int per_xcd = (p.num_tiles + 7) >> 3;
-  const int at = blockIdx.x >> 3, per_tile = p.Hkv * p.head_groups;
-  const int bucket = at / (p.bucket * per_tile);
-  const int width = min(p.bucket, per_xcd - bucket * p.bucket);   // tiles of this bucket
-  const int in_bucket = at - bucket * p.bucket * per_tile;
-  const int pair = in_bucket / width;
-  // (the parts of a tile go to XCDs one after the other: a call of one tile would otherwise run on one of them)
-  const int tile = ((blockIdx.x + blockIdx.y) & 7) * per_xcd + bucket * p.bucket + (in_bucket - pair * width);
+  const int per_tile = p.Hkv * p.head_groups;
+  int tile, pair;
+  if (HALVES && p.bucket == 0) {
+    // lists dealt longest walk first, walked in that order over all XCDs: no XCD has to itself what starts last (where all
+    // workgroups start together the order of tile_order shares keys in an XCD's L2: 12 : 4, 2048 behind 10000 75.6 us, this way 81.7)
+    const int rank = blockIdx.x / per_tile;
+    tile = (rank & 7) * per_xcd + (rank >> 3);
+    pair = blockIdx.x - rank * per_tile;
+  } else {
+    const int at = blockIdx.x >> 3;
+    const int bucket = at / (p.bucket * per_tile);
+    const int width = min(p.bucket, per_xcd - bucket * p.bucket);   // tiles of this bucket
+    const int in_bucket = at - bucket * p.bucket * per_tile;
+    pair = in_bucket / width;
+    // (the parts of a tile go to XCDs one after the other: a call of one tile would otherwise run on one of them)
+    tile = ((blockIdx.x + blockIdx.y) & 7) * per_xcd + bucket * p.bucket + (in_bucket - pair * width);
+  }
   if (tile >= p.num_tiles) return;
   const int head_group = pair / p.Hkv, kvh = pair - head_group * p.Hkv;
   const int head_begin = p.head_begin + NHEADS * head_group;
   const int nheads = ODD ? min(NHEADS, p.G - head_begin) : NHEADS;
   const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = HALVES ? wave_all / S::kSetWaves : 0, wave = HALVES ? wave_all % S::kSetWaves : wave_all;
+  char *const smem = smem_all + half * 3 * kStage;
   const int lane = tid & 63;
   const int g = lane >> 4;
   const int c = lane & 15;
@@ -222,10 +239,12 @@ void swa_prefill_kernel(const PrefillParams p) {
   // this workgroup's part of the walk
   const int part = blockIdx.y, parts = tile_parts(p, walk);
   if (part >= parts) return;  // (the whole workgroup, ahead of every barrier)
-  const int ch_begin = walk.ch_begin + part * p.part_chunks;
-  const int ch_end = part + 1 == parts ? walk.ch_end : ch_begin + p.part_chunks;
-  const int n_walk = ch_end - ch_begin;  // the walk: index x is window chunk ch_begin + x
-  const int meta_chunks = part == 0 ? (p.meta_len + 31) >> 5 : 0;
+  const int part_begin = walk.ch_begin + part * p.part_chunks;
+  const int part_end = part + 1 == parts ? walk.ch_end : part_begin + p.part_chunks;
+  // (halves are of one length: where the second has a chunk less, its last lies past every token and is masked)
+  const int n_walk = HALVES ? (part_end - part_begin + 1) >> 1 : part_end - part_begin;
+  const int ch_begin = part_begin + half * n_walk;  // the walk: index x is window chunk ch_begin + x
+  const int meta_chunks = !HALVES && part == 0 ? (p.meta_len + 31) >> 5 : 0;   // (calls with meta rows do not take halves)
 
   // Everything from here on is written for NB column blocks per wavefront: two for the wavefronts of a head
   // pair, one for those of an odd last head (four wavefronts, one per 16-token sub-tile).
@@ -276,7 +295,7 @@ void swa_prefill_kernel(const PrefillParams p) {
     // Everything that does not depend on the lane is kept in scalar registers: per chunk, the tile's byte offset
     // (one block-table entry, looked up one call ahead of its use) added to the K and V bases; a lane adds its
     // row and column as a 32-bit offset.
-    constexpr int kFetchAll = S::kFetchWaves == S::kWaves;
+    constexpr bool kFetchAll = S::kFetchWaves == S::kSetWaves;
     const bool fetcher = kFetchAll || wave < S::kFetchWaves;
     constexpr int rows_per_wave = 32 / S::kFetchWaves;                     // 4, 8 or 16
     const int tsel = (wave * rows_per_wave) >> 4;                          // which 16-key tile of a chunk this wavefront's rows are in
@@ -614,8 +633,39 @@ void swa_prefill_kernel(const PrefillParams p) {
     second_half(sa, kYes, kNo);
 
     // ---- epilogue: lane (g, c) owns token c of each block, dims 16 mt + 4g + i --------------------------
+    if constexpr (HALVES) {
+      // Each set puts one of two blocks together (the first set the only one): the other set's sums come through LDS, a
+      // wavefront's in the ring slots of its own set (read last before the barrier).
+      float *const out_acc = reinterpret_cast<float *>(smem_all + (half * S::kSetWaves + wave) * kHandOver) + lane * 4;
+      const float *const in_acc = reinterpret_cast<const float *>(smem_all + ((half ^ 1) * S::kSetWaves + wave) * kHandOver) + lane * 4;
+      auto hand_over = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int mt = 0; mt < 8; ++mt) *reinterpret_cast<f32x4_t *>(out_acc + mt * 256) = acc[b][mt];
+        *reinterpret_cast<float2 *>(out_acc + 2048) = make_float2(m[b], l[b]);
+      };
+      auto put_together = [&](int b) __attribute__((always_inline)) {
+        const float2 ml = *reinterpret_cast<const float2 *>(in_acc + 2048);
+        const float m_new = fmaxf(m[b], ml.x), m_safe = m_new == kNegInf ? 0.f : m_new;
+        const float mine = fast_exp2(m[b] - m_safe), other = fast_exp2(ml.x - m_safe);
+        m[b] = m_new;
+        l[b] = fmaf(ml.y, other, l[b] * mine);
+#pragma unroll
+        for (int mt = 0; mt < 8; ++mt) {
+          const f32x4_t x = *reinterpret_cast<const f32x4_t *>(in_acc + mt * 256);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[b][mt][i] = fmaf(x[i], other, acc[b][mt][i] * mine);
+        }
+      };
+      __syncthreads();
+      if (half) hand_over(0);
+      else if (NB == 2) hand_over(NB - 1);
+      __syncthreads();
+      if (half) { if (NB == 2) put_together(NB - 1); }
+      else put_together(0);
+    }
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
+      if (HALVES && b != half) continue;   // (wave-uniform)
       float lt = l[b];
       lt += __shfl_xor(lt, 16);
       lt += __shfl_xor(lt, 32);
@@ -710,20 +760,23 @@ __global__ __launch_bounds__(256) void swa_prefill_merge_kernel(const PrefillPar
 }
 
 template <typename E, int KVQ, bool PAGED>
-void launch_prefill_q(int nh, bool odd, dim3 grid, hipStream_t st, const PrefillParams &p) {
-  const dim3 b1(64 * Shape<1>::kWaves), b2(64 * Shape<2>::kWaves), b4(64 * Shape<4>::kWaves);
-  if (nh == 1) hipLaunchKernelGGL((swa_prefill_kernel<E, 1, KVQ, PAGED, false>), grid, b1, 0, st, p);
-  else if (nh == 2 && odd) hipLaunchKernelGGL((swa_prefill_kernel<E, 2, KVQ, PAGED, true>), grid, b2, 0, st, p);
-  else if (nh == 2) hipLaunchKernelGGL((swa_prefill_kernel<E, 2, KVQ, PAGED, false>), grid, b2, 0, st, p);
-  else if (odd) hipLaunchKernelGGL((swa_prefill_kernel<E, 4, KVQ, PAGED, true>), grid, b4, 0, st, p);
-  else hipLaunchKernelGGL((swa_prefill_kernel<E, 4, KVQ, PAGED, false>), grid, b4, 0, st, p);
+void launch_prefill_q(int nh, bool odd, bool halves, dim3 grid, hipStream_t st, const PrefillParams &p) {
+  const dim3 b4(256), b8(512);
+  if (halves && nh == 1) hipLaunchKernelGGL((swa_prefill_kernel<E, 1, KVQ, PAGED, false, true>), grid, b8, 0, st, p);
+  else if (halves && odd) hipLaunchKernelGGL((swa_prefill_kernel<E, 2, KVQ, PAGED, true, true>), grid, b8, 0, st, p);
+  else if (halves) hipLaunchKernelGGL((swa_prefill_kernel<E, 2, KVQ, PAGED, false, true>), grid, b8, 0, st, p);
+  else if (nh == 1) hipLaunchKernelGGL((swa_prefill_kernel<E, 1, KVQ, PAGED, false, false>), grid, b4, 0, st, p);
+  else if (nh == 2 && odd) hipLaunchKernelGGL((swa_prefill_kernel<E, 2, KVQ, PAGED, true, false>), grid, b4, 0, st, p);
+  else if (nh == 2) hipLaunchKernelGGL((swa_prefill_kernel<E, 2, KVQ, PAGED, false, false>), grid, b4, 0, st, p);
+  else if (odd) hipLaunchKernelGGL((swa_prefill_kernel<E, 4, KVQ, PAGED, true, false>), grid, b8, 0, st, p);
+  else hipLaunchKernelGGL((swa_prefill_kernel<E, 4, KVQ, PAGED, false, false>), grid, b8, 0, st, p);
 }
 template <typename E>
-void launch_prefill(int kv_quant, int nh, bool odd, dim3 grid, hipStream_t st, const PrefillParams &p) {
-  if (kv_quant == SB_KV_INT8) launch_prefill_q<E, SB_KV_INT8, true>(nh, odd, grid, st, p);
-  else if (kv_quant == SB_KV_FP8) launch_prefill_q<E, SB_KV_FP8, true>(nh, odd, grid, st, p);
-  else if (p.block_table) launch_prefill_q<E, SB_KV_NONE, true>(nh, odd, grid, st, p);
-  else launch_prefill_q<E, SB_KV_NONE, false>(nh, odd, grid, st, p);
+void launch_prefill(int kv_quant, int nh, bool odd, bool halves, dim3 grid, hipStream_t st, const PrefillParams &p) {
+  if (kv_quant == SB_KV_INT8) launch_prefill_q<E, SB_KV_INT8, true>(nh, odd, halves, grid, st, p);
+  else if (kv_quant == SB_KV_FP8) launch_prefill_q<E, SB_KV_FP8, true>(nh, odd, halves, grid, st, p);
+  else if (p.block_table) launch_prefill_q<E, SB_KV_NONE, true>(nh, odd, halves, grid, st, p);
+  else launch_prefill_q<E, SB_KV_NONE, false>(nh, odd, halves, grid, st, p);
 }
 
 constexpr int64_t kDealtTiles = 1024;   // shorter tile lists come dealt to the XCDs, see sb_swa_prefill_plan
@@ -747,6 +800,7 @@ int64_t most_chunks(const sb_swa_prefill_args *a, int64_t max_keys) {
 //    From 256 to 384 workgroups of four (a second round that leaves most CUs idle) they pay unless the walks are many chunks
 //    long: 3059 tokens, window 4096 92.8 -> 88.8; behind 4200, windows 512 / 1024 / 2048 / 4096 52.4 / 77.1 / 127 / 228 -> 47 / 72.9 / 124 /
 //    230; beyond that they lose (1 x 6000: 256 -> 271).
+//  * halves: workgroups of two heads that hold their four wavefronts twice, each set walking half of the keys (see halves_pay).
 //  * parts: the keys of a walk cut into parts of 8 chunks or more side by side, at the price of fp32 partials and
 //    a merge (64 / 200 / 512 / 1024 tokens behind 4200: 100 with pairs, 123 with groups of four -> 27.5 (12 parts) / 37 (8) /
 //    54 (4) / 85 (2) us; 64 tokens in 8 parts 25.7, which the estimate below does not find).
@@ -766,6 +820,25 @@ bool pairs_pay(const sb_swa_prefill_args *a, int64_t chunks, int64_t parts, int6
   const int64_t pairs_per_tile = (int64_t)a->num_kv_heads * ((a->num_q_heads / a->num_kv_heads + 1) / 2);
   const int64_t sharing = cus / pairs_per_tile;   // tiles in front of the first one that shares
   return sharing >= a->num_tiles || (double)most_chunks(a, a->tile_keys[sharing]) < 6.0 + 0.63 * (double)chunks;
+}
+// Halves: one such workgroup fills a CU and takes 8.4 + 0.525 L us for a walk of L chunks, a pair 9 + 0.69 L, so they pay wherever
+// every workgroup has a CU, from walks of 9 chunks on (28 : 4 heads, us of pairs -> halves: whole prompts of 200 / 300 / 700 / 1000
+// tokens 12.3 / 14.3 / 23.5 / 30.2 -> 12.5 / 13.4 / 20.7 / 25.5, 1024 tokens behind 10000 with a window of 512 / 4096 24.2 / 102 -> 22 / 77; 16 : 8,
+// 3000 whole 73.6 -> 54.8). A second round pays where it is short walks that are left for the CUs that come free first: with
+// the lists walked longest first over all XCDs, 1300 / 1517 / 2000 whole 38.6 / 43.3 / 54.9 -> 32.1 / 35.3 / 50.0 (38 / 40 / 54.6 with an XCD's
+// tiles to itself), 2048 behind 800 79.7 -> 77; not 2 x 1000 33.6 -> 34, 4 x 500 23 -> 26.7, 2048 behind 10000 (groups of four: 132) -> 149
+// and, in three rounds, 2560 69.7 -> 78. One head per kv head, second round: 16 : 16, 4 x 500 17 -> 19.9 (not taken).
+bool halves_pay(const sb_swa_prefill_args *a, int64_t max_keys, int64_t chunks, int64_t cus) {
+  const int64_t G = a->num_q_heads / a->num_kv_heads, per_tile = a->num_kv_heads * ((G + 1) / 2), wgs = a->num_tiles * per_tile;
+  if (a->meta_len > 0 || max_keys >= INT32_MAX || chunks < 9) return false;   // (of calls without a bound the walks are unknown)
+  if (wgs <= cus) return true;
+  if (G == 1 || wgs > 2 * cus || !a->tile_keys) return false;
+  const double l0 = (double)chunks, next = (double)most_chunks(a, a->tile_keys[cus / per_tile]),
+               first_done = (double)most_chunks(a, a->tile_keys[(cus - 1) / per_tile]);
+  const double halves = std::max(8.4 + 0.525 * l0, 14.0 + 0.55 * (first_done + next));
+  double others = 6.3 + 0.72 * l0 + 0.35 * next;   // pairs
+  if (quad_workgroups(a) <= cus) others = std::min(others, 8.4 + 0.94 * l0);
+  return halves < 0.93 * others;
 }
 // Order of a short list's tiles. Dealt to the XCDs longest walk first, in tile-major order, evens out the work of walks of
 // different lengths; in sequence order, kv heads outermost, the tiles that run on an XCD at a time are neighbours of one head and
@@ -795,7 +868,11 @@ Order tile_order(const sb_swa_prefill_args *a, int64_t max_keys, int64_t chunks,
 Spread spread_of(const sb_swa_prefill_args *a, int64_t max_keys) {
   const int64_t chunks = most_chunks(a, max_keys), wgs = quad_workgroups(a), cus = sb_host::device_cu_count();
   Spread best{1, pairs_pay(a, chunks, 1, cus)};
-  double best_us = 5.0 + (best.pairs ? 0.69 : 0.9) * (double)chunks;
+  // (parts are the better the fewer heads their workgroups have: one, 16 : 16, 512 behind 10000 in halves 64 us, in 3 parts 49; three, 12 : 4,
+  // 2048 behind 10000 78.7 and in 2 parts 75, but 1517 whole 33 and 41)
+  const int G = a->num_q_heads / a->num_kv_heads;
+  double best_us = G > 1 && halves_pay(a, max_keys, chunks, cus) ? 8.4 + (G == 3 ? 2.0 : 0.0) + 0.525 * (double)chunks
+                                                                 : 5.0 + (best.pairs ? 0.69 : 0.9) * (double)chunks;
   for (int64_t n = 2; n * wgs <= cus && 8 * n <= chunks; ++n) {
     const bool pairs = pairs_pay(a, chunks, n, cus);
     const double us = 13.5 + 0.28 * (double)n + 8.0 * (double)(n * wgs) / (double)cus +
@@ -868,7 +945,9 @@ int prefill(const sb_swa_prefill_args *a, int64_t max_keys, int n_parts, float *
   p.num_tiles = (int)a->num_tiles;
   const int64_t chunks = most_chunks(a, max_keys);
   const int64_t cus = sb_host::device_cu_count();
-  const Order order = n_parts == 1 ? tile_order(a, max_keys, chunks, cus) : Order::kDealt;
+  const bool halves = n_parts == 1 && halves_pay(a, max_keys, chunks, cus);
+  const bool rounds = halves && a->num_tiles * a->num_kv_heads * ((p.G + 1) / 2) > cus;   // more workgroups than CUs
+  const Order order = n_parts == 1 && !rounds ? tile_order(a, max_keys, chunks, cus) : Order::kDealt;
   if (order == Order::kSequence) {
     p.tile_seq = a->ordered_tile_seq;
     p.tile_q0 = a->ordered_tile_q0;
@@ -920,8 +999,8 @@ int prefill(const sb_swa_prefill_args *a, int64_t max_keys, int n_parts, float *
   // kv head at a time keep their keys in the XCD's L2).
   // Up to four query heads per kv head that is 1 to 10 % slower than all (16 : 16 3194 / 2951 us, 16 : 8 2270 / 2222, 32 : 8 4407 / 4356
   // for 10 x 8192). Shorter lists: see tile_order.
-  p.bucket = a->num_tiles >= kDealtTiles ? (p.G <= 4 ? (int)per_xcd : 4) : order == Order::kDealt ? 1 : (int)per_xcd;
-  const bool pairs = p.G > 1 && pairs_pay(a, chunks, n_parts, cus);
+  p.bucket = rounds ? 0 : a->num_tiles >= kDealtTiles ? (p.G <= 4 ? (int)per_xcd : 4) : order == Order::kDealt ? 1 : (int)per_xcd;
+  const bool pairs = p.G > 1 && (halves || pairs_pay(a, chunks, n_parts, cus));
   if (per_xcd * 8 * a->num_kv_heads * p.G > 0x7fffffffLL) return fail(SB_ERR_UNSUPPORTED, "sb_swa_prefill: grid too large");
   for (int h0 = 0; h0 < p.G;) {
     const int left = p.G - h0;
@@ -932,8 +1011,8 @@ int prefill(const sb_swa_prefill_args *a, int64_t max_keys, int n_parts, float *
     h0 += nh * groups;
     p.head_groups = groups;
     const dim3 grid((unsigned)(per_xcd * 8 * a->num_kv_heads * groups), (unsigned)n_parts);
-    if (a->dtype == SB_BF16) launch_prefill<BF16>(a->kv_quant, nh, odd, grid, (hipStream_t)a->stream, p);
-    else launch_prefill<F16>(a->kv_quant, nh, odd, grid, (hipStream_t)a->stream, p);
+    if (a->dtype == SB_BF16) launch_prefill<BF16>(a->kv_quant, nh, odd, halves, grid, (hipStream_t)a->stream, p);
+    else launch_prefill<F16>(a->kv_quant, nh, odd, halves, grid, (hipStream_t)a->stream, p);
     const int rc = check_launch("swa_prefill_kernel");
     if (rc != SB_OK) return rc;
   }
@@ -1009,7 +1088,9 @@ extern "C" int32_t sb_swa_prefill_parts(const sb_swa_prefill_args *a, int64_t ma
 
 extern "C" int32_t sb_swa_prefill_group_heads(const sb_swa_prefill_args *a, int64_t max_keys, int32_t n_parts) {
   if (!a || a->num_tiles <= 0 || a->num_kv_heads <= 0 || a->num_q_heads < a->num_kv_heads || max_keys <= 0) return 4;
-  return pairs_pay(a, most_chunks(a, max_keys < INT32_MAX ? max_keys : INT32_MAX), n_parts < 1 ? 1 : n_parts, sb_host::device_cu_count()) ? 2 : 4;
+  if (max_keys > INT32_MAX) max_keys = INT32_MAX;
+  const int64_t chunks = most_chunks(a, max_keys), cus = sb_host::device_cu_count();
+  return pairs_pay(a, chunks, n_parts < 1 ? 1 : n_parts, cus) || (n_parts < 2 && halves_pay(a, max_keys, chunks, cus)) ? 2 : 4;
 }
 
 extern "C" size_t sb_swa_prefill_workspace_bytes(const sb_swa_prefill_args *a, int64_t total_q, int32_t n_parts) {

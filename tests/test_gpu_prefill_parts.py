@@ -155,3 +155,38 @@ def test_more_parts_than_the_merge_addresses(sb, dev):
     run = lambda n: sb.ops.swa_prefill_attention(q, k, v, query_lens=[1], seq_lens_k=[300], kv_start=torch.zeros(1, dtype=torch.int64, device=dev),
                                                  window_left=4096, n_parts=n)
     assert torch.equal(run(1024), run(40))
+
+
+@pytest.mark.parametrize("kv", ["dense", "paged", "int8", "fp8"])
+@pytest.mark.parametrize("G,lens,ctx,window", [(7, [257], 0, 4096), (7, [1300], 0, 4096), (3, [65, 300], 520, 300), (2, [64], 256, 4096), (1, [290, 31], 64, -1),
+                                               (5, [33], 700, 290)])
+def test_halves_of_a_walk(sb, dev, kv, G, lens, ctx, window):
+    """Workgroups whose two sets of wavefronts each take half of the keys: odd and even numbers of chunks, a last group of one head,
+    walks whose second half is all masked for some tokens, more workgroups than CUs (1300 tokens), against the same call cut
+    into two parts; both are within 1e-2 of the mathematics, and their log-sum-exps come from the same fp32 scores (as above)."""
+    g = torch.Generator().manual_seed(G + len(lens))
+    Hkv, T, keys = 4, sum(lens), [n + ctx for n in lens]
+    q = torch.randn(T, Hkv * G, D, generator=g).bfloat16().to(dev)
+    kw = dict(query_lens=lens, seq_lens_k=keys, window_left=window, return_lse=True)
+    if kv == "dense":
+        k, v = (torch.randn(sum(keys), Hkv, D, generator=g).bfloat16().to(dev) for _ in range(2))
+        kw.update(kv_start=torch.tensor([0] + keys).cumsum(0)[:-1].to(dev), key_lo=torch.tensor([5] * len(lens), dtype=torch.int32, device=dev))
+    else:
+        width = max(-(-n // 16) for n in keys)
+        table = torch.randperm(len(lens) * width, generator=g).view(len(lens), width).int()
+        shape = (2, table.numel(), 16, Hkv, D)
+        if kv == "paged":
+            k, v = torch.randn(shape, generator=g).bfloat16().to(dev)
+        elif kv == "int8":
+            k, v = torch.randint(-127, 128, shape, generator=g).to(torch.int8).to(dev)
+            s = (torch.rand(2, table.numel(), Hkv, 16, generator=g) * 0.02).to(dev)
+            kw.update(k_scale=s[0], v_scale=s[1])
+        else:
+            k, v = torch.randn(shape, generator=g).to(torch.float8_e4m3fn).to(dev)
+            kw.update(fp8_scales=(1.0, 1.0))
+        kw.update(block_table=table.to(dev))
+    (whole, lse), (cut, lse1) = (sb.ops.swa_prefill_attention(q, k, v, n_parts=n, **kw) for n in (1, 2))
+    assert torch.isfinite(whole).all()
+    assert (whole.double() - cut.double()).norm() <= 1e-2 * cut.double().norm()
+    ok = ~torch.isneginf(lse1)
+    assert torch.equal(torch.isneginf(lse), ~ok) and (lse[ok] - lse1[ok]).abs().max() <= 1e-4
