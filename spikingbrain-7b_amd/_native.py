@@ -6,6 +6,7 @@ when the shared object is missing, and every wrapper raises when a launch is rej
 from __future__ import annotations
 
 import ctypes as C
+import importlib.util
 import os
 from typing import Optional
 
@@ -251,6 +252,27 @@ def lib() -> C.CDLL:
         raise NativeLibraryError(f"{LIB_PATH} has ABI version {got}, this package needs {ABI_VERSION}")
     _lib = handle
     return handle
+
+
+_calls_module = None
+
+
+def calls():
+    """The extension module of csrc/calls.cpp: ordinary layer calls from tensors to the C ABI in one step."""
+    global _calls_module
+    if _calls_module is None:
+        lib()
+        path = os.path.join(_HERE, "_calls.so")
+        if not os.path.exists(path):
+            raise NativeLibraryError(f"{path} is missing: build it with `make -C {os.path.join(_HERE, 'csrc')}`")
+        spec = importlib.util.spec_from_file_location("_calls", path)
+        module = importlib.util.module_from_spec(spec)
+        try:
+            spec.loader.exec_module(module)
+        except ImportError as e:
+            raise NativeLibraryError(f"cannot load {path}: {e}") from e
+        _calls_module = module
+    return _calls_module
 
 
 def last_error() -> str:

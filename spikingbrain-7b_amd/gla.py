@@ -50,6 +50,9 @@ def my_fused_recurrent_gla(
         scale = D ** -0.5
     if slot_idx is not None and slot_idx.dtype != torch.int32:
         slot_idx = slot_idx.to(torch.int32)
+    out = ops.gla_step(q, k, v, g, kv_caches, slot_idx, scale)
+    if out is not None:
+        return out
     out = ops.gla_recurrent(q, k, v, g, kv_caches, slot_idx, scale, zero_skipped=True)
     return out.view(B, H, D)
 

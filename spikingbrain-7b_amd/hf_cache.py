@@ -36,7 +36,7 @@ class _WindowBuffer:
         self.length = length
 
     def view(self) -> torch.Tensor:
-        return self.storage[:, :, self.start:self.start + self.length, :]
+        return self.storage.narrow(2, self.start, self.length)
 
 
 def _capacity_for(rows: int, window: Optional[int]) -> int:

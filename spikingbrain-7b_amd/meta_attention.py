@@ -482,6 +482,9 @@ class MetaAttentionImpl:
         """query [T, Hq, D]; key/value [T, Hkv, D]; kv_cache [2, nb, bs, Hkv, D] (numel 0 for the
         profiling run); `output` [T, Hq, D] is written in place and returned (:703-982)."""
         assert output is not None, "Output tensor must be provided."
+        if output_scale is None and query2 is None and key2 is None and value2 is None and \
+                self._pure_decode(layer, query, key, value, kv_cache, attn_metadata, output):
+            return output
         if output_scale is not None:
             raise NotImplementedError("fused output quantization is not supported in MetaAttention.")
         fp8_kv = self.kv_cache_dtype.startswith("fp8")
@@ -636,18 +639,40 @@ class MetaAttentionImpl:
                 if fuse_append:
                     fused = dict(new_key=_rows_of(key, 0, n), new_value=_rows_of(value, 0, n),
                                  new_slot_mapping=_rows_of(_flat(decode_meta.slot_mapping), 0, n).contiguous())
-                if decode_meta._decode_balanced is None:
-                    host_lens = decode_meta.host_seq_lens
-                    decode_meta._decode_balanced = bool(
-                        host_lens is not None and len(host_lens) >= n and
-                        ops.plan_decode_split(n, self.num_kv_heads, decode_meta.max_decode_seq_len or max(host_lens[:n]),
-                                              window_left, host_lens[:n]))
+                balanced = self._balanced(decode_meta, n, window_left)
                 ops.swa_decode_attention(
                     decode_query, key_cache, value_cache, _rows_of(decode_meta.seq_lens_tensor, 0, n),
                     block_table=decode_meta.block_tables, window_left=window_left, scale=self.scale,
                     out=decode_output, max_seq_len=decode_meta.max_decode_seq_len or None,
-                    balanced=False if byte_kv else decode_meta._decode_balanced, **scales, **fused, **decode_kv)
+                    balanced=False if byte_kv else balanced, **scales, **fused, **decode_kv)
         return output
+
+    def _pure_decode(self, layer, query, key, value, kv_cache, meta, output) -> bool:
+        """The layer call of a step of decoding sequences only (one token each, element caches, no score options) in one
+        native step; False, with nothing done, for any other."""
+        n = meta.num_decode_tokens
+        if meta.num_prefill_tokens or meta.num_prefills or n <= 0 or (meta.max_decode_query_len or 1) != 1 or meta.slot_mapping is None or \
+                key is None or value is None or self.attn_type != AttentionType.DECODER or self.alibi_slopes is not None or \
+                self.logits_soft_cap > 0 or self.kv_cache_dtype.startswith("fp8") or type(kv_cache) is not torch.Tensor or \
+                not query.is_cuda or query.shape != (n, self.num_heads, self.head_size) or \
+                getattr(layer, "_k_scale_float", 1.0) != 1.0 or getattr(layer, "_v_scale_float", 1.0) != 1.0:
+            return False
+        meta = meta.decode_metadata
+        if meta.max_decode_query_len is None:
+            return False
+        return ops.paged_decode_step(query, key, value, kv_cache, output, meta.slot_mapping, meta.seq_lens_tensor, meta.block_tables,
+                                     self.sliding_window[0], self.scale, meta.max_decode_seq_len or 0,
+                                     self._balanced(meta, n, self.sliding_window[0]))
+
+    def _balanced(self, decode_meta, n: int, window_left: int) -> bool:
+        """Split policy of the step's decode launch, decided once for all layers."""
+        if decode_meta._decode_balanced is None:
+            host_lens = decode_meta.host_seq_lens
+            decode_meta._decode_balanced = bool(
+                host_lens is not None and len(host_lens) >= n and
+                ops.plan_decode_split(n, self.num_kv_heads, decode_meta.max_decode_seq_len or max(host_lens[:n]),
+                                      window_left, host_lens[:n]))
+        return decode_meta._decode_balanced
 
     # -- multi-query forms: every query token becomes one row of the single-query kernel ----
     @staticmethod

@@ -60,6 +60,20 @@ def _workspace(dev: torch.device, nbytes: int, counters: bool = False) -> Option
     return ws
 
 
+def _stream_and_workspace(t: torch.Tensor):
+    """The stream a call on t's device goes to, and the scratch memory calls on it share (None before the first one)."""
+    dev = t.device
+    stream = N.stream_ptr(dev)
+    return stream, _workspaces.get((dev, stream))
+
+
+def _done(result, what: str):
+    """Result of a function of N.calls(): a status is checked, anything else (a tensor, None: not taken) handed on."""
+    if type(result) is int:
+        N.check(result, what)
+    return result
+
+
 def graph_workspace_ids(device=None):
     """Capture ids that still own split-K workspaces (one id per stream capture that ran a split decode call)."""
     return sorted(c for d, c in _graph_workspaces if device is None or d == torch.device(device))
@@ -86,6 +100,9 @@ def kv_append(key: torch.Tensor, value: torch.Tensor, key_cache: torch.Tensor, v
     """Scatter key/value [T, Hkv, D] into the paged caches [nb, bs, Hkv, D] at slot_mapping [T]
     (int64; negative = skip). Same contract as reshape_and_cache_flash at
     vllm_hymeta/attention/meta_attention.py:790-799 with an unquantised kv_cache_dtype."""
+    if key.is_cuda and _done(N.calls().append(key, value, key_cache, value_cache, slot_mapping, None, None, N.stream_ptr(key.device)),
+                             "kv_append") is not None:
+        return
     dev = N.require_gpu(key, value, key_cache, value_cache, slot_mapping)
     if key.dim() != 3 or value.shape != key.shape:
         raise ValueError(f"key/value must both be [num_tokens, num_kv_heads, head_size], got {tuple(key.shape)} "
@@ -202,6 +219,18 @@ def swa_decode_attention(
     kv_append_int8 wrote them (paged mode, bf16/fp16 queries, append not fused).
     fp8_scales (k_scale, v_scale floats): the caches are fp8 (e4m3fn) codes as kv_append_fp8 wrote them
     (float8_e4m3fn or uint8 tensors), dequantised as code * scale; same restrictions."""
+    if balanced is not None and block_table is not None and out is not None and n_split == 0 and (max_seq_len is None or max_seq_len > 0) and \
+            q.is_cuda and kv_start is None and row_seq is None and key_lo is None and kv_strides is None and meta_k is None and \
+            meta_v is None and profile_events is None and alibi_slopes is None and softcap == 0.0 and phases == 0 and \
+            (k_scale is None) == (v_scale is None) and (k_scale is None or fp8_scales is None) and \
+            not (return_lse or force_valu or merge_in_kernel or per_segment or pipeline_depth):
+        stream, ws = _stream_and_workspace(q)
+        quant = N.SB_KV_FP8 if fp8_scales is not None else N.SB_KV_INT8 if k_scale is not None else N.SB_KV_NONE
+        k8, v8 = (0.0, 0.0) if fp8_scales is None else (fp8_scales[0], fp8_scales[1])
+        if _done(N.calls().decode(q, key_cache, value_cache, out, seq_lens, block_table, new_key, new_value, new_slot_mapping, k_scale,
+                                  v_scale, quant, k8, v8, window_left, q.shape[-1] ** -0.5 if scale is None else scale,
+                                  max_seq_len or 0, balanced, ws, stream), "swa_decode") is not None:
+            return out
     dev = N.require_gpu(q, key_cache, value_cache, seq_lens, block_table, kv_start, row_seq, key_lo, out)
     if q.dim() != 3:
         raise ValueError(f"q must be [rows, num_heads, head_size], got {tuple(q.shape)}")
@@ -357,6 +386,16 @@ def swa_decode_attention(
     return (out, lse) if return_lse else out
 
 
+def paged_decode_step(q: torch.Tensor, key: torch.Tensor, value: torch.Tensor, kv_cache: torch.Tensor, out: torch.Tensor,
+                      slot_mapping: torch.Tensor, seq_lens: torch.Tensor, block_table: torch.Tensor, window_left: int, scale: float,
+                      max_seq_len: int, balanced: bool) -> bool:
+    """swa_decode_attention with its append over a cache [2, num_blocks, block_size, Hkv, D] of q's type; False where the tensors are
+    not of that form (nothing is enqueued then). max_seq_len 0: bounded by the table."""
+    stream, ws = _stream_and_workspace(q)
+    return _done(N.calls().decode(q, kv_cache, None, out, seq_lens, block_table, key, value, slot_mapping, None, None, N.SB_KV_NONE, 0.0, 0.0,
+                                  window_left, scale, max_seq_len, balanced, ws, stream), "swa_decode") is not None
+
+
 def _slopes(alibi_slopes, num_q_heads: int, device) -> Optional[torch.Tensor]:
     """ALiBi slopes as the kernels read them: fp32 [Hq], contiguous, on the queries' device."""
     if alibi_slopes is None:
@@ -396,6 +435,10 @@ def kv_append_int8(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor
                    k_scale: torch.Tensor, v_scale: torch.Tensor, slot_mapping: torch.Tensor) -> None:
     """Quantise this step's K/V rows (per row: 128 signed bytes + one fp32 scale) and store them at
     their slots; slots < 0 are skipped. Caches int8 [nb, bs, Hkv, 128], scales fp32 [nb, Hkv, bs]."""
+    if key.is_cuda and k_scale is not None and v_scale is not None and \
+            _done(N.calls().append(key, value, k_cache, v_cache, slot_mapping, k_scale, v_scale, N.stream_ptr(key.device)),
+                  "kv_append_int8") is not None:
+        return
     dev = N.require_gpu(key, value, k_cache, v_cache, k_scale, v_scale, slot_mapping)
     if key.dim() != 3 or value.shape != key.shape or value.dtype != key.dtype:
         raise ValueError("key and value must be [tokens, num_kv_heads, head_size] of one dtype")
@@ -479,6 +522,11 @@ def fp8_round(x: torch.Tensor, scale: float = 1.0, out: Optional[torch.Tensor] =
 def fp8_step(append: Optional[tuple], rounds) -> list:
     """The append (arguments of kv_append_fp8, or None) and the fp8 round trip of up to three contiguous tensors,
     rounds = [(x, scale), ...], in one launch where all are of one dtype; returns the rounded tensors."""
+    if len(rounds) == 1 and rounds[0][0].is_cuda:
+        x, scale = rounds[0]
+        out = _done(N.calls().append_fp8(*(append or (None, None, None, None, None, 1.0, 1.0)), x, scale, N.stream_ptr(x.device)), "fp8_step")
+        if out is not None:
+            return [out]
     a = None if append is None else _append_fp8_args(*append)
     outs = []
     jobs = (N.Fp8RoundArgs * max(1, len(rounds)))()
@@ -637,6 +685,16 @@ def swa_prefill_attention(
     kv_append_int8 / kv_append_fp8 wrote them; rows are dequantised on their way into the kernel.
     n_parts: cut the keys of a tile into up to this many parts that run side by side (0 = chosen by the library, 1 =
     not at all)."""
+    if plan is not None and out is not None and n_parts == 0 and q.is_cuda and not return_lse and key_lo is None and kv_strides is None and \
+            num_kv_heads is None and k_scale is None and v_scale is None and fp8_scales is None and meta_k is None and meta_v is None and \
+            softcap == 0.0 and alibi_slopes is None and (block_table is None or kv_start is None and kv_start32 is None):
+        tile_keys, ordered_seq, ordered_q0 = plan.list_ptrs()
+        starts = plan.cu_seqlens_q if block_table is None and kv_start is None and kv_start32 is None else kv_start32
+        if _done(N.calls().prefill(q, k, v, out, plan.cu_seqlens_q, plan.seq_lens_k, plan.tile_seq, plan.tile_q0, block_table, kv_start, starts,
+                                   plan.num_tiles, plan.num_seqs, plan.total_q, plan.total_k, plan.max_k, tile_keys or 0, ordered_seq or 0,
+                                   ordered_q0 or 0, window_left, q.shape[-1] ** -0.5 if scale is None else scale, N.stream_ptr(q.device)),
+                 "swa_prefill") is not None:
+            return out
     dev = N.require_gpu(q, k, v, block_table, kv_start, kv_start32, key_lo, out, k_scale, v_scale)
     kv_quant = N.SB_KV_NONE
     if fp8_scales is not None:
@@ -892,6 +950,13 @@ def gla_recurrent(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
     return out
 
 
+def gla_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor, state: torch.Tensor, slot_idx: Optional[torch.Tensor],
+             scale: float) -> Optional[torch.Tensor]:
+    """gla_recurrent for one step, zero_skipped: out [B, H, D], or None where the tensors are not of the ordinary form (nothing is
+    enqueued then)."""
+    return _done(N.calls().gla_step(q, k, v, g, state, slot_idx, scale, N.stream_ptr(q.device)), "gla_recurrent") if q.is_cuda else None
+
+
 def _launch_gla(a, dev: torch.device, total: int = 0) -> None:
     """Enqueue the recurrence; long prompts of a few sequences are cut into segments that run side by side, with
     scratch memory from torch's allocator (stream-ordered, and part of the graph under capture). total: the tokens of
@@ -931,6 +996,13 @@ def gla_recurrent_packed(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: t
     max_seq_len, an upper bound of their lengths, says (default: by the mean length, which some sequence reaches: eight
     prompts of 100 tokens are not cut like one of 800, of whose segments the first would hold all there is). Returns o [total_tokens, H, D]. Shared states as in gla_recurrent: k, v, g
     [total_tokens, Hkv, D] with state [slots, Hkv, D, D]."""
+    if out is None and per_head is None and q.is_cuda and not (vector_only or check_gates):
+        a = N.GlaRecurrentArgs()
+        o = N.calls().gla_packed(C.addressof(a), q, k, v, g, state, cu_seqlens, slot_idx, q.shape[-1] ** -0.5 if scale is None else scale,
+                                 max_seq_len or 0, N.stream_ptr(q.device))
+        if o is not None:
+            _launch_gla(a, q.device, 0 if max_seq_len or a.batch == 1 else q.shape[0])
+            return o
     dev = N.require_gpu(q, k, v, g, state, cu_seqlens, slot_idx, out)
     if q.dim() != 3 or k.dim() != 3 or v.shape != k.shape or g.shape != k.shape or \
             (k.shape[0], k.shape[2]) != (q.shape[0], q.shape[2]):
@@ -1041,6 +1113,9 @@ def window_shift(src: Optional[torch.Tensor], dst: torch.Tensor, fresh: Optional
 def window_shift_pair(k: tuple, v: tuple) -> None:
     """window_shift for a layer's K and V, each (src, dst, fresh, keep_rows, src_row0, dst_row0): one launch where both
     move the same rows of the same strides."""
+    if k[0] is None and v[0] is None and k[1].is_cuda and k[3] == v[3] == 0 and k[5] == v[5] and \
+            _done(N.calls().push(k[1], v[1], k[2], v[2], k[5], N.stream_ptr(k[1].device)), "window_shift") is not None:
+        return
     ak, _k = _window_shift_args(*k)
     av, _v = _window_shift_args(*v)
     N.check(N.lib().sb_window_shift_pair(C.byref(ak), C.byref(av)), "window_shift")
@@ -1072,6 +1147,14 @@ def dense_rows(batch: int, num_queries: int, num_keys: int, kv_step: int, device
         mask_elem_bytes=1 if mask is None else mask.element_size(), stream=N.stream_ptr(device))
     N.check(N.lib().sb_dense_rows(C.byref(a)), "dense_rows")
     return seq_lens, row_seq, None if mask is None else key_lo, kv_start
+
+
+def dense_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: Optional[torch.Tensor], window_left: int,
+                 scale: float) -> Optional[torch.Tensor]:
+    """dense_rows and swa_decode_attention for one new token of each sequence, q [B, Hq, 1, D] over k, v [B, Hkv, K, D], mask
+    [B, n] whose last K columns count: out [B, 1, Hq, D], or None where the tensors are not of that form (nothing is enqueued then)."""
+    stream, ws = _stream_and_workspace(q)
+    return _done(N.calls().dense_decode(q, k, v, mask, window_left, scale, ws, stream), "swa_decode")
 
 
 def window_advance(n_tokens: torch.Tensor, lo: torch.Tensor, hi: torch.Tensor, ring: torch.Tensor,

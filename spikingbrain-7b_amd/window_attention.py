@@ -87,6 +87,10 @@ def sliding_window_attention(
     if window_left is None:
         window_left = sliding_window if flavour == "flash" else sliding_window - 1
 
+    if Q == 1 and query_states.is_cuda:
+        out = ops.dense_decode(query_states, key_states, value_states, attention_mask, window_left, D ** -0.5)
+        if out is not None:
+            return out
     k, v = key_states, value_states
     if k.stride(3) != 1 or v.stride() != k.stride() or _kv_step_rows(k) is None:
         k, v = k.contiguous(), v.contiguous()
