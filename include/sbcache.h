@@ -185,7 +185,7 @@ typedef struct sb_swa_decode_args {
   /* Per-row INT8 cache (kv_quant = SB_KV_INT8): k_cache/v_cache hold int8 codes
    * [num_blocks, block_size, Hkv, 128] (kv strides in bytes), k_scale/v_scale the fp32 scales
    * [num_blocks, Hkv, block_size] that sb_kv_append_int8 wrote. Paged mode, q/out bf16 or fp16, fixed
-   * split; the append is not fused (new_key etc. must be NULL: quantise and append first). */
+   * split; new_key etc. must be NULL here (quantise and append first, or sb_swa_decode_append_codes). */
   const float *k_scale;
   const float *v_scale;
   int32_t kv_quant;
@@ -257,6 +257,13 @@ int32_t sb_swa_decode_prefer_balanced(const int32_t *host_seq_lens, int64_t num_
 size_t sb_swa_decode_workspace_bytes(int64_t num_rows, int32_t num_q_heads, int32_t head_size,
                                      int32_t n_split);
 int sb_swa_decode(const sb_swa_decode_args *args);
+
+/* The same over a byte-code cache (kv_quant INT8 or FP8) with the append in the launch: row r's newest key is new_key[r] /
+ * new_value[r] (of dtype), which the call quantises and stores at new_slot_mapping[r] as sb_kv_append_int8 / sb_kv_append_fp8
+ * (with k_scale_tensor / v_scale_tensor) do, and attends to those codes: the bits of that call followed by sb_swa_decode.
+ * A slot < 0 stores nothing and attends to what the cache holds. q_scale > 0 (fp8 only): the queries are first taken through
+ * sb_fp8_round with it. Paged mode, phases 0, no meta tokens, no key_lo. */
+int sb_swa_decode_append_codes(const sb_swa_decode_args *a, float q_scale);
 
 /* ------------------------------------------------------------------------------------
  * sb_swa_decode without any workspace from the caller and without any allocation.

@@ -193,6 +193,7 @@ EXPORTS = {
     "sb_swa_decode_workspace_bytes": (sz, [i64, i32, i32, i32]),
     "sb_swa_decode_prefer_balanced": (i32, [C.POINTER(i32), i64, i32, i32]),
     "sb_swa_decode": (C.c_int, [C.POINTER(SwaDecodeArgs)]),
+    "sb_swa_decode_append_codes": (C.c_int, [C.POINTER(SwaDecodeArgs), C.c_float]),
     "sb_swa_decode_static": (C.c_int, [C.POINTER(SwaDecodeArgs)]),
     "sb_gla_recurrent": (C.c_int, [C.POINTER(GlaRecurrentArgs)]),
     "sb_gla_prompt_segments": (i32, [C.POINTER(GlaRecurrentArgs)]),

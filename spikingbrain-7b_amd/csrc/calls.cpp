@@ -96,6 +96,20 @@ struct Pages {
   }
 };
 
+// The scales of an INT8 cache: two tensors [blocks, heads, block size], or both in one [2, ...]
+bool both_scales(const Tensor *ks, const Tensor *vs, const Pages &c, const float *&k, const float *&v) {
+  if (!vs) {
+    if (!ks || ks->scalar_type() != at::kFloat || !shaped(*ks, {2, c.nb, c.heads, c.bs}) || !ks->is_contiguous()) return false;
+    k = ks->data_ptr<float>();
+    v = k + c.nb * c.heads * c.bs;
+    return true;
+  }
+  if (!scales_of(ks, c.nb, c.heads, c.bs) || !scales_of(vs, c.nb, c.heads, c.bs)) return false;
+  k = ks->data_ptr<float>();
+  v = vs->data_ptr<float>();
+  return true;
+}
+
 // Whether `ws` can hold this split's partial results, outside a stream capture (a capture's scratch memory belongs to its graph)
 bool workspace_fits(const Tensor *ws, size_t bytes, void *stream) {
   if (bytes == 0) return true;
@@ -117,13 +131,13 @@ PyObject *call(PyObject *, PyObject *const *a, Py_ssize_t n) {
 }
 
 // decode(q, k_cache, v_cache | None, out, seq_lens, block_table, new_key | None, new_value | None, slots | None, k_scale | None,
-// v_scale | None, kv_quant, k_scale_tensor, v_scale_tensor, window_left, scale, max_seq_len (0: the table's), balanced, workspace | None,
-// stream): ops.swa_decode_attention over a paged cache, one query row per sequence.
+// v_scale | None, kv_quant, k_scale_tensor, v_scale_tensor, q_scale (>= 0: the append over a byte-code cache; -1: none), window_left, scale,
+// max_seq_len (0: the table's), balanced, workspace | None, stream): ops.swa_decode_attention over a paged cache, one query row per sequence.
 PyObject *decode(Args &in) {
   const Tensor *q = in.tensor(), *kc = in.tensor(), *vc = in.maybe_tensor(), *out = in.tensor(), *lens = in.tensor(), *table = in.tensor();
   const Tensor *nk = in.maybe_tensor(), *nv = in.maybe_tensor(), *slots = in.maybe_tensor(), *ks = in.maybe_tensor(), *vs = in.maybe_tensor();
   const int64_t quant = in.integer();
-  const double kst = in.number(), vst = in.number();
+  const double kst = in.number(), vst = in.number(), q_scale = in.number();
   const int64_t window = in.integer();
   const double scale = in.number();
   int64_t longest = in.integer();
@@ -133,18 +147,21 @@ PyObject *decode(Args &in) {
   Pages c;
   if (!in.ok || q->dim() != 3 || !half_type(*q) || !inner_contiguous(*q) || !c.from(kc, vc)) return not_taken();
   const int64_t R = q->size(0), Hq = q->size(1), D = q->size(2);
+  const float *k_scale = nullptr, *v_scale = nullptr;
   if (D != 128 || c.dim != D || c.nb < 1 || c.bs < 1 || c.heads <= 0 || Hq % c.heads != 0 || Hq > 16 * c.heads || R < 1 || R > INT32_MAX || window < -1 || window > INT32_MAX)
     return not_taken();
   if (quant == SB_KV_NONE ? c.type != q->scalar_type()
-                          : quant == SB_KV_INT8 ? c.type != at::kChar || !scales_of(ks, c.nb, c.heads, c.bs) || !scales_of(vs, c.nb, c.heads, c.bs)
+                          : quant == SB_KV_INT8 ? c.type != at::kChar || !both_scales(ks, vs, c, k_scale, v_scale)
                                                 : quant != SB_KV_FP8 || (c.type != at::kByte && c.type != at::kFloat8_e4m3fn))
     return not_taken();
   if (out->sizes() != q->sizes() || out->scalar_type() != q->scalar_type() || !inner_contiguous(*out) || !vector_of(*lens, at::kInt, R) ||
       table->scalar_type() != at::kInt || table->dim() != 2 || table->stride(1) != 1)
     return not_taken();
   if (!nk && (nv || slots)) return not_taken();
-  if (nk && (quant != SB_KV_NONE || !nv || !slots || nk->dim() != 3 || nk->size(0) != R || nk->size(1) != c.heads || nk->size(2) != D ||
-             nv->sizes() != nk->sizes() || nk->scalar_type() != c.type || nv->scalar_type() != c.type || !inner_contiguous(*nk) ||
+  const bool codes = quant != SB_KV_NONE;
+  if (codes ? (q_scale >= 0.0) != (nk != nullptr) : q_scale >= 0.0) return not_taken();
+  if (nk && (!nv || !slots || nk->dim() != 3 || nk->size(0) != R || nk->size(1) != c.heads || nk->size(2) != D ||
+             nv->sizes() != nk->sizes() || nk->scalar_type() != q->scalar_type() || nv->scalar_type() != q->scalar_type() || !inner_contiguous(*nk) ||
              !inner_contiguous(*nv) || !vector_of(*slots, at::kLong, R)))
     return not_taken();
   if (longest <= 0) longest = table->size(1) * c.bs;
@@ -174,9 +191,9 @@ PyObject *decode(Args &in) {
   }
   a.stream = stream;
   a.kv_quant = (int)quant;
-  if (quant == SB_KV_INT8) { a.k_scale = ks->data_ptr<float>(); a.v_scale = vs->data_ptr<float>(); }
+  a.k_scale = k_scale; a.v_scale = v_scale;
   if (quant == SB_KV_FP8) { a.k_scale_tensor = (float)kst; a.v_scale_tensor = (float)vst; }
-  return status(sb_swa_decode(&a));
+  return status(codes && nk ? sb_swa_decode_append_codes(&a, (float)q_scale) : sb_swa_decode(&a));
 }
 
 // append(key, value, k_cache, v_cache, slots, k_scale | None, v_scale | None, stream): ops.kv_append, or ops.kv_append_int8 with scales

@@ -7,11 +7,11 @@
 //
 // One wavefront quantises the rows of one (token, K|V) for up to 4 heads: 16 lanes per head, 8
 // values per lane; max|x| of a head is four xor-exchanges inside its 16 lanes.
-#include "common.h"
+#include "kv_codes.h"
 
 namespace {
 
-constexpr float kScaleMin = 1e-5f, kScaleMax = 1e4f;
+using namespace sb;
 
 template <int DT>
 __device__ __forceinline__ void load8(const char *p, float (&x)[8]) {
@@ -20,20 +20,7 @@ __device__ __forceinline__ void load8(const char *p, float (&x)[8]) {
     x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
     x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
   } else {
-    const uint4 w = *reinterpret_cast<const uint4 *>(p);
-    const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if constexpr (DT == SB_BF16) {
-        x[2 * i] = sb::bf16_lo(ws[i]);
-        x[2 * i + 1] = sb::bf16_hi(ws[i]);
-      } else {
-        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-        const h2 h = __builtin_bit_cast(h2, ws[i]);
-        x[2 * i] = (float)h.x;
-        x[2 * i + 1] = (float)h.y;
-      }
-    }
+    unpack8<DT>(*reinterpret_cast<const uint4 *>(p), x);
   }
 }
 
@@ -42,31 +29,18 @@ __device__ __forceinline__ void store8(char *p, const float (&x)[8]) {
   if constexpr (DT == SB_F32) {
     reinterpret_cast<float4 *>(p)[0] = make_float4(x[0], x[1], x[2], x[3]);
     reinterpret_cast<float4 *>(p)[1] = make_float4(x[4], x[5], x[6], x[7]);
-  } else if constexpr (DT == SB_BF16) {
-    *reinterpret_cast<uint4 *>(p) = make_uint4(sb::pack_bf16(x[0], x[1]), sb::pack_bf16(x[2], x[3]),
-                                               sb::pack_bf16(x[4], x[5]), sb::pack_bf16(x[6], x[7]));
   } else {
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    uint32_t w[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const h2 h = {(_Float16)x[2 * i], (_Float16)x[2 * i + 1]};
-      w[i] = __builtin_bit_cast(uint32_t, h);
-    }
-    *reinterpret_cast<uint4 *>(p) = make_uint4(w[0], w[1], w[2], w[3]);
+    *reinterpret_cast<uint4 *>(p) = pack8<DT>(x);
   }
 }
 
 // scale of the 128-value row this lane's 16-lane group holds, and this lane's 8 codes (as floats)
 __device__ __forceinline__ float quantise_row(const float (&x)[8], float (&code)[8]) {
-  float amax = 0.f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(x[i]));
+  float amax = max_abs8(x, 0.f);
 #pragma unroll
   for (int d = 1; d < 16; d <<= 1) amax = fmaxf(amax, __shfl_xor(amax, d));
-  const float scale = fminf(fmaxf(amax / 127.f, kScaleMin), kScaleMax);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) code[i] = fminf(fmaxf(rintf(x[i] / scale), -128.f), 127.f);
+  const float scale = int8_scale(amax);
+  int8_codes(x, scale, code);
   return scale;
 }
 
@@ -98,14 +72,8 @@ __global__ __launch_bounds__(256) void kv_append_int8_kernel(
   }
   const float scale = quantise_row(x, code);
   if (!live) return;
-  uint32_t lo = 0, hi = 0;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    lo |= ((uint32_t)(int)code[i] & 0xffu) << (8 * i);
-    hi |= ((uint32_t)(int)code[4 + i] & 0xffu) << (8 * i);
-  }
   char *dst = (which ? v_cache : k_cache) + blk * blk_b + off * row_b + h * head_b + piece * 8;
-  *reinterpret_cast<uint2 *>(dst) = make_uint2(lo, hi);
+  *reinterpret_cast<uint2 *>(dst) = int8_bytes(code);
   if (piece == 0) (which ? v_scale : k_scale)[(blk * num_kv_heads + h) * block_size + off] = scale;
 }
 
@@ -128,19 +96,6 @@ __global__ __launch_bounds__(256) void quantize_sym_kernel(const char *__restric
 #pragma unroll
   for (int i = 0; i < 8; ++i) code[i] *= scale;
   store8<DT>(out + wave * out_row_b + h * out_head_b + piece * 8 * kEsz, code);
-}
-
-// ---- fp8 (OCP e4m3fn) K/V with per-tensor scales ---------------------------------------------------
-// code = e4m3fn(clamp(x / scale, -448, 448)), round to nearest even: what the kv_cache_dtype="fp8"
-// branch of reshape_and_cache_flash stores (vllm_hymeta/attention/meta_attention.py:790-799 with
-// layer._k_scale / layer._v_scale). gfx950's v_cvt_pk_fp8_f32 is that rounding; it does not saturate,
-// hence the clamp. NaN stays NaN.
-__device__ __forceinline__ uint32_t to_fp8x4(float a, float b, float c, float d, float s) {
-  auto q = [&](float x) { return fminf(fmaxf(x / s, -448.f), 448.f); };  // fminf/fmaxf would drop a NaN: kept below
-  const float qa = a != a ? a : q(a), qb = b != b ? b : q(b), qc = c != c ? c : q(c), qd = d != d ? d : q(d);
-  int r = __builtin_amdgcn_cvt_pk_fp8_f32(qa, qb, 0, false);
-  r = __builtin_amdgcn_cvt_pk_fp8_f32(qc, qd, r, true);
-  return (uint32_t)r;
 }
 
 struct Fp8Append {
@@ -169,11 +124,11 @@ __device__ __forceinline__ void append_fp8(const Fp8Append &p, int64_t tok, int 
   load8<DT>(src + piece * 8 * kEsz, x);
   const float sc = which ? p.v_scale : p.k_scale;
   char *dst = (which ? p.v_cache : p.k_cache) + blk * p.blk_b + off * p.row_b + h * p.head_b + piece * 8;
-  *reinterpret_cast<uint2 *>(dst) = make_uint2(to_fp8x4(x[0], x[1], x[2], x[3], sc), to_fp8x4(x[4], x[5], x[6], x[7], sc));
+  *reinterpret_cast<uint2 *>(dst) = fp8_bytes(x, sc);
 }
 
-// The append alone (a captured decode step of 28 layers over an fp8 cache: through the kernel below, with its 300 bytes of
-// arguments, the step took 319 instead of 315 us).
+// The append alone (28 of them in a captured step: through the kernel below, with its 300 bytes of arguments, the step took 319 instead
+// of 315 us).
 template <int DT>
 __global__ __launch_bounds__(256) void kv_append_fp8_kernel(const Fp8Append p) {
   const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -199,11 +154,8 @@ __device__ __forceinline__ void round_fp8(const Fp8Round &p, int64_t t) {  // t:
   const float scale = p.scale;
   float x[8];
   load8<DT>(p.in + r * p.in_row_b + vec * 8 * kEsz, x);
-  const uint32_t lo = to_fp8x4(x[0], x[1], x[2], x[3], scale), hi = to_fp8x4(x[4], x[5], x[6], x[7], scale);
-  const float y[8] = {__builtin_amdgcn_cvt_f32_fp8((int)lo, 0) * scale, __builtin_amdgcn_cvt_f32_fp8((int)lo, 1) * scale,
-                      __builtin_amdgcn_cvt_f32_fp8((int)lo, 2) * scale, __builtin_amdgcn_cvt_f32_fp8((int)lo, 3) * scale,
-                      __builtin_amdgcn_cvt_f32_fp8((int)hi, 0) * scale, __builtin_amdgcn_cvt_f32_fp8((int)hi, 1) * scale,
-                      __builtin_amdgcn_cvt_f32_fp8((int)hi, 2) * scale, __builtin_amdgcn_cvt_f32_fp8((int)hi, 3) * scale};
+  float y[8];
+  fp8_values(fp8_bytes(x, scale), scale, y);
   store8<DT>(p.out + r * p.out_row_b + vec * 8 * kEsz, y);
 }
 

@@ -921,7 +921,9 @@ extern "C" size_t sb_swa_decode_workspace_bytes(int64_t num_rows, int32_t num_q_
                   round_up(num_rows * 2 * 4, 256));  // ... + per row the span of runs holding its partials (balanced split)
 }
 
-extern "C" int sb_swa_decode(const sb_swa_decode_args *a) {
+// append_codes: the step's rows are quantised and stored by this launch too (byte-code caches); q_scale > 0: over an fp8 cache the
+// queries take their round trip in it as well.
+static int swa_decode(const sb_swa_decode_args *a, bool append_codes, float q_scale) {
   using namespace sb_host;
   if (!a) return fail(SB_ERR_INVALID, "sb_swa_decode: null args");
   if (a->num_rows < 0) return fail(SB_ERR_INVALID, "sb_swa_decode: negative num_rows");
@@ -960,7 +962,7 @@ extern "C" int sb_swa_decode(const sb_swa_decode_args *a) {
       return fail(SB_ERR_UNSUPPORTED, "sb_swa_decode: the INT8 cache needs bf16 or fp16 queries on the matrix-core path");
     if (!a->block_table || (!fp8_kv && (!a->k_scale || !a->v_scale)))
       return fail(SB_ERR_INVALID, "sb_swa_decode: the INT8 cache needs paged mode and both scale tensors");
-    if (a->new_key || a->new_value || a->new_slot_mapping)
+    if (!append_codes && (a->new_key || a->new_value || a->new_slot_mapping))
       return fail(SB_ERR_UNSUPPORTED, "sb_swa_decode: no fused append into the INT8 cache (call sb_kv_append_int8 first)");
     if (!fp8_kv && ((reinterpret_cast<uintptr_t>(a->k_scale) | reinterpret_cast<uintptr_t>(a->v_scale)) & 15u))
       return fail(SB_ERR_INVALID, "sb_swa_decode: scale tensors not 16-byte aligned");
@@ -1020,6 +1022,8 @@ extern "C" int sb_swa_decode(const sb_swa_decode_args *a) {
     p.kv_out_scale = a->v_scale_tensor;
   }
 
+  p.nk_scale = a->k_scale_tensor; p.nv_scale = a->v_scale_tensor;
+  p.q_round = q_scale;
   const int G = a->num_q_heads / a->num_kv_heads;
   const dim3 grid((unsigned)a->num_rows, (unsigned)a->num_kv_heads, (unsigned)n_split);
   hipStream_t st = (hipStream_t)a->stream;
@@ -1173,6 +1177,22 @@ extern "C" int sb_swa_decode(const sb_swa_decode_args *a) {
   else if (a->dtype == SB_F16) launch_merge<F16>(mgrid, mblock, st, p);
   else launch_merge<F32>(mgrid, mblock, st, p);
   return check_launch("swa_decode_merge_kernel");
+}
+
+extern "C" int sb_swa_decode(const sb_swa_decode_args *a) { return swa_decode(a, false, 0.f); }
+
+extern "C" int sb_swa_decode_append_codes(const sb_swa_decode_args *a, float q_scale) {
+  using namespace sb_host;
+  if (!a) return fail(SB_ERR_INVALID, "sb_swa_decode_append_codes: null args");
+  if (a->kv_quant != SB_KV_INT8 && a->kv_quant != SB_KV_FP8)
+    return fail(SB_ERR_INVALID, "sb_swa_decode_append_codes: a byte-code cache is needed (sb_swa_decode appends elements)");
+  if (!a->new_key || !a->new_value || !a->new_slot_mapping)
+    return fail(SB_ERR_INVALID, "sb_swa_decode_append_codes: new_key, new_value and new_slot_mapping are needed");
+  if (a->phases != 0 || a->meta_len > 0 || a->key_lo)
+    return fail(SB_ERR_UNSUPPORTED, "sb_swa_decode_append_codes: both phases, no meta tokens, no key_lo");
+  if (!(q_scale >= 0.f) || (q_scale > 0.f && a->kv_quant != SB_KV_FP8))
+    return fail(SB_ERR_INVALID, "sb_swa_decode_append_codes: q_scale must be 0, or positive over an fp8 cache");
+  return swa_decode(a, true, q_scale);
 }
 
 // ---- sb_swa_decode_static: the same call, partial results in memory the library itself holds ------

@@ -45,11 +45,13 @@ struct DecodeParams {
   int64_t q_sr, q_sh, o_sr, o_sh;  // elements
   int64_t kv_sb, kv_sr, kv_sh;     // bytes
   int64_t bt_stride;
-  // fused append (matrix-core kernel only): this step's key/value rows and their cache slots
+  // fused append (matrix-core kernels only): this step's key/value rows and their cache slots
   const char *new_k;
   const char *new_v;
   const int64_t *slot_mapping;
   int64_t nk_st, nk_sh, nv_st, nv_sh;  // bytes
+  float nk_scale, nv_scale;  // fp8 cache: what the new rows are divided by
+  float q_round;             // fp8 cache with append: > 0 = the queries take the fp8 round trip with this scale
   // INT8 cache: per-row scales [num_blocks, Hkv, block_size]
   const float *k_scale;
   const float *v_scale;

@@ -220,21 +220,23 @@ class HybridDecodeCache:
 
     def swa_layer(self, layer_idx: int, q, k, v, meta: MetaAttentionMetadata, out) -> torch.Tensor:
         """q [B, Hq, D], k/v [B, Hkv, D]: append + window attention for one SWA layer."""
-        if self.kv_quant == "int8":
-            codes, scales = self.kv_caches[layer_idx // 2], self.kv_scales[layer_idx // 2]
-            n = q.shape[0]
-            ops.kv_append_int8(k, v, codes[0], codes[1], scales[0], scales[1], _rows_of(_flat(meta.slot_mapping), 0, n))
-            return ops.swa_decode_attention(
-                q, codes[0], codes[1], _rows_of(meta.seq_lens_tensor, 0, n), block_table=meta.block_tables, window_left=self.wl,
-                scale=self.D ** -0.5, out=out, max_seq_len=meta.max_decode_seq_len or None,
-                k_scale=scales[0], v_scale=scales[1])
-        if self.kv_quant == "fp8":
+        if self.kv_quant:
             codes = self.kv_caches[layer_idx // 2]
             n = q.shape[0]
-            ops.kv_append_fp8(k, v, codes[0], codes[1], _rows_of(_flat(meta.slot_mapping), 0, n), 1.0, 1.0)
+            how = dict(fp8_scales=(1.0, 1.0))
+            if self.kv_quant == "int8":
+                scales = self.kv_scales[layer_idx // 2]
+                how = dict(k_scale=scales[0], v_scale=scales[1])
+            slots = _rows_of(_flat(meta.slot_mapping), 0, n)
+            if k.dtype == v.dtype == q.dtype and k.shape[0] == n:
+                how.update(new_key=k, new_value=v, new_slot_mapping=slots.contiguous(), append_codes=0.0)
+            elif self.kv_quant == "int8":
+                ops.kv_append_int8(k, v, codes[0], codes[1], scales[0], scales[1], slots)
+            else:
+                ops.kv_append_fp8(k, v, codes[0], codes[1], slots, 1.0, 1.0)
             return ops.swa_decode_attention(
                 q, codes[0], codes[1], _rows_of(meta.seq_lens_tensor, 0, n), block_table=meta.block_tables, window_left=self.wl,
-                scale=self.D ** -0.5, out=out, max_seq_len=meta.max_decode_seq_len or None, fp8_scales=(1.0, 1.0))
+                scale=self.D ** -0.5, out=out, max_seq_len=meta.max_decode_seq_len or None, balanced=False, **how)
         return self.impl.forward(self._layer, q, k, v, None, None, None, self.kv_caches[layer_idx // 2], meta, out)
 
     def bytes_per_step(self) -> int:

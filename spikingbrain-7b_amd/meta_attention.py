@@ -526,6 +526,14 @@ class MetaAttentionImpl:
         # its slot. Every other step appends first, exactly as the reference does (:790-799).
         int8_kv = isinstance(kv_cache, Int8KVCache)
         scales = dict(k_scale=kv_cache.scales[0], v_scale=kv_cache.scales[1]) if int8_kv else {}
+        # the same over a byte-code cache: the launch quantises the newest row (and rounds fp8 queries) as well
+        fuse_codes = False
+        if int8_kv or fp8_kv:
+            fuse_codes = (kv_cache.numel() > 0 and key is not None and value is not None and not with_meta
+                          and attn_metadata.num_prefill_tokens == 0 and attn_metadata.num_decode_tokens == query.shape[0] == key.shape[0] > 0
+                          and (attn_metadata.max_decode_query_len or 1) == 1 and attn_metadata.slot_mapping is not None
+                          and query.dtype in (torch.bfloat16, torch.float16) and key.dtype == value.dtype == query.dtype
+                          and (query.is_contiguous() or not fp8_kv))
         if fp8_kv:
             if int8_kv:
                 raise ValueError("kv_cache_dtype says fp8 but the cache is an Int8KVCache")
@@ -544,7 +552,9 @@ class MetaAttentionImpl:
             key_cache, value_cache = (kv_cache.codes[0], kv_cache.codes[1]) if int8_kv else (kv_cache[0], kv_cache[1])
             if fp8_kv and key_cache.dtype not in (torch.uint8, torch.float8_e4m3fn):
                 raise ValueError(f"an fp8 kv-cache must be a uint8 or float8_e4m3fn tensor, got {key_cache.dtype}")
-            if key is not None and value is not None and fp8_kv:
+            if fuse_codes:
+                pass
+            elif key is not None and value is not None and fp8_kv:
                 append = (key, value, key_cache, value_cache, _flat(attn_metadata.slot_mapping), k_scale_f, v_scale_f)
             elif key is not None and value is not None and int8_kv:
                 # rows are quantised on their way in: 128 code bytes + one scale per (token, kv head)
@@ -556,7 +566,7 @@ class MetaAttentionImpl:
 
         num_prefill_query_tokens = attn_metadata.num_prefill_tokens
         num_decode_query_tokens = attn_metadata.num_decode_tokens
-        if fp8_kv:
+        if fp8_kv and not fuse_codes:
             prompts = attn_metadata.prefill_metadata
             if prompts and key is not None and _in_flight(kv_cache, prompts):
                 rounds += [(_rows_of(key, 0, num_prefill_query_tokens).contiguous(), k_scale_f),
@@ -636,8 +646,10 @@ class MetaAttentionImpl:
                 # by this very launch when the step is a pure decode step
                 n = decode_query.shape[0]
                 fused = {}
-                if fuse_append:
-                    fused = dict(new_key=_rows_of(key, 0, n), new_value=_rows_of(value, 0, n),
+                if fuse_codes:
+                    fused = dict(append_codes=float(getattr(layer, "_q_scale_float", 1.0)) if fp8_kv else 0.0)
+                if fuse_append or fuse_codes:
+                    fused.update(new_key=_rows_of(key, 0, n), new_value=_rows_of(value, 0, n),
                                  new_slot_mapping=_rows_of(_flat(decode_meta.slot_mapping), 0, n).contiguous())
                 balanced = self._balanced(decode_meta, n, window_left)
                 ops.swa_decode_attention(
@@ -648,21 +660,31 @@ class MetaAttentionImpl:
         return output
 
     def _pure_decode(self, layer, query, key, value, kv_cache, meta, output) -> bool:
-        """The layer call of a step of decoding sequences only (one token each, element caches, no score options) in one
-        native step; False, with nothing done, for any other."""
+        """The layer call of a step of decoding sequences only (one token each, no score options) in one native step; False, with
+        nothing done, for any other."""
         n = meta.num_decode_tokens
         if meta.num_prefill_tokens or meta.num_prefills or n <= 0 or (meta.max_decode_query_len or 1) != 1 or meta.slot_mapping is None or \
                 key is None or value is None or self.attn_type != AttentionType.DECODER or self.alibi_slopes is not None or \
-                self.logits_soft_cap > 0 or self.kv_cache_dtype.startswith("fp8") or type(kv_cache) is not torch.Tensor or \
-                not query.is_cuda or query.shape != (n, self.num_heads, self.head_size) or \
-                getattr(layer, "_k_scale_float", 1.0) != 1.0 or getattr(layer, "_v_scale_float", 1.0) != 1.0:
+                self.logits_soft_cap > 0 or not query.is_cuda or query.shape != (n, self.num_heads, self.head_size):
+            return False
+        k_scale, v_scale = float(getattr(layer, "_k_scale_float", 1.0)), float(getattr(layer, "_v_scale_float", 1.0))
+        codes, how = kv_cache, ()
+        if self.kv_cache_dtype.startswith("fp8"):
+            if type(kv_cache) is not torch.Tensor or not query.is_contiguous():
+                return False
+            how = (ops.N.SB_KV_FP8, None, k_scale, v_scale, float(getattr(layer, "_q_scale_float", 1.0)))
+        elif k_scale != 1.0 or v_scale != 1.0:
+            return False
+        elif type(kv_cache) is Int8KVCache:
+            codes, how = kv_cache.codes, (ops.N.SB_KV_INT8, kv_cache.scales, 0.0, 0.0, 0.0)
+        elif type(kv_cache) is not torch.Tensor:
             return False
         meta = meta.decode_metadata
         if meta.max_decode_query_len is None:
             return False
-        return ops.paged_decode_step(query, key, value, kv_cache, output, meta.slot_mapping, meta.seq_lens_tensor, meta.block_tables,
-                                     self.sliding_window[0], self.scale, meta.max_decode_seq_len or 0,
-                                     self._balanced(meta, n, self.sliding_window[0]))
+        window_left = self.sliding_window[0]
+        return ops.paged_decode_step(query, key, value, codes, output, meta.slot_mapping, meta.seq_lens_tensor, meta.block_tables, window_left,
+                                     self.scale, meta.max_decode_seq_len or 0, not how and self._balanced(meta, n, window_left), *how)
 
     def _balanced(self, decode_meta, n: int, window_left: int) -> bool:
         """Split policy of the step's decode launch, decided once for all layers."""

@@ -175,6 +175,7 @@ def swa_decode_attention(
     softcap: float = 0.0,
     alibi_slopes: Optional[torch.Tensor] = None,
     meta_bias: Optional[Tuple[int, int]] = None,
+    append_codes: Optional[float] = None,
 ):
     """Single-query window attention for each row of q [R, Hq, D].
 
@@ -216,9 +217,12 @@ def swa_decode_attention(
     a lot, a little slower when they do not. Default: decided from host_seq_lens (the same numbers
     as seq_lens, as Python ints) when the caller has them, else off.
     k_scale, v_scale (fp32 [num_blocks, Hkv, block_size]): the caches are per-row INT8 codes as
-    kv_append_int8 wrote them (paged mode, bf16/fp16 queries, append not fused).
+    kv_append_int8 wrote them (paged mode, bf16/fp16 queries; the append: see append_codes).
     fp8_scales (k_scale, v_scale floats): the caches are fp8 (e4m3fn) codes as kv_append_fp8 wrote them
-    (float8_e4m3fn or uint8 tensors), dequantised as code * scale; same restrictions."""
+    (float8_e4m3fn or uint8 tensors), dequantised as code * scale; same restrictions.
+    append_codes: the append into a byte-code cache in the same launch: new_key, new_value (elements of q's type) are quantised, stored
+    at new_slot_mapping (negative: not, and the cache's own row counts) and attended to as those codes, the bits of kv_append_int8 /
+    kv_append_fp8 before this call. Its value, positive over an fp8 cache only: q takes fp8_round with that scale first; 0 = not."""
     if balanced is not None and block_table is not None and out is not None and n_split == 0 and (max_seq_len is None or max_seq_len > 0) and \
             q.is_cuda and kv_start is None and row_seq is None and key_lo is None and kv_strides is None and meta_k is None and \
             meta_v is None and profile_events is None and alibi_slopes is None and softcap == 0.0 and phases == 0 and \
@@ -228,7 +232,7 @@ def swa_decode_attention(
         quant = N.SB_KV_FP8 if fp8_scales is not None else N.SB_KV_INT8 if k_scale is not None else N.SB_KV_NONE
         k8, v8 = (0.0, 0.0) if fp8_scales is None else (fp8_scales[0], fp8_scales[1])
         if _done(N.calls().decode(q, key_cache, value_cache, out, seq_lens, block_table, new_key, new_value, new_slot_mapping, k_scale,
-                                  v_scale, quant, k8, v8, window_left, q.shape[-1] ** -0.5 if scale is None else scale,
+                                  v_scale, quant, k8, v8, -1.0 if append_codes is None else append_codes, window_left, q.shape[-1] ** -0.5 if scale is None else scale,
                                   max_seq_len or 0, balanced, ws, stream), "swa_decode") is not None:
             return out
     dev = N.require_gpu(q, key_cache, value_cache, seq_lens, block_table, kv_start, row_seq, key_lo, out)
@@ -254,10 +258,12 @@ def swa_decode_attention(
                 raise ValueError("with k_scale/v_scale the caches must be int8")
         if q.dtype not in (torch.bfloat16, torch.float16) or force_valu:
             raise NotImplementedError("the INT8 cache needs bf16 or fp16 queries on the matrix-core path")
-        if new_key is not None or new_value is not None or new_slot_mapping is not None:
+        if append_codes is None and (new_key is not None or new_value is not None or new_slot_mapping is not None):
             raise NotImplementedError("no fused append into the INT8 cache: call kv_append_int8 first")
     elif key_cache.dtype != q.dtype or value_cache.dtype != q.dtype:
         raise ValueError("q and the caches must share one dtype")
+    if append_codes is not None and (not int8_kv or new_key is None):
+        raise ValueError("append_codes goes with a byte-code cache and new_key")
     if block_table is not None:
         if key_cache.dim() != 4 or value_cache.shape != key_cache.shape:
             raise ValueError("paged caches must be [num_blocks, block_size, num_kv_heads, head_size]")
@@ -382,18 +388,23 @@ def swa_decode_attention(
         softcap=float(softcap), alibi_slopes=N.ptr(_slopes(alibi_slopes, Hq, dev)),
         meta_bias_row0=int(meta_bias[0]) if meta_bias else 0, meta_bias_rows=int(meta_bias[1]) if meta_bias else 0,
         **fused, **_event_args(profile_events))
-    N.check(L.sb_swa_decode(C.byref(a)), "swa_decode")
+    if append_codes is not None:
+        N.check(L.sb_swa_decode_append_codes(C.byref(a), float(append_codes)), "swa_decode_append_codes")
+    else:
+        N.check(L.sb_swa_decode(C.byref(a)), "swa_decode")
     return (out, lse) if return_lse else out
 
 
 def paged_decode_step(q: torch.Tensor, key: torch.Tensor, value: torch.Tensor, kv_cache: torch.Tensor, out: torch.Tensor,
                       slot_mapping: torch.Tensor, seq_lens: torch.Tensor, block_table: torch.Tensor, window_left: int, scale: float,
-                      max_seq_len: int, balanced: bool) -> bool:
-    """swa_decode_attention with its append over a cache [2, num_blocks, block_size, Hkv, D] of q's type; False where the tensors are
-    not of that form (nothing is enqueued then). max_seq_len 0: bounded by the table."""
+                      max_seq_len: int, balanced: bool, kv_quant: int = N.SB_KV_NONE, scales: Optional[torch.Tensor] = None,
+                      k_scale: float = 0.0, v_scale: float = 0.0, append_codes: float = -1.0) -> bool:
+    """swa_decode_attention with its append over a cache [2, num_blocks, block_size, Hkv, D] of q's type or, with kv_quant, of codes
+    (scales [2, num_blocks, Hkv, block_size] of an INT8 one); False where the tensors are not of that form (nothing is enqueued
+    then). max_seq_len 0: bounded by the table."""
     stream, ws = _stream_and_workspace(q)
-    return _done(N.calls().decode(q, kv_cache, None, out, seq_lens, block_table, key, value, slot_mapping, None, None, N.SB_KV_NONE, 0.0, 0.0,
-                                  window_left, scale, max_seq_len, balanced, ws, stream), "swa_decode") is not None
+    return _done(N.calls().decode(q, kv_cache, None, out, seq_lens, block_table, key, value, slot_mapping, scales, None, kv_quant, k_scale,
+                                  v_scale, append_codes, window_left, scale, max_seq_len, balanced, ws, stream), "swa_decode") is not None
 
 
 def _slopes(alibi_slopes, num_q_heads: int, device) -> Optional[torch.Tensor]:
