@@ -552,6 +552,10 @@ int32_t sb_swa_prefill_group_heads(const sb_swa_prefill_args *args, int64_t max_
 size_t sb_swa_prefill_workspace_bytes(const sb_swa_prefill_args *args, int64_t total_q, int32_t n_parts);
 int sb_swa_prefill_parted(const sb_swa_prefill_args *args, int64_t total_q, int64_t max_keys, int32_t n_parts,
                           void *workspace, size_t workspace_bytes);
+/* sb_kv_append and sb_swa_prefill_parted, in one launch where that is faster (keys and values in flight, 16-bit elements): the
+ * attention must not read what the append writes. */
+int sb_swa_prefill_append(const sb_swa_prefill_args *args, const sb_kv_append_args *append, int64_t total_q, int64_t max_keys,
+                          int32_t n_parts, void *workspace, size_t workspace_bytes);
 
 /* ------------------------------------------------------------------------------------
  * Per-row symmetric INT8 K/V (W8ASpike/window_attention.py:183-186 with quantize_sym, :227-237):

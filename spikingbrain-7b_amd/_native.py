@@ -210,6 +210,7 @@ EXPORTS = {
     "sb_swa_prefill_group_heads": (i32, [C.POINTER(SwaPrefillArgs), i64, i32]),
     "sb_swa_prefill_workspace_bytes": (sz, [C.POINTER(SwaPrefillArgs), i64, i32]),
     "sb_swa_prefill_parted": (C.c_int, [C.POINTER(SwaPrefillArgs), i64, i64, i32, vp, sz]),
+    "sb_swa_prefill_append": (C.c_int, [C.POINTER(SwaPrefillArgs), C.POINTER(KvAppendArgs), i64, i64, i32, vp, sz]),
     "sb_window_advance": (C.c_int, [C.POINTER(WindowAdvanceArgs)]),
     "sb_lse_merge": (C.c_int, [C.POINTER(LseMergeArgs)]),
     "sb_kv_append_int8": (C.c_int, [C.POINTER(KvAppendInt8Args)]),

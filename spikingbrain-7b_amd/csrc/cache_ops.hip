@@ -123,8 +123,10 @@ inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 
 
 }  // namespace
 
-extern "C" int sb_kv_append(const sb_kv_append_args *a) {
-  using namespace sb_host;
+namespace sb_host {
+
+// Refuses what the append kernels do not take (num_tokens > 0 from here on; the prefill kernel's append goes by it too).
+int check_kv_append(const sb_kv_append_args *a) {
   if (!a) return fail(SB_ERR_INVALID, "sb_kv_append: null args");
   if (a->num_tokens < 0) return fail(SB_ERR_INVALID, "sb_kv_append: negative num_tokens");
   if (a->num_tokens == 0) return SB_OK;
@@ -152,11 +154,20 @@ extern "C" int sb_kv_append(const sb_kv_append_args *a) {
                   (long long)s);
   if (!aligned16(a->key) || !aligned16(a->value) || !aligned16(a->k_cache) || !aligned16(a->v_cache))
     return fail(SB_ERR_INVALID, "sb_kv_append: tensor base not 16-byte aligned");
-  const int chunks_per_head = (int)(head_bytes / 16);
+  if ((a->num_tokens * 2 + 3) / 4 > 0x7fffffffLL) return fail(SB_ERR_UNSUPPORTED, "sb_kv_append: too many tokens");
+  return SB_OK;
+}
+
+}  // namespace sb_host
+
+extern "C" int sb_kv_append(const sb_kv_append_args *a) {
+  using namespace sb_host;
+  if (const int rc = check_kv_append(a)) return rc;
+  if (a->num_tokens == 0) return SB_OK;
+  const int esz = a->dtype == SB_F32 ? 4 : 2;
+  const int chunks_per_head = a->head_size * esz / 16;
   const int n_chunks = chunks_per_head * a->num_kv_heads;
-  const int64_t waves = a->num_tokens * 2;
-  const int64_t blocks = (waves + 3) / 4;
-  if (blocks > 0x7fffffffLL) return fail(SB_ERR_UNSUPPORTED, "sb_kv_append: too many tokens");
+  const int64_t blocks = (a->num_tokens * 2 + 3) / 4;
   hipLaunchKernelGGL(kv_append_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)a->stream,
                      (const char *)a->key, (const char *)a->value, (char *)a->k_cache,
                      (char *)a->v_cache, a->slot_mapping, a->num_tokens, chunks_per_head, n_chunks,

@@ -196,6 +196,24 @@ PyObject *decode(Args &in) {
   return status(codes && nk ? sb_swa_decode_append_codes(&a, (float)q_scale) : sb_swa_decode(&a));
 }
 
+// The fields of an element append; false where the tensors are not of the ordinary form
+bool fill_append(sb_kv_append_args &a, const Tensor &key, const Tensor &value, const Pages &c, const Tensor &slots, void *stream) {
+  if (key.dim() != 3 || value.sizes() != key.sizes() || value.scalar_type() != key.scalar_type() || code_of(key.scalar_type()) < 0 ||
+      !inner_contiguous(key) || !inner_contiguous(value) || c.heads != key.size(1) || c.dim != key.size(2) || c.type != key.scalar_type() ||
+      !vector_of(slots, at::kLong, key.size(0)))
+    return false;
+  std::memset(&a, 0, sizeof a);
+  a.key = key.data_ptr(); a.value = value.data_ptr(); a.k_cache = const_cast<char *>(c.k); a.v_cache = const_cast<char *>(c.v);
+  a.slot_mapping = slots.data_ptr<int64_t>();
+  a.num_tokens = key.size(0); a.num_kv_heads = (int)c.heads; a.head_size = (int)c.dim; a.block_size = (int)c.bs;
+  a.dtype = code_of(key.scalar_type());
+  a.key_stride_token = key.stride(0); a.key_stride_head = key.stride(1);
+  a.value_stride_token = value.stride(0); a.value_stride_head = value.stride(1);
+  a.cache_stride_block = c.s_block; a.cache_stride_row = c.s_row; a.cache_stride_head = c.s_head;
+  a.num_blocks = c.nb; a.stream = stream;
+  return true;
+}
+
 // append(key, value, k_cache, v_cache, slots, k_scale | None, v_scale | None, stream): ops.kv_append, or ops.kv_append_int8 with scales
 PyObject *append(Args &in) {
   const Tensor *key = in.tensor(), *value = in.tensor(), *kc = in.tensor(), *vc = in.tensor(), *slots = in.tensor();
@@ -208,16 +226,8 @@ PyObject *append(Args &in) {
   const int64_t T = key->size(0), H = key->size(1), D = key->size(2);
   if (c.heads != H || c.dim != D || !vector_of(*slots, at::kLong, T)) return not_taken();
   if (!ks && !vs) {
-    if (c.type != key->scalar_type()) return not_taken();
     sb_kv_append_args a;
-    std::memset(&a, 0, sizeof a);
-    a.key = key->data_ptr(); a.value = value->data_ptr(); a.k_cache = const_cast<char *>(c.k); a.v_cache = const_cast<char *>(c.v);
-    a.slot_mapping = slots->data_ptr<int64_t>();
-    a.num_tokens = T; a.num_kv_heads = (int)H; a.head_size = (int)D; a.block_size = (int)c.bs; a.dtype = code_of(key->scalar_type());
-    a.key_stride_token = key->stride(0); a.key_stride_head = key->stride(1);
-    a.value_stride_token = value->stride(0); a.value_stride_head = value->stride(1);
-    a.cache_stride_block = c.s_block; a.cache_stride_row = c.s_row; a.cache_stride_head = c.s_head;
-    a.num_blocks = c.nb; a.stream = stream;
+    if (!fill_append(a, *key, *value, c, *slots, stream)) return not_taken();
     return status(sb_kv_append(&a));
   }
   if (c.type != at::kChar || !scales_of(ks, c.nb, H, c.bs) || !scales_of(vs, c.nb, H, c.bs)) return not_taken();
@@ -235,8 +245,8 @@ PyObject *append(Args &in) {
 }
 
 // prefill(q, k, v, out, cu_seqlens_q, seq_lens_k, tile_seq, tile_q0, block_table | None, kv_start | None, kv_start32 | None, num_tiles,
-// num_seqs, total_q, total_k, max_k, tile_keys, ordered_tile_seq, ordered_tile_q0, window_left, scale, stream): ops.swa_prefill_attention
-// over element caches or in-flight keys.
+// num_seqs, total_q, total_k, max_k, tile_keys, ordered_tile_seq, ordered_tile_q0, window_left, scale, new_key | None, new_value | None,
+// kv_cache [2, ...] | None, slots | None, stream): ops.swa_prefill_attention over element caches or in-flight keys, with or without an append.
 PyObject *prefill(Args &in) {
   const Tensor *q = in.tensor(), *k = in.tensor(), *v = in.tensor(), *out = in.tensor(), *cu = in.tensor(), *lens = in.tensor();
   const Tensor *tile_seq = in.tensor(), *tile_q0 = in.tensor(), *table = in.maybe_tensor(), *start = in.maybe_tensor(), *start32 = in.maybe_tensor();
@@ -244,6 +254,7 @@ PyObject *prefill(Args &in) {
   void *const tile_keys = in.address(), *const ordered_seq = in.address(), *const ordered_q0 = in.address();
   const int64_t window = in.integer();
   const double scale = in.number();
+  const Tensor *nk = in.maybe_tensor(), *nv = in.maybe_tensor(), *cache = in.maybe_tensor(), *slots = in.maybe_tensor();
   void *const stream = in.address();
   if (!in.ok || q->dim() != 3 || !half_type(*q) || !inner_contiguous(*q) || q->size(2) != 128 || q->size(0) != total_q || tiles < 1 ||
       max_k < 1 || max_k > INT32_MAX || window < -1 || window > INT32_MAX || k->scalar_type() != q->scalar_type() || !same_layout(*k, *v) ||
@@ -285,12 +296,18 @@ PyObject *prefill(Args &in) {
   a.tile_keys = static_cast<const int32_t *>(tile_keys);
   a.ordered_tile_seq = static_cast<const int32_t *>(ordered_seq);
   a.ordered_tile_q0 = static_cast<const int32_t *>(ordered_q0);
+  sb_kv_append_args ap;
+  Pages c;
+  if (nk && (!nv || !cache || !slots || !c.from(cache, nullptr) || !fill_append(ap, *nk, *nv, c, *slots, stream))) return not_taken();
   const int parts = sb_swa_prefill_parts(&a, max_k);
-  if (parts < 2) return status(sb_swa_prefill_parted(&a, total_q, max_k, parts, nullptr, 0));
+  auto go = [&](void *ws, size_t bytes) {
+    return status(nk ? sb_swa_prefill_append(&a, &ap, total_q, max_k, parts, ws, bytes) : sb_swa_prefill_parted(&a, total_q, max_k, parts, ws, bytes));
+  };
+  if (parts < 2) return go(nullptr, 0);
   const size_t bytes = sb_swa_prefill_workspace_bytes(&a, total_q, parts);
   const Tensor ws = at::empty({(int64_t)bytes}, q->options().dtype(at::kByte));
   if (!plain(ws)) return not_taken();
-  return status(sb_swa_prefill_parted(&a, total_q, max_k, parts, ws.data_ptr(), bytes));
+  return go(ws.data_ptr(), bytes);
 }
 
 // What the two linear-attention calls share, once their shapes are known

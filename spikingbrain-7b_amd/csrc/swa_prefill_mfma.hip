@@ -46,9 +46,25 @@
 #include "common.h"
 #include "mfma_util.h"
 
+namespace sb_host {
+int check_kv_append(const sb_kv_append_args *a);   // cache_ops.hip
+}
+
 namespace {
 
 using namespace sb;
+
+// An append of this call's keys and values that rides in the launch (see append_rides): workgroups from `first` on copy rows.
+struct Append {
+  const char *key, *value;
+  char *k_cache, *v_cache;
+  const int64_t *slots;
+  int64_t tokens;
+  unsigned first;
+  int n_chunks, block_size;    // 16-byte chunks of a row (16 per head)
+  int64_t key_st, key_sh, val_st, val_sh, blk, row, head;   // bytes
+};
+constexpr int kAppendTokens = 4;   // of a wavefront: eight rows in flight
 
 struct PrefillParams {
   const char *q;
@@ -95,6 +111,7 @@ struct PrefillParams {
   int n_parts, part_chunks;
   float *ws_acc;
   float *ws_ml;
+  Append append;              // in-flight element calls: first = ~0u where there is none
 };
 
 // The walk of a tile in 32-key chunks: every chunk that holds a key some token of the tile can see.
@@ -179,6 +196,32 @@ __device__ __forceinline__ uint4 dequant8(uint2 w, float s) {
                     Mma<E>::pack(code_value<Q, 2>(w.y) * s, code_value<Q, 3>(w.y) * s));
 }
 
+__device__ __forceinline__ void append_rows(const PrefillParams &p, int64_t wave, int lane) {
+  const int64_t tok0 = wave * kAppendTokens, last = p.append.tokens - 1;
+  if (tok0 > last) return;
+  for (int c = lane; c < p.append.n_chunks; c += 64) {
+    const int64_t h = c >> 4, w = (int64_t)(c & 15) * 16;
+    const char *const key = p.append.key + h * p.append.key_sh + w, *const value = p.append.value + h * p.append.val_sh + w;
+    u32x4_t k[kAppendTokens], v[kAppendTokens];
+#pragma unroll
+    for (int u = 0; u < kAppendTokens; ++u) {
+      const int64_t tok = min(tok0 + u, last);
+      k[u] = *reinterpret_cast<const u32x4_t *>(key + tok * p.append.key_st);
+      v[u] = *reinterpret_cast<const u32x4_t *>(value + tok * p.append.val_st);
+    }
+#pragma unroll
+    for (int u = 0; u < kAppendTokens; ++u) {
+      if (tok0 + u > last) continue;
+      const int64_t slot = p.append.slots[tok0 + u];
+      if (slot < 0) continue;   // (padded lane / token older than the window)
+      const int64_t blk = slot / p.append.block_size;
+      const int64_t at = blk * p.append.blk + (slot - blk * p.append.block_size) * p.append.row + h * p.append.head + w;
+      *reinterpret_cast<u32x4_t *>(p.append.k_cache + at) = k[u];
+      *reinterpret_cast<u32x4_t *>(p.append.v_cache + at) = v[u];
+    }
+  }
+}
+
 // ODD: the last group of heads may have one less (3 of 4, 1 of 2): a build of its own, because the second path costs
 // the kernel of two heads 5 % (16 : 8 heads, 2000 tokens behind 3000 95 -> 100 us).
 template <typename E, int NHEADS, int KVQ, bool PAGED, bool ODD, bool HALVES>
@@ -188,6 +231,14 @@ void swa_prefill_kernel(const PrefillParams p) {
   using S = Shape<NHEADS, HALVES>;
   __shared__ __attribute__((aligned(16))) char smem_all[(HALVES ? 6 : 3) * kStage];  // ring(s) of three chunks, each [K|V]
 
+  if constexpr (!PAGED) {
+    if (blockIdx.x >= p.append.first) {   // (the whole workgroup, ahead of every barrier)
+      if (blockIdx.y == 0)
+        append_rows(p, (int64_t)(blockIdx.x - p.append.first) * S::kWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6),
+                    threadIdx.x & 63);
+      return;
+    }
+  }
   // Workgroups are handed to the 8 XCDs round-robin by index, and each XCD has its own L2. Give XCD x
   // the x-th contiguous eighth of the tiles, so that the workgroups resident on one XCD at a time are
   // neighbouring tiles of one sequence and kv head, whose key windows overlap almost entirely.
@@ -885,7 +936,16 @@ Spread spread_of(const sb_swa_prefill_args *a, int64_t max_keys) {
   return best;
 }
 
-int prefill(const sb_swa_prefill_args *a, int64_t max_keys, int n_parts, float *ws_acc, float *ws_ml) {
+// The append of a call whose keys are in flight rides along as workgroups behind those of the attention: they copy on CUs that have
+// none or whose own are done, and a launch less is made. us of the layer call, append in front -> in it (28 : 4 heads): 64 / 300 / 700 / 1517 /
+// 2500 / 4000 tokens 17.8 / 18.4 / 22.2 / 36.5 / 73.0 / 143.0 -> 14.2 / 14.7 / 19.4 / 34.4 / 70.0 / 139.8, 4 x 700 30.6 -> 28.1, 8 x 2000
+// 210 -> 204. From 8000 tokens on they wait for the attention's CUs and it is level (1 x 8000 373.5 -> 373; 16 x 8192: 5925 + 62 -> 5985 by
+// the trace), the extra workgroups moving 4 to 5 TB/s as the kernel of its own did.
+bool append_rides(const sb_swa_prefill_args *a, const sb_kv_append_args *ap) {
+  return !a->block_table && ap->head_size == 128 && ap->dtype != SB_F32 && ap->stream == a->stream && a->num_tiles > 0;
+}
+
+int prefill(const sb_swa_prefill_args *a, int64_t max_keys, int n_parts, float *ws_acc, float *ws_ml, const sb_kv_append_args *ap = nullptr) {
   using namespace sb_host;
   if (!a) return fail(SB_ERR_INVALID, "sb_swa_prefill: null args");
   if (a->num_tiles < 0) return fail(SB_ERR_INVALID, "sb_swa_prefill: negative num_tiles");
@@ -952,6 +1012,8 @@ int prefill(const sb_swa_prefill_args *a, int64_t max_keys, int n_parts, float *
     p.tile_seq = a->ordered_tile_seq;
     p.tile_q0 = a->ordered_tile_q0;
   }
+  p.append = Append{};
+  p.append.first = ~0u;
   p.n_parts = n_parts; p.part_chunks = (int)((chunks + n_parts - 1) / n_parts);
   p.ws_acc = ws_acc; p.ws_ml = ws_ml;
   p.meta_k = p.meta_v = nullptr;
@@ -1010,7 +1072,19 @@ int prefill(const sb_swa_prefill_args *a, int64_t max_keys, int n_parts, float *
     p.head_begin = h0;
     h0 += nh * groups;
     p.head_groups = groups;
-    const dim3 grid((unsigned)(per_xcd * 8 * a->num_kv_heads * groups), (unsigned)n_parts);
+    dim3 grid((unsigned)(per_xcd * 8 * a->num_kv_heads * groups), (unsigned)n_parts);
+    p.append.first = ~0u;
+    if (ap && p.head_begin == 0) {   // (the first launch takes it along)
+      const int waves = nh == 4 || halves ? 8 : 4;
+      const int64_t esz = 2;
+      p.append = Append{(const char *)ap->key, (const char *)ap->value, (char *)ap->k_cache, (char *)ap->v_cache, ap->slot_mapping,
+                        ap->num_tokens, grid.x, ap->num_kv_heads * 16, ap->block_size, ap->key_stride_token * esz,
+                        ap->key_stride_head * esz, ap->value_stride_token * esz, ap->value_stride_head * esz,
+                        ap->cache_stride_block * esz, ap->cache_stride_row * esz, ap->cache_stride_head * esz};
+      const int64_t more = (ap->num_tokens + kAppendTokens * waves - 1) / (kAppendTokens * waves);
+      if (grid.x + more > 0x7fffffffLL) return fail(SB_ERR_UNSUPPORTED, "sb_swa_prefill: grid too large");
+      grid.x += (unsigned)more;
+    }
     if (a->dtype == SB_BF16) launch_prefill<BF16>(a->kv_quant, nh, odd, halves, grid, (hipStream_t)a->stream, p);
     else launch_prefill<F16>(a->kv_quant, nh, odd, halves, grid, (hipStream_t)a->stream, p);
     const int rc = check_launch("swa_prefill_kernel");
@@ -1098,14 +1172,14 @@ extern "C" size_t sb_swa_prefill_workspace_bytes(const sb_swa_prefill_args *a, i
   return (size_t)total_q * (size_t)a->num_q_heads * (size_t)n_parts * (128 + 2) * sizeof(float);
 }
 
-extern "C" int sb_swa_prefill_parted(const sb_swa_prefill_args *a, int64_t total_q, int64_t max_keys, int32_t n_parts,
-                                     void *workspace, size_t workspace_bytes) {
+static int prefill_parted(const sb_swa_prefill_args *a, int64_t total_q, int64_t max_keys, int32_t n_parts, void *workspace,
+                          size_t workspace_bytes, const sb_kv_append_args *ap) {
   using namespace sb_host;
   if (!a) return fail(SB_ERR_INVALID, "sb_swa_prefill_parted: null args");
   if (a->num_tiles <= 0) return sb_swa_prefill(a);
   if (total_q <= 0 || max_keys <= 0) return fail(SB_ERR_INVALID, "sb_swa_prefill_parted: total_q and max_keys must be positive");
   if (max_keys > INT32_MAX) max_keys = INT32_MAX;
-  if (n_parts < 2) return prefill(a, max_keys, 1, nullptr, nullptr);
+  if (n_parts < 2) return prefill(a, max_keys, 1, nullptr, nullptr, ap);
   if (n_parts > 1024 || a->num_q_heads > 65535) return fail(SB_ERR_UNSUPPORTED, "sb_swa_prefill_parted: too many parts or heads");
   if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 15u) ||
       workspace_bytes < sb_swa_prefill_workspace_bytes(a, total_q, n_parts))
@@ -1115,5 +1189,21 @@ extern "C" int sb_swa_prefill_parted(const sb_swa_prefill_args *a, int64_t total
   if (a->num_q_heads > 0)
     n_parts = (int32_t)std::max<int64_t>(1, std::min<int64_t>(n_parts, INT32_MAX / ((int64_t)8 * 512 * a->num_q_heads)));
   float *acc = static_cast<float *>(workspace);
-  return prefill(a, max_keys, n_parts, acc, acc + total_q * a->num_q_heads * n_parts * 128);
+  return prefill(a, max_keys, n_parts, acc, acc + total_q * a->num_q_heads * n_parts * 128, ap);
+}
+
+extern "C" int sb_swa_prefill_parted(const sb_swa_prefill_args *a, int64_t total_q, int64_t max_keys, int32_t n_parts, void *workspace,
+                                     size_t workspace_bytes) {
+  return prefill_parted(a, total_q, max_keys, n_parts, workspace, workspace_bytes, nullptr);
+}
+
+extern "C" int sb_swa_prefill_append(const sb_swa_prefill_args *a, const sb_kv_append_args *append, int64_t total_q, int64_t max_keys,
+                                     int32_t n_parts, void *workspace, size_t workspace_bytes) {
+  using namespace sb_host;
+  if (!a) return fail(SB_ERR_INVALID, "sb_swa_prefill_append: null args");
+  if (const int rc = check_kv_append(append)) return rc;
+  if (append->num_tokens == 0 || append_rides(a, append))
+    return prefill_parted(a, total_q, max_keys, n_parts, workspace, workspace_bytes, append->num_tokens ? append : nullptr);
+  const int rc = sb_kv_append(append);
+  return rc ? rc : prefill_parted(a, total_q, max_keys, n_parts, workspace, workspace_bytes, nullptr);
 }

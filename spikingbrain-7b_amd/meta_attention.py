@@ -548,6 +548,7 @@ class MetaAttentionImpl:
                        and (attn_metadata.max_decode_query_len or 1) == 1
                        and query.dtype in (torch.bfloat16, torch.float16)
                        and attn_metadata.slot_mapping is not None)
+        late_append = None
         if kv_cache.numel() > 0:
             key_cache, value_cache = (kv_cache.codes[0], kv_cache.codes[1]) if int8_kv else (kv_cache[0], kv_cache[1])
             if fp8_kv and key_cache.dtype not in (torch.uint8, torch.float8_e4m3fn):
@@ -561,8 +562,13 @@ class MetaAttentionImpl:
                 ops.kv_append_int8(key, value, key_cache, value_cache, scales["k_scale"], scales["v_scale"],
                                    _flat(attn_metadata.slot_mapping))
             elif key is not None and value is not None and not fuse_append:
-                # all new K/V of the step (prefill and decode tokens) go in with one launch (:790-799)
-                ops.kv_append(key, value, key_cache, value_cache, _flat(attn_metadata.slot_mapping))
+                # all new K/V of the step (prefill and decode tokens) go in with one launch (:790-799), that of the prompts where they
+                # attend to the keys and values in flight
+                prompts = attn_metadata.prefill_metadata
+                if prompts and _in_flight(kv_cache, prompts):
+                    late_append = (key, value, kv_cache, _flat(attn_metadata.slot_mapping))
+                else:
+                    ops.kv_append(key, value, key_cache, value_cache, _flat(attn_metadata.slot_mapping))
 
         num_prefill_query_tokens = attn_metadata.num_prefill_tokens
         num_decode_query_tokens = attn_metadata.num_decode_tokens
@@ -623,7 +629,7 @@ class MetaAttentionImpl:
                     pk, pv = ops.quantize_sym(pk), ops.quantize_sym(pv)
                 elif fp8_kv:  # the prompt's keys and values after their round trip
                     pk, pv = fp8_prompt
-                self._varlen_inflight(query, pk, pv, prefill_meta, prefill_output, window_left, meta_kv=prefill_kv)
+                self._varlen_inflight(query, pk, pv, prefill_meta, prefill_output, window_left, meta_kv=prefill_kv, append=late_append)
             else:
                 # prefix hit / chunked prefill: keys and values come from the paged cache (:885-919)
                 assert prefill_meta.seq_lens is not None
@@ -718,25 +724,28 @@ class MetaAttentionImpl:
             return None
         return plan
 
-    def _varlen_inflight(self, q, k, v, meta, out, window_left, return_lse=False, meta_kv=None):
+    def _varlen_inflight(self, q, k, v, meta, out, window_left, return_lse=False, meta_kv=None, append=None):
         """Returns the fp32 [T, Hq] log-sum-exp when asked for, else None. meta_kv: meta_k/meta_v for the
-        kernels to take into their softmax."""
+        kernels to take into their softmax. append: (key, value, kv_cache, slots) to append on the way."""
         meta_kv = meta_kv or {}
         T = q.shape[0]
+        plan = None if T == 0 else self._plan_for(meta, q)
+        rides = plan is not None and plan.total_k <= k.shape[0]
+        if append is not None and not rides:
+            ops.kv_append(append[0], append[1], append[2][0], append[2][1], append[3])
         if T == 0:
             return None
         if k.stride() != v.stride():
             v = v.contiguous()
             k = k.contiguous()
-        plan = self._plan_for(meta, q)
-        if plan is not None and plan.total_k <= k.shape[0]:
+        if rides:
             start = meta.seq_start_loc
             if start.dtype == torch.int32 and start.dim() == 1 and start.is_contiguous() and start.numel() > plan.num_seqs:
                 starts = dict(kv_start32=start)
             else:
                 starts = dict(kv_start=start.to(torch.int64)[:-1].contiguous())
             res = ops.swa_prefill_attention(q, k, v, plan=plan, window_left=window_left, scale=self.scale, out=out,
-                                            return_lse=return_lse, **starts, **meta_kv)
+                                            return_lse=return_lse, append=append, **starts, **meta_kv)
             return res[1] if return_lse else None
         row_seq, j, _ = self._rows(meta.query_start_loc, T)
         seq_lens_row = (j + 1).to(torch.int32)

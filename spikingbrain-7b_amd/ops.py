@@ -674,6 +674,7 @@ def swa_prefill_attention(
     meta_bias: Optional[Tuple[int, int]] = None,
     n_parts: int = 0,
     kv_start32: Optional[torch.Tensor] = None,
+    append: Optional[tuple] = None,
 ):
     """Causal sliding-window attention for q [total_q, Hq, D] packed sequence after sequence.
     softcap / alibi_slopes: as for swa_decode_attention; query j of a sequence sits at key position
@@ -695,7 +696,9 @@ def swa_prefill_attention(
     k_scale/v_scale (INT8 codes) or fp8_scales (e4m3fn codes): the paged caches are byte codes as
     kv_append_int8 / kv_append_fp8 wrote them; rows are dequantised on their way into the kernel.
     n_parts: cut the keys of a tile into up to this many parts that run side by side (0 = chosen by the library, 1 =
-    not at all)."""
+    not at all).
+    append: (key, value, kv_cache [2, num_blocks, block_size, Hkv, D], slot_mapping) of a kv_append to make as well, into
+    memory this call does not read: in the same launch where that is faster."""
     if plan is not None and out is not None and n_parts == 0 and q.is_cuda and not return_lse and key_lo is None and kv_strides is None and \
             num_kv_heads is None and k_scale is None and v_scale is None and fp8_scales is None and meta_k is None and meta_v is None and \
             softcap == 0.0 and alibi_slopes is None and (block_table is None or kv_start is None and kv_start32 is None):
@@ -703,9 +706,12 @@ def swa_prefill_attention(
         starts = plan.cu_seqlens_q if block_table is None and kv_start is None and kv_start32 is None else kv_start32
         if _done(N.calls().prefill(q, k, v, out, plan.cu_seqlens_q, plan.seq_lens_k, plan.tile_seq, plan.tile_q0, block_table, kv_start, starts,
                                    plan.num_tiles, plan.num_seqs, plan.total_q, plan.total_k, plan.max_k, tile_keys or 0, ordered_seq or 0,
-                                   ordered_q0 or 0, window_left, q.shape[-1] ** -0.5 if scale is None else scale, N.stream_ptr(q.device)),
+                                   ordered_q0 or 0, window_left, q.shape[-1] ** -0.5 if scale is None else scale, *(append or (None,) * 4),
+                                   N.stream_ptr(q.device)),
                  "swa_prefill") is not None:
             return out
+    if append is not None:
+        kv_append(append[0], append[1], append[2][0], append[2][1], append[3])
     dev = N.require_gpu(q, k, v, block_table, kv_start, kv_start32, key_lo, out, k_scale, v_scale)
     kv_quant = N.SB_KV_NONE
     if fp8_scales is not None:
