@@ -444,6 +444,9 @@ typedef struct sb_dense_rows_args {
 } sb_dense_rows_args;
 
 int sb_dense_rows(const sb_dense_rows_args *args);
+/* sb_window_shift_pair and sb_dense_rows, which need nothing of each other, in one launch where no rows are kept (a decode step behind
+ * the window's end). */
+int sb_dense_step(const sb_window_shift_args *k, const sb_window_shift_args *v, const sb_dense_rows_args *rows);
 
 /* ------------------------------------------------------------------------------------
  * Causal sliding-window attention over many query tokens per sequence (prompt prefill,

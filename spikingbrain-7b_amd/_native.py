@@ -204,6 +204,7 @@ EXPORTS = {
     "sb_window_shift": (C.c_int, [C.POINTER(WindowShiftArgs)]),
     "sb_window_shift_pair": (C.c_int, [C.POINTER(WindowShiftArgs), C.POINTER(WindowShiftArgs)]),
     "sb_dense_rows": (C.c_int, [C.POINTER(DenseRowsArgs)]),
+    "sb_dense_step": (C.c_int, [C.POINTER(WindowShiftArgs), C.POINTER(WindowShiftArgs), C.POINTER(DenseRowsArgs)]),
     "sb_swa_prefill": (C.c_int, [C.POINTER(SwaPrefillArgs)]),
     "sb_swa_prefill_plan": (C.c_int, [C.POINTER(i32), C.POINTER(i32), i64, i64, vp, vp]),
     "sb_swa_prefill_parts": (i32, [C.POINTER(SwaPrefillArgs), i64]),

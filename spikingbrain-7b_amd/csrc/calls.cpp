@@ -378,38 +378,48 @@ PyObject *gla_packed(Args &in) {
   return THPVariable_Wrap(std::move(out));
 }
 
-// push(k_storage, v_storage, key, value, row, stream): rows [row, row + n) of both window buffers [B, H, capacity, D] take the n new rows
-// of key and value [B, H, n, D]: ops.window_shift_pair without rows that stay
-PyObject *push(Args &in) {
-  const Tensor *storage[2] = {in.tensor(), in.tensor()}, *fresh[2] = {in.tensor(), in.tensor()};
-  const int64_t row = in.integer();
-  void *const stream = in.address();
-  if (!in.ok || row < 0) return not_taken();
-  sb_window_shift_args a[2];
+// Rows [row, row + n) of both window buffers [B, H, capacity, D] take the n new rows of key and value [B, H, n, D]; false where the tensors
+// are not of the ordinary form
+bool fill_push(sb_window_shift_args (&a)[2], const Tensor *const (&storage)[2], const Tensor *const (&fresh)[2], int64_t row, void *stream) {
+  if (row < 0) return false;
   std::memset(a, 0, sizeof a);
   for (int i = 0; i < 2; ++i) {
     const Tensor &s = *storage[i], &f = *fresh[i];
     if (s.dim() != 4 || f.dim() != 4 || !s.is_contiguous() || f.size(0) != s.size(0) || f.size(1) != s.size(1) || f.size(3) != s.size(3) ||
         f.scalar_type() != s.scalar_type() || f.stride(3) != 1 || f.stride(0) != f.size(1) * f.stride(1) || row + f.size(2) > s.size(2))
-      return not_taken();
+      return false;
     const int64_t e = s.element_size();
     a[i].dst = s.data_ptr(); a[i].fresh = f.data_ptr();
     a[i].planes = s.size(0) * s.size(1); a[i].dst_row0 = row; a[i].n_new = f.size(2); a[i].row_bytes = s.size(3) * e;
     a[i].dst_stride_plane_bytes = s.stride(1) * e; a[i].fresh_stride_plane_bytes = f.stride(1) * e; a[i].fresh_stride_row_bytes = f.stride(2) * e;
     a[i].stream = stream;
   }
+  return true;
+}
+
+// push(k_storage, v_storage, key, value, row, stream): ops.window_shift_pair without rows that stay
+PyObject *push(Args &in) {
+  const Tensor *storage[2] = {in.tensor(), in.tensor()}, *fresh[2] = {in.tensor(), in.tensor()};
+  const int64_t row = in.integer();
+  void *const stream = in.address();
+  sb_window_shift_args a[2];
+  if (!in.ok || !fill_push(a, storage, fresh, row, stream)) return not_taken();
   return status(sb_window_shift_pair(&a[0], &a[1]));
 }
 
-// dense_decode(q [B, Hq, 1, D], k, v [B, Hkv, K, D], mask | None, window_left, scale, workspace | None, stream): the attention of
-// window_attention.sliding_window_attention for one new token per sequence; returns out [B, 1, Hq, D], or the status of a call that was
-// refused
+// dense_decode(q [B, Hq, 1, D], k, v [B, Hkv, K, D], mask | None, window_left, scale, k_storage | None, v_storage | None, key | None,
+// value | None, row, workspace | None, stream): the attention of window_attention.sliding_window_attention for one new token per sequence,
+// and with the storage the push of the new rows; returns out [B, 1, Hq, D], or the status of a call that was refused
 PyObject *dense_decode(Args &in) {
   const Tensor *q = in.tensor(), *k = in.tensor(), *v = in.tensor(), *mask = in.maybe_tensor();
   const int64_t window = in.integer();
   const double scale = in.number();
+  const Tensor *storage[2] = {in.maybe_tensor(), in.maybe_tensor()}, *fresh[2] = {in.maybe_tensor(), in.maybe_tensor()};
+  const int64_t row = in.integer();
   const Tensor *ws = in.maybe_tensor();
   void *const stream = in.address();
+  sb_window_shift_args shift[2];
+  if (in.ok && storage[0] && (!storage[1] || !fresh[0] || !fresh[1] || !fill_push(shift, storage, fresh, row, stream))) return not_taken();
   if (!in.ok || q->dim() != 4 || k->dim() != 4 || q->size(2) != 1 || q->size(3) != 128 || q->stride(3) != 1 || code_of(q->scalar_type()) < 0)
     return not_taken();
   const int64_t B = q->size(0), Hq = q->size(1), D = 128, Hkv = k->size(1), K = k->size(2);
@@ -450,7 +460,7 @@ PyObject *dense_decode(Args &in) {
     d.mask_cols = cols; d.mask_stride_row = mask->stride(0); d.mask_stride_col = mask->stride(1); d.mask_elem_bytes = (int)mask->element_size();
   }
   d.stream = stream;
-  if (const int rc = sb_dense_rows(&d)) return status(rc);
+  if (const int rc = storage[0] ? sb_dense_step(&shift[0], &shift[1], &d) : sb_dense_rows(&d)) return status(rc);
   sb_swa_decode_args a;
   std::memset(&a, 0, sizeof a);
   a.q = q->data_ptr(); a.k_cache = k->data_ptr(); a.v_cache = v->data_ptr(); a.out = out.data_ptr();

@@ -1166,12 +1166,18 @@ def dense_rows(batch: int, num_queries: int, num_keys: int, kv_step: int, device
     return seq_lens, row_seq, None if mask is None else key_lo, kv_start
 
 
-def dense_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: Optional[torch.Tensor], window_left: int,
-                 scale: float) -> Optional[torch.Tensor]:
+def dense_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: Optional[torch.Tensor], window_left: int, scale: float,
+                 push: Optional[tuple] = None) -> Optional[torch.Tensor]:
     """dense_rows and swa_decode_attention for one new token of each sequence, q [B, Hq, 1, D] over k, v [B, Hkv, K, D], mask
-    [B, n] whose last K columns count: out [B, 1, Hq, D], or None where the tensors are not of that form (nothing is enqueued then)."""
+    [B, n] whose last K columns count, and in front of them window_shift_pair(*push) (no rows kept): out [B, 1, Hq, D], or None where the
+    tensors are not of that form (nothing is enqueued then)."""
     stream, ws = _stream_and_workspace(q)
-    return _done(N.calls().dense_decode(q, k, v, mask, window_left, scale, ws, stream), "swa_decode")
+    ks, vs, key, value, row = (None, None, None, None, 0)
+    if push is not None:
+        (k_src, ks, key, k_keep, _, row), (v_src, vs, value, v_keep, _, v_row) = push
+        if k_src is not None or v_src is not None or k_keep or v_keep or row != v_row:
+            return None
+    return _done(N.calls().dense_decode(q, k, v, mask, window_left, scale, ks, vs, key, value, row, ws, stream), "swa_decode")
 
 
 def window_advance(n_tokens: torch.Tensor, lo: torch.Tensor, hi: torch.Tensor, ring: torch.Tensor,

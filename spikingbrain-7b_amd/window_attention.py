@@ -71,15 +71,21 @@ def sliding_window_attention(
     B, Hq, Q, D = query_states.shape
     Hkv = key_states.shape[1]
 
+    push = []   # a copy into the cache that is still to be made
     if past_key_values is not None:
         cache_has_content = past_key_values.get_seq_length(layer_idx) > 0
         if cache_window_size == -1:
             cache_kwargs = {"window_size": sliding_window} if flavour == "flash" else {}
         else:
             cache_kwargs = {"window_size": cache_window_size}
-        key_cached, value_cached = past_key_values.update(
-            attn_state=(key_states, value_states), layer_idx=layer_idx, offset=Q,
-            cache_kwargs=cache_kwargs)["attn_state"]
+        if Q == 1 and cache_has_content and type(past_key_values) is Cache and query_states.is_cuda:
+            # the new rows' copy goes with the attention's first launch, below
+            key_cached, value_cached = past_key_values._update(
+                lambda *copies: push.extend(copies), None, (key_states, value_states), None, layer_idx, Q, cache_kwargs)["attn_state"]
+        else:
+            key_cached, value_cached = past_key_values.update(
+                attn_state=(key_states, value_states), layer_idx=layer_idx, offset=Q,
+                cache_kwargs=cache_kwargs)["attn_state"]
         if cache_has_content:
             key_states, value_states = key_cached, value_cached
 
@@ -88,9 +94,16 @@ def sliding_window_attention(
         window_left = sliding_window if flavour == "flash" else sliding_window - 1
 
     if Q == 1 and query_states.is_cuda:
-        out = ops.dense_decode(query_states, key_states, value_states, attention_mask, window_left, D ** -0.5)
+        try:
+            out = ops.dense_decode(query_states, key_states, value_states, attention_mask, window_left, D ** -0.5, push or None)
+        except Exception:   # (the cache counts the rows already)
+            if push:
+                ops.window_shift_pair(*push)
+            raise
         if out is not None:
             return out
+        if push:
+            ops.window_shift_pair(*push)
     k, v = key_states, value_states
     if k.stride(3) != 1 or v.stride() != k.stride() or _kv_step_rows(k) is None:
         k, v = k.contiguous(), v.contiguous()

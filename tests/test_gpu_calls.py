@@ -116,14 +116,13 @@ def test_prompts(sb, dev, both, paged, lens, ctx):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("mask", [None, torch.long, torch.bool, torch.int32])
-def test_hugging_face_decode(sb, dev, both, dtype, mask):
-    B, W = 3, 256
+@pytest.mark.parametrize("mask,B,W", [(None, 3, 256), (torch.long, 3, 256), (torch.bool, 1, 40), (torch.int32, 64, 33), (torch.int16, 5, 1)])
+def test_hugging_face_decode(sb, dev, both, dtype, mask, B, W):
     rows = [_rand(dev, B, HKV, W + 3, D, dtype=dtype, seed=s) for s in (1, 2)]
     m = None
     if mask is not None:
         m = torch.ones(B, W + 9, dtype=mask, device=dev)
-        m[1, :100] = 0
+        m[B // 2, :9 + W // 3] = 0
     new = [_rand(dev, B, 1, h, D, dtype=dtype, seed=h).transpose(1, 2) for h in (HQ, HKV, HKV)]
 
     def run():
