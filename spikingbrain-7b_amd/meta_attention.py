@@ -533,7 +533,7 @@ class MetaAttentionImpl:
                           and attn_metadata.num_prefill_tokens == 0 and attn_metadata.num_decode_tokens == query.shape[0] == key.shape[0] > 0
                           and (attn_metadata.max_decode_query_len or 1) == 1 and attn_metadata.slot_mapping is not None
                           and query.dtype in (torch.bfloat16, torch.float16) and key.dtype == value.dtype == query.dtype
-                          and (query.is_contiguous() or not fp8_kv))
+                          and (not fp8_kv or (query.is_contiguous() and float(getattr(layer, "_q_scale_float", 1.0)) > 0.0)))
         if fp8_kv:
             if int8_kv:
                 raise ValueError("kv_cache_dtype says fp8 but the cache is an Int8KVCache")
@@ -676,9 +676,10 @@ class MetaAttentionImpl:
         k_scale, v_scale = float(getattr(layer, "_k_scale_float", 1.0)), float(getattr(layer, "_v_scale_float", 1.0))
         codes, how = kv_cache, ()
         if self.kv_cache_dtype.startswith("fp8"):
-            if type(kv_cache) is not torch.Tensor or not query.is_contiguous():
+            q_scale = float(getattr(layer, "_q_scale_float", 1.0))
+            if type(kv_cache) is not torch.Tensor or not query.is_contiguous() or not q_scale > 0.0:
                 return False
-            how = (ops.N.SB_KV_FP8, None, k_scale, v_scale, float(getattr(layer, "_q_scale_float", 1.0)))
+            how = (ops.N.SB_KV_FP8, None, k_scale, v_scale, q_scale)
         elif k_scale != 1.0 or v_scale != 1.0:
             return False
         elif type(kv_cache) is Int8KVCache:

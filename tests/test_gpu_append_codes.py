@@ -82,6 +82,11 @@ def test_layer_call_under_capture(sb, dev, kv):
         want = run(q, c0, torch.zeros_like(q)).clone()
         general = run(spread[:, :HQ], c1, torch.zeros_like(q))             # fp8: the unfused form
         assert torch.equal(general, want) and all(torch.equal(a, b) for a, b in zip(held(c1), held(c0)))
+    if kv == "fp8":                                                        # (0 would mean no round trip)
+        layer._q_scale_float = 0.0
+        with pytest.raises(ValueError):
+            run(q, c1, torch.zeros_like(q))
+        layer._q_scale_float = 0.5
     out = torch.zeros_like(q)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
