@@ -593,6 +593,9 @@ typedef struct sb_kv_append_int8_args {
 } sb_kv_append_int8_args;
 
 int sb_kv_append_int8(const sb_kv_append_int8_args *args);
+/* The same, and the first round_tokens tokens' rows as the cache holds them (code * scale in the tensor's type, the bits of
+ * sb_quantize_sym) to key_out and value_out, [round_tokens, num_kv_heads, 128] contiguous: what a prompt in flight attends to. */
+int sb_kv_append_int8_round(const sb_kv_append_int8_args *args, void *key_out, void *value_out, int64_t round_tokens);
 
 typedef struct sb_quantize_sym_args {
   const void *in;  /* [rows, heads, 128] */

@@ -215,6 +215,7 @@ EXPORTS = {
     "sb_window_advance": (C.c_int, [C.POINTER(WindowAdvanceArgs)]),
     "sb_lse_merge": (C.c_int, [C.POINTER(LseMergeArgs)]),
     "sb_kv_append_int8": (C.c_int, [C.POINTER(KvAppendInt8Args)]),
+    "sb_kv_append_int8_round": (C.c_int, [C.POINTER(KvAppendInt8Args), vp, vp, i64]),
     "sb_quantize_sym": (C.c_int, [C.POINTER(QuantizeSymArgs)]),
     "sb_kv_append_fp8": (C.c_int, [C.POINTER(KvAppendFp8Args)]),
     "sb_fp8_round": (C.c_int, [vp, vp, i64, i64, i64, i64, i32, f32, vp]),

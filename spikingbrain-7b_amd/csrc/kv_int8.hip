@@ -44,20 +44,24 @@ __device__ __forceinline__ float quantise_row(const float (&x)[8], float (&code)
   return scale;
 }
 
-template <int DT>
+// ROUND: the first round_tokens tokens, a prompt that attends to its rows as the cache will hold them, also leave code * scale in the
+// tensor's type, [tokens, heads, 128] each, what quantize_sym_kernel writes in two more launches: us of a layer call, 64 / 1517 tokens
+// 34.8 / 45.7 -> 29.9 / 40.4, 8 x 2000 230 -> 222, 16 x 8192 level. Latency for small prompts, bytes (read once instead of twice) for large.
+template <int DT, bool ROUND>
 __global__ __launch_bounds__(256) void kv_append_int8_kernel(
     const char *__restrict__ key, const char *__restrict__ value, char *__restrict__ k_cache,
     char *__restrict__ v_cache, float *__restrict__ k_scale, float *__restrict__ v_scale,
     const int64_t *__restrict__ slot_mapping, int64_t num_tokens, int num_kv_heads, int block_size,
     int64_t key_tok_b, int64_t key_head_b, int64_t val_tok_b, int64_t val_head_b, int64_t blk_b, int64_t row_b,
-    int64_t head_b) {
+    int64_t head_b, char *__restrict__ k_round, char *__restrict__ v_round, int64_t round_tokens) {
   const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const int lane = threadIdx.x & 63;
   const int64_t tok = wave >> 1;
   const int which = (int)(wave & 1);
   if (tok >= num_tokens) return;
   const int64_t slot = slot_mapping[tok];
-  if (slot < 0) return;  // padded lane / token older than the window
+  const bool rounds = ROUND && tok < round_tokens;
+  if (slot < 0 && !rounds) return;  // padded lane / token older than the window
   const int64_t blk = slot / block_size;
   const int off = (int)(slot - blk * block_size);
   const int h = blockIdx.y * 4 + (lane >> 4);
@@ -72,6 +76,13 @@ __global__ __launch_bounds__(256) void kv_append_int8_kernel(
   }
   const float scale = quantise_row(x, code);
   if (!live) return;
+  if (rounds) {
+    float y[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) y[i] = code[i] * scale;
+    store8<DT>((which ? v_round : k_round) + ((tok * num_kv_heads + h) * 128 + piece * 8) * kEsz, y);
+    if (slot < 0) return;
+  }
   char *dst = (which ? v_cache : k_cache) + blk * blk_b + off * row_b + h * head_b + piece * 8;
   *reinterpret_cast<uint2 *>(dst) = int8_bytes(code);
   if (piece == 0) (which ? v_scale : k_scale)[(blk * num_kv_heads + h) * block_size + off] = scale;
@@ -199,7 +210,7 @@ inline int elem_size(int dtype) {
 
 }  // namespace
 
-extern "C" int sb_kv_append_int8(const sb_kv_append_int8_args *a) {
+static int append_int8(const sb_kv_append_int8_args *a, void *k_round, void *v_round, int64_t round_tokens) {
   using namespace sb_host;
   if (!a) return fail(SB_ERR_INVALID, "sb_kv_append_int8: null args");
   if (a->num_tokens < 0) return fail(SB_ERR_INVALID, "sb_kv_append_int8: negative num_tokens");
@@ -228,13 +239,29 @@ extern "C" int sb_kv_append_int8(const sb_kv_append_int8_args *a) {
   (const char *)a->key, (const char *)a->value, (char *)a->k_cache, (char *)a->v_cache, a->k_scale, a->v_scale, \
       a->slot_mapping, a->num_tokens, a->num_kv_heads, a->block_size, a->key_stride_token *esz,              \
       a->key_stride_head *esz, a->value_stride_token *esz, a->value_stride_head *esz, a->cache_stride_block,  \
-      a->cache_stride_row, a->cache_stride_head
+      a->cache_stride_row, a->cache_stride_head, (char *)k_round, (char *)v_round, round_tokens
   hipStream_t st = (hipStream_t)a->stream;
-  if (a->dtype == SB_BF16) hipLaunchKernelGGL(kv_append_int8_kernel<SB_BF16>, grid, dim3(256), 0, st, SB_ARGS);
-  else if (a->dtype == SB_F16) hipLaunchKernelGGL(kv_append_int8_kernel<SB_F16>, grid, dim3(256), 0, st, SB_ARGS);
-  else hipLaunchKernelGGL(kv_append_int8_kernel<SB_F32>, grid, dim3(256), 0, st, SB_ARGS);
+#define SB_APPEND(DT)                                                                                          \
+  do {                                                                                                         \
+    if (round_tokens > 0) hipLaunchKernelGGL((kv_append_int8_kernel<DT, true>), grid, dim3(256), 0, st, SB_ARGS); \
+    else hipLaunchKernelGGL((kv_append_int8_kernel<DT, false>), grid, dim3(256), 0, st, SB_ARGS);              \
+  } while (0)
+  if (a->dtype == SB_BF16) SB_APPEND(SB_BF16);
+  else if (a->dtype == SB_F16) SB_APPEND(SB_F16);
+  else SB_APPEND(SB_F32);
+#undef SB_APPEND
 #undef SB_ARGS
   return check_launch("kv_append_int8_kernel");
+}
+
+extern "C" int sb_kv_append_int8(const sb_kv_append_int8_args *a) { return append_int8(a, nullptr, nullptr, 0); }
+
+extern "C" int sb_kv_append_int8_round(const sb_kv_append_int8_args *a, void *key_out, void *value_out, int64_t round_tokens) {
+  using namespace sb_host;
+  if (!a) return fail(SB_ERR_INVALID, "sb_kv_append_int8_round: null args");
+  if (round_tokens < 0 || round_tokens > a->num_tokens || (round_tokens > 0 && (!key_out || !value_out || !aligned16(key_out) || !aligned16(value_out))))
+    return fail(SB_ERR_INVALID, "sb_kv_append_int8_round: 0 to num_tokens rounded tokens, outputs 16-byte aligned");
+  return append_int8(a, key_out, value_out, round_tokens);
 }
 
 extern "C" int sb_quantize_sym(const sb_quantize_sym_args *a) {

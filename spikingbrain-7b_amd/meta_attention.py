@@ -548,7 +548,7 @@ class MetaAttentionImpl:
                        and (attn_metadata.max_decode_query_len or 1) == 1
                        and query.dtype in (torch.bfloat16, torch.float16)
                        and attn_metadata.slot_mapping is not None)
-        late_append = None
+        late_append = rounded = None
         if kv_cache.numel() > 0:
             key_cache, value_cache = (kv_cache.codes[0], kv_cache.codes[1]) if int8_kv else (kv_cache[0], kv_cache[1])
             if fp8_kv and key_cache.dtype not in (torch.uint8, torch.float8_e4m3fn):
@@ -559,8 +559,11 @@ class MetaAttentionImpl:
                 append = (key, value, key_cache, value_cache, _flat(attn_metadata.slot_mapping), k_scale_f, v_scale_f)
             elif key is not None and value is not None and int8_kv:
                 # rows are quantised on their way in: 128 code bytes + one scale per (token, kv head)
-                ops.kv_append_int8(key, value, key_cache, value_cache, scales["k_scale"], scales["v_scale"],
-                                   _flat(attn_metadata.slot_mapping))
+                # (and a prompt that attends to them in flight takes them as the cache will hold them)
+                prompts = attn_metadata.prefill_metadata
+                rounded = ops.kv_append_int8(key, value, key_cache, value_cache, scales["k_scale"], scales["v_scale"],
+                                             _flat(attn_metadata.slot_mapping),
+                                             attn_metadata.num_prefill_tokens if prompts and _in_flight(kv_cache, prompts) else 0)
             elif key is not None and value is not None and not fuse_append:
                 # all new K/V of the step (prefill and decode tokens) go in with one launch (:790-799), that of the prompts where they
                 # attend to the keys and values in flight
@@ -626,7 +629,7 @@ class MetaAttentionImpl:
                 if not fp8_kv:
                     pk, pv = _rows_of(key, 0, num_prefill_query_tokens), _rows_of(value, 0, num_prefill_query_tokens)
                 if int8_kv:   # attend to what the cache will hold: the rows as quantize_sym returns them
-                    pk, pv = ops.quantize_sym(pk), ops.quantize_sym(pv)
+                    pk, pv = rounded if rounded is not None else (ops.quantize_sym(pk), ops.quantize_sym(pv))
                 elif fp8_kv:  # the prompt's keys and values after their round trip
                     pk, pv = fp8_prompt
                 self._varlen_inflight(query, pk, pv, prefill_meta, prefill_output, window_left, meta_kv=prefill_kv, append=late_append)

@@ -443,10 +443,11 @@ def alloc_int8_kv_cache(num_blocks: int, block_size: int, num_kv_heads: int, hea
 
 
 def kv_append_int8(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
-                   k_scale: torch.Tensor, v_scale: torch.Tensor, slot_mapping: torch.Tensor) -> None:
+                   k_scale: torch.Tensor, v_scale: torch.Tensor, slot_mapping: torch.Tensor, round_tokens: int = 0):
     """Quantise this step's K/V rows (per row: 128 signed bytes + one fp32 scale) and store them at
-    their slots; slots < 0 are skipped. Caches int8 [nb, bs, Hkv, 128], scales fp32 [nb, Hkv, bs]."""
-    if key.is_cuda and k_scale is not None and v_scale is not None and \
+    their slots; slots < 0 are skipped. Caches int8 [nb, bs, Hkv, 128], scales fp32 [nb, Hkv, bs].
+    round_tokens > 0: returns (quantize_sym(key[:round_tokens]), quantize_sym(value[:round_tokens])) of the same launch."""
+    if round_tokens == 0 and key.is_cuda and k_scale is not None and v_scale is not None and \
             _done(N.calls().append(key, value, k_cache, v_cache, slot_mapping, k_scale, v_scale, N.stream_ptr(key.device)),
                   "kv_append_int8") is not None:
         return
@@ -475,6 +476,13 @@ def kv_append_int8(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor
         value_stride_token=value.stride(0), value_stride_head=value.stride(1),
         cache_stride_block=k_cache.stride(0), cache_stride_row=k_cache.stride(1), cache_stride_head=k_cache.stride(2),
         stream=N.stream_ptr(dev))
+    if round_tokens > 0:
+        if round_tokens > T:
+            raise ValueError(f"{round_tokens} tokens to round of {T}")
+        out = torch.empty((2, round_tokens, Hkv, D), dtype=key.dtype, device=dev)
+        k_out, v_out = out[0], out[1]
+        N.check(N.lib().sb_kv_append_int8_round(C.byref(a), N.ptr(k_out), N.ptr(v_out), round_tokens), "kv_append_int8")
+        return k_out, v_out
     N.check(N.lib().sb_kv_append_int8(C.byref(a)), "kv_append_int8")
 
 

@@ -98,3 +98,23 @@ def test_layer_call_under_capture(sb, dev, kv):
         torch.cuda.synchronize()
         assert torch.equal(out, want) and all(torch.equal(a, b) for a, b in zip(held(c2), held(c0)))
     sb.ops.release_graph_workspace()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,rounded,heads", [(1, 1, 1), (9, 4, 4), (70, 70, 5), (33, 31, 2)])
+def test_append_that_rounds(sb, dev, dtype, T, rounded, heads):
+    """The rows of a prompt as the INT8 cache holds them, from the append's own launch: the bits of append and round trips by themselves."""
+    gen = torch.Generator().manual_seed(T)
+    key, value = (torch.randn(T, 3 * heads, D, generator=gen).to(dtype).to(dev)[:, heads:2 * heads] for _ in range(2))
+    key[0, 0] = 0
+    value[T - 1] *= 1e4
+    slots = torch.randperm(96, generator=gen)[:T].to(dev)
+    slots[T // 2] = -1
+    codes, scales = torch.zeros(2, 6, PAGE, heads, D, dtype=torch.int8, device=dev), torch.zeros(2, 6, heads, PAGE, device=dev)
+    c1, s1 = codes.clone(), scales.clone()
+    sb.ops.kv_append_int8(key, value, codes[0], codes[1], scales[0], scales[1], slots)
+    k, v = sb.ops.kv_append_int8(key, value, c1[0], c1[1], s1[0], s1[1], slots, rounded)
+    assert torch.equal(c1, codes) and torch.equal(s1, scales) and k.shape == (rounded, heads, D)
+    assert torch.equal(k, sb.ops.quantize_sym(key[:rounded])) and torch.equal(v, sb.ops.quantize_sym(value[:rounded]))
+    with pytest.raises(ValueError):
+        sb.ops.kv_append_int8(key, value, c1[0], c1[1], s1[0], s1[1], slots, T + 1)
