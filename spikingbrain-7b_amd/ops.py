@@ -1108,6 +1108,9 @@ def _window_shift_args(src: Optional[torch.Tensor], dst: torch.Tensor, fresh: Op
     B, H, cap_d, D = dst.shape
     if not dst.is_contiguous() or (src is not None and not src.is_contiguous()):
         raise ValueError("window_shift needs contiguous [B, H, cap, D] storage")
+    if src is not None and (src.dtype != dst.dtype or src.shape[:2] != (B, H) or src.shape[3] != D or
+                            not 0 <= src_row0 <= src_row0 + keep_rows <= src.shape[2]):
+        raise ValueError("src must be [B, H, n, D] of the cache dtype and hold the rows that are kept")
     esz = dst.element_size()
     n_new = 0 if fresh is None else fresh.shape[2]
     if fresh is not None:
