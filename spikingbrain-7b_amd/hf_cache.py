@@ -124,10 +124,12 @@ class Cache(_HFCache):
     ) -> Dict[str, Any]:
         """Same contract as cache.py:40-112. `attn_state` = (key, value), each [B, Hkv, n, D];
         `cache_kwargs['window_size']` bounds the stored rows (None = unbounded)."""
-        return self._update(ops.window_shift_pair, recurrent_state, attn_state, conv_state, layer_idx, offset, cache_kwargs)
+        return self._update(lambda k_copy, v_copy, rows: ops.window_shift_pair(k_copy, v_copy), recurrent_state, attn_state, conv_state,
+                            layer_idx, offset, cache_kwargs)
 
     def _update(self, push, recurrent_state, attn_state, conv_state, layer_idx, offset, cache_kwargs) -> Dict[str, Any]:
-        """`update`, with push(k_copy, v_copy) in place of ops.window_shift_pair for the rows of a layer that is there already."""
+        """`update`, with push(k_copy, v_copy, (keys, values)) in place of ops.window_shift_pair for the rows of a layer that is there
+        already: it makes the copies, after which keys and values are the layer's rows. Where it raises, the layer stays as it was."""
         if layer_idx == 0:
             self._seen_tokens += offset  # cache.py:70-71: only layer 0 counts tokens
 
@@ -169,9 +171,10 @@ class Cache(_HFCache):
                         "slice-assign would fail with a shape mismatch here")
                 k_copy, kb = self._push(kb, attn_state[0], drop, window_size)
                 v_copy, vb = self._push(vb, attn_state[1], drop, window_size)
-                push(k_copy, v_copy)
+                rows = (kb.view(), vb.view())
+                push(k_copy, v_copy, rows)
                 self._buffers[layer_idx] = (kb, vb)
-                state["attn_state"] = (kb.view(), vb.view())
+                state["attn_state"] = rows
             if conv_state is not None:
                 state["conv_state"] = conv_state
         return state

@@ -69,41 +69,57 @@ def sliding_window_attention(
     if flavour not in ("flash", "sdpa"):
         raise ValueError("flavour must be 'flash' or 'sdpa'")
     B, Hq, Q, D = query_states.shape
-    Hkv = key_states.shape[1]
-
-    push = []   # a copy into the cache that is still to be made
+    if window_left is None:
+        window_left = sliding_window if flavour == "flash" else sliding_window - 1
     if past_key_values is not None:
         cache_has_content = past_key_values.get_seq_length(layer_idx) > 0
         if cache_window_size == -1:
             cache_kwargs = {"window_size": sliding_window} if flavour == "flash" else {}
         else:
             cache_kwargs = {"window_size": cache_window_size}
-        if Q == 1 and cache_has_content and type(past_key_values) is Cache and query_states.is_cuda:
-            # the new rows' copy goes with the attention's first launch, below
-            key_cached, value_cached = past_key_values._update(
-                lambda *copies: push.extend(copies), None, (key_states, value_states), None, layer_idx, Q, cache_kwargs)["attn_state"]
-        else:
-            key_cached, value_cached = past_key_values.update(
-                attn_state=(key_states, value_states), layer_idx=layer_idx, offset=Q,
-                cache_kwargs=cache_kwargs)["attn_state"]
+        if Q == 1 and cache_has_content and query_states.is_cuda and type(past_key_values) is Cache and \
+                getattr(past_key_values.update, "__func__", None) is _UPDATE:
+            return _decode_step(past_key_values, layer_idx, query_states, key_states, value_states, attention_mask, window_left, cache_kwargs)
+        key_cached, value_cached = past_key_values.update(
+            attn_state=(key_states, value_states), layer_idx=layer_idx, offset=Q,
+            cache_kwargs=cache_kwargs)["attn_state"]
         if cache_has_content:
             key_states, value_states = key_cached, value_cached
 
-    K = key_states.shape[2]
-    if window_left is None:
-        window_left = sliding_window if flavour == "flash" else sliding_window - 1
-
     if Q == 1 and query_states.is_cuda:
-        try:
-            out = ops.dense_decode(query_states, key_states, value_states, attention_mask, window_left, D ** -0.5, push or None)
-        except Exception:   # (the cache counts the rows already)
-            if push:
-                ops.window_shift_pair(*push)
-            raise
+        out = ops.dense_decode(query_states, key_states, value_states, attention_mask, window_left, D ** -0.5)
         if out is not None:
             return out
-        if push:
-            ops.window_shift_pair(*push)
+    return _attend(query_states, key_states, value_states, attention_mask, window_left)
+
+
+_UPDATE = Cache.update   # (a cache with another one is updated through that)
+
+
+def _decode_step(cache: Cache, layer_idx: int, q, key, value, mask, window_left: int, cache_kwargs) -> torch.Tensor:
+    """One new token against a cache that has rows: their copy into the window goes with the attention's first launch. Refused rows leave
+    the cache as it was; where the rows are fine and the attention fails, they are in the cache, as after an `update` by itself."""
+    out = failure = None
+
+    def push(k_copy, v_copy, rows):
+        nonlocal out, failure
+        try:
+            out = ops.dense_decode(q, *rows, mask, window_left, q.shape[3] ** -0.5, (k_copy, v_copy))
+        except Exception as e:
+            failure = e
+        if out is None:
+            ops.window_shift_pair(k_copy, v_copy)
+
+    rows = cache._update(push, None, (key, value), None, layer_idx, 1, cache_kwargs)["attn_state"]
+    if failure is not None:
+        raise failure
+    return out if out is not None else _attend(q, *rows, mask, window_left)
+
+
+def _attend(query_states, key_states, value_states, attention_mask, window_left: int) -> torch.Tensor:
+    """The queries [B, Hq, Q, D] are the last Q of the keys' [B, Hkv, K, D] positions; returns [B, Q, Hq, D]."""
+    B, Hq, Q, D = query_states.shape
+    Hkv, K = key_states.shape[1], key_states.shape[2]
     k, v = key_states, value_states
     if k.stride(3) != 1 or v.stride() != k.stride() or _kv_step_rows(k) is None:
         k, v = k.contiguous(), v.contiguous()
