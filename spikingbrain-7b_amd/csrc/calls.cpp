@@ -1,9 +1,10 @@
 // The ordinary forms of the layer calls, from torch tensors to the C ABI in one step. A layer call of a small batch costs
 // more host time than GPU time, and most of it is the interpreter reading tensors attribute by attribute and filling
 // an argument structure field by field (one sequence's sliding-window decode layer 27.5 us that way and 12.8 this way, four
-// sequences' linear-attention step 14.7 and 6.3, a Hugging Face layer of four sequences 51 and 23). A function here takes the call if the tensors have the form it knows, with the checks of its counterpart in ops.py; for any
-// other it returns None and does nothing, and the caller goes on to that counterpart, which accepts more and says what is
-// wrong with the rest. Nothing is kept between calls.
+// sequences' linear-attention step 14.7 and 6.3, a Hugging Face layer of four sequences 52 and 21). A function here takes the call
+// if the tensors have the form it knows, with the checks of its counterpart in ops.py; for any other it returns None and
+// does nothing, and the caller goes on to that counterpart, which accepts more and says what is wrong with the rest. Nothing
+// is kept between calls.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -11,6 +12,7 @@
 
 #include <cmath>
 #include <cstring>
+#include <vector>
 
 #include "sbcache.h"
 
@@ -110,15 +112,46 @@ bool both_scales(const Tensor *ks, const Tensor *vs, const Pages &c, const float
   return true;
 }
 
-// Whether `ws` can hold this split's partial results, outside a stream capture (a capture's scratch memory belongs to its graph)
-bool workspace_fits(const Tensor *ws, size_t bytes, void *stream) {
-  if (bytes == 0) return true;
-  uint64_t capture = 0;
-  return ws && ws->scalar_type() == at::kByte && (size_t)ws->numel() >= bytes && sb_stream_capture_id(stream, &capture) == SB_OK && capture == 0;
+PyObject *not_taken() { Py_RETURN_NONE; }
+
+// What a call came to: not taken, a status, or (status 0) a tensor
+struct Result {
+  int rc = 0;
+  Tensor out = {};
+  bool taken = true;
+};
+
+// Lets go of the interpreter lock for allocations and library calls, as ctypes does for the general forms: a launch waits where the
+// stream's queue is full, an allocation where memory has to be given back first, and other Python threads run on meanwhile. What
+// `go` needs of the caller's tensors is read before.
+template <typename Go>
+PyObject *unlocked(Go go) {
+  Result r;
+  {
+    struct Unlock {
+      PyThreadState *const state = PyEval_SaveThread();
+      ~Unlock() { PyEval_RestoreThread(state); }
+    } unlock;
+    r = go();
+  }
+  if (!r.taken) return not_taken();
+  return r.rc || !r.out.defined() ? PyLong_FromLong(r.rc) : THPVariable_Wrap(std::move(r.out));
 }
 
-PyObject *not_taken() { Py_RETURN_NONE; }
-PyObject *status(int rc) { return PyLong_FromLong(rc); }
+// The caller's scratch memory, if any
+struct Scratch {
+  void *ptr = nullptr;
+  size_t bytes = 0;
+  explicit Scratch(const Tensor *t) {
+    if (t && t->scalar_type() == at::kByte) { ptr = t->data_ptr(); bytes = (size_t)t->numel(); }
+  }
+  // Whether it can hold `need` bytes of partial results, outside a stream capture (a capture's scratch memory belongs to its graph)
+  bool holds(size_t need, void *stream) const {
+    if (need == 0) return true;
+    uint64_t capture = 0;
+    return ptr && bytes >= need && sb_stream_capture_id(stream, &capture) == SB_OK && capture == 0;
+  }
+};
 
 template <PyObject *(*F)(Args &)>
 PyObject *call(PyObject *, PyObject *const *a, Py_ssize_t n) {
@@ -142,7 +175,7 @@ PyObject *decode(Args &in) {
   const double scale = in.number();
   int64_t longest = in.integer();
   const int64_t want_balanced = in.integer();
-  const Tensor *ws = in.maybe_tensor();
+  const Tensor *const workspace = in.maybe_tensor();
   void *const stream = in.address();
   Pages c;
   if (!in.ok || q->dim() != 3 || !half_type(*q) || !inner_contiguous(*q) || !c.from(kc, vc)) return not_taken();
@@ -172,12 +205,12 @@ PyObject *decode(Args &in) {
                        : sb_swa_decode_auto_split(R, (int)c.heads, (int)longest, (int)window);
   if (balanced && split < 2) split = 2;
   const size_t bytes = sb_swa_decode_workspace_bytes(R, (int)Hq, (int)D, split);
-  if (!workspace_fits(ws, bytes, stream)) return not_taken();
+  const Scratch ws(workspace);
   sb_swa_decode_args a;
   std::memset(&a, 0, sizeof a);
   a.q = q->data_ptr(); a.k_cache = const_cast<char *>(c.k); a.v_cache = const_cast<char *>(c.v); a.out = out->data_ptr();
   a.block_table = table->data_ptr<int32_t>(); a.seq_lens = lens->data_ptr<int32_t>();
-  if (bytes) { a.workspace = ws->data_ptr(); a.workspace_bytes = (size_t)ws->numel(); }
+  if (bytes) { a.workspace = ws.ptr; a.workspace_bytes = ws.bytes; }
   a.num_rows = R; a.num_q_heads = (int)Hq; a.num_kv_heads = (int)c.heads; a.head_size = (int)D; a.block_size = (int)c.bs;
   a.window_left = (int)window; a.max_seq_len = (int)longest; a.n_split = split; a.dtype = code_of(q->scalar_type());
   a.flags = want_balanced ? SB_DECODE_BALANCED : 0;
@@ -193,7 +226,10 @@ PyObject *decode(Args &in) {
   a.kv_quant = (int)quant;
   a.k_scale = k_scale; a.v_scale = v_scale;
   if (quant == SB_KV_FP8) { a.k_scale_tensor = (float)kst; a.v_scale_tensor = (float)vst; }
-  return status(codes && nk ? sb_swa_decode_append_codes(&a, (float)q_scale) : sb_swa_decode(&a));
+  return unlocked([&]() -> Result {
+    if (!ws.holds(bytes, stream)) return {.taken = false};
+    return {codes && nk ? sb_swa_decode_append_codes(&a, (float)q_scale) : sb_swa_decode(&a)};
+  });
 }
 
 // The fields of an element append; false where the tensors are not of the ordinary form
@@ -228,7 +264,7 @@ PyObject *append(Args &in) {
   if (!ks && !vs) {
     sb_kv_append_args a;
     if (!fill_append(a, *key, *value, c, *slots, stream)) return not_taken();
-    return status(sb_kv_append(&a));
+    return unlocked([&]() -> Result { return {sb_kv_append(&a)}; });
   }
   if (c.type != at::kChar || !scales_of(ks, c.nb, H, c.bs) || !scales_of(vs, c.nb, H, c.bs)) return not_taken();
   sb_kv_append_int8_args a;
@@ -241,7 +277,7 @@ PyObject *append(Args &in) {
   a.value_stride_token = value->stride(0); a.value_stride_head = value->stride(1);
   a.cache_stride_block = c.s_block; a.cache_stride_row = c.s_row; a.cache_stride_head = c.s_head;
   a.stream = stream;
-  return status(sb_kv_append_int8(&a));
+  return unlocked([&]() -> Result { return {sb_kv_append_int8(&a)}; });
 }
 
 // prefill(q, k, v, out, cu_seqlens_q, seq_lens_k, tile_seq, tile_q0, block_table | None, kv_start | None, kv_start32 | None, num_tiles,
@@ -300,21 +336,25 @@ PyObject *prefill(Args &in) {
   Pages c;
   if (nk && (!nv || !cache || !slots || !c.from(cache, nullptr) || !fill_append(ap, *nk, *nv, c, *slots, stream))) return not_taken();
   const int parts = sb_swa_prefill_parts(&a, max_k);
-  auto go = [&](void *ws, size_t bytes) {
-    return status(nk ? sb_swa_prefill_append(&a, &ap, total_q, max_k, parts, ws, bytes) : sb_swa_prefill_parted(&a, total_q, max_k, parts, ws, bytes));
-  };
-  if (parts < 2) return go(nullptr, 0);
-  const size_t bytes = sb_swa_prefill_workspace_bytes(&a, total_q, parts);
-  const Tensor ws = at::empty({(int64_t)bytes}, q->options().dtype(at::kByte));
-  if (!plain(ws)) return not_taken();
-  return go(ws.data_ptr(), bytes);
+  const at::TensorOptions raw = q->options().dtype(at::kByte);
+  return unlocked([&]() -> Result {
+    Tensor ws;
+    size_t bytes = 0;
+    if (parts > 1) {
+      bytes = sb_swa_prefill_workspace_bytes(&a, total_q, parts);
+      ws = at::empty({(int64_t)bytes}, raw);
+      if (!plain(ws)) return {.taken = false};
+    }
+    void *const at = parts > 1 ? ws.data_ptr() : nullptr;
+    return {nk ? sb_swa_prefill_append(&a, &ap, total_q, max_k, parts, at, bytes) : sb_swa_prefill_parted(&a, total_q, max_k, parts, at, bytes)};
+  });
 }
 
 // What the two linear-attention calls share, once their shapes are known
-void fill_gla(sb_gla_recurrent_args &a, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &g, const Tensor &state, const Tensor &out,
+void fill_gla(sb_gla_recurrent_args &a, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &g, const Tensor &state,
               const Tensor *slots, double scale, int flags, void *stream) {
   std::memset(&a, 0, sizeof a);
-  a.q = q.data_ptr(); a.k = k.data_ptr(); a.v = v.data_ptr(); a.g = g.data_ptr(); a.state = state.data_ptr(); a.out = out.data_ptr();
+  a.q = q.data_ptr(); a.k = k.data_ptr(); a.v = v.data_ptr(); a.g = g.data_ptr(); a.state = state.data_ptr();
   if (slots) a.slot_idx = slots->data_ptr<int32_t>();
   a.head_dim = 128; a.dtype = code_of(q.scalar_type()); a.g_dtype = code_of(g.scalar_type()); a.state_dtype = code_of(state.scalar_type());
   a.scale = (float)scale;
@@ -339,18 +379,22 @@ PyObject *gla_step(Args &in) {
   if (!shaped(*k, {B, Hk, 1, 128}) || v->sizes() != k->sizes() || g->sizes() != k->sizes() || !gla_types(*q, *k, *v, *g, *state, H, Hk) ||
       (slots ? !vector_of(*slots, at::kInt, B) : state->size(0) < B))
     return not_taken();
-  Tensor out = at::empty({B, H, 128}, q->options());
-  if (!plain(out)) return not_taken();
   sb_gla_recurrent_args a;
-  fill_gla(a, *q, *k, *v, *g, *state, out, slots, scale, SB_GLA_ZERO_SKIPPED, stream);
+  fill_gla(a, *q, *k, *v, *g, *state, slots, scale, SB_GLA_ZERO_SKIPPED, stream);
   a.batch = B; a.num_heads = (int)H; a.seq_len = 1; a.q_heads_per_state = (int)(H / Hk);
   a.q_stride_b = q->stride(0); a.q_stride_h = q->stride(1); a.q_stride_t = q->stride(2);
   a.k_stride_b = k->stride(0); a.k_stride_h = k->stride(1); a.k_stride_t = k->stride(2);
   a.v_stride_b = v->stride(0); a.v_stride_h = v->stride(1); a.v_stride_t = v->stride(2);
   a.g_stride_b = g->stride(0); a.g_stride_h = g->stride(1); a.g_stride_t = g->stride(2);
   a.out_stride_b = H * 128; a.out_stride_h = 128; a.out_stride_t = 128;
-  const int rc = sb_gla_recurrent(&a);
-  return rc ? status(rc) : THPVariable_Wrap(std::move(out));
+  const at::TensorOptions like = q->options();
+  return unlocked([&]() -> Result {
+    Tensor out = at::empty({B, H, 128}, like);
+    if (!plain(out)) return {.taken = false};
+    a.out = out.data_ptr();
+    const int rc = sb_gla_recurrent(&a);
+    return {rc, std::move(out)};
+  });
 }
 
 // gla_packed(args, q, k, v, g [tokens, heads, 128], state, cu_seqlens, slots | None, scale, max_seq_len (0: the mean), stream): fills the
@@ -367,15 +411,19 @@ PyObject *gla_packed(Args &in) {
       !vector_of(*cu, at::kInt, 2) || (slots ? !vector_of(*slots, at::kInt, B) : state->size(0) < B) || longest < 0 || longest > INT32_MAX ||
       T > INT32_MAX)
     return not_taken();
-  Tensor out = at::empty({T, H, 128}, q->options());
-  if (!plain(out)) return not_taken();
-  fill_gla(*a, *q, *k, *v, *g, *state, out, slots, scale, 0, stream);
+  fill_gla(*a, *q, *k, *v, *g, *state, slots, scale, 0, stream);
   a->batch = B; a->num_heads = (int)H; a->seq_len = (int)(longest ? longest : (T + B - 1) / B); a->q_heads_per_state = (int)(H / Hk);
   a->cu_seqlens = cu->data_ptr<int32_t>();
   a->q_stride_h = q->stride(1); a->q_stride_t = q->stride(0); a->k_stride_h = k->stride(1); a->k_stride_t = k->stride(0);
   a->v_stride_h = v->stride(1); a->v_stride_t = v->stride(0); a->g_stride_h = g->stride(1); a->g_stride_t = g->stride(0);
   a->out_stride_h = 128; a->out_stride_t = H * 128;
-  return THPVariable_Wrap(std::move(out));
+  const at::TensorOptions like = q->options();
+  return unlocked([&]() -> Result {
+    Tensor out = at::empty({T, H, 128}, like);
+    if (!plain(out)) return {.taken = false};
+    a->out = out.data_ptr();
+    return {0, std::move(out)};
+  });
 }
 
 // Rows [row, row + n) of both window buffers [B, H, capacity, D] take the n new rows of key and value [B, H, n, D]; false where the tensors
@@ -404,7 +452,7 @@ PyObject *push(Args &in) {
   void *const stream = in.address();
   sb_window_shift_args a[2];
   if (!in.ok || !fill_push(a, storage, fresh, row, stream)) return not_taken();
-  return status(sb_window_shift_pair(&a[0], &a[1]));
+  return unlocked([&]() -> Result { return {sb_window_shift_pair(&a[0], &a[1])}; });
 }
 
 // dense_decode(q [B, Hq, 1, D], k, v [B, Hkv, K, D], mask | None, window_left, scale, k_storage | None, v_storage | None, key | None,
@@ -416,7 +464,7 @@ PyObject *dense_decode(Args &in) {
   const double scale = in.number();
   const Tensor *storage[2] = {in.maybe_tensor(), in.maybe_tensor()}, *fresh[2] = {in.maybe_tensor(), in.maybe_tensor()};
   const int64_t row = in.integer();
-  const Tensor *ws = in.maybe_tensor();
+  const Tensor *const workspace = in.maybe_tensor();
   void *const stream = in.address();
   sb_window_shift_args shift[2];
   if (in.ok && storage[0] && (!storage[1] || !fresh[0] || !fresh[1] || !fill_push(shift, storage, fresh, row, stream))) return not_taken();
@@ -441,32 +489,21 @@ PyObject *dense_decode(Args &in) {
     if (balanced && split < 2) split = 2;
   }
   const size_t bytes = sb_swa_decode_workspace_bytes(B, (int)Hq, (int)D, split);
-  if (!workspace_fits(ws, bytes, stream)) return not_taken();
-  // [kv_start, then as 32 bits lengths, sequence numbers, padding]
-  const Tensor rows = at::empty({B + (3 * B + 1) / 2}, q->options().dtype(at::kLong));
-  Tensor out = at::empty({B, 1, Hq, D}, q->options());
-  if (!plain(rows) || !plain(out)) return not_taken();
-  int64_t *const starts = rows.data_ptr<int64_t>();
-  int32_t *const lens = reinterpret_cast<int32_t *>(starts + B);
+  const Scratch ws(workspace);
   sb_dense_rows_args d;
   std::memset(&d, 0, sizeof d);
-  d.seq_lens = lens; d.row_seq = lens + B; d.kv_start = starts;
   d.batch = B; d.num_queries = 1; d.num_keys = K; d.kv_step = B == 1 ? 0 : k->stride(0) / k->stride(2);
   d.mask_elem_bytes = 1;
   if (mask) {   // its last K columns
     const int64_t cols = mask->size(1) < K ? mask->size(1) : K;
     d.mask = static_cast<const char *>(mask->data_ptr()) + (mask->size(1) - cols) * mask->stride(1) * (int64_t)mask->element_size();
-    d.key_lo = lens + 2 * B;
     d.mask_cols = cols; d.mask_stride_row = mask->stride(0); d.mask_stride_col = mask->stride(1); d.mask_elem_bytes = (int)mask->element_size();
   }
   d.stream = stream;
-  if (const int rc = storage[0] ? sb_dense_step(&shift[0], &shift[1], &d) : sb_dense_rows(&d)) return status(rc);
   sb_swa_decode_args a;
   std::memset(&a, 0, sizeof a);
-  a.q = q->data_ptr(); a.k_cache = k->data_ptr(); a.v_cache = v->data_ptr(); a.out = out.data_ptr();
-  a.kv_start = starts; a.row_seq = lens + B; a.seq_lens = lens;
-  if (mask) a.key_lo = lens + 2 * B;
-  if (bytes) { a.workspace = ws->data_ptr(); a.workspace_bytes = (size_t)ws->numel(); }
+  a.q = q->data_ptr(); a.k_cache = k->data_ptr(); a.v_cache = v->data_ptr();
+  if (bytes) { a.workspace = ws.ptr; a.workspace_bytes = ws.bytes; }
   a.num_rows = B; a.num_q_heads = (int)Hq; a.num_kv_heads = (int)Hkv; a.head_size = (int)D; a.block_size = 16;
   a.window_left = (int)window; a.max_seq_len = (int)K; a.n_split = split; a.dtype = code_of(q->scalar_type());
   a.flags = balanced ? SB_DECODE_BALANCED : 0;
@@ -475,8 +512,24 @@ PyObject *dense_decode(Args &in) {
   a.kv_stride_row = k->stride(2); a.kv_stride_head = k->stride(1);
   a.stream = stream;
   a.kv_quant = SB_KV_NONE;
-  const int rc = sb_swa_decode(&a);
-  return rc ? status(rc) : THPVariable_Wrap(std::move(out));
+  const at::TensorOptions like = q->options();
+  const bool masked = mask != nullptr, pushes = storage[0] != nullptr;
+  return unlocked([&]() -> Result {
+    if (!ws.holds(bytes, stream)) return {.taken = false};
+    // [kv_start, then as 32 bits lengths, sequence numbers, padding]
+    const Tensor rows = at::empty({B + (3 * B + 1) / 2}, like.dtype(at::kLong));
+    Tensor out = at::empty({B, 1, Hq, D}, like);
+    if (!plain(rows) || !plain(out)) return {.taken = false};
+    d.kv_start = rows.data_ptr<int64_t>();
+    d.seq_lens = reinterpret_cast<int32_t *>(d.kv_start + B);
+    d.row_seq = d.seq_lens + B;
+    if (masked) d.key_lo = d.seq_lens + 2 * B;
+    a.kv_start = d.kv_start; a.seq_lens = d.seq_lens; a.row_seq = d.row_seq; a.key_lo = d.key_lo;
+    a.out = out.data_ptr();
+    int rc = pushes ? sb_dense_step(&shift[0], &shift[1], &d) : sb_dense_rows(&d);
+    if (rc == SB_OK) rc = sb_swa_decode(&a);
+    return {rc, std::move(out)};
+  });
 }
 
 // append_fp8(key | None, value | None, k_cache | None, v_cache | None, slots | None, k_scale, v_scale, query, query scale, stream):
@@ -506,14 +559,19 @@ PyObject *append_fp8(Args &in) {
     a.cache_stride_block = c.s_block; a.cache_stride_row = c.s_row; a.cache_stride_head = c.s_head;
     a.k_scale = (float)k_scale; a.v_scale = (float)v_scale; a.stream = stream;
   }
-  Tensor out = at::empty_like(*x);
-  if (!plain(out) || out.strides() != x->strides()) return not_taken();
   sb_fp8_round_args r;
   std::memset(&r, 0, sizeof r);
-  r.in = x->data_ptr(); r.out = out.data_ptr(); r.row_elems = r.in_stride_row = r.out_stride_row = x->size(-1);
+  r.in = x->data_ptr(); r.row_elems = r.in_stride_row = r.out_stride_row = x->size(-1);
   r.rows = x->numel() / x->size(-1); r.dtype = code_of(x->scalar_type()); r.scale = (float)x_scale;
-  const int rc = sb_fp8_step(key ? &a : nullptr, &r, 1, stream);
-  return rc ? status(rc) : THPVariable_Wrap(std::move(out));
+  const at::TensorOptions like = x->options();
+  const std::vector<int64_t> sizes = x->sizes().vec(), strides = x->strides().vec();
+  return unlocked([&]() -> Result {
+    Tensor out = at::empty(sizes, like);
+    if (!plain(out) || out.strides() != at::IntArrayRef(strides)) return {.taken = false};
+    r.out = out.data_ptr();
+    const int rc = sb_fp8_step(key ? &a : nullptr, &r, 1, stream);
+    return {rc, std::move(out)};
+  });
 }
 
 #define SB_CALL(f) {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&call<f>)), METH_FASTCALL, nullptr}
