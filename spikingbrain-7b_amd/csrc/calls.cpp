@@ -193,6 +193,7 @@ PyObject *decode(Args &in) {
   if (!nk && (nv || slots)) return not_taken();
   const bool codes = quant != SB_KV_NONE;
   if (codes ? (q_scale >= 0.0) != (nk != nullptr) : q_scale >= 0.0) return not_taken();
+  if (q_scale > 0.0 && !((float)q_scale > 0.f)) return not_taken();   // (0 as 32 bits would mean no round trip)
   if (nk && (!nv || !slots || nk->dim() != 3 || nk->size(0) != R || nk->size(1) != c.heads || nk->size(2) != D ||
              nv->sizes() != nk->sizes() || nk->scalar_type() != q->scalar_type() || nv->scalar_type() != q->scalar_type() || !inner_contiguous(*nk) ||
              !inner_contiguous(*nv) || !vector_of(*slots, at::kLong, R)))

@@ -264,6 +264,8 @@ def swa_decode_attention(
         raise ValueError("q and the caches must share one dtype")
     if append_codes is not None and (not int8_kv or new_key is None):
         raise ValueError("append_codes goes with a byte-code cache and new_key")
+    if append_codes is not None and append_codes > 0.0 and not C.c_float(append_codes).value > 0.0:
+        raise ValueError(f"append_codes {append_codes}: no positive scale in 32 bits")
     if block_table is not None:
         if key_cache.dim() != 4 or value_cache.shape != key_cache.shape:
             raise ValueError("paged caches must be [num_blocks, block_size, num_kv_heads, head_size]")
