@@ -163,6 +163,13 @@ PyObject *call(PyObject *, PyObject *const *a, Py_ssize_t n) {
   }
 }
 
+// decodes(q, k_cache): whether `decode` has a form for these queries and this cache, without looking at anything else
+PyObject *decodes(Args &in) {
+  const Tensor *q = in.tensor(), *kc = in.tensor();
+  const bool yes = in.ok && q->dim() == 3 && half_type(*q) && q->size(2) == 128 && kc->dim() == 4 && q->size(1) <= 16 * kc->size(2);
+  return PyBool_FromLong(yes);
+}
+
 // decode(q, k_cache, v_cache | None, out, seq_lens, block_table, new_key | None, new_value | None, slots | None, k_scale | None,
 // v_scale | None, kv_quant, k_scale_tensor, v_scale_tensor, q_scale (>= 0: the append over a byte-code cache; -1: none), window_left, scale,
 // max_seq_len (0: the table's), balanced, workspace | None, stream): ops.swa_decode_attention over a paged cache, one query row per sequence.
@@ -576,7 +583,7 @@ PyObject *append_fp8(Args &in) {
 }
 
 #define SB_CALL(f) {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&call<f>)), METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {SB_CALL(decode),   SB_CALL(append), SB_CALL(prefill),      SB_CALL(gla_step),
+PyMethodDef methods[] = {SB_CALL(decodes),    SB_CALL(decode), SB_CALL(append),       SB_CALL(prefill),    SB_CALL(gla_step),
                          SB_CALL(gla_packed), SB_CALL(push),   SB_CALL(dense_decode), SB_CALL(append_fp8), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_calls", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

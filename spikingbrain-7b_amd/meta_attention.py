@@ -482,7 +482,7 @@ class MetaAttentionImpl:
         """query [T, Hq, D]; key/value [T, Hkv, D]; kv_cache [2, nb, bs, Hkv, D] (numel 0 for the
         profiling run); `output` [T, Hq, D] is written in place and returned (:703-982)."""
         assert output is not None, "Output tensor must be provided."
-        if output_scale is None and query2 is None and key2 is None and value2 is None and \
+        if output_scale is None and query2 is None and key2 is None and value2 is None and self.alibi_slopes is None and self.head_size == 128 and \
                 self._pure_decode(layer, query, key, value, kv_cache, attn_metadata, output):
             return output
         if output_scale is not None:
@@ -669,12 +669,14 @@ class MetaAttentionImpl:
         return output
 
     def _pure_decode(self, layer, query, key, value, kv_cache, meta, output) -> bool:
-        """The layer call of a step of decoding sequences only (one token each, no score options) in one native step; False, with
+        """The layer call of a step of decoding sequences only (one token each, no score options, head size 128) in one native step; False, with
         nothing done, for any other."""
+        if self.num_heads > 16 * self.num_kv_heads or self.logits_soft_cap > 0 or self.attn_type != AttentionType.DECODER or \
+                not query.is_cuda or query.dtype is torch.float32:
+            return False   # (forms the step does not have, like score slopes and other head sizes: an attempt would cost 3 us of a call's 25)
         n = meta.num_decode_tokens
         if meta.num_prefill_tokens or meta.num_prefills or n <= 0 or (meta.max_decode_query_len or 1) != 1 or meta.slot_mapping is None or \
-                key is None or value is None or self.attn_type != AttentionType.DECODER or self.alibi_slopes is not None or \
-                self.logits_soft_cap > 0 or not query.is_cuda or query.shape != (n, self.num_heads, self.head_size):
+                key is None or value is None or query.shape != (n, self.num_heads, self.head_size):
             return False
         k_scale, v_scale = float(getattr(layer, "_k_scale_float", 1.0)), float(getattr(layer, "_v_scale_float", 1.0))
         codes, how = kv_cache, ()

@@ -100,10 +100,10 @@ def kv_append(key: torch.Tensor, value: torch.Tensor, key_cache: torch.Tensor, v
     """Scatter key/value [T, Hkv, D] into the paged caches [nb, bs, Hkv, D] at slot_mapping [T]
     (int64; negative = skip). Same contract as reshape_and_cache_flash at
     vllm_hymeta/attention/meta_attention.py:790-799 with an unquantised kv_cache_dtype."""
-    if key.is_cuda and _done(N.calls().append(key, value, key_cache, value_cache, slot_mapping, None, None, N.stream_ptr(key.device)),
-                             "kv_append") is not None:
+    stream = N.stream_ptr(key.device) if key.is_cuda else None
+    if stream is not None and _done(N.calls().append(key, value, key_cache, value_cache, slot_mapping, None, None, stream), "kv_append") is not None:
         return
-    dev = N.require_gpu(key, value, key_cache, value_cache, slot_mapping)
+    N.require_gpu(key, value, key_cache, value_cache, slot_mapping)
     if key.dim() != 3 or value.shape != key.shape:
         raise ValueError(f"key/value must both be [num_tokens, num_kv_heads, head_size], got {tuple(key.shape)} "
                          f"and {tuple(value.shape)}")
@@ -133,7 +133,7 @@ def kv_append(key: torch.Tensor, value: torch.Tensor, key_cache: torch.Tensor, v
         key_stride_token=key.stride(0), key_stride_head=key.stride(1),
         value_stride_token=value.stride(0), value_stride_head=value.stride(1),
         cache_stride_block=key_cache.stride(0), cache_stride_row=key_cache.stride(1),
-        cache_stride_head=key_cache.stride(2), num_blocks=nb, stream=N.stream_ptr(dev))
+        cache_stride_head=key_cache.stride(2), num_blocks=nb, stream=stream)
     N.check(N.lib().sb_kv_append(C.byref(a)), "kv_append")
 
 
@@ -223,8 +223,9 @@ def swa_decode_attention(
     append_codes: the append into a byte-code cache in the same launch: new_key, new_value (elements of q's type) are quantised, stored
     at new_slot_mapping (negative: not, and the cache's own row counts) and attended to as those codes, the bits of kv_append_int8 /
     kv_append_fp8 before this call. Its value, positive over an fp8 cache only: q takes fp8_round with that scale first; 0 = not."""
-    if balanced is not None and block_table is not None and out is not None and n_split == 0 and (max_seq_len is None or max_seq_len > 0) and \
-            q.is_cuda and kv_start is None and row_seq is None and key_lo is None and kv_strides is None and meta_k is None and \
+    # (decodes: of sizes and a type that the native step has; other calls would pay 1.3 us of 14 for the attempt)
+    if balanced is not None and block_table is not None and out is not None and n_split == 0 and N.calls().decodes(q, key_cache) and \
+            (max_seq_len is None or max_seq_len > 0) and kv_start is None and row_seq is None and key_lo is None and kv_strides is None and meta_k is None and \
             meta_v is None and profile_events is None and alibi_slopes is None and softcap == 0.0 and phases == 0 and \
             (k_scale is None) == (v_scale is None) and (k_scale is None or fp8_scales is None) and \
             not (return_lse or force_valu or merge_in_kernel or per_segment or pipeline_depth):

@@ -71,13 +71,17 @@ def sliding_window_attention(
     B, Hq, Q, D = query_states.shape
     if window_left is None:
         window_left = sliding_window if flavour == "flash" else sliding_window - 1
+    # one new token of a few sequences, in a form that the native step has (ops.dense_decode, which would turn the others down at
+    # 2 us a call)
+    one_step = Q == 1 and D == 128 and B <= 64 and query_states.is_cuda and Hq <= 16 * key_states.shape[1] and \
+        (attention_mask is None or not attention_mask.dtype.is_floating_point)
     if past_key_values is not None:
         cache_has_content = past_key_values.get_seq_length(layer_idx) > 0
         if cache_window_size == -1:
             cache_kwargs = {"window_size": sliding_window} if flavour == "flash" else {}
         else:
             cache_kwargs = {"window_size": cache_window_size}
-        if Q == 1 and cache_has_content and query_states.is_cuda and type(past_key_values) is Cache and \
+        if one_step and cache_has_content and type(past_key_values) is Cache and \
                 getattr(past_key_values.update, "__func__", None) is _UPDATE:
             return _decode_step(past_key_values, layer_idx, query_states, key_states, value_states, attention_mask, window_left, cache_kwargs)
         key_cached, value_cached = past_key_values.update(
@@ -86,7 +90,7 @@ def sliding_window_attention(
         if cache_has_content:
             key_states, value_states = key_cached, value_cached
 
-    if Q == 1 and query_states.is_cuda:
+    if one_step:
         out = ops.dense_decode(query_states, key_states, value_states, attention_mask, window_left, D ** -0.5)
         if out is not None:
             return out

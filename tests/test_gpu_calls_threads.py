@@ -47,6 +47,7 @@ def test_other_threads_run_during_a_call(sb, dev, monkeypatch):
     kept = []
     _layer_calls(sb, dev)                                                  # (scratch memory, lazy imports)
     calls = _recorded(sb, monkeypatch, lambda: kept.append(_layer_calls(sb, dev)))
+    calls = [c for c in calls if c[0] != "decodes"]                         # (asks about tensors, launches nothing)
     assert {n for n, _, _ in calls} == {"append", "decode", "append_fp8", "prefill", "gla_step", "push", "dense_decode"}
     count, stop, started = [0], [], threading.Event()
 
