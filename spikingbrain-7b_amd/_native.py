@@ -8,6 +8,7 @@ from __future__ import annotations
 import ctypes as C
 import importlib.util
 import os
+import sys
 from typing import Optional
 
 import torch  # imported first on purpose: the library must bind to the HIP runtime torch loaded
@@ -268,7 +269,7 @@ def calls():
         lib()
         path = os.path.join(_HERE, "_calls.so")
         if not os.path.exists(path):
-            raise NativeLibraryError(f"{path} is missing: build it with `make -C {os.path.join(_HERE, 'csrc')}`")
+            raise NativeLibraryError(f"{path} is missing: build it with `make -C {os.path.join(_HERE, 'csrc')} calls PY={sys.executable}`")
         spec = importlib.util.spec_from_file_location("_calls", path)
         module = importlib.util.module_from_spec(spec)
         try:
