@@ -276,6 +276,9 @@ def calls():
             spec.loader.exec_module(module)
         except ImportError as e:
             raise NativeLibraryError(f"cannot load {path}: {e}") from e
+        if module.torch_version != str(torch.__version__):   # (tensors' fields are read where that torch has them)
+            raise NativeLibraryError(f"{path} was built against torch {module.torch_version}, this is {torch.__version__}: build it again with "
+                                     f"`make -C {os.path.join(_HERE, 'csrc')} calls PY={sys.executable}`")
         _calls_module = module
     return _calls_module
 

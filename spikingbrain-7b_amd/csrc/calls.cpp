@@ -594,5 +594,11 @@ PyMODINIT_FUNC PyInit__calls() {
     PyErr_SetString(PyExc_ImportError, "libsbcache.so has another ABI version than _calls.so was built for");
     return nullptr;
   }
-  return PyModule_Create(&module);
+  PyObject *const m = PyModule_Create(&module);
+  // (the accessors of at::Tensor are compiled in: another torch may lay its tensors out otherwise)
+  if (m && PyModule_AddStringConstant(m, "torch_version", SB_TORCH_VERSION) < 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
 }
