@@ -111,7 +111,7 @@ struct PrefillParams {
   int n_parts, part_chunks;
   float *ws_acc;
   float *ws_ml;
-  Append append;              // in-flight element calls: first = ~0u where there is none
+  Append append;              // tokens 0: none
 };
 
 // The walk of a tile in 32-key chunks: every chunk that holds a key some token of the tile can see.
@@ -224,14 +224,16 @@ __device__ __forceinline__ void append_rows(const PrefillParams &p, int64_t wave
 
 // ODD: the last group of heads may have one less (3 of 4, 1 of 2): a build of its own, because the second path costs
 // the kernel of two heads 5 % (16 : 8 heads, 2000 tokens behind 3000 95 -> 100 us).
-template <typename E, int NHEADS, int KVQ, bool PAGED, bool ODD, bool HALVES>
+// APPEND: with the append that rides along (in-flight elements): builds of their own, because its code and arguments in front cost
+// the calls without one 0.5 us (64 tokens, 28 : 4 heads 8.3 -> 8.8, behind 2000 18.7 -> 19.3; 8 : 8 5.4 -> 6.0).
+template <typename E, int NHEADS, int KVQ, bool PAGED, bool ODD, bool HALVES, bool APPEND>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * Shape<NHEADS, HALVES>::kWaves, 64 * Shape<NHEADS, HALVES>::kWaves),
                           amdgpu_waves_per_eu(2, 2)))
 void swa_prefill_kernel(const PrefillParams p) {
   using S = Shape<NHEADS, HALVES>;
   __shared__ __attribute__((aligned(16))) char smem_all[(HALVES ? 6 : 3) * kStage];  // ring(s) of three chunks, each [K|V]
 
-  if constexpr (!PAGED) {
+  if constexpr (APPEND) {
     if (blockIdx.x >= p.append.first) {   // (the whole workgroup, ahead of every barrier)
       if (blockIdx.y == 0)
         append_rows(p, (int64_t)(blockIdx.x - p.append.first) * S::kWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6),
@@ -810,23 +812,24 @@ __global__ __launch_bounds__(256) void swa_prefill_merge_kernel(const PrefillPar
   if (p.lse && d4 == 0) p.lse[rh] = L > 0.f ? (M + log2f(L)) * kLn2 : kNegInf;
 }
 
-template <typename E, int KVQ, bool PAGED>
+template <typename E, int KVQ, bool PAGED, bool APPEND = false>
 void launch_prefill_q(int nh, bool odd, bool halves, dim3 grid, hipStream_t st, const PrefillParams &p) {
   const dim3 b4(256), b8(512);
-  if (halves && nh == 1) hipLaunchKernelGGL((swa_prefill_kernel<E, 1, KVQ, PAGED, false, true>), grid, b8, 0, st, p);
-  else if (halves && odd) hipLaunchKernelGGL((swa_prefill_kernel<E, 2, KVQ, PAGED, true, true>), grid, b8, 0, st, p);
-  else if (halves) hipLaunchKernelGGL((swa_prefill_kernel<E, 2, KVQ, PAGED, false, true>), grid, b8, 0, st, p);
-  else if (nh == 1) hipLaunchKernelGGL((swa_prefill_kernel<E, 1, KVQ, PAGED, false, false>), grid, b4, 0, st, p);
-  else if (nh == 2 && odd) hipLaunchKernelGGL((swa_prefill_kernel<E, 2, KVQ, PAGED, true, false>), grid, b4, 0, st, p);
-  else if (nh == 2) hipLaunchKernelGGL((swa_prefill_kernel<E, 2, KVQ, PAGED, false, false>), grid, b4, 0, st, p);
-  else if (odd) hipLaunchKernelGGL((swa_prefill_kernel<E, 4, KVQ, PAGED, true, false>), grid, b8, 0, st, p);
-  else hipLaunchKernelGGL((swa_prefill_kernel<E, 4, KVQ, PAGED, false, false>), grid, b8, 0, st, p);
+  if (halves && nh == 1) hipLaunchKernelGGL((swa_prefill_kernel<E, 1, KVQ, PAGED, false, true, APPEND>), grid, b8, 0, st, p);
+  else if (halves && odd) hipLaunchKernelGGL((swa_prefill_kernel<E, 2, KVQ, PAGED, true, true, APPEND>), grid, b8, 0, st, p);
+  else if (halves) hipLaunchKernelGGL((swa_prefill_kernel<E, 2, KVQ, PAGED, false, true, APPEND>), grid, b8, 0, st, p);
+  else if (nh == 1) hipLaunchKernelGGL((swa_prefill_kernel<E, 1, KVQ, PAGED, false, false, APPEND>), grid, b4, 0, st, p);
+  else if (nh == 2 && odd) hipLaunchKernelGGL((swa_prefill_kernel<E, 2, KVQ, PAGED, true, false, APPEND>), grid, b4, 0, st, p);
+  else if (nh == 2) hipLaunchKernelGGL((swa_prefill_kernel<E, 2, KVQ, PAGED, false, false, APPEND>), grid, b4, 0, st, p);
+  else if (odd) hipLaunchKernelGGL((swa_prefill_kernel<E, 4, KVQ, PAGED, true, false, APPEND>), grid, b8, 0, st, p);
+  else hipLaunchKernelGGL((swa_prefill_kernel<E, 4, KVQ, PAGED, false, false, APPEND>), grid, b8, 0, st, p);
 }
 template <typename E>
 void launch_prefill(int kv_quant, int nh, bool odd, bool halves, dim3 grid, hipStream_t st, const PrefillParams &p) {
   if (kv_quant == SB_KV_INT8) launch_prefill_q<E, SB_KV_INT8, true>(nh, odd, halves, grid, st, p);
   else if (kv_quant == SB_KV_FP8) launch_prefill_q<E, SB_KV_FP8, true>(nh, odd, halves, grid, st, p);
   else if (p.block_table) launch_prefill_q<E, SB_KV_NONE, true>(nh, odd, halves, grid, st, p);
+  else if (p.append.tokens > 0) launch_prefill_q<E, SB_KV_NONE, false, true>(nh, odd, halves, grid, st, p);
   else launch_prefill_q<E, SB_KV_NONE, false>(nh, odd, halves, grid, st, p);
 }
 
@@ -1012,8 +1015,6 @@ int prefill(const sb_swa_prefill_args *a, int64_t max_keys, int n_parts, float *
     p.tile_seq = a->ordered_tile_seq;
     p.tile_q0 = a->ordered_tile_q0;
   }
-  p.append = Append{};
-  p.append.first = ~0u;
   p.n_parts = n_parts; p.part_chunks = (int)((chunks + n_parts - 1) / n_parts);
   p.ws_acc = ws_acc; p.ws_ml = ws_ml;
   p.meta_k = p.meta_v = nullptr;
@@ -1073,7 +1074,7 @@ int prefill(const sb_swa_prefill_args *a, int64_t max_keys, int n_parts, float *
     h0 += nh * groups;
     p.head_groups = groups;
     dim3 grid((unsigned)(per_xcd * 8 * a->num_kv_heads * groups), (unsigned)n_parts);
-    p.append.first = ~0u;
+    p.append = Append{};
     if (ap && p.head_begin == 0) {   // (the first launch takes it along)
       const int waves = nh == 4 || halves ? 8 : 4;
       const int64_t esz = 2;
