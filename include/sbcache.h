@@ -548,10 +548,12 @@ int sb_swa_prefill_plan(const int32_t *query_lens, const int32_t *seq_lens_k, in
  * after; calls whose scratch memory overlaps must be ordered), total_q being the packed query rows (cu_seqlens_q's last
  * entry). sb_swa_prefill_parted: the call. Every part keeps its softmax in fp32 and the parts are put together in fp32.
  * n_parts < 2: sb_swa_prefill with max_keys known (workspace unused). A walk longer than max_keys allows is still
- * walked whole. sb_swa_prefill_group_heads: how many query heads a workgroup of that call takes at most, 4 or 2 (same bits; where those of two
- * heads also halve their walk, the halves are put together in fp32). */
+ * walked whole. sb_swa_prefill_group_heads: how many query heads a workgroup of that call takes at most, 4 or 2 (same bits).
+ * sb_swa_prefill_halves: 1 where those of two heads also walk half of the keys with one half of their wavefronts and half with the other
+ * (the halves are put together in fp32), else 0. */
 int32_t sb_swa_prefill_parts(const sb_swa_prefill_args *args, int64_t max_keys);
 int32_t sb_swa_prefill_group_heads(const sb_swa_prefill_args *args, int64_t max_keys, int32_t n_parts);
+int32_t sb_swa_prefill_halves(const sb_swa_prefill_args *args, int64_t max_keys, int32_t n_parts);
 size_t sb_swa_prefill_workspace_bytes(const sb_swa_prefill_args *args, int64_t total_q, int32_t n_parts);
 int sb_swa_prefill_parted(const sb_swa_prefill_args *args, int64_t total_q, int64_t max_keys, int32_t n_parts,
                           void *workspace, size_t workspace_bytes);

@@ -210,6 +210,7 @@ EXPORTS = {
     "sb_swa_prefill_plan": (C.c_int, [C.POINTER(i32), C.POINTER(i32), i64, i64, vp, vp]),
     "sb_swa_prefill_parts": (i32, [C.POINTER(SwaPrefillArgs), i64]),
     "sb_swa_prefill_group_heads": (i32, [C.POINTER(SwaPrefillArgs), i64, i32]),
+    "sb_swa_prefill_halves": (i32, [C.POINTER(SwaPrefillArgs), i64, i32]),
     "sb_swa_prefill_workspace_bytes": (sz, [C.POINTER(SwaPrefillArgs), i64, i32]),
     "sb_swa_prefill_parted": (C.c_int, [C.POINTER(SwaPrefillArgs), i64, i64, i32, vp, sz]),
     "sb_swa_prefill_append": (C.c_int, [C.POINTER(SwaPrefillArgs), C.POINTER(KvAppendArgs), i64, i64, i32, vp, sz]),

@@ -41,6 +41,7 @@
 //   has no cross-lane traffic; raising m_ref (rare after the first chunks) takes the row maximum over
 //   the four lanes of a token and rescales the output accumulators.
 #include <algorithm>
+#include <cmath>
 #include <functional>
 
 #include "common.h"
@@ -854,7 +855,7 @@ int64_t most_chunks(const sb_swa_prefill_args *a, int64_t max_keys) {
 //    From 256 to 384 workgroups of four (a second round that leaves most CUs idle) they pay unless the walks are many chunks
 //    long: 3059 tokens, window 4096 92.8 -> 88.8; behind 4200, windows 512 / 1024 / 2048 / 4096 52.4 / 77.1 / 127 / 228 -> 47 / 72.9 / 124 /
 //    230; beyond that they lose (1 x 6000: 256 -> 271).
-//  * halves: workgroups of two heads that hold their four wavefronts twice, each set walking half of the keys (see halves_pay).
+//  * halves: workgroups of two heads that hold their four wavefronts twice, each set walking half of the keys (see halves_us).
 //  * parts: the keys of a walk cut into parts of 8 chunks or more side by side, at the price of fp32 partials and
 //    a merge (64 / 200 / 512 / 1024 tokens behind 4200: 100 with pairs, 123 with groups of four -> 27.5 (12 parts) / 37 (8) /
 //    54 (4) / 85 (2) us; 64 tokens in 8 parts 25.7, which the estimate below does not find).
@@ -875,24 +876,31 @@ bool pairs_pay(const sb_swa_prefill_args *a, int64_t chunks, int64_t parts, int6
   const int64_t sharing = cus / pairs_per_tile;   // tiles in front of the first one that shares
   return sharing >= a->num_tiles || (double)most_chunks(a, a->tile_keys[sharing]) < 6.0 + 0.63 * (double)chunks;
 }
-// Halves: one such workgroup fills a CU and takes 8.4 + 0.525 L us for a walk of L chunks, a pair 9 + 0.69 L, so they pay wherever
-// every workgroup has a CU, from walks of 9 chunks on (28 : 4 heads, us of pairs -> halves: whole prompts of 200 / 300 / 700 / 1000
-// tokens 12.3 / 14.3 / 23.5 / 30.2 -> 12.5 / 13.4 / 20.7 / 25.5, 1024 tokens behind 10000 with a window of 512 / 4096 24.2 / 102 -> 22 / 77; 16 : 8,
-// 3000 whole 73.6 -> 54.8). A second round pays where it is short walks that are left for the CUs that come free first: with
-// the lists walked longest first over all XCDs, 1300 / 1517 / 2000 whole 38.6 / 43.3 / 54.9 -> 32.1 / 35.3 / 50.0 (38 / 40 / 54.6 with an XCD's
-// tiles to itself), 2048 behind 800 79.7 -> 77; not 2 x 1000 33.6 -> 34, 4 x 500 23 -> 26.7, 2048 behind 10000 (groups of four: 132) -> 149
-// and, in three rounds, 2560 69.7 -> 78. One head per kv head, second round: 16 : 16, 4 x 500 17 -> 19.9 (not taken).
-bool halves_pay(const sb_swa_prefill_args *a, int64_t max_keys, int64_t chunks, int64_t cus) {
+// Halves: us such a call takes, or infinity where it is better without. A workgroup fills a CU and takes 8.9 + 0.487 L us for a walk of L
+// chunks, a pair 9 + 0.69 L, so they pay wherever every workgroup has a CU, from walks of 9 chunks on (28 : 4 heads, us of pairs -> halves:
+// whole prompts of 200 / 300 / 700 / 1000 tokens 12.3 / 14.3 / 23.5 / 30.2 -> 12.5 / 13.4 / 20.7 / 25.5, 1024 tokens behind 10000 with a
+// window of 512 / 4096 24.2 / 102 -> 22 / 77; 16 : 8, 3000 whole 73.6 -> 54.8). A second round pays where it is short walks that are left for
+// the CUs that come free first: with the lists walked longest first over all XCDs, 1300 / 1517 / 2000 whole 38.6 / 43.3 / 54.9 -> 32.1 / 35.3 /
+// 50.0 (38 / 40 / 54.6 with an XCD's tiles to itself), 2048 behind 800 79.7 -> 77, 18 : 6, 1517 behind 2000 93 -> 81; not 2 x 1000
+// 33.6 -> 34, 4 x 500 23 -> 26.7, 2048 behind 10000 (groups of four: 132) -> 149 and, in three rounds, 2560 69.7 -> 78, nor against groups of
+// three heads, whose chunks are shorter (12 : 4, 3000 behind 2000 105 -> 111.6; 24 : 8, 1517 behind 2000 88 -> 96). One head per kv head,
+// second round: 16 : 16, 4 x 500 17 -> 19.9 (not taken).
+double halves_us(const sb_swa_prefill_args *a, int64_t max_keys, int64_t chunks, int64_t cus) {
   const int64_t G = a->num_q_heads / a->num_kv_heads, per_tile = a->num_kv_heads * ((G + 1) / 2), wgs = a->num_tiles * per_tile;
-  if (a->meta_len > 0 || max_keys >= INT32_MAX || chunks < 9) return false;   // (of calls without a bound the walks are unknown)
-  if (wgs <= cus) return true;
-  if (G == 1 || wgs > 2 * cus || !a->tile_keys) return false;
-  const double l0 = (double)chunks, next = (double)most_chunks(a, a->tile_keys[cus / per_tile]),
-               first_done = (double)most_chunks(a, a->tile_keys[(cus - 1) / per_tile]);
-  const double halves = std::max(8.4 + 0.525 * l0, 14.0 + 0.55 * (first_done + next));
+  if (a->meta_len > 0 || max_keys >= INT32_MAX || chunks < 9) return HUGE_VAL;   // (of calls without a bound the walks are unknown)
+  const double l0 = (double)chunks, alone = 8.9 + 0.487 * l0;
+  if (wgs <= cus) return alone;
+  if (G == 1 || wgs > 2 * cus || !a->tile_keys) return HUGE_VAL;
+  const double next = (double)most_chunks(a, a->tile_keys[cus / per_tile]), first_done = (double)most_chunks(a, a->tile_keys[(cus - 1) / per_tile]);
+  const double halves = std::max(alone, 13.0 + 0.51 * (first_done + next));
   double others = 6.3 + 0.72 * l0 + 0.35 * next;   // pairs
-  if (quad_workgroups(a) <= cus) others = std::min(others, 8.4 + 0.94 * l0);
-  return halves < 0.93 * others;
+  if (quad_workgroups(a) <= cus) others = std::min(others, 8.4 + (G == 3 ? 0.75 : 0.94) * l0);   // groups of three or four heads
+  return halves < 0.93 * others ? halves : HUGE_VAL;
+}
+// Whether a call in halves has more workgroups than an XCD's eighth of the tiles leaves CUs for: they are then walked over all XCDs
+// (24 : 4 heads, 800 and 300 behind 1000, 216 workgroups of which an XCD would get 36 for its 32 CUs: 55.3 -> 49.9 us).
+bool halves_in_rounds(const sb_swa_prefill_args *a, int64_t cus) {
+  return (a->num_tiles + 7) / 8 * 8 * a->num_kv_heads * ((a->num_q_heads / a->num_kv_heads + 1) / 2) > cus;
 }
 // Order of a short list's tiles. Dealt to the XCDs longest walk first, in tile-major order, evens out the work of walks of
 // different lengths; in sequence order, kv heads outermost, the tiles that run on an XCD at a time are neighbours of one head and
@@ -919,14 +927,24 @@ Order tile_order(const sb_swa_prefill_args *a, int64_t max_keys, int64_t chunks,
   return G == 1 && 2 * a->num_tiles * a->num_kv_heads >= (even >= 0.65 ? 7 : 22) * cus ? Order::kDealtByHead : Order::kDealt;
 }
 
+// What a call in parts takes, for the choice between them and halves: it goes by the heads the workgroups of the parts hold (two, and one,
+// run four wavefronts; three run eight, of which four hold one head's scores; four run eight of two). us by least squares over 1500 calls of
+// 20 head counts (G = 2 / 3 / 4 / 7 and pairs: 0.70 / 0.75 / 0.90 / 0.89 and 0.69 to 0.73 a chunk; +- 1.5 to 3.4). Parts -> halves, not
+// taken: 8 : 4, 700 behind 2000, window 1024 20.5 -> 26.4, 2048 behind 2000 59.8 -> 69.4; 16 : 8, 400 behind 800 21.1 -> 27.5; 12 : 4, 2048
+// behind 2000 66 -> 71.5; 24 : 8, 400 behind 800 26.4 -> 28.1; taken: 28 : 4, 1024 behind 10000 79.7 -> 74.1. Where few tiles leave XCDs
+// without any it is too low (30 : 10, 576 behind 2000, nine tiles on five XCDs: estimated 50, 71.5; in halves 48.9, not taken).
+double parts_us(const sb_swa_prefill_args *a, const Spread &s, int64_t chunks, int64_t cus) {
+  const int64_t G = a->num_q_heads / a->num_kv_heads;
+  const double n = (double)s.parts, fill = n * (double)quad_workgroups(a) / (double)cus, walk = (double)((chunks + s.parts - 1) / s.parts);
+  if (s.pairs || G == 2) return 9.1 + 0.11 * n + (G == 2 ? 7.0 : 15.0) * fill + 0.7 * walk;
+  return 14.0 + 0.33 * n + 6.0 * fill + (G == 3 ? 0.75 : 0.9) * walk;
+}
+
 Spread spread_of(const sb_swa_prefill_args *a, int64_t max_keys) {
-  const int64_t chunks = most_chunks(a, max_keys), wgs = quad_workgroups(a), cus = sb_host::device_cu_count();
-  Spread best{1, pairs_pay(a, chunks, 1, cus)};
-  // (parts are the better the fewer heads their workgroups have: one, 16 : 16, 512 behind 10000 in halves 64 us, in 3 parts 49; three, 12 : 4,
-  // 2048 behind 10000 78.7 and in 2 parts 75, but 1517 whole 33 and 41)
-  const int G = a->num_q_heads / a->num_kv_heads;
-  double best_us = G > 1 && halves_pay(a, max_keys, chunks, cus) ? 8.4 + (G == 3 ? 2.0 : 0.0) + 0.525 * (double)chunks
-                                                                 : 5.0 + (best.pairs ? 0.69 : 0.9) * (double)chunks;
+  const int64_t chunks = most_chunks(a, max_keys), wgs = quad_workgroups(a), cus = sb_host::device_cu_count(), G = a->num_q_heads / a->num_kv_heads;
+  const Spread whole{1, pairs_pay(a, chunks, 1, cus)};
+  Spread best = whole;
+  double best_us = 5.0 + (whole.pairs ? 0.69 : 0.9) * (double)chunks;
   for (int64_t n = 2; n * wgs <= cus && 8 * n <= chunks; ++n) {
     const bool pairs = pairs_pay(a, chunks, n, cus);
     const double us = 13.5 + 0.28 * (double)n + 8.0 * (double)(n * wgs) / (double)cus +
@@ -936,6 +954,7 @@ Spread spread_of(const sb_swa_prefill_args *a, int64_t max_keys) {
       best_us = us;
     }
   }
+  if (best.parts > 1 && G > 1 && halves_us(a, max_keys, chunks, cus) < 0.95 * parts_us(a, best, chunks, cus)) best = whole;
   return best;
 }
 
@@ -1008,8 +1027,8 @@ int prefill(const sb_swa_prefill_args *a, int64_t max_keys, int n_parts, float *
   p.num_tiles = (int)a->num_tiles;
   const int64_t chunks = most_chunks(a, max_keys);
   const int64_t cus = sb_host::device_cu_count();
-  const bool halves = n_parts == 1 && halves_pay(a, max_keys, chunks, cus);
-  const bool rounds = halves && a->num_tiles * a->num_kv_heads * ((p.G + 1) / 2) > cus;   // more workgroups than CUs
+  const bool halves = n_parts == 1 && halves_us(a, max_keys, chunks, cus) < HUGE_VAL;
+  const bool rounds = halves && halves_in_rounds(a, cus);
   const Order order = n_parts == 1 && !rounds ? tile_order(a, max_keys, chunks, cus) : Order::kDealt;
   if (order == Order::kSequence) {
     p.tile_seq = a->ordered_tile_seq;
@@ -1161,11 +1180,17 @@ extern "C" int32_t sb_swa_prefill_parts(const sb_swa_prefill_args *a, int64_t ma
   return spread_of(a, max_keys < INT32_MAX ? max_keys : INT32_MAX).parts;
 }
 
+extern "C" int32_t sb_swa_prefill_halves(const sb_swa_prefill_args *a, int64_t max_keys, int32_t n_parts) {
+  if (!a || a->num_tiles <= 0 || a->num_kv_heads <= 0 || a->num_q_heads < a->num_kv_heads || max_keys <= 0 || n_parts > 1) return 0;
+  if (max_keys > INT32_MAX) max_keys = INT32_MAX;
+  return halves_us(a, max_keys, most_chunks(a, max_keys), sb_host::device_cu_count()) < HUGE_VAL;
+}
+
 extern "C" int32_t sb_swa_prefill_group_heads(const sb_swa_prefill_args *a, int64_t max_keys, int32_t n_parts) {
   if (!a || a->num_tiles <= 0 || a->num_kv_heads <= 0 || a->num_q_heads < a->num_kv_heads || max_keys <= 0) return 4;
   if (max_keys > INT32_MAX) max_keys = INT32_MAX;
-  const int64_t chunks = most_chunks(a, max_keys), cus = sb_host::device_cu_count();
-  return pairs_pay(a, chunks, n_parts < 1 ? 1 : n_parts, cus) || (n_parts < 2 && halves_pay(a, max_keys, chunks, cus)) ? 2 : 4;
+  return sb_swa_prefill_halves(a, max_keys, n_parts) ||
+         pairs_pay(a, most_chunks(a, max_keys), n_parts < 1 ? 1 : n_parts, sb_host::device_cu_count()) ? 2 : 4;
 }
 
 extern "C" size_t sb_swa_prefill_workspace_bytes(const sb_swa_prefill_args *a, int64_t total_q, int32_t n_parts) {
