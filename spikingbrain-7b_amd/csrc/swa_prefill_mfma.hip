@@ -688,8 +688,9 @@ void swa_prefill_kernel(const PrefillParams p) {
 
     // ---- epilogue: lane (g, c) owns token c of each block, dims 16 mt + 4g + i --------------------------
     if constexpr (HALVES) {
-      // Each set puts one of two blocks together (the first set the only one): the other set's sums come through LDS, a
-      // wavefront's in the ring slots of its own set (read last before the barrier).
+      // Each set puts one of two blocks together (the first set the only one): the other set's sums come through LDS. What is handed
+      // over lies across both sets' rings, whose last slots any wavefront of either set may still be reading: the first barrier is
+      // what frees them, the second what makes the sums readable.
       float *const out_acc = reinterpret_cast<float *>(smem_all + (half * S::kSetWaves + wave) * kHandOver) + lane * 4;
       const float *const in_acc = reinterpret_cast<const float *>(smem_all + ((half ^ 1) * S::kSetWaves + wave) * kHandOver) + lane * 4;
       auto hand_over = [&](int b) __attribute__((always_inline)) {
