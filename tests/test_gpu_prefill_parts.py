@@ -3,6 +3,8 @@ against float64 attention, over dense keys and over paged element and byte-code 
 from fp32 and the probabilities on the way: 1e-2 (bf16) or 1.25e-3 (fp16, three more bits) of the 2-norm, the same bound for cut
 and uncut calls and between the two. Their log-sum-exps come from the same fp32 scores, summed in another order: terms of up to
 1100 keys, each within 2^-24 of itself, move the logarithm by 6.6e-5 at most, and a value below 16 has places of 1e-6: 1e-4."""
+import ctypes
+
 import pytest
 import torch
 
@@ -162,8 +164,10 @@ def test_more_parts_than_the_merge_addresses(sb, dev):
                                                (5, [33], 700, 290)])
 def test_halves_of_a_walk(sb, dev, kv, G, lens, ctx, window):
     """Workgroups whose two sets of wavefronts each take half of the keys: odd and even numbers of chunks, a last group of one head,
-    walks whose second half is all masked for some tokens, more workgroups than CUs (1300 tokens), against the same call cut
-    into two parts; both are within 1e-2 of the mathematics, and their log-sum-exps come from the same fp32 scores (as above)."""
+    walks whose second half is all masked for some tokens, more workgroups than CUs (1300 tokens), and the same call cut into two
+    parts, each against float64 attention element by element. A probability is rounded to bf16 (2^-8 of itself, its sum is not), so an
+    output lies within 2^-8 of the same average over |v|, and 2^-8 of itself from its own rounding; scores of up to 128 terms in
+    fp32 move both by less than 2^-12. The log-sum-exps come from the same fp32 scores (as above)."""
     g = torch.Generator().manual_seed(G + len(lens))
     Hkv, T, keys = 4, sum(lens), [n + ctx for n in lens]
     q = torch.randn(T, Hkv * G, D, generator=g).bfloat16().to(dev)
@@ -185,8 +189,17 @@ def test_halves_of_a_walk(sb, dev, kv, G, lens, ctx, window):
             k, v = torch.randn(shape, generator=g).to(torch.float8_e4m3fn).to(dev)
             kw.update(fp8_scales=(1.0, 1.0))
         kw.update(block_table=table.to(dev))
+    plan = sb.ops.PrefillPlan(lens, keys, "cpu")
+    args = sb._native.SwaPrefillArgs(num_tiles=plan.num_tiles, num_q_heads=Hkv * G, num_kv_heads=Hkv, window_left=window, tile_keys=plan.tile_keys_ptr)
+    assert sb._native.lib().sb_swa_prefill_halves(ctypes.byref(args), plan.max_k, 1) == 1
     (whole, lse), (cut, lse1) = (sb.ops.swa_prefill_attention(q, k, v, n_parts=n, **kw) for n in (1, 2))
-    assert torch.isfinite(whole).all()
-    assert (whole.double() - cut.double()).norm() <= 1e-2 * cut.double().norm()
+    rows = [x.cpu() for x in (k, v)]
+    if kv != "dense":                                                       # as the kernel takes them: in sequence, rounded to bf16
+        rows = [x.float() * (s[i].cpu().permute(0, 2, 1)[..., None] if kv == "int8" else 1.0) for i, x in enumerate(rows)]
+        rows = [torch.cat([x[t.long()].flatten(0, 1)[:n] for t, n in zip(table, keys)]).bfloat16() for x in rows]
+    ref = _reference(q.cpu(), rows[0], torch.cat([rows[1], rows[1].abs()], -1), lens, ctx, window, [5 if kv == "dense" else 0] * len(lens), G)
+    ref, bound = ref[..., :D], (2 ** -8 + 2 ** -12) * (ref[..., D:] + ref[..., :D].abs())
+    for out in (whole, cut):
+        assert ((out.cpu().double() - ref).abs() <= bound).all()
     ok = ~torch.isneginf(lse1)
     assert torch.equal(torch.isneginf(lse), ~ok) and (lse[ok] - lse1[ok]).abs().max() <= 1e-4
