@@ -32,8 +32,7 @@ def test_append_with_a_prompt(sb, dev, HQ, HKV, lens, dtype, page):
         c1 = cache.clone()
         got = call(c1, torch.zeros_like(q), append=(key, value, c1, slots), **kw)
         assert torch.equal(c1, c0)
-        if not kw:
-            assert torch.equal(got, want)
+        assert torch.equal(got, call(c0, torch.zeros_like(q), **kw) if kw else want)
     c1 = cache.clone()                                                     # a list of slots that only the general call takes
     got = call(c1, torch.zeros_like(q), append=(key, value, c1, slots.view(-1, 1)))
     assert torch.equal(c1, c0) and torch.equal(got, want)
