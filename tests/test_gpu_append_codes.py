@@ -51,6 +51,40 @@ def test_append_codes(sb, dev, kv, dtype, window, n_split):
 
 
 @pytest.mark.parametrize("kv", ["int8", "fp8"])
+@pytest.mark.parametrize("softcap,alibi", [(20.0, False), (0.0, True), (20.0, True)])
+def test_append_codes_with_score_options(sb, dev, kv, softcap, alibi):
+    """The same with a soft cap, slopes or both on the scores (of the calls with the append in front, test_gpu_score_options has the values)."""
+    gen = torch.Generator().manual_seed(7)
+    R, width = len(LENS), -(-max(LENS) // PAGE)
+    table = torch.randperm(R * width, generator=gen).view(R, width).int().to(dev)
+    lens = torch.tensor(LENS, dtype=torch.int32, device=dev)
+    last = (lens - 1).clamp(min=0)
+    slots = table[torch.arange(R, device=dev), (last // PAGE).long()].long() * PAGE + (last % PAGE)
+    q, key, value = (torch.randn(R, h, D, generator=gen).bfloat16().to(dev) for h in (HQ, HKV, HKV))
+    shape = (2, R * width, PAGE, HKV, D)
+    codes, scales = torch.randint(-127, 128, shape, dtype=torch.int8, generator=gen).to(dev), torch.full((2, R * width, HKV, PAGE), 0.02, device=dev)
+    if kv == "fp8":
+        codes = torch.randn(shape, generator=gen).to(torch.float8_e4m3fn).to(dev)
+    slopes = torch.linspace(0.01, 0.3, HQ, device=dev) if alibi else None
+    how = dict(k_scale=scales[0], v_scale=scales[1]) if kv == "int8" else dict(fp8_scales=(0.5, 2.0))
+    call = lambda c, **kw: sb.ops.swa_decode_attention(q, c[0], c[1], lens, block_table=table, window_left=200, balanced=False, return_lse=True,
+                                                       softcap=softcap, alibi_slopes=slopes, **how, **kw)
+    c0, s0 = codes.clone(), scales.clone()
+    got, lse = call(codes, new_key=key, new_value=value, new_slot_mapping=slots, append_codes=0.0)
+    if kv == "int8":
+        sb.ops.kv_append_int8(key, value, c0[0], c0[1], s0[0], s0[1], slots)
+        assert torch.equal(scales, s0)
+        how = dict(k_scale=s0[0], v_scale=s0[1])
+    else:
+        sb.ops.kv_append_fp8(key, value, c0[0], c0[1], slots, 0.5, 2.0)
+    want, want_lse = call(c0)
+    assert torch.equal(codes.view(torch.uint8), c0.view(torch.uint8))
+    assert torch.equal(got, want) and torch.equal(lse.view(torch.int32), want_lse.view(torch.int32))
+    plain = sb.ops.swa_decode_attention(q, c0[0], c0[1], lens, block_table=table, window_left=200, balanced=False, **how)
+    assert torch.isfinite(got).all() and not torch.equal(plain, want)
+
+
+@pytest.mark.parametrize("kv", ["int8", "fp8"])
 def test_layer_call_under_capture(sb, dev, kv):
     """A decode layer over byte codes through the backend: eager (native step and general form) and replayed from a graph."""
     R, keys, width = 3, 3000, 188
