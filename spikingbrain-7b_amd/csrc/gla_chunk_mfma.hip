@@ -18,9 +18,9 @@
 //
 // What bounds it is memory, and there the pattern: heads of a token lie side by side, so a workgroup reads pieces of 256
 // bytes (512 of the fp32 gates) and a wavefront's share of a row is what one of its loads finds together. A loop of the
-// same loads and stores that computes nothing takes, for 16 x 8192 tokens x 28 heads (5.64 GB), 1340 us where a
-// wavefront's load covers 64 bytes of 16 rows and its store 32, 1258 with 64 bytes per store, 1172 with 128 bytes of 8 rows
-// per load as here, 1158 with whole rows (which would cut the sum over the tokens into four wavefronts).
+// same loads and stores that computes nothing (profiles/gla_prompt_copy.hip) takes, for 16 x 8192 tokens x 28 heads (5.64 GB), 1243 us
+// where a wavefront's load covers 64 bytes of 16 rows and its store 32, 1207 with 64 bytes per store, 1164 with 128 bytes of 8 rows
+// per load as here, 1166 with whole rows (which would cut the sum over the tokens into four wavefronts).
 // Measured (us per call, blocks of 16 tokens read in 64-byte pieces -> this form): 16 x 8192 tokens 1400 -> 1240 (4.5 TB/s),
 // 8 x 4096 368 -> 283, 16 x 500 82 -> 66, 4 x 900 75 -> 68; shared states 16 x 8192 777 -> 659.
 //
@@ -102,7 +102,8 @@ struct Carry {
 // Rows are 256 bytes = all 64 banks, so piece p of row t lies at place p ^ f(t), with f such that the 16-byte accesses of 8
 // consecutive rows (matrix operands), of rows 0, 2, 4, 6 and two pieces (the stores) and the transposing loads of four rows
 // by four pieces all spread over the banks: the low two bits of t in front (a transposing load takes pieces 4 P .. 4 P + 3 of
-// rows 4 j .. 4 j + 3), bits 2 and 3 behind them. (Rows padded to 304 bytes instead spent half of the LDS cycles on conflicts.)
+// rows 4 j .. 4 j + 3), bits 2 and 3 behind them. (Rows padded to 304 bytes instead spent half of the LDS cycles on conflicts; the counter
+// still gives 0.43, 809 of a block's 1899 cycles, and where those come from is open.)
 __device__ __forceinline__ int piece_at(int t, int piece) {
   return t * 128 + ((piece ^ ((t & 3) << 2 | (t >> 1 & 2) | (t >> 3 & 1))) << 3);
 }
