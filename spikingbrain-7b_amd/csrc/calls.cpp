@@ -447,7 +447,7 @@ bool fill_push(sb_window_shift_args (&a)[2], const Tensor *const (&storage)[2], 
     const int64_t e = s.element_size();
     a[i].dst = s.data_ptr(); a[i].fresh = f.data_ptr();
     a[i].planes = s.size(0) * s.size(1); a[i].dst_row0 = row; a[i].n_new = f.size(2); a[i].row_bytes = s.size(3) * e;
-    a[i].dst_stride_plane_bytes = s.stride(1) * e; a[i].fresh_stride_plane_bytes = f.stride(1) * e; a[i].fresh_stride_row_bytes = f.stride(2) * e;
+    a[i].dst_stride_plane_bytes = s.size(2) * s.size(3) * e; a[i].fresh_stride_plane_bytes = f.stride(1) * e; a[i].fresh_stride_row_bytes = f.stride(2) * e;
     a[i].stream = stream;
   }
   return true;

@@ -1126,9 +1126,10 @@ def _window_shift_args(src: Optional[torch.Tensor], dst: torch.Tensor, fresh: Op
     return N.WindowShiftArgs(
         src=N.ptr(src), dst=N.ptr(dst), fresh=N.ptr(fresh), planes=B * H, keep_rows=keep_rows,
         src_row0=src_row0, dst_row0=dst_row0, n_new=n_new, row_bytes=D * esz,
-        src_stride_plane_bytes=0 if src is None else src.stride(1) * esz,
-        dst_stride_plane_bytes=dst.stride(1) * esz,
-        fresh_stride_plane_bytes=0 if fresh is None else fresh.stride(1) * esz,
+        # (of one head, contiguous or not, the stride between heads says nothing)
+        src_stride_plane_bytes=0 if src is None else src.shape[2] * D * esz,
+        dst_stride_plane_bytes=cap_d * D * esz,
+        fresh_stride_plane_bytes=0 if fresh is None else fresh.stride(0 if H == 1 else 1) * esz,
         fresh_stride_row_bytes=0 if fresh is None else fresh.stride(2) * esz,
         stream=N.stream_ptr(dev)), fresh
 
