@@ -435,32 +435,51 @@ PyObject *gla_packed(Args &in) {
 }
 
 // Rows [row, row + n) of both window buffers [B, H, capacity, D] take the n new rows of key and value [B, H, n, D]; false where the tensors
-// are not of the ordinary form
-bool fill_push(sb_window_shift_args (&a)[2], const Tensor *const (&storage)[2], const Tensor *const (&fresh)[2], int64_t row, void *stream) {
+// are not of the ordinary form. lay_out, if given, is set where rows first have to be laid out contiguously (no address is filled in then).
+bool fill_push(sb_window_shift_args (&a)[2], const Tensor *const (&storage)[2], const Tensor *const (&fresh)[2], int64_t row, void *stream,
+               bool *lay_out = nullptr) {
   if (row < 0) return false;
   std::memset(a, 0, sizeof a);
   for (int i = 0; i < 2; ++i) {
     const Tensor &s = *storage[i], &f = *fresh[i];
     if (s.dim() != 4 || f.dim() != 4 || !s.is_contiguous() || f.size(0) != s.size(0) || f.size(1) != s.size(1) || f.size(3) != s.size(3) ||
-        f.scalar_type() != s.scalar_type() || f.stride(3) != 1 || f.stride(0) != f.size(1) * f.stride(1) || row + f.size(2) > s.size(2))
+        f.scalar_type() != s.scalar_type() || f.stride(3) != 1 || row + f.size(2) > s.size(2))
       return false;
     const int64_t e = s.element_size();
     a[i].dst = s.data_ptr(); a[i].fresh = f.data_ptr();
     a[i].planes = s.size(0) * s.size(1); a[i].dst_row0 = row; a[i].n_new = f.size(2); a[i].row_bytes = s.size(3) * e;
     a[i].dst_stride_plane_bytes = s.size(2) * s.size(3) * e; a[i].fresh_stride_plane_bytes = f.stride(1) * e; a[i].fresh_stride_row_bytes = f.stride(2) * e;
     a[i].stream = stream;
+    if (f.stride(0) == f.size(1) * f.stride(1)) continue;
+    if (!lay_out) return false;
+    lay_out[i] = true;
+    a[i].fresh = nullptr;
+    a[i].fresh_stride_row_bytes = a[i].row_bytes;
+    a[i].fresh_stride_plane_bytes = f.size(2) * a[i].row_bytes;
   }
   return true;
 }
 
-// push(k_storage, v_storage, key, value, row, stream): ops.window_shift_pair without rows that stay
+// push(k_storage, v_storage, key, value, row, stream): ops.window_shift_pair without rows that stay (prompts' rows as a projection leaves
+// them, [B, n, H, D] transposed, are laid out on the way: the attempt was in vain for them, and two sequences of 143 tokens take 57.9 us
+// instead of 64.8 in the general form and 65.6 behind the attempt)
 PyObject *push(Args &in) {
   const Tensor *storage[2] = {in.tensor(), in.tensor()}, *fresh[2] = {in.tensor(), in.tensor()};
   const int64_t row = in.integer();
   void *const stream = in.address();
   sb_window_shift_args a[2];
-  if (!in.ok || !fill_push(a, storage, fresh, row, stream)) return not_taken();
-  return unlocked([&]() -> Result { return {sb_window_shift_pair(&a[0], &a[1])}; });
+  bool lay_out[2] = {false, false};
+  if (!in.ok || !fill_push(a, storage, fresh, row, stream, lay_out)) return not_taken();
+  return unlocked([&]() -> Result {
+    Tensor rows[2];   // (until the copy is enqueued)
+    for (int i = 0; i < 2; ++i)
+      if (lay_out[i]) {
+        rows[i] = fresh[i]->contiguous();
+        if (!plain(rows[i])) return {.taken = false};
+        a[i].fresh = rows[i].data_ptr();
+      }
+    return {sb_window_shift_pair(&a[0], &a[1])};
+  });
 }
 
 // dense_decode(q [B, Hq, 1, D], k, v [B, Hkv, K, D], mask | None, window_left, scale, k_storage | None, v_storage | None, key | None,

@@ -134,6 +134,23 @@ def test_hugging_face_decode(sb, dev, both, dtype, mask, B, W):
     both(run)
 
 
+@pytest.mark.parametrize("B,H,n", [(1, 1, 5), (1, 3, 5), (2, 1, 5), (3, 2, 1), (2, 4, 70)])
+@pytest.mark.parametrize("layout", ["transposed", "fused", "contiguous"])
+def test_new_rows(sb, dev, both, B, H, n, layout):
+    """A prompt's rows into a window buffer, also where they have to be laid out first."""
+    wide = _rand(dev, B, n, 3 * H, D, seed=n)
+    k, v = (wide[:, :, i * H:(i + 1) * H] for i in (1, 2)) if layout == "fused" else (wide[:, :, i * H:(i + 1) * H].contiguous() for i in (1, 2))
+    k, v = (x.transpose(1, 2).contiguous() if layout == "contiguous" else x.transpose(1, 2) for x in (k, v))
+
+    def push():
+        storage = [torch.zeros(B, H, n + 9, D, dtype=k.dtype, device=dev) for _ in range(2)]
+        sb.ops.window_shift_pair((None, storage[0], k, 0, 0, 4), (None, storage[1], v, 0, 0, 4))
+        assert torch.equal(storage[0][:, :, 4:4 + n], k) and torch.equal(storage[1][:, :, 4:4 + n], v)
+        assert not storage[0][:, :, :4].any() and not storage[1][:, :, 4 + n:].any()
+        return storage
+    both(push)
+
+
 @pytest.mark.parametrize("H,Hk,sdtype", [(4, 4, torch.float32), (14, 2, torch.bfloat16)])
 @pytest.mark.parametrize("slots", [None, [2, -1, 0]])
 def test_linear_attention(sb, dev, both, H, Hk, sdtype, slots):
