@@ -826,10 +826,28 @@ void launch_prefill_q(int nh, bool odd, bool halves, dim3 grid, hipStream_t st, 
   else if (odd) hipLaunchKernelGGL((swa_prefill_kernel<E, 4, KVQ, PAGED, true, false, APPEND>), grid, b8, 0, st, p);
   else hipLaunchKernelGGL((swa_prefill_kernel<E, 4, KVQ, PAGED, false, false, APPEND>), grid, b8, 0, st, p);
 }
+}  // namespace
+
+// The launches over INT8 caches, whose kernels swa_prefill_int8.hip compiles from this file; params: a PrefillParams.
+namespace sb_host {
+void launch_prefill_int8(int dtype, int nh, bool odd, bool halves, dim3 grid, hipStream_t st, const void *params)
+#ifndef SB_PREFILL_INT8
+    ;
+#else
+{
+  const PrefillParams &p = *static_cast<const PrefillParams *>(params);
+  if (dtype == SB_BF16) launch_prefill_q<BF16, SB_KV_INT8, true>(nh, odd, halves, grid, st, p);
+  else launch_prefill_q<F16, SB_KV_INT8, true>(nh, odd, halves, grid, st, p);
+}
+#endif
+}  // namespace sb_host
+
+#ifndef SB_PREFILL_INT8
+namespace {
+
 template <typename E>
 void launch_prefill(int kv_quant, int nh, bool odd, bool halves, dim3 grid, hipStream_t st, const PrefillParams &p) {
-  if (kv_quant == SB_KV_INT8) launch_prefill_q<E, SB_KV_INT8, true>(nh, odd, halves, grid, st, p);
-  else if (kv_quant == SB_KV_FP8) launch_prefill_q<E, SB_KV_FP8, true>(nh, odd, halves, grid, st, p);
+  if (kv_quant == SB_KV_FP8) launch_prefill_q<E, SB_KV_FP8, true>(nh, odd, halves, grid, st, p);
   else if (p.block_table) launch_prefill_q<E, SB_KV_NONE, true>(nh, odd, halves, grid, st, p);
   else if (p.append.tokens > 0) launch_prefill_q<E, SB_KV_NONE, false, true>(nh, odd, halves, grid, st, p);
   else launch_prefill_q<E, SB_KV_NONE, false>(nh, odd, halves, grid, st, p);
@@ -1106,7 +1124,8 @@ int prefill(const sb_swa_prefill_args *a, int64_t max_keys, int n_parts, float *
       if (grid.x + more > 0x7fffffffLL) return fail(SB_ERR_UNSUPPORTED, "sb_swa_prefill: grid too large");
       grid.x += (unsigned)more;
     }
-    if (a->dtype == SB_BF16) launch_prefill<BF16>(a->kv_quant, nh, odd, halves, grid, (hipStream_t)a->stream, p);
+    if (a->kv_quant == SB_KV_INT8) launch_prefill_int8(a->dtype, nh, odd, halves, grid, (hipStream_t)a->stream, &p);
+    else if (a->dtype == SB_BF16) launch_prefill<BF16>(a->kv_quant, nh, odd, halves, grid, (hipStream_t)a->stream, p);
     else launch_prefill<F16>(a->kv_quant, nh, odd, halves, grid, (hipStream_t)a->stream, p);
     const int rc = check_launch("swa_prefill_kernel");
     if (rc != SB_OK) return rc;
@@ -1234,3 +1253,4 @@ extern "C" int sb_swa_prefill_append(const sb_swa_prefill_args *a, const sb_kv_a
   const int rc = sb_kv_append(append);
   return rc ? rc : prefill_parted(a, total_q, max_keys, n_parts, workspace, workspace_bytes, nullptr);
 }
+#endif  // SB_PREFILL_INT8
